@@ -42,6 +42,7 @@ GLLMQ_EMBED(mm8c)
 GLLMQ_EMBED(mm8_q6k_q8_0)
 GLLMQ_EMBED(mmf)
 GLLMQ_EMBED(mmfs)
+GLLMQ_EMBED(mmfw)
 GLLMQ_EMBED(moe)
 
 namespace {
@@ -108,6 +109,15 @@ uint32_t mmf_lds_bytes(uint32_t mt, int fmt)
     return kTotal[mt - 1][fmt];
 }
 
+uint32_t mmfw_lds_bytes(int fmt, int planes, uint32_t mt)
+{
+#define GQ_ROW(F, PL) { gq::mmfw_lds<F, PL, 1>(), gq::mmfw_lds<F, PL, 2>(), gq::mmfw_lds<F, PL, 3>(), gq::mmfw_lds<F, PL, 4>() }
+    static const uint32_t kTotal[4][2][4] = { { GQ_ROW(0, 1), GQ_ROW(0, 2) }, { GQ_ROW(1, 1), GQ_ROW(1, 2) },
+                                              { GQ_ROW(2, 1), GQ_ROW(2, 2) }, { GQ_ROW(3, 1), GQ_ROW(3, 2) } };
+#undef GQ_ROW
+    return kTotal[fmt][planes - 1][mt - 1];
+}
+
 // Formats of the int8 matrix-core kernels, in the order of the kernel tables below.
 // (the grouped MoE kernels exist for the first MM8_MOE_KINDS of them)
 enum Mm8Kind { MM8_Q4K = 0, MM8_Q6K = 1, MM8_Q5K = 2, MM8_Q8_0 = 3, MM8_KINDS = 4, MM8_MOE_KINDS = 3 };
@@ -168,7 +178,7 @@ struct CachedWeights {
 
 struct gllmq_ctx {
     int device = 0;
-    hipModule_t modules[9] = {}; // one per embedded code object
+    hipModule_t modules[10] = {}; // one per embedded code object
     hipFunction_t dequant[kNumFormats][2] = {}; // [format][0 = scalar stores, 1 = float4 stores]
     hipFunction_t gather[kNumFormats][2] = {};  // quantized embedding lookup [format][0 = scalar stores, 1 = float4 stores]
     hipFunction_t gather_e16[kNumFormats][2] = {}; // the same into rows of a 16-bit element type [format][0 = scalar stores, 1 = 8-byte stores]
@@ -206,6 +216,11 @@ struct gllmq_ctx {
     uint32_t mm8s_min_rows = 8;                 // "mm8s_min_rows": fewest weight rows per CU that take the streamed form
     hipFunction_t moe_mm8_glu_fn[3][2] = {};    // gated gate/up kernels [Mm8Kind (Q4_K and Q5_K only)][passes per tile - 1]
     hipFunction_t mmf_q4k[4][2][2] = {};        // f16 matrix-core GEMM [0 = Q4_K, 1 = Q5_K, 2 = Q6_K, 3 = Q8_0][32-row activation tiles - 1][bf16 mode]
+    hipFunction_t mmfw[4][4][2] = {};           // the GEMM for more rows [format as above][32-row activation tiles - 1][0 = hi and lo plane, 1 = hi only]
+    hipFunction_t mmfw_prep[2] = {};            // its activation images [hi and lo plane, hi only]
+    bool use_mmfw = true;                       // "mmfw" = 0: 64-row passes of the other forms
+    uint32_t mmfw_min_m = 33;                   // "mmfw_min_m": fewest activation rows that take it
+    uint32_t mmfw_mt = 0, mmfw_ksplit = 0;      // "mmfw_mt", "mmfw_ksplit": activation tiles per workgroup, slices of K (0 = by the shape)
     hipFunction_t mmfs[2][2] = {};              // its streamed form [0 = Q4_K, 1 = Q5_K][bf16 mode]
     hipFunction_t mmfr[2] = {};                 // the streamed form whose waves prepare their own activations (f32, 9 to 16 rows) [0 = Q4_K, 1 = Q5_K]
     bool use_mmfr = true;                       // "mmfr" = 0: never
@@ -508,11 +523,13 @@ bool aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) &
 // Element `index` of activations or outputs whose element type is that of the call being enqueued
 // (pointers are typed for the f32 case).
 template <class T>
-T *elem_at(const gllmq_ctx *ctx, T *base, size_t index)
+T *elem_at(uint32_t elem, T *base, size_t index)
 {
     typedef typename std::conditional<std::is_const<T>::value, const uint8_t, uint8_t>::type Byte;
-    return reinterpret_cast<T *>(reinterpret_cast<Byte *>(base) + index * (ctx->call_elem ? 2u : 4u));
+    return reinterpret_cast<T *>(reinterpret_cast<Byte *>(base) + index * (elem ? 2u : 4u));
 }
+template <class T>
+T *elem_at(const gllmq_ctx *ctx, T *base, size_t index) { return elem_at(ctx->call_elem, base, index); }
 
 // Elements between activation rows of the matmul being enqueued: k unless the caller says otherwise.
 uint32_t row_stride_x(const gllmq_ctx *ctx, size_t k) { return ctx->call_ldx ? ctx->call_ldx : static_cast<uint32_t>(k); }
@@ -1014,6 +1031,176 @@ int run_mmf(gllmq_ctx *ctx, Scratch &S, const Format &f, const uint8_t *w, const
     return GLLMQ_OK;
 }
 
+// One weight matrix of a GEMM launch.
+struct MmfwMatrix {
+    const uint8_t *w;
+    float *y;
+    size_t n;
+};
+
+// Launch geometry of the GEMM for more rows (mmfw.hip.inc), for matrices of n[0 .. count) rows that
+// share their activations, and the scratch it needs.  ok = false: not for it.
+struct MmfwPlan {
+    bool ok = false;
+    uint32_t groups = 0, planes = 2, mt = 1, n_tiles = 0, ksplit = 1, bps = 0, band = 4;
+    size_t rows = 0; // activation rows per pass (all of them, unless the images would pass 1 GiB or the scratch is of fixed size)
+    size_t img_bytes = 0, inv_bytes = 0, part_bytes = 0;
+    size_t need() const { return img_bytes + inv_bytes + part_bytes; }
+};
+
+int mmf_format(uint32_t dtype) { return dtype == T_Q8_0 ? 3 : dtype == T_Q6_K ? 2 : dtype == T_Q5_K ? 1 : 0; }
+
+uint32_t mmfw_inv_ld(size_t rows) { return static_cast<uint32_t>((rows + 31) / 32 * 32); }
+
+void mmfw_size(MmfwPlan &L, size_t rows, size_t n_sum)
+{
+    L.rows = rows;
+    const size_t image = L.planes == 2 ? gq::MmfwImage<2>::bytes : gq::MmfwImage<1>::bytes;
+    L.img_bytes = (rows + 31) / 32 * L.groups * image;
+    // (a workgroup fetches the inverse scales of its rows as one KiB)
+    L.inv_bytes = (static_cast<size_t>(L.groups) * mmfw_inv_ld(rows) * 4 + 1024 + 255) & ~size_t(255);
+    L.part_bytes = L.ksplit > 1 ? static_cast<size_t>(L.ksplit) * rows * n_sum * 4 : 0;
+}
+
+MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t *n, int count, size_t k, bool hi_only,
+                   size_t scratch_limit = SIZE_MAX)
+{
+    MmfwPlan L;
+    const int fmt = mmf_format(dtype);
+    size_t n_sum = 0, tiles = 0;
+    for (int i = 0; i < count; ++i) {
+        n_sum += n[i];
+        tiles += (n[i] + gq::MMFW_TILE_ROWS - 1) / gq::MMFW_TILE_ROWS;
+    }
+    if (!ctx->use_mmf || !ctx->use_mmfw || m == 0 || n_sum == 0 || tiles > 0xFFFFFFu) return L;
+    if (fmt == 3 && k < 256) return L; // the Q8_0 window is one whole group of 8 blocks
+    if (static_cast<uint64_t>(gllmq_row_bytes(dtype, k)) * gq::MMFW_TILE_ROWS > 0xFFFFFFFFull) return L;
+    L.groups = static_cast<uint32_t>((k + 255) / 256);
+    L.planes = hi_only ? 1u : 2u;
+    L.n_tiles = static_cast<uint32_t>(tiles);
+    const uint32_t row_tiles = static_cast<uint32_t>((m + 31) / 32);
+    // Activation tiles per workgroup and slices of K by a cost model (us): a block of K takes a
+    // workgroup its matrix-core time or the weights' way from memory, whichever is longer; a
+    // workgroup starts and ends in about the time of two blocks; the slices of K meet through memory.
+    const double cus = ctx->num_cus;
+    const double w_us = find_format(dtype)->group_bytes * 256.0 * cus / 5.0e6; // 5 TB/s over all CUs
+    double best = 1e300;
+    for (uint32_t mt = 1; mt <= static_cast<uint32_t>(gq::MMFW_MAX_MT); ++mt) {
+        if (ctx->mmfw_mt ? mt != ctx->mmfw_mt : (mt > row_tiles)) continue;
+        const uint64_t m_tiles = (row_tiles + mt - 1) / mt;
+        if (m_tiles * tiles > 0x7FFFFFFu) continue;
+        for (uint32_t ks = 1; ks <= std::min(L.groups, 32u); ++ks) {
+            const uint32_t bps = (L.groups + ks - 1) / ks;
+            if ((L.groups + bps - 1) / bps != ks) continue; // every slice has a block
+            if (ctx->mmfw_ksplit && ks != std::min(ctx->mmfw_ksplit, L.groups)) continue;
+            const double rounds = std::ceil(static_cast<double>(m_tiles * tiles * ks) / cus);
+            const double busy = std::min(1.0, static_cast<double>(m_tiles * tiles * ks) / cus);
+            const double block = std::max(0.62 * mt * L.planes + 0.25 * mt, w_us * busy);
+            double us = rounds * (bps * block + 3.0);
+            if (ks > 1) us += 4.0 + 2.0 * ks * static_cast<double>(m) * static_cast<double>(n_sum) * 4.0 / 4.0e6;
+            if (us < best) {
+                best = us;
+                L.mt = mt;
+                L.ksplit = ks;
+                L.bps = bps;
+            }
+        }
+    }
+    if (best == 1e300) return L;
+    const uint32_t m_tiles = (row_tiles + L.mt - 1) / L.mt;
+    L.band = std::min(m_tiles, 4u);
+    size_t rows = m;
+    const size_t step = 32u * L.mt;
+    mmfw_size(L, rows, n_sum);
+    // fewer rows per pass where the whole does not fit: the tiles and slices stay what they are, so the results do too
+    while ((L.img_bytes > (size_t(1) << 30) || L.need() > scratch_limit) && rows > step) {
+        rows = std::max(step, (rows / 2 + step - 1) / step * step);
+        mmfw_size(L, rows, n_sum);
+    }
+    L.ok = L.img_bytes < 0xFFFFFFFFull;
+    return L;
+}
+
+// The GEMM over `count` matrices of one format and K that share their activations: one launch that
+// prepares the activation images, one that multiplies, and one that adds the slices of K where
+// there are any.  Returns -1 for what it does not take.
+// `elem_x`, `elem_y`: element types of the activations and of the outputs.
+int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats, int count, const float *x, uint32_t elem_x,
+             uint32_t elem_y, size_t m, size_t k, bool act_bf16, void *stream, size_t min_m)
+{
+    if (!ctx->use_mmf || !ctx->use_mmfw || m < min_m) return -1;
+    if (!aligned(x, 16) || k % 4 != 0) return -1; // activation rows are loaded as aligned float4
+    if (ctx->call_glu && !glu_vector_ok(ctx)) return kNeedPlainActivations;
+    size_t n[gq::MMFW_MAX_SEGS];
+    for (int i = 0; i < count; ++i) n[i] = mats[i].n;
+    const bool hi_only = act_bf16 || (elem_x && !ctx->call_glu);
+    const MmfwPlan L = plan_mmfw(ctx, f.dtype, m, n, count, k, hi_only, S.fixed ? S.mmf_bytes : SIZE_MAX);
+    if (!L.ok) return -1;
+    int rc = grow_scratch(ctx, S, &S.mmf, &S.mmf_bytes, L.need(), stream, "quantized_matmul (GEMM)");
+    if (rc != GLLMQ_OK) return rc;
+    uint8_t *scratch = static_cast<uint8_t *>(S.mmf);
+    const int fmt = mmf_format(f.dtype);
+    const uint32_t ldx = row_stride_x(ctx, k);
+    for (size_t m0 = 0; m0 < m; m0 += L.rows) {
+        const uint32_t mm = static_cast<uint32_t>(std::min(L.rows, m - m0));
+        gq::MmfwPrepParams Q{};
+        Q.x = elem_at(elem_x, x, m0 * ldx);
+        Q.ximg = scratch;
+        Q.inv = reinterpret_cast<float *>(scratch + L.img_bytes);
+        Q.m = mm;
+        Q.k = static_cast<uint32_t>(k);
+        Q.ldx = ldx;
+        Q.groups = L.groups;
+        Q.inv_ld = mmfw_inv_ld(L.rows);
+        Q.act_bf16 = act_bf16 ? 1u : 0u;
+        Q.elem = ctx->call_glu ? 0u : elem_x;
+        Q.natural = fmt == 2 ? 1u : 0u; // a sub-block of Q6_K is one K step
+        Q.glu = ctx->call_glu;
+        Q.glu_off = ctx->call_glu_off;
+        const uint32_t row_tiles = (mm + 31u) / 32u;
+        rc = launch2d(ctx, ctx->mmfw_prep[hi_only ? 1 : 0], L.groups, row_tiles, 256, 0, stream, &Q, sizeof Q, true);
+        if (rc != GLLMQ_OK) return rc;
+        gq::MmfwParams P{};
+        P.ximg = scratch;
+        P.inv = Q.inv;
+        P.segs = static_cast<uint32_t>(count);
+        P.groups = L.groups;
+        P.row_bytes = static_cast<uint32_t>(gllmq_row_bytes(f.dtype, k));
+        P.m = mm;
+        P.k = Q.k;
+        P.row_tiles = row_tiles;
+        P.inv_ld = Q.inv_ld;
+        P.m_tiles = (row_tiles + L.mt - 1u) / L.mt;
+        P.n_tiles = L.n_tiles;
+        P.ksplit = L.ksplit;
+        P.blocks_per_split = L.bps;
+        P.items = P.m_tiles * P.n_tiles * L.ksplit;
+        P.band = std::min(L.band, P.m_tiles);
+        P.elem = elem_y;
+        float *part = reinterpret_cast<float *>(scratch + L.img_bytes + L.inv_bytes);
+        uint32_t tile0 = 0;
+        for (int i = 0; i < count; ++i) {
+            gq::MmfwSeg &G = P.seg[i];
+            G.w = mats[i].w;
+            G.y = elem_at(elem_y, mats[i].y, m0 * mats[i].n);
+            G.partial = part;
+            G.n = static_cast<uint32_t>(mats[i].n);
+            G.tile0 = tile0;
+            tile0 += (G.n + gq::MMFW_TILE_ROWS - 1u) / gq::MMFW_TILE_ROWS;
+            part += static_cast<size_t>(L.ksplit) * mm * G.n;
+        }
+        rc = launch(ctx, ctx->mmfw[fmt][L.mt - 1][hi_only ? 1 : 0], (P.items + 7u) / 8u * 8u, gq::MMFW_WAVES * 64, mmfw_lds_bytes(fmt, hi_only ? 1 : 2, L.mt),
+                    stream, &P, sizeof P, true);
+        for (int i = 0; i < count && rc == GLLMQ_OK && L.ksplit > 1; ++i) {
+            MmfReduceParams R{ P.seg[i].partial, P.seg[i].y, mm, P.seg[i].n, P.seg[i].n, L.ksplit, P.elem };
+            const uint64_t quads = (static_cast<uint64_t>(mm) * P.seg[i].n + 3) / 4;
+            rc = launch(ctx, ctx->mmf_reduce, static_cast<uint32_t>((quads + 255) / 256), 256, 0, stream, &R, sizeof R, true);
+        }
+        if (rc != GLLMQ_OK) return rc;
+    }
+    return GLLMQ_OK;
+}
+
 // Launch geometry of the streamed GEMM (mmfs.hip.inc) for one matmul; ok = false when the shape is
 // left to the three-launch form.
 struct MmfsPlan {
@@ -1366,7 +1553,13 @@ int run_gemv(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
 int dispatch_matmul(gllmq_ctx *ctx, Scratch &S, const Format &f, const uint8_t *w, const float *x, float *y, size_t m,
                     size_t n, size_t k, bool bf16, void *stream)
 {
-    int rc = run_mmfr(ctx, S, f, w, x, y, m, n, k, bf16, stream);
+    int rc = -1;
+    if (!ctx->mmfs_all) {
+        const MmfwMatrix one{ w, y, n };
+        rc = run_mmfw(ctx, S, f, &one, 1, x, ctx->call_elem, ctx->call_elem, m, k, bf16, stream, ctx->mmfw_min_m);
+        if (rc >= 0 || rc == kNeedPlainActivations) return rc;
+    }
+    rc = run_mmfr(ctx, S, f, w, x, y, m, n, k, bf16, stream);
     if (rc >= 0) return rc;
     rc = run_mmfs(ctx, S, f, w, x, y, m, n, k, bf16, stream);
     if (rc >= 0 || rc == kNeedPlainActivations) return rc;
@@ -1486,9 +1679,9 @@ int gllmq_init(gllmq_ctx **out, int device)
             return GLLMQ_ERR_UNIMPLEMENTED;
         }
     }
-    const unsigned char *const images[9] = { gllmq_co_codec, gllmq_co_mm8, gllmq_co_mm8s, gllmq_co_mm8s_q8_0, gllmq_co_mm8c,
-                                             gllmq_co_mm8_q6k_q8_0, gllmq_co_mmf, gllmq_co_mmfs, gllmq_co_moe };
-    for (int i = 0; i < 9; ++i) {
+    const unsigned char *const images[10] = { gllmq_co_codec, gllmq_co_mm8, gllmq_co_mm8s, gllmq_co_mm8s_q8_0, gllmq_co_mm8c,
+                                             gllmq_co_mm8_q6k_q8_0, gllmq_co_mmf, gllmq_co_mmfs, gllmq_co_mmfw, gllmq_co_moe };
+    for (int i = 0; i < 10; ++i) {
         e = hipModuleLoadData(&ctx->modules[i], images[i]);
         if (e != hipSuccess) {
             fprintf(stderr, "gllmq_init: hipModuleLoadData: %s\n", hipGetErrorString(e));
@@ -1559,6 +1752,14 @@ int gllmq_init(gllmq_ctx **out, int device)
             snprintf(name, sizeof name, "gq_mmfs_%s%s", q ? "q5k" : "q4k", b ? "_bf16" : "");
             rc = get_function(ctx, &ctx->mmfs[q][b], name);
         }
+    if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfw_prep[0], "gq_mmfw_prep");
+    if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfw_prep[1], "gq_mmfw_prep_hi");
+    for (int q = 0; q < 4 && rc == GLLMQ_OK; ++q)
+        for (int t = 0; t < gq::MMFW_MAX_MT && rc == GLLMQ_OK; ++t)
+            for (int b = 0; b < 2 && rc == GLLMQ_OK; ++b) {
+                snprintf(name, sizeof name, "gq_mmf_%s_w%d%s", q == 3 ? "q8_0" : q == 2 ? "q6k" : q == 1 ? "q5k" : "q4k", t + 1, b ? "_hi" : "");
+                rc = get_function(ctx, &ctx->mmfw[q][t][b], name);
+            }
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfr[0], "gq_mmfr_q4k");
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfr[1], "gq_mmfr_q5k");
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->moe_plan, "gq_moe_plan");
@@ -1743,6 +1944,10 @@ int gllmq_set_option(gllmq_ctx *ctx, const char *name, long value)
     else if (n == "mm8s") ctx->use_mm8s = value != 0;
     else if (n == "mmfs") ctx->use_mmfs = value != 0;
     else if (n == "mmfr") ctx->use_mmfr = value != 0;
+    else if (n == "mmfw") ctx->use_mmfw = value != 0;
+    else if (n == "mmfw_min_m") ctx->mmfw_min_m = std::max(1u, u);
+    else if (n == "mmfw_mt") ctx->mmfw_mt = std::min(u, static_cast<uint32_t>(gq::MMFW_MAX_MT));
+    else if (n == "mmfw_ksplit") ctx->mmfw_ksplit = u;
     else if (n == "mmfr_min_rows") ctx->mmfr_min_rows = std::max(1u, u);
     else if (n == "chain") ctx->use_chain = value != 0;
     else if (n == "chain_dependent") ctx->chain_dependent = value != 0;
@@ -2048,12 +2253,14 @@ int gllmq_reserve_matmul_elem(gllmq_ctx *ctx, uint32_t dtype, size_t m, size_t n
     return grow_scratch(ctx, *S, &S->elem, &S->elem_bytes, elem_scratch_bytes(m, n, k), stream, "reserve_matmul_elem");
 }
 
-int gllmq_ffn_swiglu(gllmq_ctx *ctx, const void *gate_w, const void *up_w, size_t gate_up_bytes_each, uint32_t dtype_gate_up,
-                     const void *down_w, size_t down_bytes, uint32_t dtype_down, const float *x, float *out, size_t m,
-                     size_t hidden, size_t ffn, int relu_gate, void *stream)
+namespace {
+
+// The feed-forward block (call_mutex held).  x and out are of type `elem`; where the kernels of the
+// shape take f32 only, kNeedPlainActivations comes back and nothing has been enqueued.
+int ffn_on_stream(gllmq_ctx *ctx, const void *gate_w, const void *up_w, size_t gate_up_bytes_each, uint32_t dtype_gate_up,
+                  const void *down_w, size_t down_bytes, uint32_t dtype_down, const float *x, float *out, uint32_t elem, size_t m,
+                  size_t hidden, size_t ffn, int relu_gate, void *stream)
 {
-    if (!ctx) return GLLMQ_ERR_INVALID;
-    std::lock_guard<std::recursive_mutex> call(ctx->call_mutex);
     const Format *fg = find_format(dtype_gate_up), *fd = find_format(dtype_down);
     if (!fg || !fd)
         return fail(ctx, GLLMQ_ERR_UNIMPLEMENTED,
@@ -2085,6 +2292,37 @@ int gllmq_ffn_swiglu(gllmq_ctx *ctx, const void *gate_w, const void *up_w, size_
     float *gu = reinterpret_cast<float *>(static_cast<uint8_t *>(S.ffn) + h_bytes);
     const uint8_t *gw = static_cast<const uint8_t *>(gate_w), *uw = static_cast<const uint8_t *>(up_w);
 
+    // Prompts and larger batches: gate and up share their activation images and run as one launch; the
+    // down projection's images are prepared from the two results.
+    if (m >= ctx->mmfw_min_m && m > 8 && !ctx->mmfs_all && ffn % 4 == 0 && m * ffn <= 0xFFFFFFFFull &&
+        plan_mmfw(ctx, dtype_down, m, &hidden, 1, ffn, false).ok) {
+        const MmfwMatrix gate_up[2] = { { gw, gu, ffn }, { uw, gu + m * ffn, ffn } };
+        rc = run_mmfw(ctx, S, *fg, gate_up, 2, x, elem, 0, m, hidden, false, stream, ctx->mmfw_min_m);
+        if (rc > 0) return rc;
+        if (rc == GLLMQ_OK) {
+            const MmfwMatrix down{ static_cast<const uint8_t *>(down_w), out, hidden };
+            if (ctx->ffn_glu_load) {
+                ctx->call_glu = relu_gate ? 2u : 1u;
+                ctx->call_glu_off = static_cast<uint32_t>(m * ffn);
+                ctx->call_ldx = static_cast<uint32_t>(ffn);
+                rc = run_mmfw(ctx, S, *fd, &down, 1, gu, 0, elem, m, ffn, false, stream, ctx->mmfw_min_m);
+                ctx->call_glu = ctx->call_glu_off = ctx->call_ldx = 0;
+            } else {
+                gq::GluActParams A{};
+                A.h = h;
+                A.g = gu;
+                A.u = gu + m * ffn;
+                A.m = static_cast<uint32_t>(m);
+                A.ffn = A.ld = static_cast<uint32_t>(ffn);
+                A.relu_gate = relu_gate ? 1u : 0u;
+                rc = launch2d(ctx, ctx->glu_act, static_cast<uint32_t>((ffn + 255) / 256),
+                              static_cast<uint32_t>(std::min<size_t>(m, 65535)), 256, 0, stream, &A, sizeof A);
+                if (rc == GLLMQ_OK) rc = run_mmfw(ctx, S, *fd, &down, 1, h, 0, elem, m, ffn, false, stream, ctx->mmfw_min_m);
+            }
+            return rc >= 0 ? rc : fail(ctx, GLLMQ_ERR_BAD_SHAPE, "ffn_swiglu: the down projection has no kernel for this shape");
+        }
+    }
+    if (elem) return kNeedPlainActivations;
     // gate and up in one launch with the activation in its epilogue (Q4_K / Q5_K, up to 8 rows)
     rc = -1;
     if (ctx->ffn_fused && ctx->ffn_streamed && m <= 4) rc = run_mm8s(ctx, *fg, gw, x, h, m, ffn, hidden, false, stream, uw, relu_gate != 0);
@@ -2129,6 +2367,18 @@ int gllmq_ffn_swiglu(gllmq_ctx *ctx, const void *gate_w, const void *up_w, size_
         if (rc != GLLMQ_OK) return rc;
     }
     return dispatch_matmul(ctx, S, *fd, static_cast<const uint8_t *>(down_w), h, out, m, hidden, ffn, false, stream);
+}
+
+} // namespace
+
+int gllmq_ffn_swiglu(gllmq_ctx *ctx, const void *gate_w, const void *up_w, size_t gate_up_bytes_each, uint32_t dtype_gate_up,
+                     const void *down_w, size_t down_bytes, uint32_t dtype_down, const float *x, float *out, size_t m,
+                     size_t hidden, size_t ffn, int relu_gate, void *stream)
+{
+    if (!ctx) return GLLMQ_ERR_INVALID;
+    std::lock_guard<std::recursive_mutex> call(ctx->call_mutex);
+    return ffn_on_stream(ctx, gate_w, up_w, gate_up_bytes_each, dtype_gate_up, down_w, down_bytes, dtype_down, x, out, 0, m, hidden, ffn,
+                         relu_gate, stream);
 }
 
 namespace {
@@ -2191,8 +2441,13 @@ int gllmq_ffn_swiglu_elem(gllmq_ctx *ctx, const void *gate_w, const void *up_w, 
 {
     if (!ctx) return GLLMQ_ERR_INVALID;
     std::lock_guard<std::recursive_mutex> call(ctx->call_mutex);
+    int rc = kNeedPlainActivations;
+    if ((elem == GLLMQ_ELEM_F16 || elem == GLLMQ_ELEM_BF16) && flags == 0 && ctx->elem_fused && aligned(x, 16) && aligned(out, 4))
+        rc = ffn_on_stream(ctx, gate_w, up_w, gate_up_bytes_each, dtype_gate_up, down_w, down_bytes, dtype_down,
+                           static_cast<const float *>(x), static_cast<float *>(out), static_cast<uint32_t>(elem), m, hidden, ffn, relu_gate, stream);
+    if (rc != kNeedPlainActivations) return rc;
     ElemStage st;
-    int rc = elem_stage_begin(ctx, x, out, m * hidden, elem, flags, stream, "ffn_swiglu", &st);
+    rc = elem_stage_begin(ctx, x, out, m * hidden, elem, flags, stream, "ffn_swiglu", &st);
     if (rc != GLLMQ_OK) return rc;
     rc = gllmq_ffn_swiglu(ctx, gate_w, up_w, gate_up_bytes_each, dtype_gate_up, down_w, down_bytes, dtype_down, st.x, st.result, m,
                           hidden, ffn, relu_gate, stream);
@@ -2751,6 +3006,7 @@ int gllmq_reserve_matmul(gllmq_ctx *ctx, uint32_t dtype, size_t m, size_t n, siz
     if (m < 3) return GLLMQ_OK;
     // (either form of it: which one runs also depends on the activation pointer's alignment)
     size_t need = plan_mmf(ctx, m, n, k).need;
+    for (bool hi_only : { false, true }) need = std::max(need, plan_mmfw(ctx, dtype, m, &n, 1, k, hi_only).need());
     const MmfsPlan Ls = plan_mmfs(ctx, *find_format(dtype), m, n, k);
     if (Ls.ok) need = std::max(need, Ls.need);
     return grow_scratch(ctx, *S, &S->mmf, &S->mmf_bytes, need, stream, "reserve_matmul");
@@ -2767,6 +3023,11 @@ int gllmq_reserve_ffn(gllmq_ctx *ctx, uint32_t dtype_gate_up, uint32_t dtype_dow
     Scratch *S = nullptr;
     rc = acquire_scratch(ctx, stream, &S);
     if (rc != GLLMQ_OK) return rc;
+    const size_t both[2] = { ffn, ffn }; // gate and up in one GEMM launch
+    for (bool hi_only : { false, true }) {
+        rc = grow_scratch(ctx, *S, &S->mmf, &S->mmf_bytes, plan_mmfw(ctx, dtype_gate_up, m, both, 2, hidden, hi_only).need(), stream, "reserve_ffn");
+        if (rc != GLLMQ_OK) return rc;
+    }
     return grow_scratch(ctx, *S, &S->ffn, &S->ffn_bytes, ffn_scratch_bytes(m, ffn), stream, "reserve_ffn");
 }
 

@@ -367,6 +367,143 @@ constexpr int MMFR_LOADERS = 4;  // loader waves (MM8S_LOADERS: the loader is th
 constexpr int MMFR_RED_BUFS = 3; // tiles whose block sums can be waiting in LDS
 constexpr uint32_t MMFR_RED_WAVE = 2u * 64u * 16u; // bytes of a tile's sums in LDS per wave: [column tile][lane] float4
 
+// The GEMM for prompts and larger batches (mmfw.hip.inc).  A workgroup is eight waves of 32 weight
+// rows each and MT tiles of 32 activation rows; the activations come as images in the order the
+// lanes hold them (MmfwImage), the weight matrices of one launch share the activations.
+constexpr int MMFW_WAVES = 8;
+constexpr int MMFW_TILE_ROWS = 32 * MMFW_WAVES; // weight rows per workgroup
+constexpr int MMFW_MAX_SEGS = 3;                // weight matrices of one launch
+constexpr int MMFW_MAX_MT = 4;
+
+// Image of 32 activation rows x 256 elements of K: [K step 0..15][plane][lane] 16 bytes, then
+// [lane] 16 bytes of sub-block sums (lanes 0..31 hi, 32..63 lo); images lie [row tile][block].
+// The inverse scales are an array of their own: [block][padded rows] f32.
+template <int PL> struct MmfwImage {
+    static constexpr uint32_t sums = 16u * PL * 1024u, bytes = sums + 1024u;
+};
+
+// FMT: 0 = Q4_K, 1 = Q5_K, 2 = Q6_K, 3 = Q8_0.  A wave's weights of a block come in parts, each
+// requested again (for the next block) as soon as it has been read: the header (scales) and `PARTS`
+// equal shares of the quants, `PART` wave-loads each.
+template <int FMT> struct MmfwFormat;
+template <> struct MmfwFormat<0> { // 32 rows x 32 bytes per part, headers 16 bytes a row
+    static constexpr uint32_t BLOCK = 144, STAGE = 5u * 1024u;
+    static constexpr int PARTS = 4, PART = 1, HEAD = 1, BP = 1;
+    static constexpr bool SUMS = true;
+};
+template <> struct MmfwFormat<1> { // the fifth bits come with the header
+    static constexpr uint32_t BLOCK = 176, STAGE = 6u * 1024u;
+    static constexpr int PARTS = 4, PART = 1, HEAD = 2, BP = 1;
+    static constexpr bool SUMS = true;
+};
+template <> struct MmfwFormat<2> { // half blocks: two 32-byte pieces of low nibbles a row, one of high bits
+    static constexpr uint32_t BLOCK = 210, STAGE = 7u * 1024u;
+    static constexpr int PARTS = 2, PART = 3, HEAD = 1, BP = 2;
+    static constexpr bool SUMS = false;
+};
+template <> struct MmfwFormat<3> { // half groups: 136 bytes a row
+    static constexpr uint32_t BLOCK = 272, STAGE = 10u * 1024u;
+    static constexpr int PARTS = 2, PART = 5, HEAD = 0, BP = 1;
+    static constexpr bool SUMS = false;
+};
+
+template <int FMT, int PL, int MT>
+struct MmfwShape {
+    using F = MmfwFormat<FMT>;
+    // Activations move in chunks of UC units (32 elements of K) through a ring of R chunk slots in LDS.
+    static constexpr int UC = MT == 4 ? (PL == 2 ? 1 : 2) : MT == 3 ? (PL == 2 ? 2 : 4) : MT == 2 ? (PL == 2 ? 2 : 4) : (PL == 2 ? 4 : 8);
+    static constexpr int R = MT == 3 ? 3 : 4;
+    static constexpr int C = 8 / UC;                   // chunks per block
+    static constexpr int PIECES = MT * PL * 2 * UC;    // KiB per chunk
+    static constexpr int NA = PIECES / MMFW_WAVES;     // wave-loads per wave and chunk
+    static_assert(PIECES % MMFW_WAVES == 0, "every wave requests the same number of pieces");
+    static constexpr uint32_t CHUNK = PIECES * 1024u;
+    static constexpr uint32_t TILE_CHUNK = 2u * UC * PL * 1024u; // a row tile's share: contiguous in its image
+    static constexpr uint32_t extra = 0;               // [4][sums of MT tiles, inverse scales]
+    static constexpr uint32_t EXTRA = ((F::SUMS ? MT : 0) + 1) * 1024u;
+    static constexpr uint32_t stage = 4u * EXTRA;
+    static constexpr uint32_t ring = stage + MMFW_WAVES * F::STAGE;
+    static constexpr uint32_t total = ring + R * CHUNK;
+    static_assert(total <= 160u * 1024u, "LDS");
+
+    // ---- A block is NS stages of SG operand slots (a K step of one plane) for all row tiles; Q8_0: a
+    // stage is a unit.  What stage s + 1 multiplies is read from LDS during stage s.
+    static constexpr int SG = MT >= 3 ? 1 : MT == 2 ? 2 : 4;
+    static constexpr int NS = FMT == 3 ? 8 : 16 * PL / SG;
+    static constexpr int SPC = NS / C;                 // stages per chunk
+    static constexpr int QL = NS / F::PARTS;           // stages per weight part
+    // Q8_0 reads the quants of stage s + 1 in stage s, so a part is free a stage before the next one starts
+    static constexpr int FREE = FMT == 3 ? QL - 1 : 0; // a part (p) is requested again at stage p * QL + FREE
+    static constexpr int part_of(int s) { return s >= FREE && (s - FREE) % QL == 0 ? (s - FREE) / QL : -1; }
+
+    // ---- the wave's sequence of loads, one block being a period: stage s requests its weights (and
+    // stage 0 the extra of the block after next, first); then, in the last stage of a chunk, the
+    // next chunk is acquired: its arrival is waited for and NA pieces of the chunk R - 1 further on
+    // are requested.
+    static constexpr int stage_loads(int s) { return (s == 0 ? 1 + F::HEAD : 0) + (part_of(s) >= 0 ? F::PART : 0); }
+    static constexpr int after_weights(int s) // position behind stage s's weight requests
+    {
+        int p = 0;
+        for (int i = 0; i <= s; ++i) p += stage_loads(i) + (i < s && (i + 1) % SPC == 0 ? NA : 0);
+        return p;
+    }
+    static constexpr int period = after_weights(NS - 1) + NA;
+    static constexpr int acquired(int c) // position of the acquisition of chunk c, ahead of its requests
+    {
+        int blk = 0;
+        while (c < 0) { c += C; --blk; }
+        return blk * period + (c ? after_weights(c * SPC - 1) : -NA);
+    }
+    static constexpr int limit(int n) { return n < 0 ? 0 : n < 63 ? n : 63; }
+    // loads that may be outstanding: at the acquisition of chunk c (with chunk 0 of a block its extra
+    // has to be there, requested two blocks ago)
+    static constexpr int chunk_wait(int c)
+    {
+        int n = acquired(c) - (acquired(c - R + 1) + NA);
+        if (c == 0 && 2 * period - NA - 1 < n) n = 2 * period - NA - 1;
+        return limit(n);
+    }
+    // ... when stage s has made its requests and reads what the weight requests of stage `at`, `blocks` blocks
+    // ago (0: this block), brought
+    static constexpr int weight_wait(int s, int at, int blocks)
+    {
+        return limit(after_weights(s) + ((s + 1) % SPC == 0 ? NA : 0) - (after_weights(at) - blocks * period));
+    }
+};
+
+template <int FMT, int PL, int MT> constexpr uint32_t mmfw_lds() { return MmfwShape<FMT, PL, MT>::total; }
+
+struct MmfwSeg {
+    const uint8_t *w;
+    float *y;
+    float *partial;    // [ksplit][m][n] when ksplit > 1
+    uint32_t n, tile0; // weight rows; index of the matrix's first 256-row tile in the launch
+};
+
+struct MmfwParams {
+    MmfwSeg seg[MMFW_MAX_SEGS];
+    const uint8_t *ximg;
+    const float *inv;          // [groups][inv_ld]
+    uint32_t segs, groups, row_bytes, m, k;
+    uint32_t row_tiles;        // images per block of K = ceil(m / 32)
+    uint32_t inv_ld;
+    uint32_t m_tiles, n_tiles; // workgroup tiles of activation rows and of weight rows (all matrices)
+    uint32_t ksplit, blocks_per_split;
+    uint32_t items;            // m_tiles * n_tiles * ksplit
+    uint32_t band;             // activation tiles that neighbouring workgroups share a weight tile over
+    uint32_t elem;             // element type of y
+};
+
+struct MmfwPrepParams {
+    const float *x;
+    uint8_t *ximg;
+    float *inv;
+    uint32_t m, k, ldx, groups, inv_ld;
+    uint32_t act_bf16, elem;
+    uint32_t natural;      // K order inside 32 elements: 1: step s, half h = 16 s + 8 h; 0: 16 h + 8 s
+    uint32_t glu, glu_off; // x[i] = act(x[i]) * x[i + glu_off] (0 off, 1 SiLU, 2 SiLU behind a ReLU)
+};
+
 struct MmfPrepParams {
     const float *x;
     uint8_t *ximg;
