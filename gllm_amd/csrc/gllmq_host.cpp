@@ -217,6 +217,7 @@ struct gllmq_ctx {
     hipFunction_t moe_mm8_glu_fn[3][2] = {};    // gated gate/up kernels [Mm8Kind (Q4_K and Q5_K only)][passes per tile - 1]
     hipFunction_t mmf_q4k[4][2][2] = {};        // f16 matrix-core GEMM [0 = Q4_K, 1 = Q5_K, 2 = Q6_K, 3 = Q8_0][32-row activation tiles - 1][bf16 mode]
     hipFunction_t mmfw[4][4][2] = {};           // the GEMM for more rows [format as above][32-row activation tiles - 1][0 = hi and lo plane, 1 = hi only]
+    hipFunction_t moe_mmf[4][2] = {};           // the same over experts' rows [format][plane]
     hipFunction_t mmfw_prep[2] = {};            // its activation images [hi and lo plane, hi only]
     bool use_mmfw = true;                       // "mmfw" = 0: 64-row passes of the other forms
     uint32_t mmfw_min_m = 33;                   // "mmfw_min_m": fewest activation rows that take it
@@ -264,6 +265,8 @@ struct gllmq_ctx {
     uint32_t moe_slices = 0;                    // "moe_slices": workgroups that share a job's row tiles (0 = by the number of pairs and experts)
     bool moe_mm8_rows = true;                   // "moe_mm8_rows" = 0: no wave-per-tile kernel for short Q6_K rows
     uint32_t moe_streamed = 1;                  // "moe_streamed": the grouped kernels in the streamed form: 0 never, 1 while experts see few tokens each, 2 always
+    bool moe_wide = true;                       // "moe_wide" = 0: experts with many tokens stay on the eight-token jobs
+    uint32_t moe_wide_min = 8;                  // "moe_wide_min": fewest pairs per expert (on average) that take the GEMM
     uint32_t moe_depth = 0;                     // "moe_depth": items a loader of the streamed grouped kernels keeps unconfirmed (0 = as the dense launches)
 
     // One lock over every enqueue on this context: calls from several threads take turns on the
@@ -1760,6 +1763,11 @@ int gllmq_init(gllmq_ctx **out, int device)
                 snprintf(name, sizeof name, "gq_mmf_%s_w%d%s", q == 3 ? "q8_0" : q == 2 ? "q6k" : q == 1 ? "q5k" : "q4k", t + 1, b ? "_hi" : "");
                 rc = get_function(ctx, &ctx->mmfw[q][t][b], name);
             }
+    for (int q = 0; q < 4 && rc == GLLMQ_OK; ++q)
+        for (int b = 0; b < 2 && rc == GLLMQ_OK; ++b) {
+            snprintf(name, sizeof name, "gq_moe_mmf_%s%s", q == 3 ? "q8_0" : q == 2 ? "q6k" : q == 1 ? "q5k" : "q4k", b ? "_hi" : "");
+            rc = get_function(ctx, &ctx->moe_mmf[q][b], name);
+        }
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfr[0], "gq_mmfr_q4k");
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfr[1], "gq_mmfr_q5k");
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->moe_plan, "gq_moe_plan");
@@ -1979,6 +1987,8 @@ int gllmq_set_option(gllmq_ctx *ctx, const char *name, long value)
     else if (n == "moe_mm8_rows") ctx->moe_mm8_rows = value != 0;
     else if (n == "moe_glu") ctx->moe_glu = value != 0;
     else if (n == "moe_streamed") ctx->moe_streamed = u;
+    else if (n == "moe_wide") ctx->moe_wide = value != 0;
+    else if (n == "moe_wide_min") ctx->moe_wide_min = std::max(1u, u);
     else if (n == "moe_depth") ctx->moe_depth = u;
     else if (n == "moe_slices") ctx->moe_slices = u;
     else if (n == "prefetch") ctx->prefetch = value != 0;
@@ -2455,6 +2465,14 @@ int gllmq_ffn_swiglu_elem(gllmq_ctx *ctx, const void *gate_w, const void *up_w, 
     return elem_stage_end(ctx, st, out, m * hidden, elem, flags, stream);
 }
 
+namespace {
+int moe_on_stream(gllmq_ctx *ctx, const void *gate, size_t gate_bytes, size_t gate_expert_stride, const void *up,
+                  size_t up_bytes, size_t up_expert_stride, uint32_t dtype_gu, const void *down, size_t down_bytes,
+                  size_t down_expert_stride, uint32_t dtype_dn, const float *x, float *out, uint32_t elem, size_t tokens,
+                  size_t hidden, size_t ffn, size_t experts, size_t top_k, const uint32_t *route_expert,
+                  const float *route_weight, const uint32_t *route_len, int relu_gate, void *stream);
+}
+
 int gllmq_moe_matvec_elem(gllmq_ctx *ctx, const void *gate, size_t gate_bytes, size_t gate_expert_stride, const void *up,
                           size_t up_bytes, size_t up_expert_stride, uint32_t dtype_gu, const void *down, size_t down_bytes,
                           size_t down_expert_stride, uint32_t dtype_dn, const void *x, void *out, size_t tokens, size_t hidden,
@@ -2463,8 +2481,14 @@ int gllmq_moe_matvec_elem(gllmq_ctx *ctx, const void *gate, size_t gate_bytes, s
 {
     if (!ctx) return GLLMQ_ERR_INVALID;
     std::lock_guard<std::recursive_mutex> call(ctx->call_mutex);
+    int rc = kNeedPlainActivations;
+    if ((elem == GLLMQ_ELEM_F16 || elem == GLLMQ_ELEM_BF16) && flags == 0 && ctx->elem_fused && aligned(x, 16) && aligned(out, 4))
+        rc = moe_on_stream(ctx, gate, gate_bytes, gate_expert_stride, up, up_bytes, up_expert_stride, dtype_gu, down, down_bytes,
+                           down_expert_stride, dtype_dn, static_cast<const float *>(x), static_cast<float *>(out), static_cast<uint32_t>(elem),
+                           tokens, hidden, ffn, experts, top_k, route_expert, route_weight, route_len, relu_gate, stream);
+    if (rc != kNeedPlainActivations) return rc;
     ElemStage st;
-    int rc = elem_stage_begin(ctx, x, out, tokens * hidden, elem, flags, stream, "moe_matvec", &st);
+    rc = elem_stage_begin(ctx, x, out, tokens * hidden, elem, flags, stream, "moe_matvec", &st);
     if (rc != GLLMQ_OK) return rc;
     rc = gllmq_moe_matvec(ctx, gate, gate_bytes, gate_expert_stride, up, up_bytes, up_expert_stride, dtype_gu, down, down_bytes,
                           down_expert_stride, dtype_dn, st.x, st.result, tokens, hidden, ffn, experts, top_k, route_expert,
@@ -2660,7 +2684,7 @@ int gllmq_moe_route(gllmq_ctx *ctx, const float *logits, size_t tokens, size_t e
     if (!(cap >= 0.0f)) cap = 0.0f; // negative or NaN
     if (cap > 1.0e9f) cap = 1.0e9f;
     P.capacity = static_cast<uint32_t>(cap);
-    const uint32_t lds = static_cast<uint32_t>((gq::ROUTE_WAVES + 1) * experts * 4);
+    const uint32_t lds = static_cast<uint32_t>(((gq::ROUTE_WAVES + 1) * experts + 4) * 4);
     if (tokens <= gq::ROUTE_FUSED_MAX_TOKENS) {
         P.phases = 3u;
         return launch(ctx, ctx->moe_route, 1, gq::ROUTE_THREADS, lds, stream, &P, sizeof P);
@@ -2698,16 +2722,169 @@ MoeWorkspace moe_workspace(size_t pairs, size_t hidden, size_t ffn)
     return W;
 }
 
-} // namespace
-
-int gllmq_moe_matvec(gllmq_ctx *ctx, const void *gate, size_t gate_bytes, size_t gate_expert_stride, const void *up,
-                     size_t up_bytes, size_t up_expert_stride, uint32_t dtype_gu, const void *down, size_t down_bytes,
-                     size_t down_expert_stride, uint32_t dtype_dn, const float *x, float *out, size_t tokens,
-                     size_t hidden, size_t ffn, size_t experts, size_t top_k, const uint32_t *route_expert,
-                     const float *route_weight, const uint32_t *route_len, int relu_gate, void *stream)
+// Sorts the routed pairs by expert and writes the job tables that `P` points to.
+int launch_moe_plan(gllmq_ctx *ctx, MoePlanParams &P, const uint32_t *route_expert, const uint32_t *route_len, size_t tokens,
+                    size_t top_k, size_t experts, void *stream)
 {
-    if (!ctx) return GLLMQ_ERR_INVALID;
-    std::lock_guard<std::recursive_mutex> call(ctx->call_mutex);
+    P.route_expert = route_expert;
+    P.route_len = route_len;
+    P.tokens = static_cast<uint32_t>(tokens);
+    P.top_k = static_cast<uint32_t>(top_k);
+    P.experts = static_cast<uint32_t>(experts);
+    P.pairs = static_cast<uint32_t>(tokens * top_k);
+    // a wave per 64 pairs up to 16, as far as their counts (a word per expert each) fit the LDS; no
+    // fewer than four, which share the rest of the work
+    uint32_t waves = std::min<uint32_t>(gq::MOE_PLAN_THREADS / 64, std::max(4u, (P.pairs + 63u) / 64u));
+    while (waves > 4u && (waves + 4u) * P.experts * 4u > 128u * 1024u) waves /= 2u;
+    return launch(ctx, ctx->moe_plan, 1, waves * 64u, ((waves + 4u) * P.experts + 16u) * 4u, stream, &P, sizeof P);
+}
+
+// ---- Many tokens per expert (prompts): the GEMM of mmfw.hip.inc over the experts' own rows
+struct MoeWidePlan {
+    uint32_t max_tiles, max_jobs;
+    size_t src, pos, token, tiles, jobs, cnt, gu, o, img, inv, total;
+};
+
+MoeWidePlan plan_moe_wide(size_t pairs, size_t hidden, size_t ffn, size_t experts, bool hi_only)
+{
+    auto up256 = [](size_t v) { return (v + 255) & ~static_cast<size_t>(255); };
+    MoeWidePlan W{};
+    const size_t hit = std::min(experts, pairs);
+    W.max_tiles = static_cast<uint32_t>(pairs / 32 + hit);
+    W.max_jobs = static_cast<uint32_t>(pairs / (32 * gq::MMFW_MAX_MT) + hit);
+    const size_t gh = (hidden + 255) / 256, gf = (ffn + 255) / 256;
+    size_t off = 0;
+    W.src = off; off = up256(off + pairs * 4);
+    W.pos = off; off = up256(off + pairs * 4);
+    W.token = off; off = up256(off + pairs * 4);
+    W.tiles = off; off = up256(off + W.max_tiles * sizeof(gq::MoeTile));
+    W.jobs = off; off = up256(off + W.max_jobs * sizeof(gq::MoeWideJob));
+    W.cnt = off; off = up256(off + 4 * 4);
+    W.gu = off; off = up256(off + 2 * pairs * ffn * 4);
+    W.o = off; off = up256(off + pairs * hidden * 4);
+    W.img = off; off = up256(off + W.max_tiles * std::max(gh * (hi_only ? gq::MmfwImage<1>::bytes : gq::MmfwImage<2>::bytes), gf * gq::MmfwImage<2>::bytes));
+    W.inv = off; off = up256(off + std::max(gh, gf) * W.max_tiles * 128 + 1024);
+    W.total = off;
+    return W;
+}
+
+// From where the GEMM is ahead of jobs of eight tokens (us, whole call, jobs / GEMM): Q4_K with Q6_K down,
+// 128 experts of 4096 x 1536: 6 pairs per expert 472 / 590, 8: 617 / 602, 16: 884 / 616; 32 experts of
+// 2048 x 1024: 6: 96 / 90, 8: 124 / 96; 8 experts of 4096 x 2048: 8: 99 / 100, 12: 117 / 104.  Q8_0
+// experts, whose other form is the GEMV: 4: 1352 / 731, 129 / 94, 115 / 115.
+bool takes_moe_wide(const gllmq_ctx *ctx, uint32_t dtype_gu, uint32_t dtype_dn, const void *x, size_t hidden, size_t ffn, size_t experts,
+                    size_t pairs)
+{
+    if (!ctx->moe_wide || !ctx->use_mmf || !ctx->use_mmfw || ctx->moe_streamed == 2 || pairs < (dtype_gu == T_Q8_0 || dtype_dn == T_Q8_0 ? (ctx->moe_wide_min + 1) / 2 : ctx->moe_wide_min) * experts)
+        return false; // (the other form of Q8_0 experts is the GEMV)
+    if ((dtype_gu == T_Q8_0 && hidden < 256) || (dtype_dn == T_Q8_0 && ffn < 256)) return false; // the Q8_0 window is a whole group
+    const size_t tiles = pairs / 32 + std::min(experts, pairs), groups = std::max((hidden + 255) / 256, (ffn + 255) / 256);
+    return aligned(x, 16) && pairs * ffn <= 0xFFFFFFFFull && tiles * groups * gq::MmfwImage<2>::bytes <= 0xFFFFFFFFull;
+}
+
+int run_moe_wide(gllmq_ctx *ctx, const Format &fg, const void *gate, size_t gate_stride, const void *up, size_t up_stride, const Format &fd,
+                 const void *down, size_t down_stride, const float *x, float *out, uint32_t elem, size_t tokens, size_t hidden, size_t ffn,
+                 size_t experts, size_t top_k, const uint32_t *route_expert, const float *route_weight, const uint32_t *route_len,
+                 int relu_gate, void *stream)
+{
+    const size_t pairs = tokens * top_k;
+    const bool hi_only = elem != 0;
+    const MoeWidePlan W = plan_moe_wide(pairs, hidden, ffn, experts, hi_only);
+    Scratch *Sp = nullptr;
+    int rc = acquire_scratch(ctx, stream, &Sp);
+    if (rc != GLLMQ_OK) return rc;
+    rc = grow_scratch(ctx, *Sp, &Sp->moe, &Sp->moe_bytes, W.total, stream, "moe_matvec");
+    if (rc != GLLMQ_OK) return rc;
+    uint8_t *ws = static_cast<uint8_t *>(Sp->moe);
+    uint32_t *token = reinterpret_cast<uint32_t *>(ws + W.token), *counters = reinterpret_cast<uint32_t *>(ws + W.cnt);
+    float *gu = reinterpret_cast<float *>(ws + W.gu), *o = reinterpret_cast<float *>(ws + W.o);
+    MoePlanParams plan{};
+    plan.pair_src = reinterpret_cast<uint32_t *>(ws + W.src);
+    plan.pair_pos = reinterpret_cast<uint32_t *>(ws + W.pos);
+    plan.tiles = reinterpret_cast<gq::MoeTile *>(ws + W.tiles);
+    plan.wide = reinterpret_cast<gq::MoeWideJob *>(ws + W.jobs);
+    plan.token = token;
+    plan.counters = counters;
+    plan.job_rows = 32u * gq::MMFW_MAX_MT;
+    rc = launch_moe_plan(ctx, plan, route_expert, route_len, tokens, top_k, experts, stream);
+    if (rc != GLLMQ_OK) return rc;
+
+    // the images of the tiles' rows, then every job's products with its expert's matrices
+    auto multiply = [&](const Format &f, const MmfwMatrix *mats, const size_t *strides, int count, size_t k, bool hi, gq::MmfwPrepParams &Q) -> int {
+        const int fmt = mmf_format(f.dtype);
+        Q.ximg = ws + W.img;
+        Q.inv = reinterpret_cast<float *>(ws + W.inv);
+        Q.m = static_cast<uint32_t>(pairs);
+        Q.k = static_cast<uint32_t>(k);
+        Q.groups = static_cast<uint32_t>((k + 255) / 256);
+        Q.inv_ld = W.max_tiles * 32u;
+        Q.tiles = plan.tiles;
+        Q.counters = counters;
+        Q.natural = fmt == 2 ? 1u : 0u;
+        int r = launch2d(ctx, ctx->mmfw_prep[hi ? 1 : 0], Q.groups, W.max_tiles, 256, 0, stream, &Q, sizeof Q, true);
+        if (r != GLLMQ_OK) return r;
+        gq::MmfwParams P{};
+        P.ximg = Q.ximg;
+        P.inv = Q.inv;
+        P.segs = static_cast<uint32_t>(count);
+        P.groups = Q.groups;
+        P.row_bytes = static_cast<uint32_t>(gllmq_row_bytes(f.dtype, k));
+        P.m = Q.m;
+        P.k = Q.k;
+        P.inv_ld = Q.inv_ld;
+        P.ksplit = 1;
+        P.blocks_per_split = Q.groups;
+        P.jobs = plan.wide;
+        P.counters = counters;
+        for (int i = 0; i < count; ++i) {
+            P.seg[i].w = mats[i].w;
+            P.seg[i].y = mats[i].y;
+            P.seg[i].n = static_cast<uint32_t>(mats[i].n);
+            P.seg[i].tile0 = P.n_tiles;
+            P.seg[i].expert_stride = strides[i];
+            P.n_tiles += static_cast<uint32_t>((mats[i].n + gq::MMFW_TILE_ROWS - 1) / gq::MMFW_TILE_ROWS);
+        }
+        P.max_jobs = W.max_jobs;
+        uint32_t lds = 0;
+        for (uint32_t mt = 1; mt <= static_cast<uint32_t>(gq::MMFW_MAX_MT); ++mt) lds = std::max(lds, mmfw_lds_bytes(fmt, hi ? 1 : 2, mt));
+        return launch(ctx, ctx->moe_mmf[fmt][hi ? 1 : 0], (W.max_jobs + 7u) / 8u * 8u * P.n_tiles, gq::MMFW_WAVES * 64, lds, stream, &P,
+                      sizeof P, true);
+    };
+    {
+        gq::MmfwPrepParams Q{};
+        Q.x = x;
+        Q.ldx = static_cast<uint32_t>(hidden);
+        Q.elem = elem;
+        Q.row_of = token;
+        const MmfwMatrix mats[2] = { { static_cast<const uint8_t *>(gate), gu, ffn }, { static_cast<const uint8_t *>(up), gu + pairs * ffn, ffn } };
+        const size_t strides[2] = { gate_stride, up_stride };
+        rc = multiply(fg, mats, strides, 2, hidden, hi_only, Q);
+        if (rc != GLLMQ_OK) return rc;
+    }
+    {
+        gq::MmfwPrepParams Q{};
+        Q.x = gu;
+        Q.ldx = static_cast<uint32_t>(ffn);
+        Q.glu = relu_gate ? 2u : 1u;
+        Q.glu_off = static_cast<uint32_t>(pairs * ffn);
+        const MmfwMatrix mats[1] = { { static_cast<const uint8_t *>(down), o, hidden } };
+        const size_t strides[1] = { down_stride };
+        rc = multiply(fd, mats, strides, 1, ffn, false, Q);
+        if (rc != GLLMQ_OK) return rc;
+    }
+    MoeCombineParams C{ o, route_weight, route_len, plan.pair_pos, out, static_cast<uint32_t>(tokens), static_cast<uint32_t>(top_k),
+                        static_cast<uint32_t>(hidden), elem };
+    return launch2d(ctx, ctx->moe_combine, static_cast<uint32_t>((hidden + 255) / 256), static_cast<uint32_t>(tokens), 256, 0, stream, &C, sizeof C);
+}
+
+// The expert matvec (call_mutex held).  x and out are of type `elem`; where the kernels of the shape take
+// f32 only, kNeedPlainActivations comes back and nothing has been enqueued.
+int moe_on_stream(gllmq_ctx *ctx, const void *gate, size_t gate_bytes, size_t gate_expert_stride, const void *up,
+                  size_t up_bytes, size_t up_expert_stride, uint32_t dtype_gu, const void *down, size_t down_bytes,
+                  size_t down_expert_stride, uint32_t dtype_dn, const float *x, float *out, uint32_t elem, size_t tokens,
+                  size_t hidden, size_t ffn, size_t experts, size_t top_k, const uint32_t *route_expert,
+                  const float *route_weight, const uint32_t *route_len, int relu_gate, void *stream)
+{
     const Format *fg = find_format(dtype_gu), *fd = find_format(dtype_dn);
     if (!fg || !fd)
         return fail(ctx, GLLMQ_ERR_UNIMPLEMENTED,
@@ -2749,6 +2926,10 @@ int gllmq_moe_matvec(gllmq_ctx *ctx, const void *gate, size_t gate_bytes, size_t
     if (!aligned(x, 16) || !aligned(out, 4))
         return fail(ctx, GLLMQ_ERR_BAD_ALIGNMENT, "moe_matvec: x must be 16-byte and out 4-byte aligned");
 
+    if (takes_moe_wide(ctx, dtype_gu, dtype_dn, x, hidden, ffn, experts, pairs))
+        return run_moe_wide(ctx, *fg, gate, gate_expert_stride, up, up_expert_stride, *fd, down, down_expert_stride, x, out, elem, tokens,
+                            hidden, ffn, experts, top_k, route_expert, route_weight, route_len, relu_gate, stream);
+    if (elem) return kNeedPlainActivations;
     const MoeWorkspace W = moe_workspace(pairs, hidden, ffn);
     Scratch *Sp = nullptr;
     int rc = acquire_scratch(ctx, stream, &Sp);
@@ -2771,12 +2952,15 @@ int gllmq_moe_matvec(gllmq_ctx *ctx, const void *gate, size_t gate_bytes, size_t
     // average: decode batches); with more, jobs of eight read the weights half as often.
     const bool streamed_jobs = ctx->use_mm8s && (ctx->moe_streamed == 2 || (ctx->moe_streamed == 1 && pairs <= 2 * experts));
     const uint32_t job_shift = streamed_jobs ? 2u : 3u;
-    const uint32_t fast = pairs <= 4096 ? 1u : 0u; // per-pair placement: quadratic in the pairs, but without serial LDS walks
     {
-        MoePlanParams P{ route_expert, route_len, pair_src, pair_pos, jobs, jobs8, counters, static_cast<uint32_t>(tokens),
-                         static_cast<uint32_t>(top_k), static_cast<uint32_t>(experts), static_cast<uint32_t>(pairs), fast, job_shift };
-        const uint32_t lds = static_cast<uint32_t>((pairs + 4 * experts + 4 + (fast ? 2 * pairs : 0)) * 4);
-        rc = launch(ctx, ctx->moe_plan, 1, 256, lds, stream, &P, sizeof P);
+        MoePlanParams P{};
+        P.pair_src = pair_src;
+        P.pair_pos = pair_pos;
+        P.jobs = jobs;
+        P.jobs8 = jobs8;
+        P.counters = counters;
+        P.job_rows = 1u << job_shift;
+        rc = launch_moe_plan(ctx, P, route_expert, route_len, tokens, top_k, experts, stream);
         if (rc != GLLMQ_OK) return rc;
     }
     // Waves per job: the device takes about 8 waves per CU of these kernels; the jobs that
@@ -2877,7 +3061,7 @@ int gllmq_moe_matvec(gllmq_ctx *ctx, const void *gate, size_t gate_bytes, size_t
         const uint32_t groups = static_cast<uint32_t>((k + 255) / 256);
         const int kind = mm8_kind(f.dtype);
         if (glu && !(ctx->moe_glu && (kind == MM8_Q4K || kind == MM8_Q5K))) return false;
-        if (!(fast && ctx->use_mm8 && ctx->moe_mm8) || kind < 0 || kind >= MM8_MOE_KINDS || groups > 16 || k % 8 != 0) return false;
+        if (!(ctx->use_mm8 && ctx->moe_mm8) || kind < 0 || kind >= MM8_MOE_KINDS || groups > 16 || k % 8 != 0) return false;
         if (kind == MM8_Q6K && !ctx->moe_mm8_q6k) return false;
         return mm8_lds_bytes(groups, 8, 4, kind) <= 160u * 1024u;
     };
@@ -2909,8 +3093,23 @@ int gllmq_moe_matvec(gllmq_ctx *ctx, const void *gate, size_t gate_bytes, size_t
     else rc = grouped(*fd, down, down_expert_stride, rb_dn, H, F, h, false, o, H);
     if (rc != GLLMQ_OK) return rc;
     MoeCombineParams C{ o, route_weight, route_len, pair_pos, out, static_cast<uint32_t>(tokens),
-                        static_cast<uint32_t>(top_k), H };
+                        static_cast<uint32_t>(top_k), H, 0 };
     return launch2d(ctx, ctx->moe_combine, (H + 255u) / 256u, static_cast<uint32_t>(tokens), 256, 0, stream, &C, sizeof C);
+}
+
+} // namespace
+
+int gllmq_moe_matvec(gllmq_ctx *ctx, const void *gate, size_t gate_bytes, size_t gate_expert_stride, const void *up,
+                     size_t up_bytes, size_t up_expert_stride, uint32_t dtype_gu, const void *down, size_t down_bytes,
+                     size_t down_expert_stride, uint32_t dtype_dn, const float *x, float *out, size_t tokens,
+                     size_t hidden, size_t ffn, size_t experts, size_t top_k, const uint32_t *route_expert,
+                     const float *route_weight, const uint32_t *route_len, int relu_gate, void *stream)
+{
+    if (!ctx) return GLLMQ_ERR_INVALID;
+    std::lock_guard<std::recursive_mutex> call(ctx->call_mutex);
+    return moe_on_stream(ctx, gate, gate_bytes, gate_expert_stride, up, up_bytes, up_expert_stride, dtype_gu, down, down_bytes,
+                         down_expert_stride, dtype_dn, x, out, 0, tokens, hidden, ffn, experts, top_k, route_expert, route_weight, route_len,
+                         relu_gate, stream);
 }
 
 int gq_quantized_matmul_on_block(gllmq_ctx *ctx, const void *w, size_t w_bytes, const float *x, float *y, uint32_t dtype,
@@ -3038,8 +3237,11 @@ int gllmq_reserve_moe(gllmq_ctx *ctx, size_t tokens, size_t top_k, size_t hidden
     Scratch *S = nullptr;
     int rc = acquire_scratch(ctx, stream, &S);
     if (rc != GLLMQ_OK || tokens == 0 || top_k == 0) return rc;
-    return grow_scratch(ctx, *S, &S->moe, &S->moe_bytes, moe_workspace(tokens * top_k, hidden, ffn).total, stream,
-                        "reserve_moe");
+    // (the GEMM form is for calls with at least moe_wide_min pairs per expert)
+    const size_t pairs = tokens * top_k, most_experts = std::max<size_t>(1, 2 * pairs / ctx->moe_wide_min);
+    size_t need = moe_workspace(pairs, hidden, ffn).total;
+    for (size_t e = most_experts; e > 0; e /= 2) need = std::max(need, plan_moe_wide(pairs, hidden, ffn, e, false).total);
+    return grow_scratch(ctx, *S, &S->moe, &S->moe_bytes, need, stream, "reserve_moe");
 }
 
 int gllmq_dequantize_host(gllmq_ctx *ctx, const void *blocks, size_t n_bytes, float *out, size_t n_out,

@@ -478,6 +478,7 @@ struct MmfwSeg {
     float *y;
     float *partial;    // [ksplit][m][n] when ksplit > 1
     uint32_t n, tile0; // weight rows; index of the matrix's first 256-row tile in the launch
+    uint64_t expert_stride; // grouped: bytes between the experts' matrices
 };
 
 struct MmfwParams {
@@ -492,6 +493,11 @@ struct MmfwParams {
     uint32_t items;            // m_tiles * n_tiles * ksplit
     uint32_t band;             // activation tiles that neighbouring workgroups share a weight tile over
     uint32_t elem;             // element type of y
+    // Grouped launch (experts): jobs[0 .. counters[2]) take the place of the activation tiles, row r of job J
+    // is output row J.p0 + r.
+    const struct MoeWideJob *jobs;
+    const uint32_t *counters;
+    uint32_t max_jobs;         // entries of `jobs` that exist at most
 };
 
 struct MmfwPrepParams {
@@ -500,6 +506,10 @@ struct MmfwPrepParams {
     float *inv;
     uint32_t m, k, ldx, groups, inv_ld;
     uint32_t act_bf16, elem;
+    // grouped launch: image t (below counters[3]) holds the rows tiles[t].p0 + r; their activations are row
+    // row_of[that], or that row itself
+    const struct MoeTile *tiles;
+    const uint32_t *row_of, *counters;
     uint32_t natural;      // K order inside 32 elements: 1: step s, half h = 16 s + 8 h; 0: 16 h + 8 s
     uint32_t glu, glu_off; // x[i] = act(x[i]) * x[i + glu_off] (0 off, 1 SiLU, 2 SiLU behind a ReLU)
 };
@@ -575,17 +585,30 @@ struct MoeJob8 {
     uint32_t tok[8]; // their tokens (entries past m repeat the last one)
 };
 
+// The GEMM's view of the sorted pairs (mmfw.hip.inc): a tile is up to 32 of them, of one expert; a job
+// is an expert's consecutive tiles that a workgroup multiplies together.
+struct MoeTile {
+    uint32_t p0, rows; // first sorted position, pairs
+};
+struct MoeWideJob {
+    uint32_t expert, tile0, p0, rows;
+};
+
+constexpr int MOE_PLAN_THREADS = 1024;
+
 struct MoePlanParams {
     const uint32_t *route_expert; // [tokens][top_k]
     const uint32_t *route_len;    // [tokens]
     uint32_t *pair_src;
     uint32_t *pair_pos;
     MoeJob *jobs;
-    MoeJob8 *jobs8;   // written when P.fast
-    uint32_t *counters; // [0] jobs, [1] routed pairs, [2] eight-token jobs
+    MoeJob8 *jobs8;
+    MoeTile *tiles;     // null, or the GEMM's tables are written instead of the two job lists
+    MoeWideJob *wide;
+    uint32_t *token;    // [pairs] token of each sorted position
+    uint32_t *counters; // [0] jobs, [1] routed pairs, [2] matrix-core (or GEMM) jobs, [3] tiles of 32
     uint32_t tokens, top_k, experts, pairs;
-    uint32_t fast; // pairs are few enough for the per-pair placement (LDS has two more arrays of `pairs` words)
-    uint32_t job_shift; // a matrix-core job takes up to 1 << job_shift tokens of an expert (3, or 2 for the streamed kernels)
+    uint32_t job_rows;  // a matrix-core job takes up to that many tokens of an expert
 };
 
 constexpr uint32_t MOE_NONE = 0xFFFFFFFFu;
@@ -647,6 +670,7 @@ struct MoeCombineParams {
     const uint32_t *pair_pos;     // [tokens][top_k]
     float *out;                   // [tokens][hidden]
     uint32_t tokens, top_k, hidden;
+    uint32_t elem;                // element type of out
 };
 
 } // namespace gq

@@ -84,3 +84,62 @@ def test_passes_of_fewer_rows(torch, dtype):
     hip.quantized_matmul_noalloc(w, x, got, dtype, m, n, k)
     torch.cuda.synchronize()
     assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.parametrize("t_gu, t_dn, hidden, ffn, experts, top_k, tokens, elem", [
+    (Q4_K, Q6_K, 512, 256, 4, 2, 70, "float32"),     # jobs of one and two tiles
+    (Q5_K, Q4_K, 768, 520, 3, 2, 200, "bfloat16"),   # of four tiles and a fifth; a ragged ffn
+    (Q8_0, Q8_0, 288, 352, 2, 1, 190, "float16"),    # short last groups; four tiles in two halves
+    (Q6_K, Q5_K, 256, 256, 40, 8, 45, "float32"),    # few rows per tile
+])
+def test_experts_with_many_tokens(torch, oracle, t_gu, t_dn, hidden, ffn, experts, top_k, tokens, elem):
+    """moe_matvec through the GEMM (from `moe_wide_min` pairs per expert up) against the oracle, with an
+    expert nobody chose, routes dropped (length below top_k) and separate gate and up tensors."""
+    from gllm_amd.backend import HipBackend
+    from gllm_amd.ggml import row_bytes
+    hip = HipBackend(0, options={"moe_wide_min": 1})
+    rng = np.random.default_rng(tokens)
+    gate = random_weight(t_gu, experts * ffn, hidden, seed=1)
+    up = random_weight(t_gu, experts * ffn, hidden, seed=2)
+    down = random_weight(t_dn, experts * hidden, ffn, seed=3)
+    t = getattr(torch, elem)
+    x = torch.from_numpy(random_activations(tokens, hidden, seed=4) * 1e-3).to(t)
+    expert = np.stack([rng.permutation(max(1, experts - 1))[np.arange(top_k) % max(1, experts - 1)] for _ in range(tokens)]).astype(np.int32)
+    weight = rng.uniform(0.1, 1.0, (tokens, top_k)).astype(np.float32)
+    length = np.full(tokens, top_k, np.int32)
+    length[::7] = max(1, top_k - 1)
+    out = torch.full((tokens, hidden), float("nan"), dtype=t, device="cuda")
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    print(f"wide experts {t_gu}/{t_dn} hidden={hidden} ffn={ffn} tokens={tokens} {elem}", flush=True)
+    hip.moe_matvec(dev(gate), t_gu, dev(down), t_dn, x.cuda(), out, hidden, ffn, experts, dev(expert), dev(weight), dev(length), up=dev(up))
+    torch.cuda.synchronize()
+    got = out.float().cpu().numpy()
+    xf = x.float().numpy()
+    want = np.zeros((tokens, hidden), np.float64)
+    gb, db = ffn * row_bytes(t_gu, hidden), hidden * row_bytes(t_dn, ffn)
+    for e in range(experts):
+        pairs = [(a, i) for a in range(tokens) for i in range(length[a]) if expert[a, i] == e]
+        if not pairs:
+            continue
+        rows = oracle.ffn_swiglu(gate[e * gb:(e + 1) * gb], up[e * gb:(e + 1) * gb], t_gu, down[e * db:(e + 1) * db], t_dn,
+                                 np.ascontiguousarray(xf[[a for a, _ in pairs]]), len(pairs), hidden, ffn, acc=oracle.ACC_F64, threads=16)
+        for (a, i), r in zip(pairs, rows.reshape(len(pairs), hidden)):
+            want[a] += weight[a, i] * r.astype(np.float64)
+    rel = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert rel <= {"float32": 1e-5, "float16": 1e-3, "bfloat16": 5e-3}[elem], rel
+
+
+def test_router_walks_from_the_first_token_without_a_place(torch, oracle):
+    """Ranks in parallel up to the first token that loses all its choices, the serial walk from there:
+    capacities from none to plenty, top_k that does not divide 64, more tokens than a wave's run."""
+    from gllm_amd.backend import HipBackend
+    from tests.test_gpu_route import check_against_oracle, route
+    hip = HipBackend(0)
+    rng = np.random.default_rng(5)
+    for tokens, experts, top_k in ((65, 8, 2), (300, 16, 3), (777, 5, 5), (130, 128, 8), (1000, 600, 7), (90, 4, 8)):
+        logits = rng.standard_normal((tokens, experts)).astype(np.float32)
+        logits[:, 0] += 2.0  # a favourite
+        for factor in (0.0, 0.4, 1.0, 1.25, 3.0, 1e9):
+            print(f"route tokens={tokens} experts={experts} top_k={top_k} capacity={factor}", flush=True)
+            got = route(hip, torch, logits, top_k, capacity_factor=factor)
+            check_against_oracle(oracle, got, logits, top_k, factor, f"{tokens} {experts} {top_k} {factor}")
