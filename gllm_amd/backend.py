@@ -165,13 +165,18 @@ EXPORTED_SYMBOLS = [
 
 
 def _dtype_id(quant_type) -> int:
+    if type(quant_type) is int:
+        return quant_type
     if isinstance(quant_type, QuantType):
         return quant_type.ggml_dtype
     return int(quant_type)
 
 
+_tensor_type = None  # torch.Tensor, once a backend exists
+
+
 def _is_torch(t) -> bool:
-    return type(t).__module__.startswith("torch")
+    return type(t) is _tensor_type or type(t).__module__.startswith("torch")
 
 
 def _host_bytes(buf) -> np.ndarray:
@@ -190,8 +195,16 @@ class HipBackend:
         import torch
         if not torch.cuda.is_available():
             raise HipError("no HIP device is visible; this backend has no CPU path")
+        global _tensor_type
+        _tensor_type = torch.Tensor
         self._torch = torch
         self.device = device
+        # A call of a few microseconds is bound by what happens around it: the current stream's handle
+        # comes straight from torch's binding (0.1 us; a Stream object costs 1.3), and the element types
+        # are looked up in a table made once.
+        self._raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+            lambda d: torch.cuda.current_stream(d).cuda_stream)
+        self._elems = {torch.float32: ELEM_F32, torch.float16: ELEM_F16, torch.bfloat16: ELEM_BF16}
         ctx = C.c_void_p()
         rc = self._lib.gllmq_init(C.byref(ctx), device)
         if rc != OK:
@@ -253,8 +266,8 @@ class HipBackend:
             raise HipError(msg)
         raise OtherError(f"{self._lib.gllmq_status_string(rc).decode()}: {msg}")
 
-    def _stream(self):
-        return C.c_void_p(self._torch.cuda.current_stream(self.device).cuda_stream)
+    def _stream(self) -> int:
+        return self._raw_stream(self.device)
 
     def upload_weights(self, weight_blocks):
         """Raw GGUF block bytes -> device buffer, untouched (the reference passes quantized
@@ -271,7 +284,7 @@ class HipBackend:
             w, x, y = weight_blocks, input, output
             if not (w.is_cuda and x.is_cuda and y.is_cuda):
                 raise OtherError("quantized_matmul: tensors must live on the GPU")
-            elem = self._elem_of(x.dtype)
+            elem = self._elems.get(x.dtype)
             if elem is None or y.dtype != x.dtype:
                 raise Unimplemented("quantized_matmul: activations and outputs are f32, f16 or bf16, both of one type")
             if not (w.is_contiguous() and x.is_contiguous() and y.is_contiguous()):
@@ -281,13 +294,11 @@ class HipBackend:
             if elem != ELEM_F32:
                 if act_mode != ACT_F32_SPLIT:
                     raise Unimplemented("quantized_matmul: the bf16 activation mode is for f32 tensors")
-                rc = self._lib.gllmq_quantized_matmul_elem(
-                    self._ctx, w.data_ptr(), w.numel() * w.element_size(), x.data_ptr(), y.data_ptr(),
-                    dt, m, n, k, elem, self._stream())
+                rc = self._lib.gllmq_quantized_matmul_elem(self._ctx, w.data_ptr(), w.nbytes, x.data_ptr(), y.data_ptr(), dt, m, n, k,
+                                                           elem, self._raw_stream(self.device))
             else:
-                rc = self._lib.gllmq_quantized_matmul_ex(
-                    self._ctx, w.data_ptr(), w.numel() * w.element_size(), x.data_ptr(), y.data_ptr(),
-                    dt, m, n, k, act_mode, self._stream())
+                rc = self._lib.gllmq_quantized_matmul_ex(self._ctx, w.data_ptr(), w.nbytes, x.data_ptr(), y.data_ptr(), dt, m, n, k,
+                                                         act_mode, self._raw_stream(self.device))
         else:
             w = _host_bytes(weight_blocks)
             x = np.ascontiguousarray(input, np.float32).reshape(-1)
@@ -302,8 +313,7 @@ class HipBackend:
 
     def _elem_of(self, torch_dtype):
         """Backend<E>: the element types the reference instantiates (src/compat/mod.rs:376-378)."""
-        t = self._torch
-        return {t.float32: ELEM_F32, t.float16: ELEM_F16, t.bfloat16: ELEM_BF16}.get(torch_dtype)
+        return self._elems.get(torch_dtype)
 
     def quantized_matmul_noalloc(self, weight_blocks, input, output, quant_type, m: int, n: int, k: int) -> None:
         """``quantized_matmul`` on device tensors through the entry point that allocates nothing
@@ -315,7 +325,7 @@ class HipBackend:
             raise Unimplemented("quantized_matmul_noalloc: activations and outputs are f32 on this backend")
         if x.numel() < m * k or y.numel() < m * n:
             raise OtherError("quantized_matmul_noalloc: input/output shorter than m*k / m*n")
-        rc = self._lib.gllmq_quantized_matmul_noalloc(self._ctx, w.data_ptr(), w.numel() * w.element_size(), x.data_ptr(),
+        rc = self._lib.gllmq_quantized_matmul_noalloc(self._ctx, w.data_ptr(), w.nbytes, x.data_ptr(),
                                                       y.data_ptr(), _dtype_id(quant_type), m, n, k, self._stream())
         if rc != OK:
             self._raise(rc, "quantized_matmul_noalloc")
@@ -327,7 +337,7 @@ class HipBackend:
             b, o = block_data, output
             if not (b.is_cuda and o.is_cuda and o.dtype == self._torch.float32):
                 raise OtherError("dequantize: tensors must live on the GPU, output f32")
-            rc = self._lib.gllmq_dequantize(self._ctx, b.data_ptr(), b.numel() * b.element_size(),
+            rc = self._lib.gllmq_dequantize(self._ctx, b.data_ptr(), b.nbytes,
                                             o.data_ptr(), o.numel(), dt, self._stream())
         else:
             b = _host_bytes(block_data)
@@ -352,7 +362,7 @@ class HipBackend:
             if elem is None or y.dtype != x.dtype:
                 raise Unimplemented("make_batch: activations and outputs are f32, f16 or bf16, both of one type")
             flags |= {ELEM_F32: 0, ELEM_F16: DESC_ELEM_F16, ELEM_BF16: DESC_ELEM_BF16}[elem]
-            arr[i] = MatmulDesc(w.data_ptr(), w.numel() * w.element_size(), x.data_ptr(), y.data_ptr(),
+            arr[i] = MatmulDesc(w.data_ptr(), w.nbytes, x.data_ptr(), y.data_ptr(),
                                 _dtype_id(qt), flags, m, n, k)
         return arr
 
@@ -392,11 +402,11 @@ class HipBackend:
         if output.numel() < count * hidden_dim:
             raise OtherError("quant_gather: output shorter than len(ids) * hidden_dim")
         if elem == ELEM_F32:
-            rc = self._lib.gllmq_quant_gather(self._ctx, table.data_ptr(), table.numel() * table.element_size(), dt,
+            rc = self._lib.gllmq_quant_gather(self._ctx, table.data_ptr(), table.nbytes, dt,
                                               vocab_size, hidden_dim, token_ids.data_ptr(), count,
                                               1.0 if scale is None else float(scale), output.data_ptr(), self._stream())
         else:
-            rc = self._lib.gllmq_quant_gather_elem(self._ctx, table.data_ptr(), table.numel() * table.element_size(), dt,
+            rc = self._lib.gllmq_quant_gather_elem(self._ctx, table.data_ptr(), table.nbytes, dt,
                                                    vocab_size, hidden_dim, token_ids.data_ptr(), count,
                                                    1.0 if scale is None else float(scale), output.data_ptr(), elem, self._stream())
         if rc != OK:
@@ -417,15 +427,15 @@ class HipBackend:
             raise OtherError("ffn_swiglu: x and out must be f32, f16 or bf16, both of one type")
         if x.numel() < m * hidden or out.numel() < m * hidden:
             raise OtherError("ffn_swiglu: x/out shorter than m * hidden")
-        gb, ub = gate.numel() * gate.element_size(), up.numel() * up.element_size()
+        gb, ub = gate.nbytes, up.nbytes
         if elem == ELEM_F32 and not accumulate:
             rc = self._lib.gllmq_ffn_swiglu(self._ctx, gate.data_ptr(), up.data_ptr(), min(gb, ub), _dtype_id(dtype_gate_up),
-                                            down.data_ptr(), down.numel() * down.element_size(), _dtype_id(dtype_down),
+                                            down.data_ptr(), down.nbytes, _dtype_id(dtype_down),
                                             x.data_ptr(), out.data_ptr(), m, hidden, ffn, 1 if relu_gate else 0,
                                             self._stream())
         else:
             rc = self._lib.gllmq_ffn_swiglu_elem(self._ctx, gate.data_ptr(), up.data_ptr(), min(gb, ub), _dtype_id(dtype_gate_up),
-                                                 down.data_ptr(), down.numel() * down.element_size(), _dtype_id(dtype_down),
+                                                 down.data_ptr(), down.nbytes, _dtype_id(dtype_down),
                                                  x.data_ptr(), out.data_ptr(), m, hidden, ffn, 1 if relu_gate else 0,
                                                  elem, OUT_ACCUMULATE if accumulate else 0, self._stream())
         if rc != OK:
@@ -464,7 +474,7 @@ class HipBackend:
             raise OtherError("lm_head_argmax: logits must be a contiguous device f32 tensor of n entries")
         if value is not None and not (value.is_cuda and value.dtype == self._torch.float32 and value.numel() >= 1):
             raise OtherError("lm_head_argmax: value must be a device f32 tensor")
-        rc = self._lib.gllmq_lm_head_argmax(self._ctx, w.data_ptr(), w.numel() * w.element_size(), x.data_ptr(),
+        rc = self._lib.gllmq_lm_head_argmax(self._ctx, w.data_ptr(), w.nbytes, x.data_ptr(),
                                             _dtype_id(quant_type), n, k, logits.data_ptr() if logits is not None else None,
                                             token.data_ptr(), value.data_ptr() if value is not None else None,
                                             self._stream())
@@ -502,16 +512,16 @@ class HipBackend:
         if elem is None or out.dtype != x.dtype:
             raise OtherError("moe_matvec: x and out must be f32, f16 or bf16, both of one type")
         dgu, ddn = _dtype_id(dtype_gate_up), _dtype_id(dtype_down)
-        each = ffn * self._lib.gllmq_row_bytes(dgu, hidden)  # 0 for a dtype the library does not cover
-        gbytes = gate_up.numel() * gate_up.element_size()
+        each = ffn * row_bytes(dgu, hidden) if supported(dgu) else 0  # (the library refuses other dtypes)
+        gbytes = gate_up.nbytes
         if up is None:
             gate_ptr, gate_b, gate_st = gate_up.data_ptr(), max(gbytes - each, 0), 2 * each
             up_ptr, up_b, up_st = gate_up.data_ptr() + each, max(gbytes - each, 0), 2 * each
         else:
             gate_ptr, gate_b, gate_st = gate_up.data_ptr(), gbytes, each
-            up_ptr, up_b, up_st = up.data_ptr(), up.numel() * up.element_size(), each
+            up_ptr, up_b, up_st = up.data_ptr(), up.nbytes, each
         args = (self._ctx, gate_ptr, gate_b, gate_st, up_ptr, up_b, up_st, dgu,
-                down.data_ptr(), down.numel() * down.element_size(), hidden * self._lib.gllmq_row_bytes(ddn, ffn), ddn,
+                down.data_ptr(), down.nbytes, hidden * row_bytes(ddn, ffn) if supported(ddn) else 0, ddn,
                 x.data_ptr(), out.data_ptr(), tokens, hidden, ffn, experts, top_k, route_expert.data_ptr(),
                 route_weight.data_ptr(), route_len.data_ptr(), int(relu_gate))
         if elem == ELEM_F32 and not accumulate:
