@@ -1025,7 +1025,12 @@ int run_mmf(gllmq_ctx *ctx, Scratch &S, const Format &f, const uint8_t *w, const
         rc = launch(ctx, ctx->mmf_q4k[fmt][mt - 1][act_bf16 ? 1 : 0], row_tiles * ksplit, 512, mmf_lds_bytes(mt, fmt), stream,
                     &P, sizeof P, true);
         if (rc == GLLMQ_OK && ksplit > 1) {
-            MmfReduceParams R{ P.partial, P.y, mm, P.n, P.ldy, ksplit, P.elem };
+            MmfReduceParams R{};
+            R.seg[0] = gq::MmfReduceSeg{ P.partial, P.y, P.n, 0u };
+            R.segs = 1;
+            R.m = mm;
+            R.ksplit = ksplit;
+            R.elem = P.elem;
             const uint64_t quads = (static_cast<uint64_t>(mm) * n + 3) / 4;
             rc = launch(ctx, ctx->mmf_reduce, static_cast<uint32_t>((quads + 255) / 256), 256, 0, stream, &R, sizeof R, true);
         }
@@ -1083,10 +1088,16 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
     L.n_tiles = static_cast<uint32_t>(tiles);
     const uint32_t row_tiles = static_cast<uint32_t>((m + 31) / 32);
     // Activation tiles per workgroup and slices of K by a cost model (us): a block of K takes a
-    // workgroup its matrix-core time or the weights' way from memory, whichever is longer; a
-    // workgroup starts and ends in about the time of two blocks; the slices of K meet through memory.
+    // workgroup its products (Q6_K: one more operand; Q8_0: its scales), the way of one wave's block through
+    // unpacking and LDS, which a tile or two do not cover, or the weights' way from memory, whichever
+    // is longest; a workgroup starts and ends in `start`; the slices of K meet through memory.  Slopes over
+    // K measured with one tile on 16 CUs: 1.5 (Q4_K), 2.7 (Q6_K), 2.4 (Q8_0) a block; two tiles,
+    // one plane and two: 1.8 and 2.4, 2.9 and 3.9, 3.4 and 4.2.
     const double cus = ctx->num_cus;
     const double w_us = find_format(dtype)->group_bytes * 256.0 * cus / 5.0e6; // 5 TB/s over all CUs
+    static const double chain_us[4] = { 1.5, 1.6, 2.7, 2.4 };
+    const double tile_us = fmt == 3 ? 1.2 + 0.45 * L.planes : 0.25 + 0.62 * (L.planes + (fmt == 2 ? 1u : 0u));
+    const double start = 5.0;
     double best = 1e300;
     for (uint32_t mt = 1; mt <= static_cast<uint32_t>(gq::MMFW_MAX_MT); ++mt) {
         if (ctx->mmfw_mt ? mt != ctx->mmfw_mt : (mt > row_tiles)) continue;
@@ -1098,8 +1109,8 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
             if (ctx->mmfw_ksplit && ks != std::min(ctx->mmfw_ksplit, L.groups)) continue;
             const double rounds = std::ceil(static_cast<double>(m_tiles * tiles * ks) / cus);
             const double busy = std::min(1.0, static_cast<double>(m_tiles * tiles * ks) / cus);
-            const double block = std::max(0.62 * mt * L.planes + 0.25 * mt, w_us * busy);
-            double us = rounds * (bps * block + 3.0);
+            const double block = std::max({ mt * tile_us, chain_us[fmt], w_us * busy });
+            double us = rounds * (bps * block + start);
             if (ks > 1) us += 4.0 + 2.0 * ks * static_cast<double>(m) * static_cast<double>(n_sum) * 4.0 / 4.0e6;
             if (us < best) {
                 best = us;
@@ -1161,7 +1172,7 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
         Q.glu = ctx->call_glu;
         Q.glu_off = ctx->call_glu_off;
         const uint32_t row_tiles = (mm + 31u) / 32u;
-        rc = launch2d(ctx, ctx->mmfw_prep[hi_only ? 1 : 0], L.groups, row_tiles, 256, 0, stream, &Q, sizeof Q, true);
+        rc = launch2d(ctx, ctx->mmfw_prep[hi_only ? 1 : 0], L.groups, row_tiles, gq::MMFW_PREP_WAVES * 64, 0, stream, &Q, sizeof Q, true);
         if (rc != GLLMQ_OK) return rc;
         gq::MmfwParams P{};
         P.ximg = scratch;
@@ -1194,10 +1205,18 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
         }
         rc = launch(ctx, ctx->mmfw[fmt][L.mt - 1][hi_only ? 1 : 0], (P.items + 7u) / 8u * 8u, gq::MMFW_WAVES * 64, mmfw_lds_bytes(fmt, hi_only ? 1 : 2, L.mt),
                     stream, &P, sizeof P, true);
-        for (int i = 0; i < count && rc == GLLMQ_OK && L.ksplit > 1; ++i) {
-            MmfReduceParams R{ P.seg[i].partial, P.seg[i].y, mm, P.seg[i].n, P.seg[i].n, L.ksplit, P.elem };
-            const uint64_t quads = (static_cast<uint64_t>(mm) * P.seg[i].n + 3) / 4;
-            rc = launch(ctx, ctx->mmf_reduce, static_cast<uint32_t>((quads + 255) / 256), 256, 0, stream, &R, sizeof R, true);
+        if (rc == GLLMQ_OK && L.ksplit > 1) {
+            gq::MmfReduceParams R{};
+            uint32_t wgs = 0;
+            for (int i = 0; i < count; ++i) {
+                R.seg[i] = gq::MmfReduceSeg{ P.seg[i].partial, P.seg[i].y, P.seg[i].n, wgs };
+                wgs += static_cast<uint32_t>((static_cast<uint64_t>(mm) * P.seg[i].n + 1023) / 1024);
+            }
+            R.segs = P.segs;
+            R.m = mm;
+            R.ksplit = L.ksplit;
+            R.elem = P.elem;
+            rc = launch(ctx, ctx->mmf_reduce, wgs, 256, 0, stream, &R, sizeof R, true);
         }
         if (rc != GLLMQ_OK) return rc;
     }
@@ -2821,7 +2840,7 @@ int run_moe_wide(gllmq_ctx *ctx, const Format &fg, const void *gate, size_t gate
         Q.tiles = plan.tiles;
         Q.counters = counters;
         Q.natural = fmt == 2 ? 1u : 0u;
-        int r = launch2d(ctx, ctx->mmfw_prep[hi ? 1 : 0], Q.groups, W.max_tiles, 256, 0, stream, &Q, sizeof Q, true);
+        int r = launch2d(ctx, ctx->mmfw_prep[hi ? 1 : 0], Q.groups, W.max_tiles, gq::MMFW_PREP_WAVES * 64, 0, stream, &Q, sizeof Q, true);
         if (r != GLLMQ_OK) return r;
         gq::MmfwParams P{};
         P.ximg = Q.ximg;

@@ -374,6 +374,7 @@ constexpr int MMFW_WAVES = 8;
 constexpr int MMFW_TILE_ROWS = 32 * MMFW_WAVES; // weight rows per workgroup
 constexpr int MMFW_MAX_SEGS = 3;                // weight matrices of one launch
 constexpr int MMFW_MAX_MT = 4;
+constexpr uint32_t MMFW_PREP_WAVES = 16;        // of a workgroup that prepares an image
 
 // Image of 32 activation rows x 256 elements of K: [K step 0..15][plane][lane] 16 bytes, then
 // [lane] 16 bytes of sub-block sums (lanes 0..31 hi, 32..63 lo); images lie [row tile][block].
@@ -522,10 +523,15 @@ struct MmfPrepParams {
     uint32_t glu, glu_off; // x[i] = act(x[i]) * x[i + glu_off] (0 off, 1 SiLU, 2 SiLU behind a ReLU)
 };
 
-struct MmfReduceParams {
+struct MmfReduceSeg {
     const float *partial; // [ksplit][m][n]
-    float *y;             // [m][ldy]
-    uint32_t m, n, ldy, ksplit;
+    float *y;             // [m][n]
+    uint32_t n, first_wg; // the matrix's first workgroup
+};
+
+struct MmfReduceParams {
+    MmfReduceSeg seg[MMFW_MAX_SEGS];
+    uint32_t segs, m, ksplit;
     uint32_t elem; // element type of y
 };
 
