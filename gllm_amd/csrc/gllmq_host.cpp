@@ -221,6 +221,8 @@ struct gllmq_ctx {
     hipFunction_t mmfw_prep[2] = {};            // its activation images [hi and lo plane, hi only]
     bool use_mmfw = true;                       // "mmfw" = 0: 64-row passes of the other forms
     uint32_t mmfw_min_m = 33;                   // "mmfw_min_m": fewest activation rows that take it
+    bool batch_group = true;                    // "batch_group": independent entries over the same rows as one GEMM
+    uint32_t mmfw_small_min_m = 9;              // "mmfw_small_min_m": ... where the streamed GEMMs do not take the call
     uint32_t mmfw_mt = 0, mmfw_ksplit = 0;      // "mmfw_mt", "mmfw_ksplit": activation tiles per workgroup, slices of K (0 = by the shape)
     hipFunction_t mmfs[2][2] = {};              // its streamed form [0 = Q4_K, 1 = Q5_K][bf16 mode]
     hipFunction_t mmfr[2] = {};                 // the streamed form whose waves prepare their own activations (f32, 9 to 16 rows) [0 = Q4_K, 1 = Q5_K]
@@ -1070,6 +1072,13 @@ void mmfw_size(MmfwPlan &L, size_t rows, size_t n_sum)
     L.part_bytes = L.ksplit > 1 ? static_cast<size_t>(L.ksplit) * rows * n_sum * 4 : 0;
 }
 
+// Whether the GEMM's scratch for this plan is there or can be had now: a capture cannot allocate, and what was
+// reserved for the kernels of fewer rows has to go on serving them.
+bool mmfw_scratch_ok(const gllmq_ctx *ctx, const Scratch &S, const MmfwPlan &L, void *stream)
+{
+    return L.need() <= S.mmf_bytes || ctx->probe || !(S.fixed || stream_is_capturing(stream));
+}
+
 MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t *n, int count, size_t k, bool hi_only,
                    size_t scratch_limit = SIZE_MAX)
 {
@@ -1131,7 +1140,7 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
         rows = std::max(step, (rows / 2 + step - 1) / step * step);
         mmfw_size(L, rows, n_sum);
     }
-    L.ok = L.img_bytes < 0xFFFFFFFFull;
+    L.ok = L.img_bytes < 0xFFFFFFFFull && L.need() <= scratch_limit;
     return L;
 }
 
@@ -1150,6 +1159,7 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
     const bool hi_only = act_bf16 || (elem_x && !ctx->call_glu);
     const MmfwPlan L = plan_mmfw(ctx, f.dtype, m, n, count, k, hi_only, S.fixed ? S.mmf_bytes : SIZE_MAX);
     if (!L.ok) return -1;
+    if (m < ctx->mmfw_min_m && !mmfw_scratch_ok(ctx, S, L, stream)) return -1;
     int rc = grow_scratch(ctx, S, &S.mmf, &S.mmf_bytes, L.need(), stream, "quantized_matmul (GEMM)");
     if (rc != GLLMQ_OK) return rc;
     uint8_t *scratch = static_cast<uint8_t *>(S.mmf);
@@ -1585,6 +1595,15 @@ int dispatch_matmul(gllmq_ctx *ctx, Scratch &S, const Format &f, const uint8_t *
     if (rc >= 0) return rc;
     rc = run_mmfs(ctx, S, f, w, x, y, m, n, k, bf16, stream);
     if (rc >= 0 || rc == kNeedPlainActivations) return rc;
+    // 9 to 32 rows of what the streamed GEMMs leave: one row tile of the GEMM for more rows.  us per call at 16 and
+    // 32 bf16 rows against run_mmf's: Q6_K 14336 x 4096 24.7, 26.0 (27.7, 29.0), 4096 x 4096 18.8, 20.9 (21.3, 22.3);
+    // Q8_0 14336 x 4096 24.9, 27.0 (33.0, 34.3); Q4_K 4096 x 14336 19.5, 20.8 (22.2, 22.3), 1024 x 4096 the same.
+    // f32, 32 rows, Q4_K 14336 x 4096 21.2 (20.9).
+    if (!ctx->mmfs_all) {
+        const MmfwMatrix one{ w, y, n };
+        rc = run_mmfw(ctx, S, f, &one, 1, x, ctx->call_elem, ctx->call_elem, m, k, bf16, stream, std::max(9u, ctx->mmfw_small_min_m));
+        if (rc >= 0 || rc == kNeedPlainActivations) return rc;
+    }
     rc = run_mmf(ctx, S, f, w, x, y, m, n, k, bf16, stream);
     if (rc >= 0 || rc == kNeedPlainActivations) return rc;
     // up to 8 rows: the int8 kernels when one pass over the weights does it, else the GEMM
@@ -1973,6 +1992,8 @@ int gllmq_set_option(gllmq_ctx *ctx, const char *name, long value)
     else if (n == "mmfr") ctx->use_mmfr = value != 0;
     else if (n == "mmfw") ctx->use_mmfw = value != 0;
     else if (n == "mmfw_min_m") ctx->mmfw_min_m = std::max(1u, u);
+    else if (n == "batch_group") ctx->batch_group = value != 0;
+    else if (n == "mmfw_small_min_m") ctx->mmfw_small_min_m = std::max(1u, u);
     else if (n == "mmfw_mt") ctx->mmfw_mt = std::min(u, static_cast<uint32_t>(gq::MMFW_MAX_MT));
     else if (n == "mmfw_ksplit") ctx->mmfw_ksplit = u;
     else if (n == "mmfr_min_rows") ctx->mmfr_min_rows = std::max(1u, u);
@@ -2323,10 +2344,19 @@ int ffn_on_stream(gllmq_ctx *ctx, const void *gate_w, const void *up_w, size_t g
 
     // Prompts and larger batches: gate and up share their activation images and run as one launch; the
     // down projection's images are prepared from the two results.
-    if (m >= ctx->mmfw_min_m && m > 8 && !ctx->mmfs_all && ffn % 4 == 0 && m * ffn <= 0xFFFFFFFFull &&
-        plan_mmfw(ctx, dtype_down, m, &hidden, 1, ffn, false).ok) {
+    const size_t gate_up_n[2] = { ffn, ffn };
+    const uint32_t wide_min = std::max(9u, std::min(ctx->mmfw_min_m, ctx->mmfw_small_min_m));
+    auto down_fits = [&] {
+        const MmfwPlan L = plan_mmfw(ctx, dtype_down, m, &hidden, 1, ffn, false, S.fixed ? S.mmf_bytes : SIZE_MAX);
+        return L.ok && mmfw_scratch_ok(ctx, S, L, stream);
+    };
+    auto gate_up_fits = [&] {
+        const MmfwPlan L = plan_mmfw(ctx, dtype_gate_up, m, gate_up_n, 2, hidden, elem != 0, S.fixed ? S.mmf_bytes : SIZE_MAX);
+        return L.ok && mmfw_scratch_ok(ctx, S, L, stream);
+    };
+    if (m >= wide_min && !ctx->mmfs_all && ffn % 4 == 0 && m * ffn <= 0xFFFFFFFFull && down_fits() && gate_up_fits()) {
         const MmfwMatrix gate_up[2] = { { gw, gu, ffn }, { uw, gu + m * ffn, ffn } };
-        rc = run_mmfw(ctx, S, *fg, gate_up, 2, x, elem, 0, m, hidden, false, stream, ctx->mmfw_min_m);
+        rc = run_mmfw(ctx, S, *fg, gate_up, 2, x, elem, 0, m, hidden, false, stream, wide_min);
         if (rc > 0) return rc;
         if (rc == GLLMQ_OK) {
             const MmfwMatrix down{ static_cast<const uint8_t *>(down_w), out, hidden };
@@ -2334,7 +2364,7 @@ int ffn_on_stream(gllmq_ctx *ctx, const void *gate_w, const void *up_w, size_t g
                 ctx->call_glu = relu_gate ? 2u : 1u;
                 ctx->call_glu_off = static_cast<uint32_t>(m * ffn);
                 ctx->call_ldx = static_cast<uint32_t>(ffn);
-                rc = run_mmfw(ctx, S, *fd, &down, 1, gu, 0, elem, m, ffn, false, stream, ctx->mmfw_min_m);
+                rc = run_mmfw(ctx, S, *fd, &down, 1, gu, 0, elem, m, ffn, false, stream, wide_min);
                 ctx->call_glu = ctx->call_glu_off = ctx->call_ldx = 0;
             } else {
                 gq::GluActParams A{};
@@ -2346,7 +2376,7 @@ int ffn_on_stream(gllmq_ctx *ctx, const void *gate_w, const void *up_w, size_t g
                 A.relu_gate = relu_gate ? 1u : 0u;
                 rc = launch2d(ctx, ctx->glu_act, static_cast<uint32_t>((ffn + 255) / 256),
                               static_cast<uint32_t>(std::min<size_t>(m, 65535)), 256, 0, stream, &A, sizeof A);
-                if (rc == GLLMQ_OK) rc = run_mmfw(ctx, S, *fd, &down, 1, h, 0, elem, m, ffn, false, stream, ctx->mmfw_min_m);
+                if (rc == GLLMQ_OK) rc = run_mmfw(ctx, S, *fd, &down, 1, h, 0, elem, m, ffn, false, stream, wide_min);
             }
             return rc >= 0 ? rc : fail(ctx, GLLMQ_ERR_BAD_SHAPE, "ffn_swiglu: the down projection has no kernel for this shape");
         }
@@ -2541,6 +2571,54 @@ int batch_entry(gllmq_ctx *ctx, Scratch &S, const gllmq_matmul_desc &d, void *st
     return matmul_on_scratch(ctx, S, d.w_dev, d.w_bytes, d.x_dev, d.y_dev, d.ggml_dtype, d.m, d.n, d.k, GLLMQ_ACT_F32_SPLIT, stream);
 }
 
+// Entries from `descs` on that one GEMM launch can multiply: independent matmuls of one format over the same 9 or
+// more activation rows (a layer's Q, K and V projections).  0 or 1: none.
+size_t group_length(const gllmq_ctx *ctx, const gllmq_matmul_desc *descs, size_t count)
+{
+    constexpr uint32_t kElemBits = GLLMQ_DESC_ELEM_F16 | GLLMQ_DESC_ELEM_BF16;
+    const gllmq_matmul_desc &first = descs[0];
+    const uint32_t elem = first.flags & kElemBits;
+    if (count < 2 || !ctx->batch_group || ctx->mmfs_all || first.m < std::max(9u, std::min(ctx->mmfw_min_m, ctx->mmfw_small_min_m)) ||
+        first.k == 0 || !first.x_dev || elem == kElemBits || (elem && !elem_in_kernel(ctx, first.m, first.k)))
+        return 0;
+    const size_t e = elem ? 2 : 4;
+    size_t len = 0;
+    while (len < count && len < static_cast<size_t>(gq::MMFW_MAX_SEGS)) {
+        const gllmq_matmul_desc &d = descs[len];
+        const uint32_t known = elem | (len == 0 ? static_cast<uint32_t>(GLLMQ_DESC_AFTER_PREVIOUS) : 0u);
+        if ((d.flags & ~known) || (d.flags & kElemBits) != elem || d.ggml_dtype != first.ggml_dtype || d.m != first.m || d.k != first.k ||
+            d.x_dev != first.x_dev || d.n == 0 || !d.y_dev || d.m > 0x7FFFFFFFu || d.n > 0x7FFFFFFFu || d.k > 0x7FFFFFFFu)
+            break;
+        bool apart = !ranges_meet(d.y_dev, d.m * d.n * e, d.x_dev, d.m * d.k * e);
+        for (size_t i = 0; i < len; ++i) apart = apart && !ranges_meet(d.y_dev, d.m * d.n * e, descs[i].y_dev, descs[i].m * descs[i].n * e);
+        if (!apart) break;
+        ++len;
+    }
+    return len;
+}
+
+// The group as one GEMM.  -1: its entries go through the dispatch one by one (which also reports what is wrong with them).
+int run_group(gllmq_ctx *ctx, Scratch &S, const gllmq_matmul_desc *descs, size_t len, void *stream)
+{
+    const gllmq_matmul_desc &first = descs[0];
+    const Format *f = find_format(first.ggml_dtype);
+    if (!f) return -1;
+    MmfwMatrix mats[gq::MMFW_MAX_SEGS];
+    size_t n[gq::MMFW_MAX_SEGS];
+    const size_t rb = gllmq_row_bytes(first.ggml_dtype, first.k);
+    for (size_t i = 0; i < len; ++i) {
+        const gllmq_matmul_desc &d = descs[i];
+        if (!d.w_dev || rb > (size_t(1) << 26) || d.w_bytes < d.n * rb || !aligned(d.w_dev, f->w_align) || rb % f->w_align != 0 || !aligned(d.y_dev, 4))
+            return -1;
+        mats[i] = MmfwMatrix{ static_cast<const uint8_t *>(d.w_dev), d.y_dev, d.n };
+        n[i] = d.n;
+    }
+    const uint32_t elem = (first.flags & GLLMQ_DESC_ELEM_F16) ? GLLMQ_ELEM_F16 : (first.flags & GLLMQ_DESC_ELEM_BF16) ? GLLMQ_ELEM_BF16 : 0u;
+    const MmfwPlan L = plan_mmfw(ctx, first.ggml_dtype, first.m, n, static_cast<int>(len), first.k, elem != 0, S.fixed ? S.mmf_bytes : SIZE_MAX);
+    if (!L.ok || !mmfw_scratch_ok(ctx, S, L, stream)) return -1;
+    return run_mmfw(ctx, S, *f, mats, static_cast<int>(len), first.x_dev, elem, elem, first.m, first.k, false, stream, 9);
+}
+
 // The launches a batch will make, and which of them get their weights prefetched: an ordered
 // launch whose kernel and whose predecessor's kernel both say when they start (the predecessor's
 // start is the prefetch's cue, its own start tells a late prefetch to give up).  Nothing is
@@ -2638,6 +2716,16 @@ int gllmq_quantized_matmul_batch(gllmq_ctx *ctx, const gllmq_matmul_desc *descs,
                 ctx->overlap = gllmq_ctx::Overlap{};
                 ctx->overlap.on = overlap_on;
                 i += chain - 1;
+                continue;
+            }
+        }
+        const size_t group = group_length(ctx, descs + i, count - i);
+        if (group >= 2) {
+            ctx->overlap.entry_first = !(d.flags & GLLMQ_DESC_AFTER_PREVIOUS);
+            const int grc = run_group(ctx, *S, descs + i, group, stream);
+            if (grc >= 0) {
+                rc = grc;
+                i += group - 1;
                 continue;
             }
         }

@@ -143,3 +143,93 @@ def test_router_walks_from_the_first_token_without_a_place(torch, oracle):
             print(f"route tokens={tokens} experts={experts} top_k={top_k} capacity={factor}", flush=True)
             got = route(hip, torch, logits, top_k, capacity_factor=factor)
             check_against_oracle(oracle, got, logits, top_k, factor, f"{tokens} {experts} {top_k} {factor}")
+
+
+def element_bar(elem):
+    """The rounding of the output to its type (2^-11, 2^-9 of a value at most), over the f32 bar."""
+    return {"float32": 1e-5, "float16": 1e-3, "bfloat16": 5e-3}[elem]
+
+
+@pytest.mark.parametrize("dtype", ALL)
+@pytest.mark.parametrize("elem", ["float32", "float16", "bfloat16"])
+def test_nine_to_32_rows(torch, oracle, dtype, elem):
+    """One row tile, where the streamed GEMMs do not take the call: few weight rows, Q6_K and Q8_0."""
+    from gllm_amd.backend import HipBackend
+    hip = HipBackend(0)
+    t = getattr(torch, elem)
+    for m, n, k in ((9, 257, 1280), (16, 1000, 2080 if dtype == Q8_0 else 2048), (31, 40, 256), (32, 513, 4864)):
+        print(f"one tile dtype={dtype} {elem} m={m} n={n} k={k}", flush=True)
+        w, x = random_weight(dtype, n, k, seed=m + n), torch.from_numpy(random_activations(m, k, seed=k + m) * 1e-2).to(t)
+        y = torch.full((m, n), float("nan"), dtype=t, device="cuda")
+        hip.quantized_matmul(torch.from_numpy(w.view(np.uint8).reshape(-1)).cuda(), x.cuda(), y, dtype, m, n, k)
+        assert hip.last_kernel_name() == "gq_mmf_reduce" or "_w1" in hip.last_kernel_name(), hip.last_kernel_name()
+        want = oracle.quantized_matmul(w, x.float().numpy(), dtype, m, n, k, acc=oracle.ACC_F64, threads=16)
+        rel = np.linalg.norm(y.float().cpu().numpy() - want) / np.linalg.norm(want)
+        assert rel <= element_bar(elem), f"m={m} n={n} k={k}: {rel}"
+
+
+@pytest.mark.parametrize("dtype", ALL)
+@pytest.mark.parametrize("m, elem", [(9, "float32"), (16, "bfloat16"), (33, "float16"), (100, "float32")])
+def test_projections_as_one_launch(torch, oracle, dtype, m, elem):
+    """Independent batch entries over the same rows: two and three of them (a fourth starts the next group), rows
+    that fill no tile, an entry that waits for the ones before it, one with other activations; entries that write
+    the same output stay apart and in order."""
+    from gllm_amd.backend import HipBackend
+    hip = HipBackend(0)
+    t, k = getattr(torch, elem), 1280
+    sizes = [300, 40, 257, 33, 256, 70]
+    host_x = [torch.from_numpy(random_activations(m, k, seed=s + m) * 1e-2).to(t) for s in (1, 2)]
+    xs = [x.cuda() for x in host_x]
+    which = [0, 0, 0, 0, 1, 1]
+    ws = [random_weight(dtype, n, k, seed=n) for n in sizes]
+    dev = [torch.from_numpy(w.view(np.uint8).reshape(-1)).cuda() for w in ws]
+    ys = [torch.full((m, n), float("nan"), dtype=t, device="cuda") for n in sizes]
+    entries = [(d, xs[i], y, dtype, m, n, k) for d, i, y, n in zip(dev, which, ys, sizes)]
+    print(f"group dtype={dtype} m={m} {elem}", flush=True)
+    hip.run_batch(hip.make_batch(entries, after_previous=lambda i: i == 2))
+    torch.cuda.synchronize()
+    for w, i, y, n in zip(ws, which, ys, sizes):
+        want = oracle.quantized_matmul(w, host_x[i].float().numpy(), dtype, m, n, k, acc=oracle.ACC_F64, threads=16)
+        rel = np.linalg.norm(y.float().cpu().numpy() - want) / np.linalg.norm(want)
+        assert rel <= element_bar(elem), f"n={n}: {rel}"
+    # the second writes over the first: not one launch, whose tiles would finish in any order
+    twice = torch.full((m, 300), float("nan"), dtype=t, device="cuda")
+    w2 = torch.from_numpy(random_weight(dtype, 300, k, seed=99).view(np.uint8).reshape(-1)).cuda()
+    alone = torch.full((m, 300), float("nan"), dtype=t, device="cuda")
+    hip.quantized_matmul(w2, xs[0], alone, dtype, m, 300, k)
+    hip.run_batch(hip.make_batch([(dev[0], xs[0], twice, dtype, m, 300, k), (w2, xs[0], twice, dtype, m, 300, k)]))
+    torch.cuda.synchronize()
+    assert torch.equal(twice, alone)
+
+
+def test_group_under_capture_keeps_to_the_reserved_scratch(torch):
+    """What was reserved entry by entry serves the captured batch; replays, with eager work between them, give the
+    eager results."""
+    from gllm_amd.backend import HipBackend
+    hip = HipBackend(0)
+    m, k, sizes = 24, 1024, [512, 128, 128]
+    x = torch.from_numpy(random_activations(m, k, seed=3)).cuda()
+    dev = [torch.from_numpy(random_weight(Q4_K, n, k, seed=n + i).view(np.uint8).reshape(-1)).cuda() for i, n in enumerate(sizes)]
+    ys = [torch.zeros(m, n, device="cuda") for n in sizes]
+    batch = hip.make_batch([(d, x, y, Q4_K, m, n, k) for d, y, n in zip(dev, ys, sizes)])
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        hip.reserve_matmul(Q4_K, m, max(sizes), k)
+        graph = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            hip.run_batch(batch)
+    torch.cuda.synchronize()
+    plain = HipBackend(0)
+    for trial in range(3):
+        x.copy_(torch.from_numpy(random_activations(m, k, seed=10 + trial)))
+        for y in ys:
+            y.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        for d, y, n in zip(dev, ys, sizes):
+            want = torch.zeros(m, n, device="cuda")
+            plain.quantized_matmul(d, x, want, Q4_K, m, n, k)
+            torch.cuda.synchronize()
+            # two orders of the same f32 sums
+            assert float((y - want).norm() / want.norm()) <= 1e-6
