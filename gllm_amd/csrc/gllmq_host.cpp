@@ -2792,7 +2792,11 @@ int gllmq_moe_route(gllmq_ctx *ctx, const float *logits, size_t tokens, size_t e
     if (cap > 1.0e9f) cap = 1.0e9f;
     P.capacity = static_cast<uint32_t>(cap);
     const uint32_t lds = static_cast<uint32_t>(((gq::ROUTE_WAVES + 1) * experts + 4) * 4);
-    if (tokens <= gq::ROUTE_FUSED_MAX_TOKENS) {
+    // A token chooses an expert once, so with room for every token in every expert nothing is dropped and the choices
+    // stand as phase 1 leaves them; phase 2 would only count.  (16 tokens of 128 experts: 7.7 us against 19.4; 512: 8
+    // against 24.)
+    const bool no_drop = P.capacity >= P.tokens && !route_pos && !expert_counts;
+    if (tokens <= gq::ROUTE_FUSED_MAX_TOKENS && !no_drop) {
         P.phases = 3u;
         return launch(ctx, ctx->moe_route, 1, gq::ROUTE_THREADS, lds, stream, &P, sizeof P);
     }
@@ -2800,7 +2804,7 @@ int gllmq_moe_route(gllmq_ctx *ctx, const float *logits, size_t tokens, size_t e
     const uint32_t grid = static_cast<uint32_t>(std::min<size_t>((tokens + gq::ROUTE_WAVES - 1) / gq::ROUTE_WAVES,
                                                                  static_cast<size_t>(ctx->num_cus) * 4));
     int rc = launch(ctx, ctx->moe_route, grid, gq::ROUTE_THREADS, lds, stream, &P, sizeof P);
-    if (rc != GLLMQ_OK) return rc;
+    if (rc != GLLMQ_OK || no_drop) return rc;
     P.phases = 2u;
     return launch(ctx, ctx->moe_route, 1, gq::ROUTE_THREADS, lds, stream, &P, sizeof P);
 }
@@ -2843,7 +2847,9 @@ int launch_moe_plan(gllmq_ctx *ctx, MoePlanParams &P, const uint32_t *route_expe
     // fewer than four, which share the rest of the work
     uint32_t waves = std::min<uint32_t>(gq::MOE_PLAN_THREADS / 64, std::max(4u, (P.pairs + 63u) / 64u));
     while (waves > 4u && (waves + 4u) * P.experts * 4u > 128u * 1024u) waves /= 2u;
-    return launch(ctx, ctx->moe_plan, 1, waves * 64u, ((waves + 4u) * P.experts + 16u) * 4u, stream, &P, sizeof P);
+    const uint64_t words = static_cast<uint64_t>(waves + 4u) * P.experts + 16u, with_pairs = words + 2ull * P.pairs;
+    P.in_lds = with_pairs * 4u <= 128u * 1024u ? 1u : 0u;
+    return launch(ctx, ctx->moe_plan, 1, waves * 64u, static_cast<uint32_t>(P.in_lds ? with_pairs : words) * 4u, stream, &P, sizeof P);
 }
 
 // ---- Many tokens per expert (prompts): the GEMM of mmfw.hip.inc over the experts' own rows

@@ -615,6 +615,7 @@ struct MoePlanParams {
     uint32_t *counters; // [0] jobs, [1] routed pairs, [2] matrix-core (or GEMM) jobs, [3] tiles of 32
     uint32_t tokens, top_k, experts, pairs;
     uint32_t job_rows;  // a matrix-core job takes up to that many tokens of an expert
+    uint32_t in_lds;    // the pairs' experts and the sorted order fit the LDS
 };
 
 constexpr uint32_t MOE_NONE = 0xFFFFFFFFu;

@@ -307,3 +307,27 @@ def test_moe_shapes_from_a_seeded_generator(hip, torch, oracle, seed):
         want = oracle.moe_ffn(gu, dt_gu, dn, dt_dn, x, hidden, ffn, experts, r["expert"], r["weight"], r["len"], relu_gate=relu)
         got = run_gpu(hip, torch, gu, dt_gu, dn, dt_dn, x, hidden, ffn, experts, *dev, relu_gate=relu, split=bool(i & 1))
         check_close(got, want, f"moe seeded {seed}/{i}")
+
+
+def test_plan_of_more_pairs_than_the_lds_holds(torch):
+    """16384 pairs are planned through memory, the two halves of the call in LDS: the same rows."""
+    from gllm_amd.backend import HipBackend
+    hip = HipBackend(0)
+    tokens, top_k, experts, hidden, ffn = 4096, 4, 6, 256, 256
+    rng = np.random.default_rng(3)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    gate_up = dev(random_weight(Q4_K, experts * 2 * ffn, hidden, seed=1).view(np.uint8).reshape(-1))
+    down = dev(random_weight(Q4_K, experts * hidden, ffn, seed=2).view(np.uint8).reshape(-1))
+    x = dev(random_activations(tokens, hidden, seed=3) * 1e-3)
+    expert = dev(np.stack([rng.permutation(experts)[:top_k] for _ in range(tokens)]).astype(np.int32))
+    weight = dev(rng.uniform(0.1, 1.0, (tokens, top_k)).astype(np.float32))
+    length = torch.full((tokens,), top_k, dtype=torch.int32, device="cuda")
+    got, want = torch.full((tokens, hidden), float("nan"), device="cuda"), torch.full((tokens, hidden), float("nan"), device="cuda")
+    hip.moe_matvec(gate_up, Q4_K, down, Q4_K, x, got, hidden, ffn, experts, expert, weight, length)
+    half = tokens // 2
+    for a in (0, half):
+        part = slice(a, a + half)
+        hip.moe_matvec(gate_up, Q4_K, down, Q4_K, x[part], want[part], hidden, ffn, experts, expert[part].contiguous(), weight[part].contiguous(), length[part].contiguous())
+    torch.cuda.synchronize()
+    # (a row's sums do not depend on the rows it is multiplied with, up to the small products' own accumulators)
+    assert float((got - want).norm() / want.norm()) <= 1e-6

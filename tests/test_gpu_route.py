@@ -148,3 +148,23 @@ def test_route_error_behaviour(hip, torch):
         hip.moe_route(lg, 2, re, rw, rl)  # more experts than this build routes
     with pytest.raises(OtherError):
         hip.moe_route(lg[:, :8].contiguous(), 2, re[:1], rw, rl)  # outputs too short
+
+
+def test_route_without_drops_and_without_places(hip, torch, oracle):
+    """Room for every token in every expert and nobody who asks for places or counts: the choices of the first phase
+    are the table.  One token, more choices than experts, more experts than registers hold, capacity exactly the tokens."""
+    rng = np.random.default_rng(11)
+    for tokens, experts, top_k in ((1, 4, 2), (7, 8, 2), (16, 128, 8), (33, 5, 9), (300, 600, 7), (65, 1, 1)):
+        print(f"route without drops tokens={tokens} experts={experts} top_k={top_k}", flush=True)
+        logits = rng.standard_normal((tokens, experts)).astype(np.float32)
+        logits[0, 0] = np.nan if tokens > 1 else logits[0, 0]
+        re = torch.full((tokens, top_k), -7, dtype=torch.int32, device="cuda")
+        rw = torch.full((tokens, top_k), 777.0, device="cuda")
+        rl, ov = torch.full((tokens,), -7, dtype=torch.int32, device="cuda"), torch.full((1,), -7, dtype=torch.int32, device="cuda")
+        hip.moe_route(torch.from_numpy(logits).cuda(), top_k, re, rw, rl, capacity_factor=float(experts), overflow=ov)
+        full = route(hip, torch, logits, top_k, float(experts))
+        torch.cuda.synchronize()
+        assert np.array_equal(re.cpu().numpy(), full["expert"].view(np.int32)) and int(ov[0]) == 0
+        assert np.array_equal(rw.cpu().numpy().view(np.uint32), np.ascontiguousarray(full["weight"]).view(np.uint32))
+        assert (rl.cpu().numpy() == min(top_k, experts)).all()
+        check_against_oracle(oracle, full, logits, top_k, float(experts), f"{tokens} {experts} {top_k}")
