@@ -307,6 +307,7 @@ struct gllmq_ctx {
     // streamed kernels whose workgroups share a row range and take a slice of K each (two to four
     // activation rows over few weight rows) [format][p1_e4, p2_e4][plain, gated activations]
     hipFunction_t mm8s_split[4][2][2] = {};
+    hipFunction_t mm8s_group[4][2] = {};        // several matrices over the same one or two rows [format, not Q6_K][p1_e1_a, p1_e2_a]
     bool mm8s_q8_0 = true;                      // "mm8s_q8_0" = 0: Q8_0 never takes the streamed form
     bool mm8s_split_on = true;                  // "mm8s_split" = 0: such shapes stay on the fetch-and-compute form
     bool mm8s_fold_on = true;                   // "mm8s_fold" = 0: such tiles go block by block, half of the matrix-core columns idle
@@ -649,7 +650,8 @@ int check_matmul_args(gllmq_ctx *ctx, const Format *f, const void *w, size_t w_b
 // `S` != null lets few weight rows under two to four rows of long activations share a row range
 // among workgroups, a slice of K each (the sums meet in S->mm8_part).
 int run_mm8s(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, float *y, size_t m, size_t n, size_t k,
-             bool act_bf16, void *stream, const uint8_t *w2 = nullptr, bool glu_relu = false, Scratch *S = nullptr)
+             bool act_bf16, void *stream, const uint8_t *w2 = nullptr, bool glu_relu = false, Scratch *S = nullptr,
+             gq::Mm8sGroupParams *group = nullptr)
 {
     const int kind = mm8_kind(f.dtype);
     const bool glu = w2 != nullptr;
@@ -693,8 +695,18 @@ int run_mm8s(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
     if (ksplit > 1 && !ctx->mm8s_all && ksplit * tiles * 4u < cus * 3u) ksplit = 1;
     const bool split = ksplit > 1;
     const uint32_t kslice = (groups + ksplit - 1u) / ksplit, lds_groups = split ? kslice : groups; // blocks a workgroup prepares
-    const uint32_t rows_per_wg = split ? 32u : static_cast<uint32_t>((n + cus - 1) / cus);
-    const uint32_t grid = static_cast<uint32_t>((n + rows_per_wg - 1) / rows_per_wg);
+    uint32_t rows_per_wg = split ? 32u : static_cast<uint32_t>((n + cus - 1) / cus);
+    uint32_t grid = static_cast<uint32_t>((n + rows_per_wg - 1) / rows_per_wg);
+    if (group) { // a workgroup's rows are of one matrix: the smallest share for which a workgroup per CU is enough
+        for (;; ++rows_per_wg) {
+            grid = 0;
+            for (uint32_t i = 0; i < group->segs; ++i) {
+                group->seg[i].first_wg = grid;
+                grid += (group->seg[i].n + rows_per_wg - 1u) / rows_per_wg;
+            }
+            if (grid <= cus) break;
+        }
+    }
     const uint32_t wg_tiles = (rows_per_wg + 31u) / 32u, tile_rows = (rows_per_wg + wg_tiles - 1u) / wg_tiles;
     // One activation row over tiles of at most 16 weight rows: an item is a pair of blocks of the
     // tile, so that all 32 columns of the matrix cores carry weights (14336 -> 4096 is bound by the
@@ -822,6 +834,11 @@ int run_mm8s(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
     P.progress = ctx->call_seq && ctx->prefetch_announce ? ctx->progress : nullptr;
     P.progress_seq = ctx->call_seq;
     const uint32_t lds = L.total;
+    if (group) {
+        if (split || fold || !areg || variant > 1 || sfmt == 2 || act_bf16) return -1;
+        group->p = P;
+        return launch(ctx, ctx->mm8s_group[sfmt][variant], grid, (gq::MM8S_CWAVES + gq::MM8S_LOADERS) * 64, lds, stream, group, sizeof *group, false);
+    }
     if (split) {
         P.ksplit = ksplit;
         P.kslice_groups = kslice;
@@ -1913,6 +1930,11 @@ int gllmq_init(gllmq_ctx **out, int device)
                 snprintf(name, sizeof name, "gq_mm8s_%s_p%d_e4%s_s", kMm8sFormat[q], 1 + (v & 1), (v & 2) ? "_g" : "");
                 rc = get_function(ctx, &ctx->mm8s_split[q][v & 1][v >> 1], name);
             }
+        for (int q = 0; q < 4; ++q)
+            for (int v = 0; v < 2 && rc == GLLMQ_OK && q != 2; ++v) {
+                snprintf(name, sizeof name, "gq_mm8s_%s_p1_e%d_a_q", kMm8sFormat[q], v + 1);
+                rc = get_function(ctx, &ctx->mm8s_group[q][v], name);
+            }
         static const char *const kMm8sGlu[4] = { "p1_e2_g", "p2_e4_g", "p1_e4_g", "p4_e4_g" };
         for (int q = 0; q < 4; ++q)
             for (int v = 0; v < 4 && rc == GLLMQ_OK; ++v) {
@@ -1925,6 +1947,7 @@ int gllmq_init(gllmq_ctx **out, int device)
         auto add = [&](hipFunction_t f) { if (f) ctx->announces.insert(f); };
         for (auto &q : ctx->mm8s) for (hipFunction_t f : q) add(f);
         for (auto &q : ctx->mm8s_gated) for (hipFunction_t f : q) add(f);
+        for (auto &q : ctx->mm8s_group) for (hipFunction_t f : q) add(f);
         for (auto &q : ctx->mm8s_e16) for (hipFunction_t f : q) add(f);
         for (auto &q : ctx->mm8s_glu) for (hipFunction_t f : q) add(f);
         for (auto &q : ctx->mm8s_fold) for (hipFunction_t f : q) add(f);
@@ -2710,7 +2733,28 @@ int gllmq_quantized_matmul_batch(gllmq_ctx *ctx, const gllmq_matmul_desc *descs,
         // consecutive one-row matmuls of one kind run as one launch whose weight stream never stops
         const size_t chain = chain_length(ctx, descs + i, count - i);
         if (chain >= 2) {
-            const int crc = run_chain(ctx, *S, descs + i, chain, stream);
+            int crc = -1;
+            bool same_x = ctx->batch_group && chain <= static_cast<size_t>(gq::MM8S_MAX_SEGS);
+            for (size_t j = 0; j < chain && same_x; ++j) {
+                const gllmq_matmul_desc &e = descs[i + j];
+                same_x = e.x_dev == d.x_dev && (j == 0 || !(e.flags & GLLMQ_DESC_AFTER_PREVIOUS)) && !ranges_meet(e.y_dev, e.m * e.n * 4, e.x_dev, e.m * e.k * 4);
+                for (size_t o = 0; o < j; ++o) same_x = same_x && !ranges_meet(e.y_dev, e.m * e.n * 4, descs[i + o].y_dev, e.m * descs[i + o].n * 4);
+            }
+            if (same_x) { // Q, K and V (or gate and up): one streamed launch over their rows
+                gq::Mm8sGroupParams G{};
+                G.segs = static_cast<uint32_t>(chain);
+                size_t rows = 0;
+                for (size_t j = 0; j < chain; ++j) {
+                    G.seg[j] = gq::Mm8sSeg{ static_cast<const uint8_t *>(descs[i + j].w_dev), descs[i + j].y_dev, static_cast<uint32_t>(descs[i + j].n), 0u };
+                    rows += descs[i + j].n;
+                }
+                ctx->overlap.entry_first = !(d.flags & GLLMQ_DESC_AFTER_PREVIOUS);
+                if (rows <= 0x7FFFFFFFu)
+                    crc = run_mm8s(ctx, *find_format(d.ggml_dtype), G.seg[0].w, d.x_dev, d.y_dev, d.m, rows, d.k, false, stream, nullptr, false, nullptr, &G);
+                if (crc < 0) crc = -1;
+                ctx->overlap.entry_first = false;
+            }
+            if (crc < 0) crc = run_chain(ctx, *S, descs + i, chain, stream);
             if (crc >= 0) {
                 rc = crc;
                 ctx->overlap = gllmq_ctx::Overlap{};

@@ -83,6 +83,20 @@ struct Mm8Params {
     unsigned long long progress_seq;
 };
 
+// Several weight matrices over the same activations in one streamed launch: the row ranges of a matrix are
+// those of workgroups first_wg .. up to the next matrix's; p.w, p.y, p.n and p.ldy are each workgroup's own.
+constexpr int MM8S_MAX_SEGS = 3;
+struct Mm8sSeg {
+    const uint8_t *w;
+    float *y;
+    uint32_t n, first_wg;
+};
+struct Mm8sGroupParams {
+    Mm8Params p;
+    Mm8sSeg seg[MM8S_MAX_SEGS];
+    uint32_t segs;
+};
+
 // The weight prefetch that runs beside a sequence of dependent launches (touch.hip.inc): for each
 // entry, in order, wait until launch number `seq - 1` of the context has started (`progress`, see
 // Mm8Params), then pull the entry's bytes into the memory-side cache by reading one word of every

@@ -333,3 +333,34 @@ def test_open_requests_per_loader_change_no_bit(torch, dtype, m):
     for depth, out in enumerate(outs[1:], 1):
         for i in range(len(ns)):
             assert np.array_equal(out[i].view(np.uint32), outs[0][i].view(np.uint32)), f"entry {i}, depth {depth}"
+
+
+@pytest.mark.parametrize("dtype,m", [(Q4_K, 1), (Q5_K, 1), (Q8_0, 1), (Q4_K, 2), (Q5_K, 2), (Q8_0, 2)])
+def test_two_or_three_matrices_over_the_same_rows(torch, oracle, dtype, m):
+    """Q, K and V (or gate and up) as one streamed launch: row ranges that end inside a matrix, a last range of
+    one row, matrices of fewer rows than a range; short rows; outputs in one buffer side by side.  Entries that
+    write the same output, one after the other, go on as a chain."""
+    from gllm_amd.backend import HipBackend
+    hip = HipBackend(0)
+    c = cus(torch)
+    seen = set()
+    for k, ns in ((4096, [16 * c, 4 * c, 4 * c]), (4096, [17 * c + 1, 5 * c + 7]), (2048, [24 * c, c // 2, 8 * c + 1]), (264 if dtype != Q8_0 else 288, [7 * c, 6 * c, 3 * c]),
+                  (1024, [56 * c + 3, 56 * c + 3])):
+        print(f"group dtype={dtype} m={m} k={k} ns={ns}", flush=True)
+        host = [random_weight(dtype, n, k, seed=60 + i) for i, n in enumerate(ns)]
+        x_host = random_activations(m, k, seed=70)
+        x = torch.from_numpy(x_host).cuda()
+        y = torch.full((m * sum(ns) + 64,), 7.0, device="cuda")
+        y[:m * sum(ns)] = float("nan")
+        at = np.cumsum([0] + [m * n for n in ns])
+        entries = [(dev_weight(torch, w), x, y[a:b].view(m, n), dtype, m, n, k) for w, n, a, b in zip(host, ns, at, at[1:])]
+        run_batch(hip, torch, entries, after_previous=None)
+        seen.add(hip.last_kernel_name())
+        assert bool((y[m * sum(ns):] == 7.0).all())
+        for w, n, e in zip(host, ns, entries):
+            want = oracle.quantized_matmul(w, x_host, dtype, m, n, k, acc=oracle.ACC_F64, threads=16)
+            check_close(e[2].cpu().numpy(), want, f"k={k} n={n}")
+        twice = [entries[0], (entries[0][0], x, entries[0][2], dtype, m, ns[0], k)]
+        run_batch(hip, torch, twice, after_previous=None)
+        assert not hip.last_kernel_name().endswith("_q")
+    assert any(name.endswith("_q") for name in seen), seen
