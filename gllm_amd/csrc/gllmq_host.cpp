@@ -307,7 +307,7 @@ struct gllmq_ctx {
     // streamed kernels whose workgroups share a row range and take a slice of K each (two to four
     // activation rows over few weight rows) [format][p1_e4, p2_e4][plain, gated activations]
     hipFunction_t mm8s_split[4][2][2] = {};
-    hipFunction_t mm8s_group[4][2] = {};        // several matrices over the same one or two rows [format, not Q6_K][p1_e1_a, p1_e2_a]
+    hipFunction_t mm8s_group[4][2][3] = {};     // several matrices over the same rows [format, not Q6_K][f32, 16-bit][p1_e1_a, p1_e2_a, p2_e4_a]
     bool mm8s_q8_0 = true;                      // "mm8s_q8_0" = 0: Q8_0 never takes the streamed form
     bool mm8s_split_on = true;                  // "mm8s_split" = 0: such shapes stay on the fetch-and-compute form
     bool mm8s_fold_on = true;                   // "mm8s_fold" = 0: such tiles go block by block, half of the matrix-core columns idle
@@ -835,9 +835,9 @@ int run_mm8s(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
     P.progress_seq = ctx->call_seq;
     const uint32_t lds = L.total;
     if (group) {
-        if (split || fold || !areg || variant > 1 || sfmt == 2 || act_bf16) return -1;
+        if (split || fold || !areg || variant > 2 || sfmt == 2 || act_bf16) return -1;
         group->p = P;
-        return launch(ctx, ctx->mm8s_group[sfmt][variant], grid, (gq::MM8S_CWAVES + gq::MM8S_LOADERS) * 64, lds, stream, group, sizeof *group, false);
+        return launch(ctx, ctx->mm8s_group[sfmt][ctx->call_elem ? 1 : 0][variant], grid, (gq::MM8S_CWAVES + gq::MM8S_LOADERS) * 64, lds, stream, group, sizeof *group, false);
     }
     if (split) {
         P.ksplit = ksplit;
@@ -1931,9 +1931,10 @@ int gllmq_init(gllmq_ctx **out, int device)
                 rc = get_function(ctx, &ctx->mm8s_split[q][v & 1][v >> 1], name);
             }
         for (int q = 0; q < 4; ++q)
-            for (int v = 0; v < 2 && rc == GLLMQ_OK && q != 2; ++v) {
-                snprintf(name, sizeof name, "gq_mm8s_%s_p1_e%d_a_q", kMm8sFormat[q], v + 1);
-                rc = get_function(ctx, &ctx->mm8s_group[q][v], name);
+            for (int v = 0; v < 6 && rc == GLLMQ_OK && q != 2; ++v) {
+                static const char *const kGroup[3] = { "p1_e1_a", "p1_e2_a", "p2_e4_a" };
+                snprintf(name, sizeof name, "gq_mm8s_%s_%s%s_q", kMm8sFormat[q], kGroup[v % 3], v >= 3 ? "_e16" : "");
+                rc = get_function(ctx, &ctx->mm8s_group[q][v / 3][v % 3], name);
             }
         static const char *const kMm8sGlu[4] = { "p1_e2_g", "p2_e4_g", "p1_e4_g", "p4_e4_g" };
         for (int q = 0; q < 4; ++q)
@@ -1947,7 +1948,7 @@ int gllmq_init(gllmq_ctx **out, int device)
         auto add = [&](hipFunction_t f) { if (f) ctx->announces.insert(f); };
         for (auto &q : ctx->mm8s) for (hipFunction_t f : q) add(f);
         for (auto &q : ctx->mm8s_gated) for (hipFunction_t f : q) add(f);
-        for (auto &q : ctx->mm8s_group) for (hipFunction_t f : q) add(f);
+        for (auto &q : ctx->mm8s_group) for (auto &e : q) for (hipFunction_t f : e) add(f);
         for (auto &q : ctx->mm8s_e16) for (hipFunction_t f : q) add(f);
         for (auto &q : ctx->mm8s_glu) for (hipFunction_t f : q) add(f);
         for (auto &q : ctx->mm8s_fold) for (hipFunction_t f : q) add(f);
@@ -2594,15 +2595,16 @@ int batch_entry(gllmq_ctx *ctx, Scratch &S, const gllmq_matmul_desc &d, void *st
     return matmul_on_scratch(ctx, S, d.w_dev, d.w_bytes, d.x_dev, d.y_dev, d.ggml_dtype, d.m, d.n, d.k, GLLMQ_ACT_F32_SPLIT, stream);
 }
 
-// Entries from `descs` on that one GEMM launch can multiply: independent matmuls of one format over the same 9 or
-// more activation rows (a layer's Q, K and V projections).  0 or 1: none.
+// Entries from `descs` on that one launch can multiply: independent matmuls of one format over the same
+// activation rows (a layer's Q, K and V projections), 9 and more for the GEMM, up to four for the streamed
+// kernels.  0 or 1: none.
 size_t group_length(const gllmq_ctx *ctx, const gllmq_matmul_desc *descs, size_t count)
 {
     constexpr uint32_t kElemBits = GLLMQ_DESC_ELEM_F16 | GLLMQ_DESC_ELEM_BF16;
     const gllmq_matmul_desc &first = descs[0];
     const uint32_t elem = first.flags & kElemBits;
-    if (count < 2 || !ctx->batch_group || ctx->mmfs_all || first.m < std::max(9u, std::min(ctx->mmfw_min_m, ctx->mmfw_small_min_m)) ||
-        first.k == 0 || !first.x_dev || elem == kElemBits || (elem && !elem_in_kernel(ctx, first.m, first.k)))
+    if (count < 2 || !ctx->batch_group || first.m == 0 || (first.m <= 4 && !ctx->use_chain) || // (option "chain" off: a streamed launch per entry)
+        (first.m > 4 && (ctx->mmfs_all || first.m < std::max(9u, std::min(ctx->mmfw_min_m, ctx->mmfw_small_min_m)))) || first.k == 0 || !first.x_dev || elem == kElemBits || (elem && !elem_in_kernel(ctx, first.m, first.k)))
         return 0;
     const size_t e = elem ? 2 : 4;
     size_t len = 0;
@@ -2620,7 +2622,7 @@ size_t group_length(const gllmq_ctx *ctx, const gllmq_matmul_desc *descs, size_t
     return len;
 }
 
-// The group as one GEMM.  -1: its entries go through the dispatch one by one (which also reports what is wrong with them).
+// The group as one launch.  -1: its entries go through the dispatch one by one (which also reports what is wrong with them).
 int run_group(gllmq_ctx *ctx, Scratch &S, const gllmq_matmul_desc *descs, size_t len, void *stream)
 {
     const gllmq_matmul_desc &first = descs[0];
@@ -2637,6 +2639,20 @@ int run_group(gllmq_ctx *ctx, Scratch &S, const gllmq_matmul_desc *descs, size_t
         n[i] = d.n;
     }
     const uint32_t elem = (first.flags & GLLMQ_DESC_ELEM_F16) ? GLLMQ_ELEM_F16 : (first.flags & GLLMQ_DESC_ELEM_BF16) ? GLLMQ_ELEM_BF16 : 0u;
+    if (first.m <= 4) {
+        gq::Mm8sGroupParams G{};
+        G.segs = static_cast<uint32_t>(len);
+        size_t rows = 0;
+        for (size_t i = 0; i < len; ++i) {
+            G.seg[i] = gq::Mm8sSeg{ mats[i].w, mats[i].y, static_cast<uint32_t>(n[i]), 0u };
+            rows += n[i];
+        }
+        if (rows > 0x7FFFFFFFu || !ctx->use_mm8 || !ctx->use_mm8s) return -1;
+        ctx->call_elem = elem;
+        const int rc = run_mm8s(ctx, *f, G.seg[0].w, first.x_dev, first.y_dev, first.m, rows, first.k, false, stream, nullptr, false, nullptr, &G);
+        ctx->call_elem = 0;
+        return rc;
+    }
     const MmfwPlan L = plan_mmfw(ctx, first.ggml_dtype, first.m, n, static_cast<int>(len), first.k, elem != 0, S.fixed ? S.mmf_bytes : SIZE_MAX);
     if (!L.ok || !mmfw_scratch_ok(ctx, S, L, stream)) return -1;
     return run_mmfw(ctx, S, *f, mats, static_cast<int>(len), first.x_dev, elem, elem, first.m, first.k, false, stream, 9);
@@ -2734,24 +2750,9 @@ int gllmq_quantized_matmul_batch(gllmq_ctx *ctx, const gllmq_matmul_desc *descs,
         const size_t chain = chain_length(ctx, descs + i, count - i);
         if (chain >= 2) {
             int crc = -1;
-            bool same_x = ctx->batch_group && chain <= static_cast<size_t>(gq::MM8S_MAX_SEGS);
-            for (size_t j = 0; j < chain && same_x; ++j) {
-                const gllmq_matmul_desc &e = descs[i + j];
-                same_x = e.x_dev == d.x_dev && (j == 0 || !(e.flags & GLLMQ_DESC_AFTER_PREVIOUS)) && !ranges_meet(e.y_dev, e.m * e.n * 4, e.x_dev, e.m * e.k * 4);
-                for (size_t o = 0; o < j; ++o) same_x = same_x && !ranges_meet(e.y_dev, e.m * e.n * 4, descs[i + o].y_dev, e.m * descs[i + o].n * 4);
-            }
-            if (same_x) { // Q, K and V (or gate and up): one streamed launch over their rows
-                gq::Mm8sGroupParams G{};
-                G.segs = static_cast<uint32_t>(chain);
-                size_t rows = 0;
-                for (size_t j = 0; j < chain; ++j) {
-                    G.seg[j] = gq::Mm8sSeg{ static_cast<const uint8_t *>(descs[i + j].w_dev), descs[i + j].y_dev, static_cast<uint32_t>(descs[i + j].n), 0u };
-                    rows += descs[i + j].n;
-                }
+            if (chain <= static_cast<size_t>(gq::MMFW_MAX_SEGS) && group_length(ctx, descs + i, chain) == chain) { // Q, K and V, or gate and up
                 ctx->overlap.entry_first = !(d.flags & GLLMQ_DESC_AFTER_PREVIOUS);
-                if (rows <= 0x7FFFFFFFu)
-                    crc = run_mm8s(ctx, *find_format(d.ggml_dtype), G.seg[0].w, d.x_dev, d.y_dev, d.m, rows, d.k, false, stream, nullptr, false, nullptr, &G);
-                if (crc < 0) crc = -1;
+                crc = run_group(ctx, *S, descs + i, chain, stream);
                 ctx->overlap.entry_first = false;
             }
             if (crc < 0) crc = run_chain(ctx, *S, descs + i, chain, stream);
@@ -2763,7 +2764,7 @@ int gllmq_quantized_matmul_batch(gllmq_ctx *ctx, const gllmq_matmul_desc *descs,
                 continue;
             }
         }
-        const size_t group = group_length(ctx, descs + i, count - i);
+        const size_t group = chain >= 2 ? 0 : group_length(ctx, descs + i, count - i);
         if (group >= 2) {
             ctx->overlap.entry_first = !(d.flags & GLLMQ_DESC_AFTER_PREVIOUS);
             const int grc = run_group(ctx, *S, descs + i, group, stream);

@@ -364,3 +364,28 @@ def test_two_or_three_matrices_over_the_same_rows(torch, oracle, dtype, m):
         run_batch(hip, torch, twice, after_previous=None)
         assert not hip.last_kernel_name().endswith("_q")
     assert any(name.endswith("_q") for name in seen), seen
+
+
+@pytest.mark.parametrize("dtype", [Q4_K, Q5_K, Q8_0])
+@pytest.mark.parametrize("m,elem", [(1, "bfloat16"), (2, "float16"), (3, "float32"), (4, "bfloat16"), (4, "float32")])
+def test_matrices_over_the_same_rows_of_any_element_type(torch, oracle, dtype, m, elem):
+    """The same for 16-bit elements and three and four rows; a fourth entry and one that waits start a launch of
+    their own, entries over other activations too."""
+    from gllm_amd.backend import HipBackend
+    hip = HipBackend(0)
+    c, t = cus(torch), getattr(torch, elem)
+    k, ns, which = 1280, [17 * c + 3, 4 * c, 5 * c + 1, 9 * c, 8 * c, 8 * c], [0, 0, 0, 0, 0, 1]
+    x_host = [torch.from_numpy(random_activations(m, k, seed=70 + i) * 1e-2).to(t) for i in range(2)]
+    xs = [x.cuda() for x in x_host]
+    ws = [random_weight(dtype, n, k, seed=60 + i) for i, n in enumerate(ns)]
+    ys = [torch.full((m, n), float("nan"), dtype=t, device="cuda") for n in ns]
+    print(f"group dtype={dtype} m={m} {elem}", flush=True)
+    entries = [(dev_weight(torch, w), xs[i], y, dtype, m, n, k) for w, i, y, n in zip(ws, which, ys, ns)]
+    run_batch(hip, torch, entries, after_previous=lambda i: i == 4)
+    for w, i, y, n in zip(ws, which, ys, ns):
+        want = oracle.quantized_matmul(w, x_host[i].float().numpy(), dtype, m, n, k, acc=oracle.ACC_F64, threads=16)
+        rel = np.linalg.norm(y.float().cpu().numpy() - want) / np.linalg.norm(want)
+        # the output's rounding: 2^-11, 2^-9 of a value at most
+        assert rel <= {"float32": 1e-5, "float16": 1e-3, "bfloat16": 5e-3}[elem], f"n={n}: {rel}"
+    run_batch(hip, torch, entries[:3], after_previous=None)
+    assert hip.last_kernel_name().endswith("_q"), hip.last_kernel_name()
