@@ -88,6 +88,8 @@ const char *gllmq_version(void);
  * Supported (kept stable):
  *   "weights_cache_mib"  MiB of uploaded weights the host-slice calls keep (default 65536)
  *   "chain"              0: every entry of a batch is a launch of its own (default 1)
+ *   "batch_group"        0: independent entries of a batch over the same activations are
+ *                        not multiplied by one launch (default 1)
  *   "batch_overlap"      0: the kernels of a batch run strictly one after the other (default 1)
  *   "ffn_fused"          0: the feed-forward block as separate products (default 1)
  *   "chain_dependent"    1: an entry whose activations are the output of the entry before it stays
