@@ -1598,6 +1598,17 @@ int run_gemv(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
     return GLLMQ_OK;
 }
 
+// Whether 5 to 8 activation rows go to the wide GEMM.  The int8 kernels take up to eight rows of Q4_K, seven of Q5_K and
+// six of Q6_K and Q8_0 in a pass, and read the weights twice beyond that.  f32, us per call on 4096 x 14336: Q8_0 six rows
+// 24.0 (28.5 here), seven 31.6 (28.6), Q6_K seven 30.4 (27.4), Q5_K eight 26.3 (22.1); 16-bit activations, which the
+// GEMM takes as one plane, five rows 27.5 (25.8), 26.4 (26.3), 22.2 (20.7), Q4_K 21.1 (19.4).  Single matmuls of shorter
+// rows stay: 14336 x 4096 the same either way, 4096 x 4096 five rows 9.7 (15.2).
+bool mmfw_takes_few(const gllmq_ctx *ctx, uint32_t dtype, size_t m, bool one_plane)
+{
+    const size_t pass = dtype == T_Q4_K ? 8 : dtype == T_Q5_K ? 7 : 6;
+    return ctx->mmfw_small_min_m <= 9 && m >= 5 && (one_plane || m > pass);
+}
+
 // One quantized matmul on validated arguments: the kernel family by format, rows and shape.
 int dispatch_matmul(gllmq_ctx *ctx, Scratch &S, const Format &f, const uint8_t *w, const float *x, float *y, size_t m,
                     size_t n, size_t k, bool bf16, void *stream)
@@ -1616,9 +1627,9 @@ int dispatch_matmul(gllmq_ctx *ctx, Scratch &S, const Format &f, const uint8_t *
     // 32 bf16 rows against run_mmf's: Q6_K 14336 x 4096 24.7, 26.0 (27.7, 29.0), 4096 x 4096 18.8, 20.9 (21.3, 22.3);
     // Q8_0 14336 x 4096 24.9, 27.0 (33.0, 34.3); Q4_K 4096 x 14336 19.5, 20.8 (22.2, 22.3), 1024 x 4096 the same.
     // f32, 32 rows, Q4_K 14336 x 4096 21.2 (20.9).
-    if (!ctx->mmfs_all) {
+    if (!ctx->mmfs_all && (m >= ctx->mmfw_small_min_m || (!bf16 && k > 10240 && mmfw_takes_few(ctx, f.dtype, m, ctx->call_elem && !ctx->call_glu)))) {
         const MmfwMatrix one{ w, y, n };
-        rc = run_mmfw(ctx, S, f, &one, 1, x, ctx->call_elem, ctx->call_elem, m, k, bf16, stream, std::max(9u, ctx->mmfw_small_min_m));
+        rc = run_mmfw(ctx, S, f, &one, 1, x, ctx->call_elem, ctx->call_elem, m, k, bf16, stream, 5);
         if (rc >= 0 || rc == kNeedPlainActivations) return rc;
     }
     rc = run_mmf(ctx, S, f, w, x, y, m, n, k, bf16, stream);
@@ -2369,7 +2380,8 @@ int ffn_on_stream(gllmq_ctx *ctx, const void *gate_w, const void *up_w, size_t g
     // Prompts and larger batches: gate and up share their activation images and run as one launch; the
     // down projection's images are prepared from the two results.
     const size_t gate_up_n[2] = { ffn, ffn };
-    const uint32_t wide_min = std::max(9u, std::min(ctx->mmfw_min_m, ctx->mmfw_small_min_m));
+    const bool wide = m >= std::max(5u, std::min(ctx->mmfw_min_m, ctx->mmfw_small_min_m)) ||
+                      (ctx->ffn_fused && mmfw_takes_few(ctx, dtype_gate_up, m, elem != 0)); // ("ffn_fused" off: up to 8 rows in separate steps)
     auto down_fits = [&] {
         const MmfwPlan L = plan_mmfw(ctx, dtype_down, m, &hidden, 1, ffn, false, S.fixed ? S.mmf_bytes : SIZE_MAX);
         return L.ok && mmfw_scratch_ok(ctx, S, L, stream);
@@ -2378,9 +2390,9 @@ int ffn_on_stream(gllmq_ctx *ctx, const void *gate_w, const void *up_w, size_t g
         const MmfwPlan L = plan_mmfw(ctx, dtype_gate_up, m, gate_up_n, 2, hidden, elem != 0, S.fixed ? S.mmf_bytes : SIZE_MAX);
         return L.ok && mmfw_scratch_ok(ctx, S, L, stream);
     };
-    if (m >= wide_min && !ctx->mmfs_all && ffn % 4 == 0 && m * ffn <= 0xFFFFFFFFull && down_fits() && gate_up_fits()) {
+    if (wide && !ctx->mmfs_all && ffn % 4 == 0 && m * ffn <= 0xFFFFFFFFull && down_fits() && gate_up_fits()) {
         const MmfwMatrix gate_up[2] = { { gw, gu, ffn }, { uw, gu + m * ffn, ffn } };
-        rc = run_mmfw(ctx, S, *fg, gate_up, 2, x, elem, 0, m, hidden, false, stream, wide_min);
+        rc = run_mmfw(ctx, S, *fg, gate_up, 2, x, elem, 0, m, hidden, false, stream, 5);
         if (rc > 0) return rc;
         if (rc == GLLMQ_OK) {
             const MmfwMatrix down{ static_cast<const uint8_t *>(down_w), out, hidden };
@@ -2388,7 +2400,7 @@ int ffn_on_stream(gllmq_ctx *ctx, const void *gate_w, const void *up_w, size_t g
                 ctx->call_glu = relu_gate ? 2u : 1u;
                 ctx->call_glu_off = static_cast<uint32_t>(m * ffn);
                 ctx->call_ldx = static_cast<uint32_t>(ffn);
-                rc = run_mmfw(ctx, S, *fd, &down, 1, gu, 0, elem, m, ffn, false, stream, wide_min);
+                rc = run_mmfw(ctx, S, *fd, &down, 1, gu, 0, elem, m, ffn, false, stream, 5);
                 ctx->call_glu = ctx->call_glu_off = ctx->call_ldx = 0;
             } else {
                 gq::GluActParams A{};
@@ -2400,7 +2412,7 @@ int ffn_on_stream(gllmq_ctx *ctx, const void *gate_w, const void *up_w, size_t g
                 A.relu_gate = relu_gate ? 1u : 0u;
                 rc = launch2d(ctx, ctx->glu_act, static_cast<uint32_t>((ffn + 255) / 256),
                               static_cast<uint32_t>(std::min<size_t>(m, 65535)), 256, 0, stream, &A, sizeof A);
-                if (rc == GLLMQ_OK) rc = run_mmfw(ctx, S, *fd, &down, 1, h, 0, elem, m, ffn, false, stream, wide_min);
+                if (rc == GLLMQ_OK) rc = run_mmfw(ctx, S, *fd, &down, 1, h, 0, elem, m, ffn, false, stream, 5);
             }
             return rc >= 0 ? rc : fail(ctx, GLLMQ_ERR_BAD_SHAPE, "ffn_swiglu: the down projection has no kernel for this shape");
         }
@@ -2596,15 +2608,15 @@ int batch_entry(gllmq_ctx *ctx, Scratch &S, const gllmq_matmul_desc &d, void *st
 }
 
 // Entries from `descs` on that one launch can multiply: independent matmuls of one format over the same
-// activation rows (a layer's Q, K and V projections), 9 and more for the GEMM, up to four for the streamed
-// kernels.  0 or 1: none.
+// activation rows (a layer's Q, K and V projections), five and more for the GEMM (4096 + 1024 + 1024 rows of 4096 Q4_K,
+// f32, five rows 18 us against 28 one by one), up to four for the streamed kernels.  0 or 1: none.
 size_t group_length(const gllmq_ctx *ctx, const gllmq_matmul_desc *descs, size_t count)
 {
     constexpr uint32_t kElemBits = GLLMQ_DESC_ELEM_F16 | GLLMQ_DESC_ELEM_BF16;
     const gllmq_matmul_desc &first = descs[0];
     const uint32_t elem = first.flags & kElemBits;
     if (count < 2 || !ctx->batch_group || first.m == 0 || (first.m <= 4 && !ctx->use_chain) || // (option "chain" off: a streamed launch per entry)
-        (first.m > 4 && (ctx->mmfs_all || first.m < std::max(9u, std::min(ctx->mmfw_min_m, ctx->mmfw_small_min_m)))) || first.k == 0 || !first.x_dev || elem == kElemBits || (elem && !elem_in_kernel(ctx, first.m, first.k)))
+        (first.m > 4 && (ctx->mmfs_all || (first.m < std::min(ctx->mmfw_min_m, ctx->mmfw_small_min_m) && ctx->mmfw_small_min_m > 9))) || first.k == 0 || !first.x_dev || elem == kElemBits || (elem && !elem_in_kernel(ctx, first.m, first.k)))
         return 0;
     const size_t e = elem ? 2 : 4;
     size_t len = 0;
@@ -2655,7 +2667,7 @@ int run_group(gllmq_ctx *ctx, Scratch &S, const gllmq_matmul_desc *descs, size_t
     }
     const MmfwPlan L = plan_mmfw(ctx, first.ggml_dtype, first.m, n, static_cast<int>(len), first.k, elem != 0, S.fixed ? S.mmf_bytes : SIZE_MAX);
     if (!L.ok || !mmfw_scratch_ok(ctx, S, L, stream)) return -1;
-    return run_mmfw(ctx, S, *f, mats, static_cast<int>(len), first.x_dev, elem, elem, first.m, first.k, false, stream, 9);
+    return run_mmfw(ctx, S, *f, mats, static_cast<int>(len), first.x_dev, elem, elem, first.m, first.k, false, stream, 5);
 }
 
 // The launches a batch will make, and which of them get their weights prefetched: an ordered

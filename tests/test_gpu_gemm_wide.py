@@ -233,3 +233,43 @@ def test_group_under_capture_keeps_to_the_reserved_scratch(torch):
             torch.cuda.synchronize()
             # two orders of the same f32 sums
             assert float((y - want).norm() / want.norm()) <= 1e-6
+
+
+@pytest.mark.parametrize("dtype", ALL)
+def test_five_to_eight_rows(torch, oracle, dtype):
+    """Long rows of more activation rows than one pass of the int8 kernels takes, and of any five in 16 bits; a group of
+    projections, and the feed-forward block, of as many rows."""
+    from gllm_amd.backend import HipBackend
+    hip = HipBackend(0)
+    passes = {Q4_K: 8, Q5_K: 7, Q6_K: 6, Q8_0: 6}[dtype]
+    n, k = 300, 10240 + 256
+    w = random_weight(dtype, n, k, seed=5)
+    wd = torch.from_numpy(w.view(np.uint8).reshape(-1)).cuda()
+    for elem in ("float32", "bfloat16"):
+        t = getattr(torch, elem)
+        for m in (4, 5, 6, 7, 8):
+            print(f"few rows dtype={dtype} {elem} m={m}", flush=True)
+            x = torch.from_numpy(random_activations(m, k, seed=m) * 1e-2).to(t)
+            y = torch.full((m, n), float("nan"), dtype=t, device="cuda")
+            hip.quantized_matmul(wd, x.cuda(), y, dtype, m, n, k)
+            wide = m >= 5 if elem == "bfloat16" else m > passes
+            assert (hip.last_kernel_name() == "gq_mmf_reduce" or "_w1" in hip.last_kernel_name()) == wide, hip.last_kernel_name()
+            want = oracle.quantized_matmul(w, x.float().numpy(), dtype, m, n, k, acc=oracle.ACC_F64, threads=16)
+            rel = np.linalg.norm(y.float().cpu().numpy() - want) / np.linalg.norm(want)
+            assert rel <= element_bar(elem), f"m={m}: {rel}"
+            hidden, ffn = 512, 768
+            g, u, d = (random_weight(dtype, a, b, seed=i) for i, (a, b) in enumerate(((ffn, hidden), (ffn, hidden), (hidden, ffn))))
+            xf = torch.from_numpy(random_activations(m, hidden, seed=m) * 1e-2).to(t)
+            out = torch.full((m, hidden), float("nan"), dtype=t, device="cuda")
+            dev = [torch.from_numpy(a.view(np.uint8).reshape(-1)).cuda() for a in (g, u, d)]
+            hip.ffn_swiglu(dev[0], dev[1], dtype, dev[2], dtype, xf.cuda(), out, m, hidden, ffn)
+            want = oracle.ffn_swiglu(g, u, dtype, d, dtype, xf.float().numpy(), m, hidden, ffn, acc=oracle.ACC_F64, threads=16)
+            rel = np.linalg.norm(out.float().cpu().numpy() - want.reshape(m, hidden)) / np.linalg.norm(want)
+            assert rel <= element_bar(elem), f"ffn m={m}: {rel}"
+            ys = [torch.full((m, r), float("nan"), dtype=t, device="cuda") for r in (ffn, ffn)]
+            xg = xf.cuda()
+            hip.run_batch(hip.make_batch([(dev[0], xg, ys[0], dtype, m, ffn, hidden), (dev[1], xg, ys[1], dtype, m, ffn, hidden)]))
+            for wi, yi in zip((g, u), ys):
+                want = oracle.quantized_matmul(wi, xf.float().numpy(), dtype, m, ffn, hidden, acc=oracle.ACC_F64, threads=16)
+                rel = np.linalg.norm(yi.float().cpu().numpy() - want) / np.linalg.norm(want)
+                assert rel <= element_bar(elem), f"group m={m}: {rel}"
