@@ -2663,11 +2663,14 @@ int run_group(gllmq_ctx *ctx, Scratch &S, const gllmq_matmul_desc *descs, size_t
         ctx->call_elem = elem;
         const int rc = run_mm8s(ctx, *f, G.seg[0].w, first.x_dev, first.y_dev, first.m, rows, first.k, false, stream, nullptr, false, nullptr, &G);
         ctx->call_elem = 0;
-        return rc;
+        // Rows of more than 4096 elements, which these kernels leave: the GEMM from three rows on, 16 bits from two.  us per
+        // call, one by one in brackets, 5120 + 1024 + 1024 rows of 5120: Q4_K three f32 rows 17.7 (28.7), two bf16 16.5 (34.1), Q8_0
+        // 24.7 (41.2), 23.1 (34.3); 8192 + 2 x 1024 rows of 8192 Q4_K 28.7 (32.6), 27.0 (39.1), but two f32 rows 28.5 (27.2).
+        if (rc >= 0 || first.k <= 4096 || first.m < (elem ? 2u : 3u) || ctx->mmfw_small_min_m > 9) return rc;
     }
     const MmfwPlan L = plan_mmfw(ctx, first.ggml_dtype, first.m, n, static_cast<int>(len), first.k, elem != 0, S.fixed ? S.mmf_bytes : SIZE_MAX);
     if (!L.ok || !mmfw_scratch_ok(ctx, S, L, stream)) return -1;
-    return run_mmfw(ctx, S, *f, mats, static_cast<int>(len), first.x_dev, elem, elem, first.m, first.k, false, stream, 5);
+    return run_mmfw(ctx, S, *f, mats, static_cast<int>(len), first.x_dev, elem, elem, first.m, first.k, false, stream, 2);
 }
 
 // The launches a batch will make, and which of them get their weights prefetched: an ordered

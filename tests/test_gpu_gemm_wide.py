@@ -273,3 +273,26 @@ def test_five_to_eight_rows(torch, oracle, dtype):
                 want = oracle.quantized_matmul(wi, xf.float().numpy(), dtype, m, ffn, hidden, acc=oracle.ACC_F64, threads=16)
                 rel = np.linalg.norm(yi.float().cpu().numpy() - want) / np.linalg.norm(want)
                 assert rel <= element_bar(elem), f"group m={m}: {rel}"
+
+
+@pytest.mark.parametrize("dtype", ALL)
+def test_projections_of_two_to_four_long_rows(torch, oracle, dtype):
+    """Rows beyond what the streamed launch over several matrices takes: the GEMM from three rows on, in 16 bits from two."""
+    from gllm_amd.backend import HipBackend
+    hip = HipBackend(0)
+    k, sizes = 4352, [300, 40, 257]
+    ws = [random_weight(dtype, n, k, seed=n) for n in sizes]
+    dev = [torch.from_numpy(w.view(np.uint8).reshape(-1)).cuda() for w in ws]
+    for elem in ("float32", "float16"):
+        t = getattr(torch, elem)
+        for m in (1, 2, 3, 4):
+            print(f"long rows dtype={dtype} {elem} m={m}", flush=True)
+            x = torch.from_numpy(random_activations(m, k, seed=m) * 1e-2).to(t)
+            xd, ys = x.cuda(), [torch.full((m, n), float("nan"), dtype=t, device="cuda") for n in sizes]
+            hip.run_batch(hip.make_batch([(d, xd, y, dtype, m, n, k) for d, y, n in zip(dev, ys, sizes)]))
+            grouped = hip.last_kernel_name() == "gq_mmf_reduce"
+            assert grouped == (m >= (2 if elem == "float16" else 3)), hip.last_kernel_name()
+            for w, y, n in zip(ws, ys, sizes):
+                want = oracle.quantized_matmul(w, x.float().numpy(), dtype, m, n, k, acc=oracle.ACC_F64, threads=16)
+                rel = np.linalg.norm(y.float().cpu().numpy() - want) / np.linalg.norm(want)
+                assert rel <= element_bar(elem), f"m={m} n={n}: {rel}"
