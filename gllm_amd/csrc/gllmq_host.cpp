@@ -268,6 +268,7 @@ struct gllmq_ctx {
     bool moe_mm8_rows = true;                   // "moe_mm8_rows" = 0: no wave-per-tile kernel for short Q6_K rows
     uint32_t moe_streamed = 1;                  // "moe_streamed": the grouped kernels in the streamed form: 0 never, 1 while experts see few tokens each, 2 always
     bool moe_wide = true;                       // "moe_wide" = 0: experts with many tokens stay on the eight-token jobs
+    bool moe_wide_cost = true;                  // ... and only where it is estimated to be ahead (off once "moe_wide_min" is set)
     uint32_t moe_wide_min = 8;                  // "moe_wide_min": fewest pairs per expert (on average) that take the GEMM
     uint32_t moe_depth = 0;                     // "moe_depth": items a loader of the streamed grouped kernels keeps unconfirmed (0 = as the dense launches)
 
@@ -2063,7 +2064,10 @@ int gllmq_set_option(gllmq_ctx *ctx, const char *name, long value)
     else if (n == "moe_glu") ctx->moe_glu = value != 0;
     else if (n == "moe_streamed") ctx->moe_streamed = u;
     else if (n == "moe_wide") ctx->moe_wide = value != 0;
-    else if (n == "moe_wide_min") ctx->moe_wide_min = std::max(1u, u);
+    else if (n == "moe_wide_min") {
+        ctx->moe_wide_min = std::max(1u, u);
+        ctx->moe_wide_cost = false;
+    }
     else if (n == "moe_depth") ctx->moe_depth = u;
     else if (n == "moe_slices") ctx->moe_slices = u;
     else if (n == "prefetch") ctx->prefetch = value != 0;
@@ -2951,6 +2955,23 @@ bool takes_moe_wide(const gllmq_ctx *ctx, uint32_t dtype_gu, uint32_t dtype_dn, 
     if (!ctx->moe_wide || !ctx->use_mmf || !ctx->use_mmfw || ctx->moe_streamed == 2 || pairs < (dtype_gu == T_Q8_0 || dtype_dn == T_Q8_0 ? (ctx->moe_wide_min + 1) / 2 : ctx->moe_wide_min) * experts)
         return false; // (the other form of Q8_0 experts is the GEMV)
     if ((dtype_gu == T_Q8_0 && hidden < 256) || (dtype_dn == T_Q8_0 && ffn < 256)) return false; // the Q8_0 window is a whole group
+    if (ctx->moe_wide_cost) {
+        // Few experts, or small ones, do not fill the device with one workgroup per 256 weight rows and all of K, which the
+        // int8 kernels do; those take time with every pair.  Estimates in us.  GEMM: a block of K 2.5 (Q6_K, Q8_0: 3.3), 0.6 more
+        // with every CU busy, 5 for a workgroup's start and end, 20 for the launches beside the two.  int8: 25, the weights at 5
+        // TB/s, the products at 100 TFLOP/s (Q5_K 60, Q8_0 26).  Measured / estimated, 8 experts of 3072 x 512, eight pairs each: Q4_K
+        // GEMM 60 / 67, int8 45 / 36; 8 of 4096 x 2048, sixteen: 104 / 104, 143 / 115; 32 of 2048 x 1024, eight: 78 / 70, 106 / 83; 128 of
+        // 4096 x 1536, eight: 570 / 575, 615 / 726, Q8_0 four: 685 / 651, 1272 / 1281; Q8_0 8 of 3072 x 512, four: 76 / 78, 47 / 45.
+        const double e = static_cast<double>(std::min(experts, pairs)), cus = ctx->num_cus;
+        auto launch_us = [&](uint32_t dtype, size_t rows, size_t k) {
+            const double wgs = std::ceil(rows / 256.0) * e, block = (dtype == T_Q6_K || dtype == T_Q8_0 ? 3.3 : 2.5) + 0.6 * std::min(1.0, wgs / cus);
+            return std::ceil(wgs / cus) * (static_cast<double>((k + 255) / 256) * block + 5.0);
+        };
+        const double wide = 20.0 + launch_us(dtype_gu, 2 * ffn, hidden) + launch_us(dtype_dn, hidden, ffn);
+        const double bytes = e * (2.0 * ffn * gllmq_row_bytes(dtype_gu, hidden) + static_cast<double>(hidden) * gllmq_row_bytes(dtype_dn, ffn));
+        const double rate = dtype_gu == T_Q8_0 || dtype_dn == T_Q8_0 ? 26e6 : dtype_gu == T_Q5_K || dtype_dn == T_Q5_K ? 60e6 : 100e6;
+        if (wide > 25.0 + bytes / 5e6 + 6.0 * pairs * static_cast<double>(hidden) * ffn / rate) return false;
+    }
     const size_t tiles = pairs / 32 + std::min(experts, pairs), groups = std::max((hidden + 255) / 256, (ffn + 255) / 256);
     return aligned(x, 16) && pairs * ffn <= 0xFFFFFFFFull && tiles * groups * gq::MmfwImage<2>::bytes <= 0xFFFFFFFFull;
 }
