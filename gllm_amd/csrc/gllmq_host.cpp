@@ -1601,9 +1601,10 @@ int run_gemv(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
 
 // Whether 5 to 8 activation rows go to the wide GEMM.  The int8 kernels take up to eight rows of Q4_K, seven of Q5_K and
 // six of Q6_K and Q8_0 in a pass, and read the weights twice beyond that.  f32, us per call on 4096 x 14336: Q8_0 six rows
-// 24.0 (28.5 here), seven 31.6 (28.6), Q6_K seven 30.4 (27.4), Q5_K eight 26.3 (22.1); 16-bit activations, which the
-// GEMM takes as one plane, five rows 27.5 (25.8), 26.4 (26.3), 22.2 (20.7), Q4_K 21.1 (19.4).  Single matmuls of shorter
-// rows stay: 14336 x 4096 the same either way, 4096 x 4096 five rows 9.7 (15.2).
+// 24.0 (28.5 here), seven 31.6 (28.6), Q6_K seven 30.4 (27.4), Q5_K eight 26.3 (22.1); with 16-bit elements seven 35.7
+// (26.1), 34.7 (26.2), eight 30.6 (20.8).  Single matmuls of fewer weights or shorter rows stay: 14336 x 4096 f32 the same either
+// way, 2390 x 11520 Q4_K five bf16 rows 16.5 (21.0).  `one_plane`: a feed-forward block of 16-bit elements, whose other form
+// converts them in launches of its own.
 bool mmfw_takes_few(const gllmq_ctx *ctx, uint32_t dtype, size_t m, bool one_plane)
 {
     const size_t pass = dtype == T_Q4_K ? 8 : dtype == T_Q5_K ? 7 : 6;
@@ -1628,7 +1629,7 @@ int dispatch_matmul(gllmq_ctx *ctx, Scratch &S, const Format &f, const uint8_t *
     // 32 bf16 rows against run_mmf's: Q6_K 14336 x 4096 24.7, 26.0 (27.7, 29.0), 4096 x 4096 18.8, 20.9 (21.3, 22.3);
     // Q8_0 14336 x 4096 24.9, 27.0 (33.0, 34.3); Q4_K 4096 x 14336 19.5, 20.8 (22.2, 22.3), 1024 x 4096 the same.
     // f32, 32 rows, Q4_K 14336 x 4096 21.2 (20.9).
-    if (!ctx->mmfs_all && (m >= ctx->mmfw_small_min_m || (!bf16 && k > 10240 && mmfw_takes_few(ctx, f.dtype, m, ctx->call_elem && !ctx->call_glu)))) {
+    if (!ctx->mmfs_all && (m >= ctx->mmfw_small_min_m || (!bf16 && k > 10240 && n * k >= (48ull << 20) && mmfw_takes_few(ctx, f.dtype, m, false)))) {
         const MmfwMatrix one{ w, y, n };
         rc = run_mmfw(ctx, S, f, &one, 1, x, ctx->call_elem, ctx->call_elem, m, k, bf16, stream, 5);
         if (rc >= 0 || rc == kNeedPlainActivations) return rc;
