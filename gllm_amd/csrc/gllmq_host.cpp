@@ -1115,7 +1115,7 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
     L.n_tiles = static_cast<uint32_t>(tiles);
     const uint32_t row_tiles = static_cast<uint32_t>((m + 31) / 32);
     // Activation tiles per workgroup and slices of K by a cost model (us): a block of K takes a
-    // workgroup its products (Q6_K: one more operand; Q8_0: its scales), the way of one wave's block through
+    // workgroup its products (Q6_K, Q8_0: and their scales), the way of one wave's block through
     // unpacking and LDS, which a tile or two do not cover, or the weights' way from memory, whichever
     // is longest; a workgroup starts and ends in `start`; the slices of K meet through memory.  Slopes over
     // K measured with one tile on 16 CUs: 1.5 (Q4_K), 2.7 (Q6_K), 2.4 (Q8_0) a block; two tiles,
@@ -1123,7 +1123,7 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
     const double cus = ctx->num_cus;
     const double w_us = find_format(dtype)->group_bytes * 256.0 * cus / 5.0e6; // 5 TB/s over all CUs
     static const double chain_us[4] = { 1.5, 1.6, 2.7, 2.4 };
-    const double tile_us = fmt == 3 ? 1.2 + 0.45 * L.planes : 0.25 + 0.62 * (L.planes + (fmt == 2 ? 1u : 0u));
+    const double tile_us = fmt >= 2 ? (fmt == 3 ? 1.2 : 1.45) + 0.45 * L.planes : 0.25 + 0.62 * L.planes;
     const double start = 5.0;
     double best = 1e300;
     for (uint32_t mt = 1; mt <= static_cast<uint32_t>(gq::MMFW_MAX_MT); ++mt) {

@@ -403,22 +403,22 @@ template <int PL> struct MmfwImage {
 template <int FMT> struct MmfwFormat;
 template <> struct MmfwFormat<0> { // 32 rows x 32 bytes per part, headers 16 bytes a row
     static constexpr uint32_t BLOCK = 144, STAGE = 5u * 1024u;
-    static constexpr int PARTS = 4, PART = 1, HEAD = 1, BP = 1;
+    static constexpr int PARTS = 4, PART = 1, HEAD = 1;
     static constexpr bool SUMS = true;
 };
 template <> struct MmfwFormat<1> { // the fifth bits come with the header
     static constexpr uint32_t BLOCK = 176, STAGE = 6u * 1024u;
-    static constexpr int PARTS = 4, PART = 1, HEAD = 2, BP = 1;
+    static constexpr int PARTS = 4, PART = 1, HEAD = 2;
     static constexpr bool SUMS = true;
 };
 template <> struct MmfwFormat<2> { // half blocks: two 32-byte pieces of low nibbles a row, one of high bits
     static constexpr uint32_t BLOCK = 210, STAGE = 7u * 1024u;
-    static constexpr int PARTS = 2, PART = 3, HEAD = 1, BP = 2;
+    static constexpr int PARTS = 2, PART = 3, HEAD = 1;
     static constexpr bool SUMS = false;
 };
 template <> struct MmfwFormat<3> { // half groups: 136 bytes a row
     static constexpr uint32_t BLOCK = 272, STAGE = 10u * 1024u;
-    static constexpr int PARTS = 2, PART = 5, HEAD = 0, BP = 1;
+    static constexpr int PARTS = 2, PART = 5, HEAD = 0;
     static constexpr bool SUMS = false;
 };
 
@@ -441,10 +441,10 @@ struct MmfwShape {
     static constexpr uint32_t total = ring + R * CHUNK;
     static_assert(total <= 160u * 1024u, "LDS");
 
-    // ---- A block is NS stages of SG operand slots (a K step of one plane) for all row tiles; Q8_0: a
-    // stage is a unit.  What stage s + 1 multiplies is read from LDS during stage s.
+    // ---- A block is NS stages of SG operand slots (a K step of one plane) for all row tiles; Q6_K, Q8_0:
+    // a stage is a unit.  What stage s + 1 multiplies is read from LDS during stage s.
     static constexpr int SG = MT >= 3 ? 1 : MT == 2 ? 2 : 4;
-    static constexpr int NS = FMT == 3 ? 8 : 16 * PL / SG;
+    static constexpr int NS = FMT >= 2 ? 8 : 16 * PL / SG;
     static constexpr int SPC = NS / C;                 // stages per chunk
     static constexpr int QL = NS / F::PARTS;           // stages per weight part
     // Q8_0 reads the quants of stage s + 1 in stage s, so a part is free a stage before the next one starts
