@@ -1071,6 +1071,7 @@ struct MmfwMatrix {
 struct MmfwPlan {
     bool ok = false;
     uint32_t groups = 0, planes = 2, mt = 1, n_tiles = 0, ksplit = 1, bps = 0, band = 4;
+    uint32_t run = 0; // blocks whose sums are taken in one run; 0: all of a slice's
     size_t rows = 0; // activation rows per pass (all of them, unless the images would pass 1 GiB or the scratch is of fixed size)
     size_t img_bytes = 0, inv_bytes = 0, part_bytes = 0;
     size_t need() const { return img_bytes + inv_bytes + part_bytes; }
@@ -1088,6 +1089,39 @@ void mmfw_size(MmfwPlan &L, size_t rows, size_t n_sum)
     // (a workgroup fetches the inverse scales of its rows as one KiB)
     L.inv_bytes = (static_cast<size_t>(L.groups) * mmfw_inv_ld(rows) * 4 + 1024 + 255) & ~size_t(255);
     L.part_bytes = L.ksplit > 1 ? static_cast<size_t>(L.ksplit) * rows * n_sum * 4 : 0;
+}
+
+// Additions one after the other, in the mean over the blocks, when `blocks` of them are added up in runs of `run`
+// (0: in one), and `slices` of such sums.
+double mmfw_chain(uint32_t blocks, uint32_t run, uint32_t slices)
+{
+    const double slice = slices > 1u ? 0.5 * (slices + 1u) : 0.0;
+    if (run == 0u || run >= blocks) return 0.5 * (blocks + 1u) + slice;
+    return 0.5 * (run + 1u) + 0.5 * ((blocks + run - 1u) / run + 1u) + slice;
+}
+
+// Q6_K and Q8_0: blocks of a run, such that no output's additions form a longer chain than in the form of 64-row passes,
+// whose slices of K are short because it has few workgroups otherwise.  Error against 64 bits, 2048 f32 rows of 4096 x 14336:
+// Q6_K 1.64e-7 in one run, 1.18e-7 in runs of eight, 1.23e-7 in that form; Q8_0 1.64e-7, 1.19e-7, 1.23e-7.  It takes
+// registers that four row tiles do not have: 571 -> 657 us, 535 -> 626.  Q4_K and Q5_K, whose blocks themselves cost more,
+// stay below that form without (2.27e-7 against 2.33e-7).
+// `bar`: that form's shortest chain over the launch's matrices (mmfw_chain_bar).
+uint32_t mmfw_run(uint32_t bps, uint32_t ksplit, double bar)
+{
+    if (mmfw_chain(bps, 0, ksplit) <= bar) return 0;
+    uint32_t run = 2;
+    for (uint32_t r = 4; r <= 16; r *= 2) // the longest that is short enough, else the best
+        if (mmfw_chain(bps, r, ksplit) <= std::max(bar, mmfw_chain(bps, run, ksplit))) run = r;
+    return run;
+}
+double mmfw_chain_bar(const gllmq_ctx *ctx, int fmt, const size_t *n, int count, size_t k)
+{
+    double bar = 1e300;
+    for (int i = 0; i < count && fmt >= 2; ++i) {
+        const MmfPlan O = plan_mmf(ctx, 64, n[i], k);
+        bar = std::min(bar, mmfw_chain(O.bps, 0, O.ksplit));
+    }
+    return bar;
 }
 
 // Whether the GEMM's scratch for this plan is there or can be had now: a capture cannot allocate, and what was
@@ -1124,7 +1158,7 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
     const double w_us = find_format(dtype)->group_bytes * 256.0 * cus / 5.0e6; // 5 TB/s over all CUs
     static const double chain_us[4] = { 1.5, 1.6, 2.7, 2.4 };
     const double tile_us = fmt >= 2 ? (fmt == 3 ? 1.2 : 1.45) + 0.45 * L.planes : 0.25 + 0.62 * L.planes;
-    const double start = 5.0;
+    const double start = 5.0, bar = mmfw_chain_bar(ctx, fmt, n, count, k);
     double best = 1e300;
     for (uint32_t mt = 1; mt <= static_cast<uint32_t>(gq::MMFW_MAX_MT); ++mt) {
         if (ctx->mmfw_mt ? mt != ctx->mmfw_mt : (mt > row_tiles)) continue;
@@ -1134,6 +1168,8 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
             const uint32_t bps = (L.groups + ks - 1) / ks;
             if ((L.groups + bps - 1) / bps != ks) continue; // every slice has a block
             if (ctx->mmfw_ksplit && ks != std::min(ctx->mmfw_ksplit, L.groups)) continue;
+            const uint32_t run = mmfw_run(bps, ks, bar);
+            if (run && !gq::mmfw_runs(static_cast<int>(mt)) && !ctx->mmfw_mt) continue;
             const double rounds = std::ceil(static_cast<double>(m_tiles * tiles * ks) / cus);
             const double busy = std::min(1.0, static_cast<double>(m_tiles * tiles * ks) / cus);
             const double block = std::max({ mt * tile_us, chain_us[fmt], w_us * busy });
@@ -1144,6 +1180,7 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
                 L.mt = mt;
                 L.ksplit = ks;
                 L.bps = bps;
+                L.run = run;
             }
         }
     }
@@ -1216,6 +1253,7 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
         P.n_tiles = L.n_tiles;
         P.ksplit = L.ksplit;
         P.blocks_per_split = L.bps;
+        P.run_mask = L.run ? L.run - 1u : ~0u;
         P.items = P.m_tiles * P.n_tiles * L.ksplit;
         P.band = std::min(L.band, P.m_tiles);
         P.elem = elem_y;

@@ -388,6 +388,7 @@ constexpr int MMFW_WAVES = 8;
 constexpr int MMFW_TILE_ROWS = 32 * MMFW_WAVES; // weight rows per workgroup
 constexpr int MMFW_MAX_SEGS = 3;                // weight matrices of one launch
 constexpr int MMFW_MAX_MT = 4;
+constexpr bool mmfw_runs(int mt) { return mt <= 3; } // Q6_K, Q8_0: registers for sums of runs (MmfwParams::run_mask)
 constexpr uint32_t MMFW_PREP_WAVES = 16;        // of a workgroup that prepares an image
 
 // Image of 32 activation rows x 256 elements of K: [K step 0..15][plane][lane] 16 bytes, then
@@ -505,6 +506,7 @@ struct MmfwParams {
     uint32_t inv_ld;
     uint32_t m_tiles, n_tiles; // workgroup tiles of activation rows and of weight rows (all matrices)
     uint32_t ksplit, blocks_per_split;
+    uint32_t run_mask;         // blocks whose sums are taken in one run, less one (a power of two less one; all ones: a slice's all)
     uint32_t items;            // m_tiles * n_tiles * ksplit
     uint32_t band;             // activation tiles that neighbouring workgroups share a weight tile over
     uint32_t elem;             // element type of y

@@ -8,7 +8,7 @@ from gllm_amd.synth import random_activations, random_weight
 
 pytestmark = pytest.mark.gpu
 
-Q6_K = 14
+Q8_0, Q6_K = 8, 14
 
 # Root mean squares over 1e5 outputs and more, which share rows of weights and of activations: their ratio is good to about 1 %.
 SPREAD = 1.03
@@ -43,3 +43,13 @@ def test_q6_k(torch, m, n, k, bf16):
     before, *here = errors(torch, Q6_K, m, n, k, bf16, (0, 1, 2, 3, 4))
     print(f"q6_k {m} {n} {k} bf16={bf16}: {before:.3e} here {[f'{e:.3e}' for e in here]}", flush=True)
     assert max(here) <= SPREAD * before
+
+
+@pytest.mark.parametrize("dtype", [Q6_K, Q8_0])
+@pytest.mark.parametrize("m, n, k", [(200, 14336, 4096), (2048, 4096, 14336), (300, 28672, 2560)])
+def test_long_rows(torch, dtype, m, n, k):
+    """Many blocks in one slice of K: their sums are taken in runs."""
+    for bf16 in (False, True):
+        before, *here = errors(torch, dtype, m, n, k, bf16, (0, 1, 2, 3))
+        print(f"{dtype} {m} {n} {k} bf16={bf16}: {before:.3e} here {[f'{e:.3e}' for e in here]}", flush=True)
+        assert max(here) <= SPREAD * before
