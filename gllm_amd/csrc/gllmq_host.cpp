@@ -1234,6 +1234,7 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
         Q.act_bf16 = act_bf16 ? 1u : 0u;
         Q.elem = ctx->call_glu ? 0u : elem_x;
         Q.natural = fmt == 2 ? 1u : 0u; // a sub-block of Q6_K is one K step
+        Q.lo_first = gq::mmfw_lo_first(fmt, static_cast<int>(L.planes), static_cast<int>(L.mt)) ? 1u : 0u;
         Q.glu = ctx->call_glu;
         Q.glu_off = ctx->call_glu_off;
         const uint32_t row_tiles = (mm + 31u) / 32u;

@@ -391,7 +391,13 @@ constexpr int MMFW_MAX_MT = 4;
 constexpr bool mmfw_runs(int mt) { return mt <= 3; } // Q6_K, Q8_0: registers for sums of runs (MmfwParams::run_mask)
 constexpr uint32_t MMFW_PREP_WAVES = 16;        // of a workgroup that prepares an image
 
-// Image of 32 activation rows x 256 elements of K: [K step 0..15][plane][lane] 16 bytes, then
+// Four tiles of Q4_K and Q5_K: no registers for sums of the lo plane's products, which therefore come ahead of the hi
+// plane's (a block's weights are unpacked twice).  In turn with them, where each costs the sum a rounding at its full size,
+// the error was 2.43e-7 (512 f32 rows of 14336 x 4096 Q4_K; so 1.92e-7, the 64-row form 2.17e-7) and the call 3 % shorter
+// (123 us, so 126; three tiles, which have the registers, 177, two 143).
+constexpr bool mmfw_lo_first(int fmt, int planes, int mt) { return fmt <= 1 && planes == 2 && mt == 4; }
+
+// Image of 32 activation rows x 256 elements of K: [K step 0..15][plane][lane] 16 bytes (lo first: [lo, hi][K step]), then
 // [lane] 16 bytes of sub-block sums (lanes 0..31 hi, 32..63 lo); images lie [row tile][block].
 // The inverse scales are an array of their own: [block][padded rows] f32.
 template <int PL> struct MmfwImage {
@@ -423,9 +429,10 @@ template <> struct MmfwFormat<3> { // half groups: 136 bytes a row
     static constexpr bool SUMS = false;
 };
 
-template <int FMT, int PL, int MT>
+template <int FMT, int PL, int MT, bool LO_FIRST = false>
 struct MmfwShape {
     using F = MmfwFormat<FMT>;
+    static_assert(!LO_FIRST || mmfw_lo_first(FMT, PL, MT), "");
     // Activations move in chunks of UC units (32 elements of K) through a ring of R chunk slots in LDS.
     static constexpr int UC = MT == 4 ? (PL == 2 ? 1 : 2) : MT == 3 ? (PL == 2 ? 2 : 4) : MT == 2 ? (PL == 2 ? 2 : 4) : (PL == 2 ? 4 : 8);
     static constexpr int R = MT == 3 ? 3 : 4;
@@ -447,10 +454,12 @@ struct MmfwShape {
     static constexpr int SG = MT >= 3 ? 1 : MT == 2 ? 2 : 4;
     static constexpr int NS = FMT >= 2 ? 8 : 16 * PL / SG;
     static constexpr int SPC = NS / C;                 // stages per chunk
-    static constexpr int QL = NS / F::PARTS;           // stages per weight part
+    static constexpr int PASS = LO_FIRST ? NS / 2 : NS; // stages in which the block's weights are read once
+    static constexpr int QL = PASS / F::PARTS;         // stages per weight part
     // Q8_0 reads the quants of stage s + 1 in stage s, so a part is free a stage before the next one starts
-    static constexpr int FREE = FMT == 3 ? QL - 1 : 0; // a part (p) is requested again at stage p * QL + FREE
-    static constexpr int part_of(int s) { return s >= FREE && (s - FREE) % QL == 0 ? (s - FREE) / QL : -1; }
+    static constexpr int FREE = FMT == 3 ? QL - 1 : 0; // a part is requested again that far behind its first stage
+    static constexpr int requested(int p) { return NS - PASS + p * QL + FREE; } // (lo first: behind its second read)
+    static constexpr int part_of(int s) { return s >= requested(0) && (s - requested(0)) % QL == 0 ? (s - requested(0)) / QL : -1; }
 
     // ---- the wave's sequence of loads, one block being a period: stage s requests its weights (and
     // stage 0 the extra of the block after next, first); then, in the last stage of a chunk, the
@@ -527,6 +536,7 @@ struct MmfwPrepParams {
     // row_of[that], or that row itself
     const struct MoeTile *tiles;
     const uint32_t *row_of, *counters;
+    uint32_t lo_first;     // two planes: see mmfw_lo_first
     uint32_t natural;      // K order inside 32 elements: 1: step s, half h = 16 s + 8 h; 0: 16 h + 8 s
     uint32_t glu, glu_off; // x[i] = act(x[i]) * x[i + glu_off] (0 off, 1 SiLU, 2 SiLU behind a ReLU)
 };

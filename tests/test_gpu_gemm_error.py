@@ -8,7 +8,7 @@ from gllm_amd.synth import random_activations, random_weight
 
 pytestmark = pytest.mark.gpu
 
-Q8_0, Q6_K = 8, 14
+Q8_0, Q4_K, Q5_K, Q6_K = 8, 12, 13, 14
 
 # Root mean squares over 1e5 outputs and more, which share rows of weights and of activations: their ratio is good to about 1 %.
 SPREAD = 1.03
@@ -53,3 +53,12 @@ def test_long_rows(torch, dtype, m, n, k):
         before, *here = errors(torch, dtype, m, n, k, bf16, (0, 1, 2, 3))
         print(f"{dtype} {m} {n} {k} bf16={bf16}: {before:.3e} here {[f'{e:.3e}' for e in here]}", flush=True)
         assert max(here) <= SPREAD * before
+
+
+@pytest.mark.parametrize("dtype", [Q4_K, Q5_K])
+@pytest.mark.parametrize("m, n, k", [(64, 2000, 2048), (512, 14336, 4096), (1024, 4096, 14336)])
+def test_q4_k_q5_k(torch, dtype, m, n, k):
+    """Up to three row tiles with sums of their own for the lo plane's products, four with those ahead of the others."""
+    before, *here = errors(torch, dtype, m, n, k, False, (0, 1, 2, 3, 4))
+    print(f"{dtype} {m} {n} {k}: {before:.3e} here {[f'{e:.3e}' for e in here]}", flush=True)
+    assert max(here) <= SPREAD * before
