@@ -1072,7 +1072,8 @@ struct MmfwPlan {
     bool ok = false;
     uint32_t groups = 0, planes = 2, mt = 1, n_tiles = 0, ksplit = 1, bps = 0, band = 4;
     uint32_t run = 0; // blocks whose sums are taken in one run; 0: all of a slice's
-    size_t rows = 0; // activation rows per pass (all of them, unless the images would pass 1 GiB or the scratch is of fixed size)
+    size_t n_sum = 0; // weight rows of all matrices
+    size_t rows = 0; // activation rows per pass (all of them, unless the images would pass 1 GiB or the scratch has no room: mmfw_fit)
     size_t img_bytes = 0, inv_bytes = 0, part_bytes = 0;
     size_t need() const { return img_bytes + inv_bytes + part_bytes; }
 };
@@ -1081,14 +1082,39 @@ int mmf_format(uint32_t dtype) { return dtype == T_Q8_0 ? 3 : dtype == T_Q6_K ? 
 
 uint32_t mmfw_inv_ld(size_t rows) { return static_cast<uint32_t>((rows + 31) / 32 * 32); }
 
-void mmfw_size(MmfwPlan &L, size_t rows, size_t n_sum)
+void mmfw_size(MmfwPlan &L, size_t rows)
 {
     L.rows = rows;
     const size_t image = L.planes == 2 ? gq::MmfwImage<2>::bytes : gq::MmfwImage<1>::bytes;
     L.img_bytes = (rows + 31) / 32 * L.groups * image;
     // (a workgroup fetches the inverse scales of its rows as one KiB)
     L.inv_bytes = (static_cast<size_t>(L.groups) * mmfw_inv_ld(rows) * 4 + 1024 + 255) & ~size_t(255);
-    L.part_bytes = L.ksplit > 1 ? static_cast<size_t>(L.ksplit) * rows * n_sum * 4 : 0;
+    L.part_bytes = L.ksplit > 1 ? static_cast<size_t>(L.ksplit) * rows * L.n_sum * 4 : 0;
+}
+
+constexpr size_t kMmfwMaxImages = size_t(1) << 30;
+
+// Fewer rows per pass, until the pass needs `limit` bytes at most (false: one row of tiles needs more).  Tiles and slices stay
+// what they are, so the results do.
+bool mmfw_shrink(MmfwPlan &L, size_t limit)
+{
+    const size_t step = 32u * L.mt;
+    while ((L.img_bytes > kMmfwMaxImages || L.need() > limit) && L.rows > step)
+        mmfw_size(L, std::max(step, (L.rows / 2 + step - 1) / step * step));
+    return L.img_bytes < 0xFFFFFFFFull && L.need() <= limit;
+}
+
+// Most bytes that the sums of K slices take; a plan has no more slices than that allows.  32 MiB cost 3000 plans of 9 to 2048
+// rows 0.6 % in the mean by the cost model, 16 MiB 1.3 %, 64 MiB 0.5 %.
+size_t mmfw_most_slices(const gllmq_ctx *ctx, size_t m) { return static_cast<size_t>(ctx->num_cus) * 1024u * (m <= 32 ? 32u : 128u); }
+
+// Scratch that any call of up to `m` rows of `k` elements fits, in one pass, and from 33 rows on any call of more rows in passes:
+// what is grown for one call or reserved serves every other one of as many rows, whatever its weight rows, matrices, slices
+// and element type.
+size_t mmfw_reserve(const gllmq_ctx *ctx, size_t m, size_t k)
+{
+    const size_t groups = (k + 255) / 256, tiles = m <= 32 ? 1 : std::max<size_t>((m + 31) / 32, gq::MMFW_MAX_MT);
+    return std::min(tiles * groups * gq::MmfwImage<2>::bytes, kMmfwMaxImages) + ((groups * tiles * 128 + 1024 + 255) & ~size_t(255)) + mmfw_most_slices(ctx, m);
 }
 
 // Additions one after the other, in the mean over the blocks, when `blocks` of them are added up in runs of `run`
@@ -1124,19 +1150,19 @@ double mmfw_chain_bar(const gllmq_ctx *ctx, int fmt, const size_t *n, int count,
     return bar;
 }
 
-// Whether the GEMM's scratch for this plan is there or can be had now: a capture cannot allocate, and what was
-// reserved for the kernels of fewer rows has to go on serving them.
-bool mmfw_scratch_ok(const gllmq_ctx *ctx, const Scratch &S, const MmfwPlan &L, void *stream)
+// Sizes the plan's passes for the scratch that there is, where no more can be had: a capture cannot allocate, and a block of fixed
+// size does not grow.  False: not even the smallest pass fits.
+bool mmfw_fit(const gllmq_ctx *ctx, const Scratch &S, MmfwPlan &L, void *stream)
 {
-    return L.need() <= S.mmf_bytes || ctx->probe || !(S.fixed || stream_is_capturing(stream));
+    if (L.need() <= S.mmf_bytes || ctx->probe || !(S.fixed || stream_is_capturing(stream))) return true;
+    return mmfw_shrink(L, S.mmf_bytes);
 }
 
-MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t *n, int count, size_t k, bool hi_only,
-                   size_t scratch_limit = SIZE_MAX)
+MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t *n, int count, size_t k, bool hi_only)
 {
     MmfwPlan L;
     const int fmt = mmf_format(dtype);
-    size_t n_sum = 0, tiles = 0;
+    size_t &n_sum = L.n_sum, tiles = 0;
     for (int i = 0; i < count; ++i) {
         n_sum += n[i];
         tiles += (n[i] + gq::MMFW_TILE_ROWS - 1) / gq::MMFW_TILE_ROWS;
@@ -1170,6 +1196,10 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
             if (ctx->mmfw_ksplit && ks != std::min(ctx->mmfw_ksplit, L.groups)) continue;
             const uint32_t run = mmfw_run(bps, ks, bar);
             if (run && !gq::mmfw_runs(static_cast<int>(mt)) && !ctx->mmfw_mt) continue;
+            // no plan that the fixed scratch cannot take in passes of one row of tiles (the call through it has the same one)
+            const size_t slices = ks > 1 ? static_cast<size_t>(ks) * n_sum * 4 : 0, pass_rows = std::min<size_t>(m, 32u * mt);
+            if (slices * m > mmfw_most_slices(ctx, m) && !ctx->mmfw_ksplit) continue;
+            if (static_cast<size_t>(L.groups) * mt * (gq::MmfwImage<2>::bytes + 128u) + 2048u + slices * pass_rows > GLLMQ_NOALLOC_SCRATCH_BYTES - kScratchFixedBytes) continue;
             const double rounds = std::ceil(static_cast<double>(m_tiles * tiles * ks) / cus);
             const double busy = std::min(1.0, static_cast<double>(m_tiles * tiles * ks) / cus);
             const double block = std::max({ mt * tile_us, chain_us[fmt], w_us * busy });
@@ -1187,15 +1217,8 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
     if (best == 1e300) return L;
     const uint32_t m_tiles = (row_tiles + L.mt - 1) / L.mt;
     L.band = std::min(m_tiles, 4u);
-    size_t rows = m;
-    const size_t step = 32u * L.mt;
-    mmfw_size(L, rows, n_sum);
-    // fewer rows per pass where the whole does not fit: the tiles and slices stay what they are, so the results do too
-    while ((L.img_bytes > (size_t(1) << 30) || L.need() > scratch_limit) && rows > step) {
-        rows = std::max(step, (rows / 2 + step - 1) / step * step);
-        mmfw_size(L, rows, n_sum);
-    }
-    L.ok = L.img_bytes < 0xFFFFFFFFull && L.need() <= scratch_limit;
+    mmfw_size(L, m);
+    L.ok = mmfw_shrink(L, SIZE_MAX);
     return L;
 }
 
@@ -1212,10 +1235,12 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
     size_t n[gq::MMFW_MAX_SEGS];
     for (int i = 0; i < count; ++i) n[i] = mats[i].n;
     const bool hi_only = act_bf16 || (elem_x && !ctx->call_glu);
-    const MmfwPlan L = plan_mmfw(ctx, f.dtype, m, n, count, k, hi_only, S.fixed ? S.mmf_bytes : SIZE_MAX);
-    if (!L.ok) return -1;
-    if (m < ctx->mmfw_min_m && !mmfw_scratch_ok(ctx, S, L, stream)) return -1;
-    int rc = grow_scratch(ctx, S, &S.mmf, &S.mmf_bytes, L.need(), stream, "quantized_matmul (GEMM)");
+    MmfwPlan L = plan_mmfw(ctx, f.dtype, m, n, count, k, hi_only);
+    if (!L.ok || !mmfw_fit(ctx, S, L, stream)) return -1;
+    if (S.fixed && plan_mmf(ctx, m, n[0], k).need > S.mmf_bytes) return -1; // beyond what that entry point takes, in passes or not
+    int rc = GLLMQ_OK;
+    const size_t reserve = std::max(L.need(), mmfw_reserve(ctx, m, k));
+    if (S.mmf_bytes < reserve && !S.fixed && !stream_is_capturing(stream)) rc = grow_scratch(ctx, S, &S.mmf, &S.mmf_bytes, reserve, stream, "quantized_matmul (GEMM)");
     if (rc != GLLMQ_OK) return rc;
     uint8_t *scratch = static_cast<uint8_t *>(S.mmf);
     const int fmt = mmf_format(f.dtype);
@@ -2427,12 +2452,12 @@ int ffn_on_stream(gllmq_ctx *ctx, const void *gate_w, const void *up_w, size_t g
     const bool wide = m >= std::max(5u, std::min(ctx->mmfw_min_m, ctx->mmfw_small_min_m)) ||
                       (ctx->ffn_fused && mmfw_takes_few(ctx, dtype_gate_up, m, elem != 0)); // ("ffn_fused" off: up to 8 rows in separate steps)
     auto down_fits = [&] {
-        const MmfwPlan L = plan_mmfw(ctx, dtype_down, m, &hidden, 1, ffn, false, S.fixed ? S.mmf_bytes : SIZE_MAX);
-        return L.ok && mmfw_scratch_ok(ctx, S, L, stream);
+        MmfwPlan L = plan_mmfw(ctx, dtype_down, m, &hidden, 1, ffn, false);
+        return L.ok && mmfw_fit(ctx, S, L, stream);
     };
     auto gate_up_fits = [&] {
-        const MmfwPlan L = plan_mmfw(ctx, dtype_gate_up, m, gate_up_n, 2, hidden, elem != 0, S.fixed ? S.mmf_bytes : SIZE_MAX);
-        return L.ok && mmfw_scratch_ok(ctx, S, L, stream);
+        MmfwPlan L = plan_mmfw(ctx, dtype_gate_up, m, gate_up_n, 2, hidden, elem != 0);
+        return L.ok && mmfw_fit(ctx, S, L, stream);
     };
     if (wide && !ctx->mmfs_all && ffn % 4 == 0 && m * ffn <= 0xFFFFFFFFull && down_fits() && gate_up_fits()) {
         const MmfwMatrix gate_up[2] = { { gw, gu, ffn }, { uw, gu + m * ffn, ffn } };
@@ -2712,8 +2737,6 @@ int run_group(gllmq_ctx *ctx, Scratch &S, const gllmq_matmul_desc *descs, size_t
         // 24.7 (41.2), 23.1 (34.3); 8192 + 2 x 1024 rows of 8192 Q4_K 28.7 (32.6), 27.0 (39.1), but two f32 rows 28.5 (27.2).
         if (rc >= 0 || first.k <= 4096 || first.m < (elem ? 2u : 3u) || ctx->mmfw_small_min_m > 9) return rc;
     }
-    const MmfwPlan L = plan_mmfw(ctx, first.ggml_dtype, first.m, n, static_cast<int>(len), first.k, elem != 0, S.fixed ? S.mmf_bytes : SIZE_MAX);
-    if (!L.ok || !mmfw_scratch_ok(ctx, S, L, stream)) return -1;
     return run_mmfw(ctx, S, *f, mats, static_cast<int>(len), first.x_dev, elem, elem, first.m, first.k, false, stream, 2);
 }
 
@@ -3435,11 +3458,11 @@ int gllmq_reserve_matmul(gllmq_ctx *ctx, uint32_t dtype, size_t m, size_t n, siz
     int rc = acquire_scratch(ctx, stream, &S);
     if (rc != GLLMQ_OK || m == 0 || n == 0 || k == 0) return rc;
     // the GEMM is the only matmul kernel family whose scratch depends on the shape; it may take
-    // any call of 3 rows and more
-    if (m < 3) return GLLMQ_OK;
-    // (either form of it: which one runs also depends on the activation pointer's alignment)
+    // any call of 3 rows and more, and a batch's matrices over the same two
+    if (m < 2) return GLLMQ_OK;
+    // (any form of it: which one runs also depends on the activation pointer's alignment)
     size_t need = plan_mmf(ctx, m, n, k).need;
-    for (bool hi_only : { false, true }) need = std::max(need, plan_mmfw(ctx, dtype, m, &n, 1, k, hi_only).need());
+    if (ctx->use_mmf && ctx->use_mmfw) need = std::max(need, mmfw_reserve(ctx, m, k));
     const MmfsPlan Ls = plan_mmfs(ctx, *find_format(dtype), m, n, k);
     if (Ls.ok) need = std::max(need, Ls.need);
     return grow_scratch(ctx, *S, &S->mmf, &S->mmf_bytes, need, stream, "reserve_matmul");
@@ -3456,11 +3479,6 @@ int gllmq_reserve_ffn(gllmq_ctx *ctx, uint32_t dtype_gate_up, uint32_t dtype_dow
     Scratch *S = nullptr;
     rc = acquire_scratch(ctx, stream, &S);
     if (rc != GLLMQ_OK) return rc;
-    const size_t both[2] = { ffn, ffn }; // gate and up in one GEMM launch
-    for (bool hi_only : { false, true }) {
-        rc = grow_scratch(ctx, *S, &S->mmf, &S->mmf_bytes, plan_mmfw(ctx, dtype_gate_up, m, both, 2, hidden, hi_only).need(), stream, "reserve_ffn");
-        if (rc != GLLMQ_OK) return rc;
-    }
     return grow_scratch(ctx, *S, &S->ffn, &S->ffn_bytes, ffn_scratch_bytes(m, ffn), stream, "reserve_ffn");
 }
 

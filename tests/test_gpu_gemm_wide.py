@@ -296,3 +296,68 @@ def test_projections_of_two_to_four_long_rows(torch, oracle, dtype):
                 want = oracle.quantized_matmul(w, x.float().numpy(), dtype, m, n, k, acc=oracle.ACC_F64, threads=16)
                 rel = np.linalg.norm(y.float().cpu().numpy() - want) / np.linalg.norm(want)
                 assert rel <= element_bar(elem), f"m={m} n={n}: {rel}"
+
+
+def captured(torch, hip, stream, call, outputs):
+    """The call captured on `stream`, replayed three times with eager work between: its outputs of every replay."""
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream), torch.cuda.graph(graph, stream=stream):
+        call()
+    found = []
+    for _ in range(3):
+        for y in outputs:
+            y.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        found.append([y.clone() for y in outputs])
+    return found
+
+
+@pytest.mark.parametrize("dtype, n, k, first, elem", [
+    (Q4_K, 2000, 2048, 64, "float32"), (Q6_K, 14336, 1024, 512, "float32"), (Q8_0, 1280, 5120, 2048, "float32"), (Q5_K, 700, 1024, 33, "bfloat16")])
+def test_capture_of_any_rows_behind_one_call(torch, dtype, n, k, first, elem):
+    """A call of 33 rows and more, or a reserved one, leaves scratch for any number of rows: fewer, more (in passes), of the
+    other element types, over other weight rows.  The captured call gives the eager bits."""
+    from gllm_amd.backend import HipBackend
+    plain, t = HipBackend(0), getattr(torch, elem)
+    w = torch.from_numpy(random_weight(dtype, n, k, seed=5).view(np.uint8).reshape(-1)).cuda()
+    x = torch.from_numpy(random_activations(2100, k, seed=6)).cuda()
+    for reserve in (True, False):
+        hip, stream = HipBackend(0), torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            if reserve:
+                hip.reserve_matmul(dtype, first, n, k)
+            else:
+                y = torch.zeros(first, n, dtype=t, device="cuda")
+                hip.quantized_matmul(w, x[:first].to(t), y, dtype, first, n, k)
+        for m in (12, 33, 64, 65, 100, 129, 192, 700, 2100):
+            for e in {torch.float32, t}:
+                print(f"capture dtype={dtype} first={first} reserve={reserve} m={m} {e}", flush=True)
+                xm, y, want = x[:m].to(e), torch.zeros(m, n, dtype=e, device="cuda"), torch.zeros(m, n, dtype=e, device="cuda")
+                plain.quantized_matmul(w, xm, want, dtype, m, n, k)
+                for got, in captured(torch, hip, stream, lambda: hip.quantized_matmul(w, xm, y, dtype, m, n, k), [y]):
+                    assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+
+
+@pytest.mark.parametrize("dtype", ALL)
+@pytest.mark.parametrize("m, elem", [(2, "bfloat16"), (4, "float32"), (24, "float32"), (24, "float16"), (70, "float32")])
+def test_captured_group_gives_the_eager_bits(torch, dtype, m, elem):
+    """Reserved entry by entry, a batch of projections is captured as the one launch that it is eagerly."""
+    from gllm_amd.backend import HipBackend
+    t, k, sizes = getattr(torch, elem), 4352, [512, 128, 130]
+    x = torch.from_numpy(random_activations(m, k, seed=3)).cuda().to(t)
+    dev = [torch.from_numpy(random_weight(dtype, n, k, seed=n + i).view(np.uint8).reshape(-1)).cuda() for i, n in enumerate(sizes)]
+    ys, want = ([torch.zeros(m, n, dtype=t, device="cuda") for n in sizes] for _ in range(2))
+    plain, hip, stream = HipBackend(0), HipBackend(0), torch.cuda.Stream()
+    plain.run_batch(plain.make_batch([(d, x, y, dtype, m, n, k) for d, y, n in zip(dev, want, sizes)]))
+    eager = plain.last_kernel_name()
+    with torch.cuda.stream(stream):
+        for n in sizes:
+            hip.reserve_matmul(dtype, m, n, k)
+    batch = hip.make_batch([(d, x, y, dtype, m, n, k) for d, y, n in zip(dev, ys, sizes)])
+    print(f"captured group dtype={dtype} m={m} {elem}", flush=True)
+    for got in captured(torch, hip, stream, lambda: hip.run_batch(batch), ys):
+        assert hip.last_kernel_name() == eager
+        assert all(torch.equal(g.view(torch.uint8), a.view(torch.uint8)) for g, a in zip(got, want))
