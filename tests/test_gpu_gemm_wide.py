@@ -361,3 +361,28 @@ def test_captured_group_gives_the_eager_bits(torch, dtype, m, elem):
     for got in captured(torch, hip, stream, lambda: hip.run_batch(batch), ys):
         assert hip.last_kernel_name() == eager
         assert all(torch.equal(g.view(torch.uint8), a.view(torch.uint8)) for g, a in zip(got, want))
+
+
+def rounded_f32_call(torch, hip, w, x16, dtype, m, n, k):
+    """The call over 16-bit elements, and the f32 call on the widened activations rounded to them."""
+    y16, y32 = torch.zeros(m, n, dtype=x16.dtype, device="cuda"), torch.zeros(m, n, device="cuda")
+    hip.quantized_matmul(w, x16, y16, dtype, m, n, k)
+    hip.quantized_matmul(w, x16.float(), y32, dtype, m, n, k)
+    torch.cuda.synchronize()
+    return y16.view(torch.int16), y32.to(x16.dtype).view(torch.int16)
+
+
+@pytest.mark.parametrize("dtype, n, k, rows", [
+    (Q4_K, 4096, 4096, (33, 48, 100, 200)), (Q8_0, 4999, 2880, (77, 40)), (Q6_K, 4096, 4096, (20, 128, 77)), (Q5_K, 700, 14336, (33, 64, 300)),
+    (Q8_0, 2000, 8192, (17, 64, 130)), (Q6_K, 3000, 11008, (9, 33, 257))])
+@pytest.mark.parametrize("elem", ["float16", "bfloat16"])
+def test_element_types_have_the_slices_of_the_f32_call(torch, dtype, n, k, rows, elem):
+    """Tiles and slices as the shape gets them: the 16-bit call is the rounded f32 call, bit for bit."""
+    from gllm_amd.backend import HipBackend
+    hip = HipBackend(0)
+    w = torch.from_numpy(random_weight(dtype, n, k, seed=5).view(np.uint8).reshape(-1)).cuda()
+    x = torch.from_numpy(random_activations(max(rows), k, seed=6)).cuda().to(getattr(torch, elem))
+    for m in rows:
+        print(f"slices dtype={dtype} m={m} n={n} k={k} {elem}", flush=True)
+        got, want = rounded_f32_call(torch, hip, w, x[:m].contiguous(), dtype, m, n, k)
+        assert torch.equal(got, want)
