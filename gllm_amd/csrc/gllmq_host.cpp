@@ -225,7 +225,7 @@ struct gllmq_ctx {
     uint32_t mmfw_small_min_m = 9;              // "mmfw_small_min_m": ... where the streamed GEMMs do not take the call
     uint32_t mmfw_mt = 0, mmfw_ksplit = 0;      // "mmfw_mt", "mmfw_ksplit": activation tiles per workgroup, slices of K (0 = by the shape)
     hipFunction_t mmfs[2][2] = {};              // its streamed form [0 = Q4_K, 1 = Q5_K][bf16 mode]
-    hipFunction_t mmfr[2] = {};                 // the streamed form whose waves prepare their own activations (f32, 9 to 16 rows) [0 = Q4_K, 1 = Q5_K]
+    hipFunction_t mmfr[2][2] = {};              // the streamed form whose waves prepare their own activations (9 to 16 rows) [0 = Q4_K, 1 = Q5_K][f32, 16-bit]
     bool use_mmfr = true;                       // "mmfr" = 0: never
     uint32_t mmfr_min_rows = 8;                 // "mmfr_min_rows": fewest weight rows per CU that take it
     hipFunction_t mm8c[3][2][2] = {};           // chains of streamed matmuls in one launch [0 = Q4_K, 1 = Q5_K, 2 = Q8_0][some entry in pairs of blocks][some entry waits for the one before it]
@@ -1432,7 +1432,7 @@ int run_mmfs(gllmq_ctx *ctx, Scratch &S, const Format &f, const uint8_t *w, cons
     return GLLMQ_OK;
 }
 
-// Q4_K and Q5_K, 9 to 16 rows of f32 activations, from `mmfr_min_rows` weight rows per CU up: the
+// Q4_K and Q5_K, 9 to 16 rows of plain activations, from `mmfr_min_rows` weight rows per CU up: the
 // streamed GEMM whose arithmetic waves prepare their own activations (mmfr.hip.inc), one launch and
 // nothing else.  A workgroup multiplies a slice of K of eight blocks (a block per arithmetic wave);
 // the slices of a row range meet through the scratch.  Returns -1 for what it does not take.
@@ -1442,7 +1442,7 @@ int run_mmfr(gllmq_ctx *ctx, Scratch &S, const Format &f, const uint8_t *w, cons
     const int fmt = f.dtype == T_Q5_K ? 1 : f.dtype == T_Q4_K ? 0 : -1;
     // (17 rows and more: two ways of sharing a block between two waves were built and timed slower than the three-launch form)
     if (!ctx->use_mmf || !ctx->use_mmfr || fmt < 0 || m < min_m || m > 16 || n == 0) return -1;
-    if (act_bf16 || ctx->call_elem || ctx->call_glu) return -1; // plain f32 activations and outputs
+    if (act_bf16 || ctx->call_glu) return -1; // plain activations
     const uint32_t ldx = row_stride_x(ctx, k);
     if (!aligned(x, 16) || k % 4 != 0 || ldx % 4 != 0) return -1; // activation rows are loaded as aligned float4
     const uint32_t cus = static_cast<uint32_t>(ctx->num_cus);
@@ -1498,7 +1498,8 @@ int run_mmfr(gllmq_ctx *ctx, Scratch &S, const Format &f, const uint8_t *w, cons
     P.lds_ctrl = 0;
     P.lds_ring = lds_ring;
     P.depth = depth;
-    return launch(ctx, ctx->mmfr[fmt], grid * ksplit, (gq::MMFR_CWAVES + gq::MMFR_LOADERS) * 64, lds_ring + slots * item_bytes, stream, &P,
+    P.elem = ctx->call_elem;
+    return launch(ctx, ctx->mmfr[fmt][ctx->call_elem ? 1 : 0], grid * ksplit, (gq::MMFR_CWAVES + gq::MMFR_LOADERS) * 64, lds_ring + slots * item_bytes, stream, &P,
                   sizeof P, ksplit > 1);
 }
 
@@ -1912,8 +1913,10 @@ int gllmq_init(gllmq_ctx **out, int device)
             snprintf(name, sizeof name, "gq_moe_mmf_%s%s", q == 3 ? "q8_0" : q == 2 ? "q6k" : q == 1 ? "q5k" : "q4k", b ? "_hi" : "");
             rc = get_function(ctx, &ctx->moe_mmf[q][b], name);
         }
-    if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfr[0], "gq_mmfr_q4k");
-    if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfr[1], "gq_mmfr_q5k");
+    if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfr[0][0], "gq_mmfr_q4k");
+    if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfr[0][1], "gq_mmfr_q4k_e16");
+    if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfr[1][0], "gq_mmfr_q5k");
+    if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfr[1][1], "gq_mmfr_q5k_e16");
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->moe_plan, "gq_moe_plan");
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->moe_act, "gq_moe_act");
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->moe_combine, "gq_moe_combine");

@@ -1,5 +1,5 @@
 """GPU parity of the f16 matrix-core GEMM whose arithmetic waves prepare their own activations
-(mmfr.hip.inc: Q4_K and Q5_K, 9 to 16 rows of f32 activations, from 8 weight rows per CU up;
+(mmfr.hip.inc: Q4_K and Q5_K, 9 to 16 rows of activations, from 8 weight rows per CU up;
 eight arithmetic waves with sixteen activation rows of one block of K in registers each, loader
 waves streaming the weight items through an LDS ring, the slices of K meeting inside the one
 launch) against the oracle, through the C ABI.  Reference: Backend::quantized_matmul with m > 1
@@ -100,3 +100,26 @@ def test_against_the_three_launch_form_and_what_it_leaves(hip, torch):
     w = random_weight(Q4_K, 16 * c, 1024, seed=2)
     gpu_matmul(hip, torch, w, random_activations(17, 1024, seed=1), Q4_K, 17, 16 * c, 1024)
     assert not hip.last_kernel_name().startswith("gq_mmfr_")
+
+
+@pytest.mark.parametrize("dtype", [Q4_K, Q5_K])
+@pytest.mark.parametrize("elem", ["float16", "bfloat16"])
+def test_element_types_give_the_rounded_f32_result(hip, torch, dtype, elem):
+    """16-bit activations and outputs take the same kernel: the f32 call on the widened activations, rounded, bit
+    for bit; one slice and several, last quads of a row, ragged workgroups, rows with an infinity and of zeros."""
+    c, t = cus(torch), getattr(torch, elem)
+    for m, n, k in ((16, 16 * c, 1024), (9, 24 * c + 7, 2048), (13, 9 * c + 1, 1024 - 28), (12, 8 * c, 4096 + 256), (16, 40 * c + 3, 2304)):
+        print(f"gemm rows dtype={dtype} {elem} m={m} n={n} k={k}", flush=True)
+        w = torch.from_numpy(random_weight(dtype, n, k, seed=m + n).view(np.uint8).reshape(-1)).cuda()
+        x = torch.from_numpy(random_activations(m, k, seed=k + m) * 1e-2).cuda().to(t)
+        x[3], x[5, 7] = 0.0, float("inf")
+        y, full = torch.zeros(m, n, dtype=t, device="cuda"), torch.zeros(m, n, device="cuda")
+        hip.quantized_matmul(w, x, y, dtype, m, n, k)
+        assert hip.last_kernel_name().startswith("gq_mmfr_") and hip.last_kernel_name().endswith("_e16"), hip.last_kernel_name()
+        hip.quantized_matmul(w, x.float(), full, dtype, m, n, k)
+        assert hip.last_kernel_name().startswith("gq_mmfr_")
+        torch.cuda.synchronize()
+        want = full.to(t)
+        assert torch.equal(torch.isnan(y), torch.isnan(want))
+        same = (y.view(torch.int16) == want.view(torch.int16)) | torch.isnan(y)
+        assert bool(same.all()), int((~same).sum())
