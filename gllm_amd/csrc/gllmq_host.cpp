@@ -1676,16 +1676,12 @@ int run_gemv(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
     return GLLMQ_OK;
 }
 
-// Whether 5 to 8 activation rows go to the wide GEMM.  The int8 kernels take up to eight rows of Q4_K, seven of Q5_K and
-// six of Q6_K and Q8_0 in a pass, and read the weights twice beyond that.  f32, us per call on 4096 x 14336: Q8_0 six rows
-// 24.0 (28.5 here), seven 31.6 (28.6), Q6_K seven 30.4 (27.4), Q5_K eight 26.3 (22.1); with 16-bit elements seven 35.7
-// (26.1), 34.7 (26.2), eight 30.6 (20.8).  Single matmuls of fewer weights or shorter rows stay: 14336 x 4096 f32 the same either
-// way, 2390 x 11520 Q4_K five bf16 rows 16.5 (21.0).  `one_plane`: a feed-forward block of 16-bit elements, whose other form
-// converts them in launches of its own.
-bool mmfw_takes_few(const gllmq_ctx *ctx, uint32_t dtype, size_t m, bool one_plane)
+// Whether 5 to 8 activation rows are more than the int8 kernels take in a pass (up to eight of Q4_K, seven of Q5_K and six
+// of Q6_K and Q8_0); beyond it they read the weights twice, and the wide GEMM is ahead from some size on.
+bool mmfw_takes_few(const gllmq_ctx *ctx, uint32_t dtype, size_t m)
 {
     const size_t pass = dtype == T_Q4_K ? 8 : dtype == T_Q5_K ? 7 : 6;
-    return ctx->mmfw_small_min_m <= 9 && m >= 5 && (one_plane || m > pass);
+    return ctx->mmfw_small_min_m <= 9 && m >= 5 && m > pass;
 }
 
 // One quantized matmul on validated arguments: the kernel family by format, rows and shape.
@@ -1706,7 +1702,9 @@ int dispatch_matmul(gllmq_ctx *ctx, Scratch &S, const Format &f, const uint8_t *
     // 32 bf16 rows against run_mmf's: Q6_K 14336 x 4096 24.7, 26.0 (27.7, 29.0), 4096 x 4096 18.8, 20.9 (21.3, 22.3);
     // Q8_0 14336 x 4096 24.9, 27.0 (33.0, 34.3); Q4_K 4096 x 14336 19.5, 20.8 (22.2, 22.3), 1024 x 4096 the same.
     // f32, 32 rows, Q4_K 14336 x 4096 21.2 (20.9).
-    if (!ctx->mmfs_all && (m >= ctx->mmfw_small_min_m || (!bf16 && k > 10240 && n * k >= (48ull << 20) && mmfw_takes_few(ctx, f.dtype, m, false)))) {
+    // Five to eight rows beyond a pass of the int8 kernels: f32, us per call on 4096 x 14336: Q8_0 six rows
+    // 24.0 (28.5 here), seven 31.6 (28.6), Q6_K seven 30.4 (27.4), Q5_K eight 26.3 (22.1); 14336 x 4096 the same either way.
+    if (!ctx->mmfs_all && (m >= ctx->mmfw_small_min_m || (!bf16 && k > 10240 && n * k >= (48ull << 20) && mmfw_takes_few(ctx, f.dtype, m)))) {
         const MmfwMatrix one{ w, y, n };
         rc = run_mmfw(ctx, S, f, &one, 1, x, ctx->call_elem, ctx->call_elem, m, k, bf16, stream, 5);
         if (rc >= 0 || rc == kNeedPlainActivations) return rc;
@@ -2464,8 +2462,13 @@ int ffn_on_stream(gllmq_ctx *ctx, const void *gate_w, const void *up_w, size_t g
     // Prompts and larger batches: gate and up share their activation images and run as one launch; the
     // down projection's images are prepared from the two results.
     const size_t gate_up_n[2] = { ffn, ffn };
+    // 5 to 8 rows, from 64 M gate and up weights on and whatever the element type (16-bit results are the f32 block's, rounded).
+    // us per call, int8 and GEMM, f32: Q5_K with Q6_K down eight rows 2 x 2048 x 5632 28.8, 35.1, 2 x 3072 x 8192 34.8, 40.3, 2 x 4096 x
+    // 8192 49.7, 43.6, 2 x 4096 x 14336 79, 67; Q6_K seven rows 44.1, 44.0 (3072 x 8192), 53.5, 51.3 (4096 x 8192), 88, 77 (4096 x 14336); Q8_0 45.7,
+    // 48.8, 54.3, 55.9, 95, 75.  16-bit blocks of fewer rows are ahead on the int8 kernels with conversions (Q4_K with Q6_K
+    // down 2 x 4096 x 14336, five bf16 rows 47.5, 61.1; eight 59.9, 61.7).
     const bool wide = m >= std::max(5u, std::min(ctx->mmfw_min_m, ctx->mmfw_small_min_m)) ||
-                      (ctx->ffn_fused && mmfw_takes_few(ctx, dtype_gate_up, m, elem != 0)); // ("ffn_fused" off: up to 8 rows in separate steps)
+                      (ctx->ffn_fused && 2 * ffn * hidden >= (64ull << 20) && mmfw_takes_few(ctx, dtype_gate_up, m)); // ("ffn_fused" off: up to 8 rows in separate steps)
     auto down_fits = [&] {
         MmfwPlan L = plan_mmfw(ctx, dtype_down, m, &hidden, 1, ffn, false);
         return L.ok && mmfw_fit(ctx, S, L, stream);

@@ -386,3 +386,22 @@ def test_element_types_have_the_slices_of_the_f32_call(torch, dtype, n, k, rows,
         print(f"slices dtype={dtype} m={m} n={n} k={k} {elem}", flush=True)
         got, want = rounded_f32_call(torch, hip, w, x[:m].contiguous(), dtype, m, n, k)
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("t_gu, t_dn", [(Q4_K, Q6_K), (Q5_K, Q6_K), (Q6_K, Q6_K), (Q8_0, Q8_0)])
+@pytest.mark.parametrize("hidden, ffn", [(1024, 1280), (4096, 8192)])
+def test_feed_forward_of_16_bit_elements_is_the_rounded_f32_block(torch, t_gu, t_dn, hidden, ffn):
+    """Whatever kernels the rows and the size take: the int8 kernels and the GEMM for 5 to 8 rows, the GEMM beyond."""
+    from gllm_amd.backend import HipBackend
+    hip = HipBackend(0)
+    g, u, d = (torch.from_numpy(random_weight(t, a, b, seed=i).view(np.uint8).reshape(-1)).cuda()
+               for i, (t, a, b) in enumerate(((t_gu, ffn, hidden), (t_gu, ffn, hidden), (t_dn, hidden, ffn))))
+    for m in (1, 4, 5, 6, 7, 8, 9, 24, 70):
+        for t in (torch.float16, torch.bfloat16):
+            print(f"ffn {t_gu}/{t_dn} {hidden} {ffn} m={m} {t}", flush=True)
+            x = (torch.from_numpy(random_activations(m, hidden, seed=m)) * 1e-2).cuda().to(t)
+            out, full = torch.zeros(m, hidden, dtype=t, device="cuda"), torch.zeros(m, hidden, device="cuda")
+            hip.ffn_swiglu(g, u, t_gu, d, t_dn, x, out, m, hidden, ffn)
+            hip.ffn_swiglu(g, u, t_gu, d, t_dn, x.float(), full, m, hidden, ffn)
+            torch.cuda.synchronize()
+            assert torch.equal(out.view(torch.int16), full.to(t).view(torch.int16))
