@@ -1702,9 +1702,13 @@ int dispatch_matmul(gllmq_ctx *ctx, Scratch &S, const Format &f, const uint8_t *
     // 32 bf16 rows against run_mmf's: Q6_K 14336 x 4096 24.7, 26.0 (27.7, 29.0), 4096 x 4096 18.8, 20.9 (21.3, 22.3);
     // Q8_0 14336 x 4096 24.9, 27.0 (33.0, 34.3); Q4_K 4096 x 14336 19.5, 20.8 (22.2, 22.3), 1024 x 4096 the same.
     // f32, 32 rows, Q4_K 14336 x 4096 21.2 (20.9).
-    // Five to eight rows beyond a pass of the int8 kernels: f32, us per call on 4096 x 14336: Q8_0 six rows
-    // 24.0 (28.5 here), seven 31.6 (28.6), Q6_K seven 30.4 (27.4), Q5_K eight 26.3 (22.1); 14336 x 4096 the same either way.
-    if (!ctx->mmfs_all && (m >= ctx->mmfw_small_min_m || (!bf16 && k > 10240 && n * k >= (48ull << 20) && mmfw_takes_few(ctx, f.dtype, m)))) {
+    // Five to eight rows beyond a pass of the int8 kernels: from 10240 elements a row and 40 M weights on.  f32, us per call, here and in
+    // brackets there (eight rows of Q5_K, seven of Q6_K and of Q8_0): 4096 x 10240 20.1 (21.4), 23.6 (24.2), 24.3 (24.9); 4096 x 11520 20.5 (24.6), 25.3
+    // (28.7), 25.2 (29.9); 14336 x 14336 54.7 (66.2), 71.6 (86.4), 69.6 (96.0); below, 2390 x 11520 23.4 (18.7), 26.9 (20.0), 26.4 (20.1); 4096 x 6144 17.6
+    // (16.6), 19.8 (17.7), 20.3 (18.3); 8192 x 8192 22.3 (23.3), 27.2 (27.6), 28.0 (29.5); 28672 x 8192 60.5 (57.5), 77.2 (79.1), 75.9 (89.9); 28672 x 4096
+    // 31.1 (30.3), 44.3 (40.5), 44.8 (47.0).  16-bit calls gain more (8192 x 8192 21.0 (27.4), 25.7 (31.5), 25.4 (33.3)), but share the f32 call's bits
+    // and so its kernel.  In a pass: Q8_0 six rows of 4096 x 14336 28.5 (24.0).
+    if (!ctx->mmfs_all && (m >= ctx->mmfw_small_min_m || (!bf16 && k >= 10240 && n * k >= (40ull << 20) && mmfw_takes_few(ctx, f.dtype, m)))) {
         const MmfwMatrix one{ w, y, n };
         rc = run_mmfw(ctx, S, f, &one, 1, x, ctx->call_elem, ctx->call_elem, m, k, bf16, stream, 5);
         if (rc >= 0 || rc == kNeedPlainActivations) return rc;
@@ -2738,7 +2742,8 @@ int run_group(gllmq_ctx *ctx, Scratch &S, const gllmq_matmul_desc *descs, size_t
         n[i] = d.n;
     }
     const uint32_t elem = (first.flags & GLLMQ_DESC_ELEM_F16) ? GLLMQ_ELEM_F16 : (first.flags & GLLMQ_DESC_ELEM_BF16) ? GLLMQ_ELEM_BF16 : 0u;
-    if (first.m <= 4) {
+    // Lines by measurement, us per call, one by one and here, two and three matrices over the same rows.
+    if (first.m <= 4) { // rows of up to 4096 elements, any number of weight rows: f32, one row, Q4_K 2 x 14336 x 4096 12.5, 11.9 (a chain before), 2 x 28672 26.1, 24.4, Q8_0 25.0, 24.3, 47.5, 46.2; four rows Q4_K 17.9, 13.5, 29.4, 27.1
         gq::Mm8sGroupParams G{};
         G.segs = static_cast<uint32_t>(len);
         size_t rows = 0;
@@ -2755,6 +2760,15 @@ int run_group(gllmq_ctx *ctx, Scratch &S, const gllmq_matmul_desc *descs, size_t
         // 24.7 (41.2), 23.1 (34.3); 8192 + 2 x 1024 rows of 8192 Q4_K 28.7 (32.6), 27.0 (39.1), but two f32 rows 28.5 (27.2).
         if (rc >= 0 || first.k <= 4096 || first.m < (elem ? 2u : 3u) || ctx->mmfw_small_min_m > 9) return rc;
     }
+    size_t n_sum = 0;
+    for (size_t i = 0; i < len; ++i) n_sum += n[i];
+    // The GEMM.  Up to eight rows it takes up to 72 and 48 weight tiles, beyond which its few slices of K leave the int8 kernels ahead: three f32
+    // rows Q4_K 3 x 6144 x 6144 33.1, 27.7, 3 x 8192 x 8192 39.8, 50.0, 2 x 14336 x 4352 26.0, 28.7; five rows 3 x 4096 x 4096 28.8, 20.2, 2 x 8192 x 4096 19.8,
+    // 21.9 (Q6_K 25.1, 27.2), 2 x 28672 x 4096 41.7, 50.0.
+    if (first.m <= 8 && n_sum > (first.m <= 4 ? 72u : 48u) * gq::MMFW_TILE_ROWS) return -1;
+    // Nine to sixteen rows of Q4_K and Q5_K, which have a one-launch kernel alone: up to 128 M weights.  Nine f32 rows 2 x 14336 x 4096 31.3, 27.8 and 34.1, 33.9;
+    // 2 x 14336 x 8192 47.6, 53.0 and 53.7, 62.2; 2 x 28672 x 4096 48.9, 50.3 and 54.0, 57.6.
+    if (first.m >= 9 && first.m <= 16 && (first.ggml_dtype == T_Q4_K || first.ggml_dtype == T_Q5_K) && n_sum * first.k > (128ull << 20)) return -1;
     return run_mmfw(ctx, S, *f, mats, static_cast<int>(len), first.x_dev, elem, elem, first.m, first.k, false, stream, 2);
 }
 
@@ -2840,7 +2854,7 @@ int gllmq_quantized_matmul_batch(gllmq_ctx *ctx, const gllmq_matmul_desc *descs,
         rc = launch_prefetch(ctx, touch);
         if (rc != GLLMQ_OK) return rc;
     }
-    size_t unit = 0;
+    size_t unit = 0, alone = 0; // `alone`: entries before this one are of a group that no launch takes
     for (size_t i = 0; i < count && rc == GLLMQ_OK; ++i) {
         const gllmq_matmul_desc &d = descs[i];
         while (unit < units.size() && units[unit].first < i) ++unit;
@@ -2864,7 +2878,7 @@ int gllmq_quantized_matmul_batch(gllmq_ctx *ctx, const gllmq_matmul_desc *descs,
                 continue;
             }
         }
-        const size_t group = chain >= 2 ? 0 : group_length(ctx, descs + i, count - i);
+        const size_t group = chain >= 2 || i < alone ? 0 : group_length(ctx, descs + i, count - i);
         if (group >= 2) {
             ctx->overlap.entry_first = !(d.flags & GLLMQ_DESC_AFTER_PREVIOUS);
             const int grc = run_group(ctx, *S, descs + i, group, stream);
@@ -2873,6 +2887,7 @@ int gllmq_quantized_matmul_batch(gllmq_ctx *ctx, const gllmq_matmul_desc *descs,
                 i += group - 1;
                 continue;
             }
+            alone = i + group;
         }
         constexpr uint32_t kElemBits = GLLMQ_DESC_ELEM_F16 | GLLMQ_DESC_ELEM_BF16;
         if ((d.flags & ~(static_cast<uint32_t>(GLLMQ_DESC_AFTER_PREVIOUS) | kElemBits)) || (d.flags & kElemBits) == kElemBits) {

@@ -405,3 +405,26 @@ def test_feed_forward_of_16_bit_elements_is_the_rounded_f32_block(torch, t_gu, t
             hip.ffn_swiglu(g, u, t_gu, d, t_dn, x.float(), full, m, hidden, ffn)
             torch.cuda.synchronize()
             assert torch.equal(out.view(torch.int16), full.to(t).view(torch.int16))
+
+
+@pytest.mark.parametrize("dtype, m, k, sizes, one", [
+    (Q4_K, 5, 512, [8192, 4096], True), (Q4_K, 5, 512, [8192, 4097], False), (Q6_K, 8, 256, [4096, 4096, 4096], True), (Q6_K, 8, 256, [4096, 4096, 4097], False),
+    (Q5_K, 3, 4352, [9216, 9216], True), (Q5_K, 3, 4352, [9216, 9217], False), (Q4_K, 16, 4096, [16384, 16384], True), (Q4_K, 16, 4096, [16384, 16385], False),
+    (Q8_0, 9, 4096, [16384, 16385], True)])
+def test_lines_of_the_launch_over_several_matrices(torch, dtype, m, k, sizes, one):
+    """On both sides of the most weight rows that the GEMM takes as one launch."""
+    from gllm_amd.backend import HipBackend
+    hip = HipBackend(0)
+    x = torch.from_numpy(random_activations(m, k, seed=3)).cuda()
+    dev = [torch.from_numpy(random_weight(dtype, n, k, seed=n + i).view(np.uint8).reshape(-1)).cuda() for i, n in enumerate(sizes)]
+    ys, alone = ([torch.full((m, n), float("nan"), device="cuda") for n in sizes] for _ in range(2))
+    print(f"lines dtype={dtype} m={m} k={k} {sizes}", flush=True)
+    for d, y, n in zip(dev, alone, sizes):
+        hip.quantized_matmul(d, x, y, dtype, m, n, k)
+    hip.run_batch(hip.make_batch([(d, x, y, dtype, m, n, k) for d, y, n in zip(dev, ys, sizes)]))
+    torch.cuda.synchronize()
+    for a, b in zip(ys, alone):
+        if one:
+            assert float((a - b).norm() / b.norm()) <= 4e-6 # (the int8 kernels' 1.2e-6, twice, over the GEMM's)
+        else:
+            assert torch.equal(a, b)
