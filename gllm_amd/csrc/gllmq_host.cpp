@@ -2780,16 +2780,28 @@ void plan_prefetch(gllmq_ctx *ctx, Scratch &S, const gllmq_matmul_desc *descs, s
                    std::vector<BatchUnit> &units, std::vector<gq::TouchEntry> &touch)
 {
     constexpr uint32_t kKnown = GLLMQ_DESC_AFTER_PREVIOUS | GLLMQ_DESC_ELEM_F16 | GLLMQ_DESC_ELEM_BF16;
+    size_t alone = 0; // as in gllmq_quantized_matmul_batch, whose launches these are
     for (size_t i = 0; i < count;) {
         BatchUnit u{ i, 1, true, false, 0 };
         const size_t chain = chain_length(ctx, descs + i, count - i);
-        if (chain >= 2) {
+        const size_t group = i < alone && chain < 2 ? 0 : group_length(ctx, descs + i, chain >= 2 ? chain : count - i);
+        const bool starts_anywhere = !(descs[i].flags & GLLMQ_DESC_AFTER_PREVIOUS) && i > 0 && ctx->batch_overlap;
+        DispatchChoice c{};
+        if (group >= 2 && (chain < 2 || group == chain)) c = dispatch_choice(ctx, [&] { return run_group(ctx, S, descs + i, group, stream); });
+        if (c.launches) { // several matrices over the same rows: one number, that of the launch
+            u.len = group;
+            u.ordered = !starts_anywhere;
+            u.announces = c.fn != nullptr && ctx->announces.count(c.fn) != 0;
+        } else if (chain >= 2) {
             u.len = chain;
             u.announces = true;
-        } else if (!(descs[i].flags & ~kKnown)) {
-            u.ordered = (descs[i].flags & GLLMQ_DESC_AFTER_PREVIOUS) != 0 || i == 0 || !ctx->batch_overlap;
-            const DispatchChoice c = dispatch_choice(ctx, [&] { return batch_entry(ctx, S, descs[i], stream); });
-            u.announces = c.fn != nullptr && ctx->announces.count(c.fn) != 0;
+        } else {
+            if (group >= 2) alone = i + group;
+            if (!(descs[i].flags & ~kKnown)) {
+                u.ordered = !starts_anywhere;
+                c = dispatch_choice(ctx, [&] { return batch_entry(ctx, S, descs[i], stream); });
+                u.announces = c.fn != nullptr && ctx->announces.count(c.fn) != 0;
+            }
         }
         u.seq = ++ctx->launch_seq;
         units.push_back(u);

@@ -309,6 +309,35 @@ def test_the_weight_prefetch_beside_dependent_launches_changes_no_bit(torch):
     assert torch.equal(ya.view(torch.int32), yb.view(torch.int32))
 
 
+@pytest.mark.parametrize("elem,m", [("bfloat16", 1), ("float32", 1), ("float16", 4)])
+def test_the_weight_prefetch_waits_for_no_entry_of_a_shared_launch(torch, elem, m):
+    """Projections over the same rows are one launch, which announces one number: the prefetch behind them has to know.  A wait
+    for the number of an entry that is never launched would last the whole time-out, half a second here; the stream
+    waits behind the prefetch."""
+    import time
+
+    from gllm_amd.backend import HipBackend
+    hip = HipBackend(0, options={"prefetch": 1, "prefetch_min_kib": 1, "batch_overlap": 0, "prefetch_timeout_us": 500000})
+    plain, t, k, ns = HipBackend(0), getattr(torch, elem), 4096, [4096, 6144, 6144, 8192]
+    xs = [torch.from_numpy(random_activations(m, k, seed=s) * 1e-2).cuda().to(t) for s in (1, 2)]
+    ws = [dev_weight(torch, random_weight(Q4_K, n, k, seed=i)) for i, n in enumerate(ns)]
+    for after in (lambda i: i == 1, None):
+        outs = []
+        for backend in (hip, plain):
+            ys = [torch.full((m, n), float("nan"), dtype=t, device="cuda") for n in ns]
+            batch = backend.make_batch([(w, xs[min(i, 1)], y, Q4_K, m, n, k) for i, (w, y, n) in enumerate(zip(ws, ys, ns))], after_previous=after)
+            print(f"prefetch over a shared launch {elem} m={m}", flush=True)
+            backend.run_batch(batch)
+            torch.cuda.synchronize()
+            start = time.monotonic()
+            backend.run_batch(batch)
+            torch.cuda.synchronize()
+            assert time.monotonic() - start < 0.25
+            outs.append(ys)
+        for a, b in zip(*outs):
+            assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dtype,m", [(Q4_K, 1), (Q5_K, 2), (Q8_0, 1)])
 def test_open_requests_per_loader_change_no_bit(torch, dtype, m):
     """By default a loader of the chained launch keeps one item open on entries of full tiles and
