@@ -241,7 +241,7 @@ struct gllmq_ctx {
     hipFunction_t mmf_prep_lanes = nullptr;     // the images of the streamed form
     hipFunction_t mmf_prep[2] = {};             // its activation preparation [32-row activation tiles - 1]
     hipFunction_t mmf_reduce = nullptr;         // and the in-order sum of its K-split partial results
-    hipFunction_t moe_plan = nullptr, moe_act = nullptr, moe_combine = nullptr, moe_route = nullptr;
+    hipFunction_t moe_plan = nullptr, moe_plan_few = nullptr, moe_act = nullptr, moe_combine = nullptr, moe_route = nullptr;
     hipFunction_t moe_gemv[kNumFormats] = {};
     hipFunction_t moe_mm8_fn[MM8_KINDS][2] = {}; // grouped int8 matrix-core kernels [Mm8Kind][passes per tile - 1]
     hipFunction_t moe_mm8_q6k_rows = nullptr;   // Q6_K rows of at most 8 blocks: a wave per 32-row tile
@@ -1920,6 +1920,7 @@ int gllmq_init(gllmq_ctx **out, int device)
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfr[1][0], "gq_mmfr_q5k");
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfr[1][1], "gq_mmfr_q5k_e16");
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->moe_plan, "gq_moe_plan");
+    if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->moe_plan_few, "gq_moe_plan_few");
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->moe_act, "gq_moe_act");
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->moe_combine, "gq_moe_combine");
     for (int i = 0; i < kNumFormats && rc == GLLMQ_OK; ++i) {
@@ -3015,6 +3016,11 @@ int launch_moe_plan(gllmq_ctx *ctx, MoePlanParams &P, const uint32_t *route_expe
     P.top_k = static_cast<uint32_t>(top_k);
     P.experts = static_cast<uint32_t>(experts);
     P.pairs = static_cast<uint32_t>(tokens * top_k);
+    if (P.pairs <= gq::MOE_PLAN_FEW) { // (from 256 pairs on the two take the same time)
+        const uint32_t padded = (P.pairs + 63u) & ~63u;
+        const uint32_t threads = std::max(padded, std::min(gq::MOE_PLAN_FEW_THREADS, (P.experts + 63u) & ~63u));
+        return launch(ctx, ctx->moe_plan_few, 1, threads, (2u * P.experts + 2u * padded + 16u) * 4u, stream, &P, sizeof P);
+    }
     // a wave per 64 pairs up to 16, as far as their counts (a word per expert each) fit the LDS; no
     // fewer than four, which share the rest of the work
     uint32_t waves = std::min<uint32_t>(gq::MOE_PLAN_THREADS / 64, std::max(4u, (P.pairs + 63u) / 64u));

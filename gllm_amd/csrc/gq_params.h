@@ -627,6 +627,8 @@ struct MoeWideJob {
 };
 
 constexpr int MOE_PLAN_THREADS = 1024;
+constexpr uint32_t MOE_PLAN_FEW = 192, MOE_PLAN_FEW_THREADS = 256; // most pairs of gq_moe_plan_few, a thread each
+static_assert(MOE_PLAN_FEW <= 255, "counts of a byte");
 
 struct MoePlanParams {
     const uint32_t *route_expert; // [tokens][top_k]

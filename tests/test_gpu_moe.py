@@ -331,3 +331,39 @@ def test_plan_of_more_pairs_than_the_lds_holds(torch):
     torch.cuda.synchronize()
     # (a row's sums do not depend on the rows it is multiplied with, up to the small products' own accumulators)
     assert float((got - want).norm() / want.norm()) <= 1e-6
+
+
+@pytest.mark.parametrize("options, dtype", [({"moe_streamed": 2, "moe_wide": 0}, Q4_K), ({"moe_streamed": 0, "moe_wide": 0}, Q4_K), ({"moe_wide": 0}, 8), ({"moe_wide_min": 1}, Q4_K)])
+def test_plan_of_few_pairs_is_the_plan_of_many(torch, options, dtype):
+    """Up to 192 pairs are planned by a thread each.  The same tokens with others behind them that are routed nowhere go through
+    the plan of many: the same rows, for one pair and for every number of waves, experts that nobody
+    chooses, more experts than threads, tokens of no route, experts that are not there."""
+    from gllm_amd.backend import HipBackend
+    hip, hidden, ffn = HipBackend(0, options=options), 256, 256
+    rng = np.random.default_rng(7)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    for tokens, top_k, experts in ((1, 1, 1), (1, 8, 8), (3, 5, 40), (16, 4, 8), (13, 5, 3), (32, 6, 300), (48, 4, 60), (191, 1, 2), (24, 8, 64)):
+        if "moe_wide_min" in options and tokens * top_k < experts:
+            continue
+        print(f"plan tokens={tokens} top_k={top_k} experts={experts} {options}", flush=True)
+        gate_up = dev(random_weight(dtype, experts * 2 * ffn, hidden, seed=1).view(np.uint8).reshape(-1))
+        down = dev(random_weight(dtype, experts * hidden, ffn, seed=2).view(np.uint8).reshape(-1))
+        many = tokens + 193 // top_k + 1
+        x = dev(random_activations(many, hidden, seed=3) * 1e-3)
+        expert = np.stack([rng.permutation(max(experts, top_k))[:top_k] for _ in range(many)]).astype(np.int32)
+        expert[rng.random(expert.shape) < 0.1] = experts + 5  # (routes nowhere)
+        length = rng.integers(0, top_k + 1, many).astype(np.int32)
+        length[:max(1, tokens // 2)] = top_k
+        length[tokens:] = 0
+        weight = rng.uniform(0.1, 1.0, (many, top_k)).astype(np.float32)
+        outs = []
+        for count in (tokens, many):
+            out = torch.full((count, hidden), float("nan"), device="cuda")
+            hip.moe_matvec(gate_up, dtype, down, dtype, x[:count].contiguous(), out, hidden, ffn, experts, dev(expert[:count]), dev(weight[:count]), dev(length[:count]))
+            outs.append(out)
+        torch.cuda.synchronize()
+        assert not bool(outs[1][tokens:].any())
+        if dtype == 8:  # the GEMV, whose waves share rows by the number of pairs: sums in another order, of two products of errors of about 1e-6
+            assert float((outs[0] - outs[1][:tokens]).norm()) <= 4e-6 * float(outs[0].norm())
+        else:
+            assert torch.equal(outs[0], outs[1][:tokens])
