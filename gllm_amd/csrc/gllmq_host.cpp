@@ -3540,10 +3540,9 @@ int gllmq_reserve_moe(gllmq_ctx *ctx, size_t tokens, size_t top_k, size_t hidden
     Scratch *S = nullptr;
     int rc = acquire_scratch(ctx, stream, &S);
     if (rc != GLLMQ_OK || tokens == 0 || top_k == 0) return rc;
-    // (the GEMM form is for calls with at least moe_wide_min pairs per expert)
+    // (the GEMM form is for calls with at least moe_wide_min pairs per expert, half as many of Q8_0, and takes the more the more experts)
     const size_t pairs = tokens * top_k, most_experts = std::max<size_t>(1, 2 * pairs / ctx->moe_wide_min);
-    size_t need = moe_workspace(pairs, hidden, ffn).total;
-    for (size_t e = most_experts; e > 0; e /= 2) need = std::max(need, plan_moe_wide(pairs, hidden, ffn, e, false).total);
+    const size_t need = std::max(moe_workspace(pairs, hidden, ffn).total, plan_moe_wide(pairs, hidden, ffn, most_experts, false).total);
     return grow_scratch(ctx, *S, &S->moe, &S->moe_bytes, need, stream, "reserve_moe");
 }
 

@@ -58,6 +58,20 @@ __device__ __forceinline__ void store_elem(float *y, size_t idx, float v, uint32
     else reinterpret_cast<uint16_t *>(y)[idx] = f32_to_elem16(v, elem);
 }
 
+// Largest value of the wave, in every lane.
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v)
+{
+#define GQ_DPP_MAX(CTRL, ROWS) v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, ROWS, 0xF, false)))
+    GQ_DPP_MAX(0x111, 0xF); // row_shr:1, 2, 4, 8: lane 15 of each row of 16
+    GQ_DPP_MAX(0x112, 0xF);
+    GQ_DPP_MAX(0x114, 0xF);
+    GQ_DPP_MAX(0x118, 0xF);
+    GQ_DPP_MAX(0x142, 0xA); // row_bcast:15
+    GQ_DPP_MAX(0x143, 0xC); // row_bcast:31
+#undef GQ_DPP_MAX
+    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), 63));
+}
+
 // Eight consecutive activations from element `idx` on (16-byte aligned for f32 and for 16-bit
 // elements alike: two quads or one).
 __device__ __forceinline__ void load_elem8(const float *x, size_t idx, uint32_t elem, float (&v)[8])
