@@ -1698,10 +1698,12 @@ int dispatch_matmul(gllmq_ctx *ctx, Scratch &S, const Format &f, const uint8_t *
     if (rc >= 0) return rc;
     rc = run_mmfs(ctx, S, f, w, x, y, m, n, k, bf16, stream);
     if (rc >= 0 || rc == kNeedPlainActivations) return rc;
-    // 9 to 32 rows of what the streamed GEMMs leave: one row tile of the GEMM for more rows.  us per call at 16 and
-    // 32 bf16 rows against run_mmf's: Q6_K 14336 x 4096 24.7, 26.0 (27.7, 29.0), 4096 x 4096 18.8, 20.9 (21.3, 22.3);
-    // Q8_0 14336 x 4096 24.9, 27.0 (33.0, 34.3); Q4_K 4096 x 14336 19.5, 20.8 (22.2, 22.3), 1024 x 4096 the same.
-    // f32, 32 rows, Q4_K 14336 x 4096 21.2 (20.9).
+    // 9 to 32 rows of what the streamed GEMMs leave: row tiles of the GEMM for more rows.  us per call with weights that are
+    // not in the caches, f32 and bf16, against run_mmf's in brackets.  32 rows: Q6_K 13824 x 5120 36.5, 34.6 (41.0, 40.8),
+    // 4096 x 4096 21.3, 20.7 (22.7, 22.6); Q8_0 14336 x 4096 31.7, 30.1 (36.5, 36.1); Q4_K 13824 x 5120 28.0, 26.0 (29.3,
+    // 28.6), 14336 x 4096 25.6, 23.7 (25.3, 24.3).  It is not ahead everywhere: of Q4_K and Q5_K with 17 to 32 rows f32 calls
+    // of k = 4096 are 1 to 8 % behind (28672 x 4096 34.3 (33.5), 39.8 (37.3)) where bf16 calls of Q4_K are up to 6 % ahead
+    // (31.2 (33.0)) and of Q5_K level (37.2 (37.1)); both take one kernel, so that they share their bits.
     // Five to eight rows beyond a pass of the int8 kernels: from 10240 elements a row and 40 M weights on.  f32, us per call, here and in
     // brackets there (eight rows of Q5_K, seven of Q6_K and of Q8_0): 4096 x 10240 20.1 (21.4), 23.6 (24.2), 24.3 (24.9); 4096 x 11520 20.5 (24.6), 25.3
     // (28.7), 25.2 (29.9); 14336 x 14336 54.7 (66.2), 71.6 (86.4), 69.6 (96.0); below, 2390 x 11520 23.4 (18.7), 26.9 (20.0), 26.4 (20.1); 4096 x 6144 17.6

@@ -104,14 +104,15 @@ const char *gllmq_version(void);
  * Development switches (UNSTABLE: they exist so that the test-suite and the measurements can reach
  * every kernel family through the public entry points; names and meaning may change with any
  * version, and a production caller should set none of them):
- *   kernel families on/off: "gemv_f32", "mm8", "mmf", "mm8s", "mm8s_q8_0", "mmfs", "mmfr",
- *     "moe_mm8", "moe_mm8_q6k", "moe_mm8_rows", "moe_glu", "moe_streamed", "lm_head_fused",
+ *   kernel families on/off: "gemv_f32", "mm8", "mmf", "mm8s", "mm8s_q8_0", "mmfs", "mmfr", "mmfw",
+ *     "moe_wide", "moe_mm8", "moe_mm8_q6k", "moe_mm8_rows", "moe_glu", "moe_streamed", "lm_head_fused",
  *     "elem_fused", "ffn_glu_load", "ffn_streamed", "mm8s_areg", "mm8s_fold", "mm8s_split",
  *     "mm8_small_to_gemv"
  *   shape thresholds: "mm8s_min_rows", "mmfs_min_rows", "mmfr_min_rows", "chain_min_rows",
+ *     "mmfw_min_m", "mmfw_small_min_m", "moe_wide_min",
  *     "mm8_q5k_min_m", "mm8_q6k_min_m", "mm8_q8_0_min_m", "mmf_small_min_m", "mm8_ksplit",
  *     "mm8s_all", "mmfs_all" (1: that form wherever the shape fits it, also where another was timed faster)
- *   launch parameters: "mm8s_depth", "moe_depth", "moe_slices", "prefetch_wgs", "prefetch_threads",
+ *   launch parameters: "mmfw_mt", "mmfw_ksplit", "mm8s_depth", "moe_depth", "moe_slices", "prefetch_wgs", "prefetch_threads",
  *     "prefetch_timeout_us", "prefetch_flags", "prefetch_announce", "prefetch_min_kib" */
 int gllmq_set_option(gllmq_ctx *ctx, const char *name, long value);
 /* Name of the kernel the context launched last ("" before the first launch): lets a profile be
@@ -119,7 +120,10 @@ int gllmq_set_option(gllmq_ctx *ctx, const char *name, long value);
 const char *gllmq_last_kernel_name(const gllmq_ctx *ctx);
 
 /* Sizes the stream's scratch for a later call of that shape, so that the call itself allocates
- * nothing (needed before a stream capture).  No counterpart in the reference, whose scratch is
+ * nothing (needed before a stream capture).  What the GEMM needs depends on m and k alone, and 33 rows
+ * serve any number (a captured call of more goes in passes, with the same bits), so one reserved or
+ * eager call per k covers other matrices, element types and batches over the same rows too.  No
+ * counterpart in the reference, whose scratch is
  * sized when the graph is compiled (src/compat/gpu_backend_macro.rs:82-87). */
 int gllmq_reserve_matmul(gllmq_ctx *ctx, uint32_t ggml_dtype, size_t m, size_t n, size_t k, void *stream);
 int gllmq_reserve_ffn(gllmq_ctx *ctx, uint32_t dtype_gate_up, uint32_t dtype_down, size_t m, size_t hidden,
@@ -171,9 +175,12 @@ int gllmq_quant_gather_elem(gllmq_ctx *ctx, const void *table_dev, size_t table_
  * each of gate_up_bytes_each bytes; Wdown is [hidden x ffn] of dtype_down; x and out are f32.
  * Q4_K / Q5_K gate and up with up to 8 rows run as ONE launch of the int8 matrix-core kernel
  * with the activation in its epilogue (a workgroup runs the gate tile and the up tile of a
- * row range back to back); other shapes run the two products (one matmul when the up rows
- * follow the gate rows in memory), an activation kernel and the down projection, each with
- * the kernels gllmq_quantized_matmul would pick.  Intermediates live in the stream's scratch. */
+ * row range back to back); more than 8 rows, and 5 to 8 that such a kernel would take in two
+ * passes over large matrices, run gate and up as one launch of the f16 matrix-core GEMM, whose
+ * down projection applies the activation while it prepares its own; other shapes run the two
+ * products (one matmul when the up rows follow the gate rows in memory), an activation kernel
+ * and the down projection, each with the kernels gllmq_quantized_matmul would pick.
+ * Intermediates live in the stream's scratch. */
 int gllmq_ffn_swiglu(gllmq_ctx *ctx, const void *gate_dev, const void *up_dev, size_t gate_up_bytes_each,
                      uint32_t dtype_gate_up, const void *down_dev, size_t down_bytes, uint32_t dtype_down,
                      const float *x_dev, float *out_dev, size_t m, size_t hidden, size_t ffn, int relu_gate,
@@ -186,7 +193,8 @@ int gllmq_ffn_swiglu(gllmq_ctx *ctx, const void *gate_dev, const void *up_dev, s
  * exactly; the block runs in f32 as gllmq_ffn_swiglu does; out = round(result) or
  * out = round(widen(out) + result), one rounding to nearest, ties to even (f32: none beyond the
  * addition's).  Bit for bit: the result of gllmq_ffn_swiglu on the widened activations, added and
- * rounded.  The conversions are small launches of their own around the block's kernels. */
+ * rounded.  Where gate, up and down run on the GEMM and nothing is added, its kernels convert; elsewhere
+ * the conversions are small launches of their own around the block's kernels. */
 #define GLLMQ_OUT_ACCUMULATE 1
 int gllmq_ffn_swiglu_elem(gllmq_ctx *ctx, const void *gate_dev, const void *up_dev, size_t gate_up_bytes_each,
                           uint32_t dtype_gate_up, const void *down_dev, size_t down_bytes, uint32_t dtype_down,
@@ -212,8 +220,9 @@ int gllmq_argmax(gllmq_ctx *ctx, const float *logits_dev, size_t rows, size_t n,
  * x_dev holds m x k and y_dev m x n elements of type `elem`; 16-bit activations widen exactly,
  * the arithmetic is that of gllmq_quantized_matmul, and a result is rounded to the nearest
  * element, ties to even (what E::from_f32 does; NaN stays NaN, f16 overflows to infinity): y is
- * bit for bit the rounded result of the f32 call on the widened activations.  The streamed
- * kernels, the GEMV (rows that are aligned vectors, k <= 16384) and the GEMM convert in their own
+ * bit for bit the rounded result of the f32 call on the widened activations (at a 16-byte aligned
+ * address, which the fast kernels need).  The streamed
+ * kernels, the GEMV (rows that are aligned vectors, k <= 16384) and the GEMMs convert in their own
  * loads and stores; other shapes take a widening and a rounding launch around the f32 kernels,
  * through scratch of the stream (gllmq_reserve_matmul_elem before capturing such a shape).
  * Both pointers 4-byte aligned. */
@@ -249,10 +258,11 @@ int gllmq_lm_head_argmax(gllmq_ctx *ctx, const void *w_dev, size_t w_bytes, cons
  * final sum are f32; one pass over the weights serves up to 8 activation rows.  Q5_K with 2
  * or more rows, Q6_K and Q8_0 with 3 or more run the same scheme (Q8_0: one matrix-core step
  * per 32-element block, its f16 scale applied in f32).  More than 8 rows run a GEMM on the
- * f16 matrix cores, 64 rows per pass: weights as the exact integers sc*q in f16 (Q6_K: q-32,
+ * f16 matrix cores, up to 128 rows per workgroup and all of them in one launch: weights as the exact
+ * integers sc*q in f16 (Q6_K: q-32,
  * Q8_0: q, their scales applied per 16 or 32 elements in f32), activations as two f16 terms
  * (22 significant bits) of a per-block scaled value, f32 accumulation; its activation images
- * and the partial sums of its K split live in the stream's scratch.  The GEMM also takes 3..8 rows when the rows are so
+ * and the partial sums of its K split live in the stream's scratch.  A GEMM also takes 3..8 rows when the rows are so
  * long that the prepared activations do not fit the LDS of one 8-row pass (K above about
  * 4096..12288, by format and rows).  Q5_K with one row, Q6_K and Q8_0 with one or two, and
  * Q8_0 rows shorter than 256 elements run integer-dot GEMV kernels, two activation rows per
@@ -295,11 +305,16 @@ int gllmq_quantized_matmul_noalloc(gllmq_ctx *ctx, const void *w_dev, size_t w_b
  * of each other (no entry reads what another writes): their kernels may overlap in time on the
  * device, and consecutive one- or two-row Q4_K / Q5_K entries of one K <= 4096 run as ONE launch
  * whose loaders go straight on from one matrix to the next (up to 32 entries per launch), which
- * saves the gaps between kernels and keeps the weight stream going.  An entry that does depend on the entries before it carries
+ * saves the gaps between kernels and keeps the weight stream going.  Two or three consecutive entries of
+ * one format, element type and K over the SAME rows (one x_dev: a layer's Q, K and V; gate and up) are
+ * multiplied by one launch where that is ahead (option "batch_group"); its sums are in another order than a
+ * single call's, so such an entry agrees with the single call to the error of the kernels (f32: about 1e-6
+ * of the result's norm), not bit for bit.  The same batch gives the same bits each time, also captured,
+ * once the stream's scratch is there.  An entry that does depend on the entries before it carries
  * GLLMQ_DESC_AFTER_PREVIOUS in `flags`: it starts after they have finished.  The batch as a whole
  * is ordered like any other call: it starts after the stream's earlier work and later work
  * starts after all of it.  GLLMQ_DESC_ELEM_F16 / _BF16: x_dev and y_dev of the entry hold elements
- * of that type (as for gllmq_quantized_matmul_elem; such an entry is a launch of its own). */
+ * of that type (as for gllmq_quantized_matmul_elem). */
 #define GLLMQ_DESC_AFTER_PREVIOUS 1u
 #define GLLMQ_DESC_ELEM_F16 0x100u
 #define GLLMQ_DESC_ELEM_BF16 0x200u
@@ -356,7 +371,9 @@ int gllmq_moe_route(gllmq_ctx *ctx, const float *logits_dev, size_t tokens, size
  * runs every expert on every token and masks, build_graph.inc.rs:2076-2123).  Q4_K, Q5_K and
  * Q6_K rows of at most 4096 elements run on the int8 matrix cores, all tokens of an expert
  * (eight per pass) against one read of its weights, Q4_K / Q5_K gate and up with the activation
- * in the same launch; other shapes run the integer-dot GEMV, two tokens per pass.
+ * in the same launch; other shapes run the integer-dot GEMV, two tokens per pass.  A prompt's many
+ * tokens per expert (about eight and more, four of Q8_0, where the experts are large or many enough)
+ * run the f16 matrix-core GEMM of gllmq_quantized_matmul over each expert's rows.
  * Expert e's gate rows ([ffn x hidden] blocks of dtype_gate_up) start at gate_dev +
  * e * gate_expert_stride, its up rows at up_dev + e * up_expert_stride, its down rows
  * ([hidden x ffn] of dtype_down) at down_dev + e * down_expert_stride; *_bytes are the sizes of

@@ -54,8 +54,8 @@ def test_non_finite_rows_stay_in_their_rows(torch, oracle, dtype):
 @pytest.mark.parametrize("dtype", ALL)
 @pytest.mark.parametrize("elem", ["float16", "bfloat16"])
 def test_one_plane_gives_the_bits_of_two(torch, dtype, elem):
-    """16-bit activations leave nothing for the lo plane: y is the rounded f32 result, bit for bit,
-    for values over the whole range of the element type."""
+    """16-bit activations leave nothing for the lo plane: with the same tiles and slices y is the rounded f32 result, bit for
+    bit, for values over 23 powers of two."""
     from gllm_amd.backend import HipBackend
     hip = HipBackend(0, options={"mmfw_mt": 2, "mmfw_ksplit": 2})
     m, n, k = 67, 270, 1024
@@ -204,7 +204,7 @@ def test_projections_as_one_launch(torch, oracle, dtype, m, elem):
 
 def test_group_under_capture_keeps_to_the_reserved_scratch(torch):
     """What was reserved entry by entry serves the captured batch; replays, with eager work between them, give the
-    eager results."""
+    results of the single calls (of the eager batch, bit for bit: test_captured_group_gives_the_eager_bits)."""
     from gllm_amd.backend import HipBackend
     hip = HipBackend(0)
     m, k, sizes = 24, 1024, [512, 128, 128]
