@@ -181,7 +181,7 @@ struct gllmq_ctx {
     hipModule_t modules[10] = {}; // one per embedded code object
     hipFunction_t dequant[kNumFormats][2] = {}; // [format][0 = scalar stores, 1 = float4 stores]
     hipFunction_t gather[kNumFormats][2] = {};  // quantized embedding lookup [format][0 = scalar stores, 1 = float4 stores]
-    hipFunction_t gather_e16[kNumFormats][2] = {}; // the same into rows of a 16-bit element type [format][0 = scalar stores, 1 = 8-byte stores]
+    hipFunction_t gather_e16[kNumFormats][3] = {}; // the same into rows of a 16-bit element type [format][0 = scalar stores, 1 = 8-byte stores, 2 = 16-byte stores]
     hipFunction_t finish_elem = nullptr;        // f32 result in scratch -> output of any element type, plain or added to it
     // gated form of the int8 kernels (gate and up rows in one launch, act(gate) * up out):
     // [0 = Q4_K, 1 = Q5_K][pairs 1,2,4][early steps 1,2,4] and the register-operand variants
@@ -1863,6 +1863,9 @@ int gllmq_init(gllmq_ctx **out, int device)
         if (rc != GLLMQ_OK) break;
         snprintf(name, sizeof name, "gq_gather_%s_e16_v4", kFormats[i].tag);
         rc = get_function(ctx, &ctx->gather_e16[i][1], name);
+        if (rc != GLLMQ_OK) break;
+        snprintf(name, sizeof name, "gq_gather_%s_e16_v8", kFormats[i].tag);
+        rc = get_function(ctx, &ctx->gather_e16[i][2], name);
         for (int m = 1; m <= 2 && rc == GLLMQ_OK; ++m) {
             snprintf(name, sizeof name, "gq_gemv_%s_m%d", kFormats[i].tag, m);
             rc = get_function(ctx, &ctx->gemv[i][m - 1], name);
@@ -2238,10 +2241,14 @@ int gllmq_quant_gather_elem(gllmq_ctx *ctx, const void *table, size_t table_byte
     P.count = static_cast<uint32_t>(count);
     P.scale = scale;
     P.elem = static_cast<uint32_t>(elem);
-    const int vec = aligned(out, e16 ? 8 : 16) ? 1 : 0; // hidden is a multiple of 4, so every row then is
-    // (a one-block-per-wave form as in gq_dequant_q4k_wave measured the same: 15.9 against 16.0 us)
-    return launch2d(ctx, (e16 ? ctx->gather_e16 : ctx->gather)[format_index(dtype)][vec], (P.quads_per_row + 255u) / 256u,
-                    static_cast<uint32_t>(std::min<size_t>(count, 65535)), 256, 0, stream, &P, sizeof P);
+    // hidden is a multiple of 4, so every row is as aligned as the first; of 8: 16-bit rows go in 16-byte stores
+    const int vec = e16 && aligned(out, 16) && hidden % 8 == 0 ? 2 : aligned(out, e16 ? 8 : 16) ? 1 : 0;
+    // As many rows per workgroup as let all of them be on the chip at once (eight workgroups of 256 threads a CU).
+    const uint32_t runs = vec == 2 ? P.quads_per_row / 2u : P.quads_per_row, across = (runs + 255u) / 256u, round = 8u * static_cast<uint32_t>(ctx->num_cus);
+    P.rows = static_cast<uint32_t>(std::min<uint64_t>(gq::GATHER_ROWS, (static_cast<uint64_t>(across) * count + round - 1) / round));
+    const size_t groups = (count + P.rows - 1) / P.rows;
+    return launch2d(ctx, (e16 ? ctx->gather_e16[format_index(dtype)] : ctx->gather[format_index(dtype)])[vec], across,
+                    static_cast<uint32_t>(std::min<size_t>(groups, 65535)), 256, 0, stream, &P, sizeof P);
 }
 
 int gllmq_argmax(gllmq_ctx *ctx, const float *logits, size_t rows, size_t n, size_t ld, uint32_t *token, float *value,

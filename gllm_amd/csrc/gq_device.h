@@ -46,9 +46,7 @@ __device__ __forceinline__ float elem16_to_f32(uint32_t bits, uint32_t elem)
 __device__ __forceinline__ uint16_t f32_to_elem16(float v, uint32_t elem)
 {
     if (elem == ELEM_F16) return __builtin_bit_cast(uint16_t, static_cast<_Float16>(v));
-    const uint32_t b = __builtin_bit_cast(uint32_t, v);
-    if ((b & 0x7FFFFFFFu) > 0x7F800000u) return static_cast<uint16_t>((b >> 16) | 0x0040u); // NaN, made quiet
-    return static_cast<uint16_t>((b + 0x7FFFu + ((b >> 16) & 1u)) >> 16);
+    return __builtin_bit_cast(uint16_t, static_cast<__bf16>(v)); // (v_cvt_pk_bf16_f32)
 }
 
 // y[idx] of an output whose elements are of type `elem` (y is typed for the f32 case)

@@ -570,7 +570,9 @@ struct GatherParams {
     uint32_t count;
     float scale;            // 1.0f when the lookup is not scaled
     uint32_t elem;          // the 16-bit kernels: element type of out (ELEM_F16 / ELEM_BF16)
+    uint32_t rows;          // looked-up rows per workgroup, at most GATHER_ROWS
 };
+constexpr uint32_t GATHER_ROWS = 2;
 
 struct GluActParams {
     const float *g; // gate results, row r at g + r * ld

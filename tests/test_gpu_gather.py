@@ -79,6 +79,32 @@ def test_gather_padded_rows(hip, torch, oracle, dtype, hidden):
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("dtype", ALL)
+@pytest.mark.parametrize("hidden,count", [(8, 1), (36, 3), (264, 2049), (512, 2050), (4096, 1025), (4104, 5)])
+def test_gather_16_bit_rows(hip, torch, oracle, dtype, hidden, count):
+    """16-bit rows: sixteen-byte stores (rows of a multiple of eight elements, aligned), eight-byte and scalar ones; one or two
+    rows per workgroup, an odd one left over; ids outside the table among them."""
+    vocab = 77
+    table = random_weight(dtype, vocab, hidden, seed=hidden)
+    ids = np.random.default_rng(count).integers(0, vocab, count).astype(np.uint32)
+    want = torch.from_numpy(oracle.quant_gather(table, dtype, vocab, hidden, ids))
+    if count > 2:
+        ids[1], ids[-1] = vocab, 0xFFFFFFFF
+        want[1], want[-1] = float("nan"), float("nan")
+    tbuf = torch.from_numpy(np.asarray(table).view(np.uint8).reshape(-1)).cuda()
+    idd = torch.from_numpy(ids.view(np.int32)).cuda()
+    for elem in (torch.float16, torch.bfloat16):
+        for offset in (0, 4, 1):
+            print(f"gather 16 bit dtype={dtype} hidden={hidden} count={count} {elem} offset={offset}", flush=True)
+            n = count * hidden
+            buf = torch.full((offset + n + GUARD,), 7.0, dtype=elem, device="cuda")
+            hip.quant_gather(tbuf, dtype, vocab, hidden, idd, buf[offset:offset + n])
+            torch.cuda.synchronize()
+            got = buf.cpu()
+            assert bool(torch.all(got[:offset] == 7.0)) and bool(torch.all(got[offset + n:] == 7.0))
+            assert torch.allclose(got[offset:offset + n].view(count, hidden).float(), want.to(elem).float(), rtol=0, atol=0, equal_nan=True)
+
+
 def test_gather_more_rows_than_one_grid_covers(hip, torch, oracle):
     # 70000 looked-up rows: the grid's second dimension ends at 65535 and walks the rest
     vocab, hidden, count = 500, 32, 70000
