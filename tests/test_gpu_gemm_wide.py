@@ -37,6 +37,31 @@ def test_tile_edges(torch, oracle, dtype, tiles, ksplit):
             check_close(got, want, f"dtype={dtype} m={m} n={n} k={k} bf16={bf16}")
 
 
+@pytest.mark.parametrize("ksplit", [2, 4, 5, 8, 9, 15])
+@pytest.mark.parametrize("m, n", [(33, 33), (34, 1), (35, 257), (36, 260)])
+def test_sums_of_slices_at_any_place(torch, oracle, ksplit, m, n):
+    """The sums over K slices go by fours of the m x n outputs in a row, wherever they start and end: outputs at every
+    alignment of their type, a last few that are no four, nothing written around them; 16-bit outputs are the rounded f32 ones."""
+    from gllm_amd.backend import HipBackend
+    hip = HipBackend(0, options={"mmfw_mt": 1, "mmfw_ksplit": ksplit})
+    k = 256 * 15
+    w, x = random_weight(Q4_K, n, k, seed=n), random_activations(m, k, seed=m).astype(np.float16).astype(np.float32)
+    want = oracle.quantized_matmul(w, x, Q4_K, m, n, k, acc=oracle.ACC_F64, threads=16)
+    wd, xd, f32 = torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda(), None
+    for t in (torch.float32, torch.float16):
+        for offset in ((0, 1, 3) if t is torch.float32 else (0, 2, 6)):  # (outputs are four-byte aligned)
+            print(f"slices={ksplit} m={m} n={n} {t} offset={offset}", flush=True)
+            buf = torch.full((offset + m * n + 64,), 7.0, dtype=t, device="cuda")
+            hip.quantized_matmul(wd, xd.to(t), buf[offset:offset + m * n].view(m, n), Q4_K, m, n, k)
+            torch.cuda.synchronize()
+            got = buf[offset:offset + m * n].cpu().view(m, n)
+            assert bool(torch.all(buf[:offset] == 7.0)) and bool(torch.all(buf[offset + m * n:] == 7.0))
+            if f32 is None:
+                check_close(got.numpy(), want, f"slices={ksplit} m={m} n={n}")
+                f32 = got
+            assert torch.equal(got, f32.to(t))
+
+
 @pytest.mark.parametrize("dtype", ALL)
 def test_non_finite_rows_stay_in_their_rows(torch, oracle, dtype):
     from gllm_amd.backend import HipBackend
