@@ -1234,12 +1234,23 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
     return L;
 }
 
+// The sums of K slices of a feed-forward block's gate and up rows, left in the scratch for the preparation of the down
+// projection, which adds them up while it applies the gate: a launch less, and the sums' way to memory and back.
+struct MmfwSlices {
+    size_t next_need = 0;    // scratch that the down projection needs
+    const float *at = nullptr;
+    uint32_t slices = 0;     // 0: none were left
+    size_t used = 0;         // bytes of the scratch in use
+};
+
 // The GEMM over `count` matrices of one format and K that share their activations: one launch that
 // prepares the activation images, one that multiplies, and one that adds the slices of K where
 // there are any.  Returns -1 for what it does not take.
 // `elem_x`, `elem_y`: element types of the activations and of the outputs.
+// `leave`: the sums of slices may stay where they are (where both calls fit the scratch in one pass each); `take`: the
+// activations are such sums.
 int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats, int count, const float *x, uint32_t elem_x,
-             uint32_t elem_y, size_t m, size_t k, bool act_bf16, void *stream, size_t min_m)
+             uint32_t elem_y, size_t m, size_t k, bool act_bf16, void *stream, size_t min_m, MmfwSlices *leave = nullptr, const MmfwSlices *take = nullptr)
 {
     if (!ctx->use_mmf || !ctx->use_mmfw || m < min_m) return -1;
     if (!aligned(x, 16) || k % 4 != 0) return -1; // activation rows are loaded as aligned float4
@@ -1248,13 +1259,17 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
     for (int i = 0; i < count; ++i) n[i] = mats[i].n;
     const bool hi_only = act_bf16 || (elem_x && !ctx->call_glu);
     MmfwPlan L = plan_mmfw(ctx, f.dtype, m, n, count, k, hi_only);
-    if (!L.ok || !mmfw_fit(ctx, S, L, stream)) return -1;
+    if (!L.ok || (!take && !mmfw_fit(ctx, S, L, stream))) return -1;
     if (S.fixed && plan_mmf(ctx, m, n[0], k).need > S.mmf_bytes) return -1; // beyond what that entry point takes, in passes or not
     int rc = GLLMQ_OK;
-    const size_t reserve = std::max(L.need(), mmfw_reserve(ctx, m, k));
-    if (S.mmf_bytes < reserve && !S.fixed && !stream_is_capturing(stream)) rc = grow_scratch(ctx, S, &S.mmf, &S.mmf_bytes, reserve, stream, "quantized_matmul (GEMM)");
+    const bool may_leave = leave && L.ksplit > 1 && L.rows >= m;
+    const size_t used = (L.need() + 255) & ~size_t(255);
+    size_t reserve = std::max(L.need(), mmfw_reserve(ctx, m, k));
+    if (may_leave) reserve = std::max(reserve, used + leave->next_need);
+    if (!take && S.mmf_bytes < reserve && !S.fixed && !stream_is_capturing(stream)) rc = grow_scratch(ctx, S, &S.mmf, &S.mmf_bytes, reserve, stream, "quantized_matmul (GEMM)");
     if (rc != GLLMQ_OK) return rc;
-    uint8_t *scratch = static_cast<uint8_t *>(S.mmf);
+    const bool leaves = may_leave && used + leave->next_need <= S.mmf_bytes;
+    uint8_t *scratch = static_cast<uint8_t *>(S.mmf) + (take ? take->used : 0);
     const int fmt = mmf_format(f.dtype);
     const uint32_t ldx = row_stride_x(ctx, k);
     for (size_t m0 = 0; m0 < m; m0 += L.rows) {
@@ -1274,6 +1289,10 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
         Q.lo_first = gq::mmfw_lo_first(fmt, static_cast<int>(L.planes), static_cast<int>(L.mt)) ? 1u : 0u;
         Q.glu = ctx->call_glu;
         Q.glu_off = ctx->call_glu_off;
+        if (take) {
+            Q.slices = take->slices;
+            Q.slice_ld = static_cast<uint32_t>(m * k);
+        }
         const uint32_t row_tiles = (mm + 31u) / 32u;
         rc = launch2d(ctx, ctx->mmfw_prep[hi_only ? 1 : 0], L.groups, row_tiles, gq::MMFW_PREP_WAVES * 64, 0, stream, &Q, sizeof Q, true);
         if (rc != GLLMQ_OK) return rc;
@@ -1309,7 +1328,11 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
         }
         rc = launch(ctx, ctx->mmfw[fmt][L.mt - 1][hi_only ? 1 : 0], (P.items + 7u) / 8u * 8u, gq::MMFW_WAVES * 64, mmfw_lds_bytes(fmt, hi_only ? 1 : 2, L.mt),
                     stream, &P, sizeof P, true);
-        if (rc == GLLMQ_OK && L.ksplit > 1) {
+        if (leaves) {
+            leave->at = P.seg[0].partial;
+            leave->slices = L.ksplit;
+            leave->used = used;
+        } else if (rc == GLLMQ_OK && L.ksplit > 1) {
             gq::MmfReduceParams R{};
             uint32_t wgs = 0;
             for (int i = 0; i < count; ++i) {
@@ -2493,7 +2516,10 @@ int ffn_on_stream(gllmq_ctx *ctx, const void *gate_w, const void *up_w, size_t g
     };
     if (wide && !ctx->mmfs_all && ffn % 4 == 0 && m * ffn <= 0xFFFFFFFFull && down_fits() && gate_up_fits()) {
         const MmfwMatrix gate_up[2] = { { gw, gu, ffn }, { uw, gu + m * ffn, ffn } };
-        rc = run_mmfw(ctx, S, *fg, gate_up, 2, x, elem, 0, m, hidden, false, stream, 5);
+        MmfwSlices sums;
+        const MmfwPlan L = plan_mmfw(ctx, dtype_down, m, &hidden, 1, ffn, false);
+        sums.next_need = std::max(L.need(), mmfw_reserve(ctx, m, ffn)); // (what the down projection would grow the scratch to)
+        rc = run_mmfw(ctx, S, *fg, gate_up, 2, x, elem, 0, m, hidden, false, stream, 5, ctx->ffn_glu_load && L.rows >= m ? &sums : nullptr);
         if (rc > 0) return rc;
         if (rc == GLLMQ_OK) {
             const MmfwMatrix down{ static_cast<const uint8_t *>(down_w), out, hidden };
@@ -2501,7 +2527,12 @@ int ffn_on_stream(gllmq_ctx *ctx, const void *gate_w, const void *up_w, size_t g
                 ctx->call_glu = relu_gate ? 2u : 1u;
                 ctx->call_glu_off = static_cast<uint32_t>(m * ffn);
                 ctx->call_ldx = static_cast<uint32_t>(ffn);
-                rc = run_mmfw(ctx, S, *fd, &down, 1, gu, 0, elem, m, ffn, false, stream, 5);
+                if (sums.slices) { // [gate, up][slice][m][ffn]
+                    ctx->call_glu_off = static_cast<uint32_t>(sums.slices * m * ffn);
+                    rc = run_mmfw(ctx, S, *fd, &down, 1, sums.at, 0, elem, m, ffn, false, stream, 5, nullptr, &sums);
+                } else {
+                    rc = run_mmfw(ctx, S, *fd, &down, 1, gu, 0, elem, m, ffn, false, stream, 5);
+                }
                 ctx->call_glu = ctx->call_glu_off = ctx->call_ldx = 0;
             } else {
                 gq::GluActParams A{};
@@ -3539,6 +3570,13 @@ int gllmq_reserve_ffn(gllmq_ctx *ctx, uint32_t dtype_gate_up, uint32_t dtype_dow
     Scratch *S = nullptr;
     rc = acquire_scratch(ctx, stream, &S);
     if (rc != GLLMQ_OK) return rc;
+    // (gate's and up's sums of slices beside what the down projection takes)
+    const size_t gate_up_n[2] = { ffn, ffn };
+    const MmfwPlan L = plan_mmfw(ctx, dtype_gate_up, m, gate_up_n, 2, hidden, false);
+    if (m >= 5 && L.ok && L.ksplit > 1) {
+        rc = grow_scratch(ctx, *S, &S->mmf, &S->mmf_bytes, ((L.need() + 255) & ~size_t(255)) + mmfw_reserve(ctx, m, ffn), stream, "reserve_ffn");
+        if (rc != GLLMQ_OK) return rc;
+    }
     return grow_scratch(ctx, *S, &S->ffn, &S->ffn_bytes, ffn_scratch_bytes(m, ffn), stream, "reserve_ffn");
 }
 

@@ -539,6 +539,8 @@ struct MmfwPrepParams {
     uint32_t lo_first;     // two planes: see mmfw_lo_first
     uint32_t natural;      // K order inside 32 elements: 1: step s, half h = 16 s + 8 h; 0: 16 h + 8 s
     uint32_t glu, glu_off; // x[i] = act(x[i]) * x[i + glu_off] (0 off, 1 SiLU, 2 SiLU behind a ReLU)
+    uint32_t slices;       // ... where both are sums of K slices, `slice_ld` elements apart, that nobody has added up yet (0, 1: they are whole)
+    uint32_t slice_ld;
 };
 
 struct MmfPrepParams {

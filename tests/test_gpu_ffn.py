@@ -192,3 +192,44 @@ def test_ffn_shapes_from_a_seeded_generator(hip, torch, oracle, seed):
         check(got, want, f"ffn seeded {seed}/{i} kernel={hip.last_kernel_name()}")
         seen.add(hip.last_kernel_name())
     print("last kernels met:", sorted(seen), flush=True)
+
+
+@pytest.mark.parametrize("t_gu,t_dn", [(Q4_K, Q6_K), (Q8_0, Q4_K), (Q6_K, Q5_K)])
+@pytest.mark.parametrize("m,hidden,ffn,ksplit", [(9, 512, 260, 2), (33, 1024, 512, 3), (65, 1536, 264, 6), (40, 1280, 300, 5)])
+def test_gate_and_up_left_as_sums_of_slices(torch, t_gu, t_dn, m, hidden, ffn, ksplit):
+    """Gate's and up's K slices are added up by the preparation of the down projection: the bits of the form in which they are
+    added up, gated and written out first; eager, captured behind a reservation, and captured with no room for both."""
+    from gllm_amd.backend import HipBackend
+    ref = HipBackend(0, options={"mmfw_ksplit": ksplit, "mmfw_small_min_m": 9, "ffn_glu_load": 0})
+    gate, up = dev_bytes(torch, random_weight(t_gu, ffn, hidden, seed=1)), dev_bytes(torch, random_weight(t_gu, ffn, hidden, seed=2))
+    down = dev_bytes(torch, random_weight(t_dn, hidden, ffn, seed=3))
+    x = torch.from_numpy(random_activations(m, hidden, seed=4) * 1e-2).cuda()
+    want = torch.zeros(m, hidden, device="cuda")
+    ref.ffn_swiglu(gate, up, t_gu, down, t_dn, x, want, m, hidden, ffn)
+    torch.cuda.synchronize()
+    for way in ("eager", "reserved", "no room"):
+        print(f"ffn slices {t_gu}/{t_dn} m={m} {way}", flush=True)
+        hip = HipBackend(0, options={"mmfw_ksplit": ksplit, "mmfw_small_min_m": 9})
+        got = torch.full((m, hidden), float("nan"), device="cuda")
+        args = (gate, up, t_gu, down, t_dn, x, got, m, hidden, ffn)
+        if way == "eager":
+            hip.ffn_swiglu(*args)
+        else:
+            stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+            stream.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(stream):
+                hip.reserve_ffn(t_gu, t_dn, m if way == "reserved" else 8, hidden, ffn)
+                if way == "no room":  # each product by itself has room, the two together do not
+                    hip.reserve_matmul(t_gu, m, 2 * ffn, hidden)
+                    hip.reserve_matmul(t_dn, m, hidden, ffn)
+                    hip.reserve_ffn(t_gu, t_dn, 1, hidden, ffn * m)  # (the intermediate results' buffer)
+                torch.cuda.synchronize()
+                with torch.cuda.graph(graph, stream=stream):
+                    hip.ffn_swiglu(*args)
+            for _ in range(3):
+                got.fill_(float("nan"))
+                graph.replay()
+                torch.cuda.synchronize()
+                assert torch.equal(got, want), way
+        torch.cuda.synchronize()
+        assert torch.equal(got, want), way
