@@ -496,7 +496,81 @@ struct MmfwShape {
     }
 };
 
-template <int FMT, int PL, int MT> constexpr uint32_t mmfw_lds() { return MmfwShape<FMT, PL, MT>::total; }
+// Few row tiles: a wave's weights come in units, whole rows of one block of K, or of two (Q4_K and Q5_K against one tile of one
+// plane), and a unit is read into registers before the next one is requested into the same place.  What that is for is the
+// CU's requests: 32 rows x 32 bytes a wave-load, as the parts have them, keep its address unit busy 79 % of a launch that streams
+// (a stream of 28672 x 4096 Q4_K weights alone, eight waves a CU: 17.5 us so, whole rows 14.3, two blocks of a row 13.0).
+// us a launch, parts, units of one block, of two (bits are the same):
+//   Q4_K 16 rows 28672 x 4096, one plane        26.9, 27.1, 25.1     Q5_K 16 rows 13824 x 5120, one plane  21.5, 21.2, 19.8
+//   Q4_K 16 rows 57344 x 8192, one plane        85.9, 86.1, 76.7     Q5_K 32 rows, two planes              23.7, 23.8, 24.1
+//   Q4_K 32 rows 14336 x 4096, two planes       18.2, 17.9, 18.9     Q5_K 48 rows, two planes              31.5, 31.1, 32.9
+//   Q4_K 64 rows 28672 x 4096, two planes       43.2, 40.8, 44.1     Q4_K 64 rows, one plane               32.8, 33.2, 33.4
+//   Q6_K 16 rows 4096 x 14336, two planes       26.2, 24.5           Q6_K 64 rows 14336 x 4096, one plane  31.4, 28.5
+//   Q6_K 2048 rows 4096 x 14336, two planes     610, 585             Q6_K 48 rows 14336 x 4096, two planes 35.3, 32.6
+//   Q8_0 64 rows 28672 x 4096, one plane        48.4, 50.6           (its rows' quants are off any alignment in LDS)
+constexpr bool mmfw_units(int fmt, int planes, int mt) { return fmt == 2 ? mt <= 2 : fmt <= 1 && mt <= planes; }
+template <int FMT, int PL, int MT>
+struct MmfwUnitShape {
+    using F = MmfwFormat<FMT>;
+    using W = MmfwShape<FMT, PL, MT>;
+    static constexpr int UB = FMT <= 1 && PL == 1 ? 2 : 1;                            // blocks of K in a unit
+    static constexpr uint32_t ROW = FMT == 2 ? 224u : UB * F::BLOCK;                  // bytes of a row in LDS (Q6_K: 208 and a window of 16 that ends with the block)
+    static constexpr int ROW_PIECES = ROW / 16u;
+    static constexpr int LW = (32 * ROW_PIECES + 63) / 64;                            // wave-loads of a unit
+    static constexpr uint32_t STAGE = LW * 1024u;
+    static constexpr int UC = W::UC, R = FMT == 1 && UB == 2 ? 3 : 4, C = W::C, NA = W::NA;      // the activations' ring, as above
+    static constexpr uint32_t CHUNK = W::CHUNK, TILE_CHUNK = W::TILE_CHUNK, EXTRA = W::EXTRA, extra = 0;
+    static_assert(TILE_CHUNK % (NA * 1024u) == 0, "a wave's pieces of a chunk are neighbours");
+    static constexpr uint32_t stage = 4u * EXTRA;
+    static constexpr uint32_t ring = stage + MMFW_WAVES * STAGE;
+    static constexpr uint32_t total = ring + R * CHUNK;
+    static_assert(total <= 160u * 1024u, "LDS");
+    static constexpr int SG = W::SG, NS = W::NS, SPC = W::SPC;
+    static constexpr int QL = NS / 4;              // K-quants: stages per quarter of a block
+    static constexpr int T = UB * NS;              // stages of a unit
+    static constexpr int REQUEST = 1;              // first stage that requests of the next unit; the last reads of this one are in stage 0
+    static constexpr int SPREAD = T - 2 - REQUEST > LW ? LW : T - 2 - REQUEST; // stages that share the requests
+    static constexpr int asked(int t) { return t <= REQUEST ? 0 : t - REQUEST >= SPREAD ? LW : (t - REQUEST) * LW / SPREAD; } // wave-loads requested ahead of stage t
+
+    // ---- the wave's sequence of loads, a unit being a period: stage t requests weights (t = REQUEST), then the extra of the
+    // block after next (first stage of a block); then, in the last stage of a chunk, the next chunk is acquired: its arrival is
+    // waited for and NA pieces of the chunk R - 1 further on are requested.
+    static constexpr int own(int t) { return asked(t + 1) - asked(t) + (t % NS == 0 ? 1 : 0); }
+    static constexpr bool acquires(int t) { return (t + 1) % SPC == 0; }
+    static constexpr int ahead_of(int t) // loads ahead of stage t
+    {
+        int blk = 0, n = 0;
+        while (t < 0) { t += T; --blk; }
+        for (int i = 0; i < t; ++i) n += own(i) + (acquires(i) ? NA : 0);
+        int period = 0;
+        for (int i = 0; i < T; ++i) period += own(i) + (acquires(i) ? NA : 0);
+        return n + blk * period;
+    }
+    static constexpr int own_at(int t) { return own((t + T) % T); }
+    static constexpr int limit(int n) { return n < 0 ? 0 : n < 63 ? n : 63; }
+    // loads that may be outstanding at stage t's acquisition; with the first chunk of a block its extra has to be there,
+    // requested in the first stage of the block before this one
+    static constexpr int chunk_wait(int t)
+    {
+        const int now = ahead_of(t) + own(t), from = t - (R - 1) * SPC;
+        int n = now - (ahead_of(from) + own_at((from % T + T) % T) + NA);
+        const int ex = t - (NS - 1) - NS;
+        if ((t + 1) % NS == 0 && now - (ahead_of(ex) + own_at((ex % T + T) % T)) < n) n = now - (ahead_of(ex) + own_at((ex % T + T) % T));
+        return limit(n);
+    }
+    // ... in stage t, behind its acquisition, where the unit requested in stage REQUEST of this period is read
+    static constexpr int weight_wait(int t)
+    {
+        const int last = REQUEST + SPREAD - 1;
+        return limit(ahead_of(t) + own(t) + (acquires(t) ? NA : 0) - (ahead_of(last) + asked(last + 1) - asked(last)));
+    }
+};
+
+template <int FMT, int PL, int MT> constexpr uint32_t mmfw_lds()
+{
+    if constexpr (mmfw_units(FMT, PL, MT)) return MmfwUnitShape<FMT, PL, MT>::total > MmfwShape<FMT, PL, MT>::total ? MmfwUnitShape<FMT, PL, MT>::total : MmfwShape<FMT, PL, MT>::total;
+    else return MmfwShape<FMT, PL, MT>::total;
+}
 
 struct MmfwSeg {
     const uint8_t *w;

@@ -37,6 +37,24 @@ def test_tile_edges(torch, oracle, dtype, tiles, ksplit):
             check_close(got, want, f"dtype={dtype} m={m} n={n} k={k} bf16={bf16}")
 
 
+@pytest.mark.parametrize("dtype", [Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("tiles", [1, 2])
+@pytest.mark.parametrize("blocks", [1, 3, 4, 5, 8, 9])
+def test_weights_in_units(torch, oracle, dtype, tiles, blocks):
+    """Whole rows of one or two blocks of K at a time: an odd block left over, one block in all, rows past the last one, a last
+    block that K does not fill; a matrix that ends with its allocation."""
+    from gllm_amd.backend import ACT_BF16, HipBackend
+    from oracle import npref
+    hip = HipBackend(0, options={"mmfw_mt": tiles, "mmfw_ksplit": 1})
+    for m, n, k in ((33, 257, 256 * blocks), (40, 1, 256 * blocks - 192)):
+        for bf16 in (False, True):
+            print(f"units dtype={dtype} tiles={tiles} m={m} n={n} k={k} bf16={bf16}", flush=True)
+            w, x = random_weight(dtype, n, k, seed=m + n), random_activations(m, k, seed=k + m)
+            want = oracle.quantized_matmul(w, npref.bf16_rne(x) if bf16 else x, dtype, m, n, k, acc=oracle.ACC_F64, threads=16)
+            got = gpu_matmul(hip, torch, w, x, dtype, m, n, k, **({"act_mode": ACT_BF16} if bf16 else {}))
+            check_close(got, want, f"dtype={dtype} m={m} n={n} k={k} bf16={bf16}")
+
+
 @pytest.mark.parametrize("ksplit", [2, 4, 5, 8, 9, 15])
 @pytest.mark.parametrize("m, n", [(33, 33), (34, 1), (35, 257), (36, 260)])
 def test_sums_of_slices_at_any_place(torch, oracle, ksplit, m, n):
