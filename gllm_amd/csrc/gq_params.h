@@ -397,6 +397,12 @@ constexpr uint32_t MMFW_PREP_WAVES = 16;        // of a workgroup that prepares 
 // (123 us, so 126; three tiles, which have the registers, 177, two 143).
 constexpr bool mmfw_lo_first(int fmt, int planes, int mt) { return fmt <= 1 && planes == 2 && mt == 4; }
 
+// Q8_0 against two planes: quants two units of 32 elements ahead, a unit's last sums scaled behind the next one's products.  A unit
+// is a chain of LDS read, unpacking, products and scaling that two waves a SIMD do not hide: 512 rows of 14336 x 4096 in two
+// tiles 172 us, so 165, in three 212, 206; 64 rows of 28672 x 4096 59.2, 57.7.  One plane 1 to 3 % longer (64 rows 48.4, 49.2), four
+// tiles have no registers for it.
+constexpr bool mmfw_q8_ahead(int planes, int mt) { return planes == 2 && mt <= 3; }
+
 // Image of 32 activation rows x 256 elements of K: [K step 0..15][plane][lane] 16 bytes (lo first: [lo, hi][K step]), then
 // [lane] 16 bytes of sub-block sums (lanes 0..31 hi, 32..63 lo); images lie [row tile][block].
 // The inverse scales are an array of their own: [block][padded rows] f32.
@@ -456,8 +462,8 @@ struct MmfwShape {
     static constexpr int SPC = NS / C;                 // stages per chunk
     static constexpr int PASS = LO_FIRST ? NS / 2 : NS; // stages in which the block's weights are read once
     static constexpr int QL = PASS / F::PARTS;         // stages per weight part
-    // Q8_0 reads the quants of stage s + 1 in stage s, so a part is free a stage before the next one starts
-    static constexpr int FREE = FMT == 3 ? QL - 1 : 0; // a part is requested again that far behind its first stage
+    // Q8_0 reads the quants of stage s + 1 (s + 2) in stage s, so a part is free a stage (two) before the next one starts
+    static constexpr int FREE = FMT == 3 ? QL - (mmfw_q8_ahead(PL, MT) ? 2 : 1) : 0; // a part is requested again that far behind its first stage
     static constexpr int requested(int p) { return NS - PASS + p * QL + FREE; } // (lo first: behind its second read)
     static constexpr int part_of(int s) { return s >= requested(0) && (s - requested(0)) % QL == 0 ? (s - requested(0)) / QL : -1; }
 

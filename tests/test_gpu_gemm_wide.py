@@ -55,6 +55,20 @@ def test_weights_in_units(torch, oracle, dtype, tiles, blocks):
             check_close(got, want, f"dtype={dtype} m={m} n={n} k={k} bf16={bf16}")
 
 
+@pytest.mark.parametrize("tiles", [1, 2, 3])
+@pytest.mark.parametrize("tail", [1, 3, 4, 5, 7, 8])
+def test_q8_0_short_last_groups(torch, oracle, tiles, tail):
+    """Quants are read ahead of a unit into a last group that holds `tail` blocks, windowed to end with the row."""
+    from gllm_amd.backend import HipBackend
+    hip = HipBackend(0, options={"mmfw_mt": tiles, "mmfw_ksplit": 1})
+    for m, n, groups in ((33, 257, 1), (97, 3, 3)):
+        k = 256 * groups + 32 * tail
+        print(f"q8_0 tail={tail} tiles={tiles} m={m} n={n} k={k}", flush=True)
+        w, x = random_weight(Q8_0, n, k, seed=m + n), random_activations(m, k, seed=k + m)
+        want = oracle.quantized_matmul(w, x, Q8_0, m, n, k, acc=oracle.ACC_F64, threads=16)
+        check_close(gpu_matmul(hip, torch, w, x, Q8_0, m, n, k), want, f"m={m} n={n} k={k}")
+
+
 @pytest.mark.parametrize("ksplit", [2, 4, 5, 8, 9, 15])
 @pytest.mark.parametrize("m, n", [(33, 33), (34, 1), (35, 257), (36, 260)])
 def test_sums_of_slices_at_any_place(torch, oracle, ksplit, m, n):
