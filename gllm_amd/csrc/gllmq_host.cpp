@@ -224,6 +224,7 @@ struct gllmq_ctx {
     bool batch_group = true;                    // "batch_group": independent entries over the same rows as one GEMM
     uint32_t mmfw_small_min_m = 9;              // "mmfw_small_min_m": ... where the streamed GEMMs do not take the call
     uint32_t mmfw_mt = 0, mmfw_ksplit = 0;      // "mmfw_mt", "mmfw_ksplit": activation tiles per workgroup, slices of K (0 = by the shape)
+    uint32_t mmfw_run = 0;                      // "mmfw_run": weight tiles per workgroup, one after the other, where the kernel can (0 = by the shape)
     hipFunction_t mmfs[2][2] = {};              // its streamed form [0 = Q4_K, 1 = Q5_K][bf16 mode]
     hipFunction_t mmfr[2][2] = {};              // the streamed form whose waves prepare their own activations (9 to 16 rows) [0 = Q4_K, 1 = Q5_K][f32, 16-bit]
     bool use_mmfr = true;                       // "mmfr" = 0: never
@@ -1072,6 +1073,7 @@ struct MmfwPlan {
     bool ok = false;
     uint32_t groups = 0, planes = 2, mt = 1, n_tiles = 0, ksplit = 1, bps = 0, band = 4;
     uint32_t run = 0; // blocks whose sums are taken in one run; 0: all of a slice's
+    uint32_t run_tiles = 1; // weight tiles that a workgroup multiplies one after the other
     size_t n_sum = 0; // weight rows of all matrices
     size_t rows = 0; // activation rows per pass (all of them, unless the images would pass 1 GiB or the scratch has no room: mmfw_fit)
     size_t img_bytes = 0, inv_bytes = 0, part_bytes = 0;
@@ -1079,6 +1081,13 @@ struct MmfwPlan {
 };
 
 int mmf_format(uint32_t dtype) { return dtype == T_Q8_0 ? 3 : dtype == T_Q6_K ? 2 : dtype == T_Q5_K ? 1 : 0; }
+
+// Whether a workgroup may take several weight tiles one after the other (mmfw_may_run): all of K, long enough for requests to reach
+// into the next tile only, and no unit of two blocks across its end.
+bool mmfw_run_ok(int fmt, int planes, uint32_t mt, uint32_t groups, uint32_t ksplit)
+{
+    return ksplit == 1 && groups >= 4 && groups % 2 == 0 && gq::mmfw_may_run(fmt, planes, static_cast<int>(mt), false);
+}
 
 uint32_t mmfw_inv_ld(size_t rows) { return static_cast<uint32_t>((rows + 31) / 32 * 32); }
 
@@ -1199,7 +1208,7 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
         const double meet = ks > 1 ? 4.0 + 2.0 * ks * static_cast<double>(m) * static_cast<double>(n_sum) * 4.0 / 4.0e6 : 0.0;
         const uint32_t run = mmfw_run(bps, ks, bar);
         double of[2] = { 1e300, 1e300 }; // one plane, two
-        uint32_t of_mt[2] = { 0, 0 };
+        uint32_t of_mt[2] = { 0, 0 }, of_run[2] = { 1, 1 };
         for (uint32_t mt = 1; mt <= static_cast<uint32_t>(gq::MMFW_MAX_MT); ++mt) {
             if (ctx->mmfw_mt ? mt != ctx->mmfw_mt : (mt > row_tiles)) continue;
             if (run && !gq::mmfw_runs(static_cast<int>(mt)) && !ctx->mmfw_mt) continue;
@@ -1209,18 +1218,25 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
             if (static_cast<size_t>(L.groups) * mt * (gq::MmfwImage<2>::bytes + 128u) + 2048u + slices * std::min<size_t>(m, 32u * mt) >
                 GLLMQ_NOALLOC_SCRATCH_BYTES - kScratchFixedBytes)
                 continue;
-            const double rounds = std::ceil(static_cast<double>(items) / cus), busy = std::min(1.0, static_cast<double>(items) / cus);
+            const double busy = std::min(1.0, static_cast<double>(items) / cus);
             for (int pl = 0; pl < 2; ++pl) {
-                const double us = rounds * (bps * std::max({ mt * tile_us[pl], chain_us[fmt], w_us * busy }) + start) + meet;
-                if (us < of[pl]) {
-                    of[pl] = us;
-                    of_mt[pl] = mt;
+                const double tile = bps * std::max({ mt * tile_us[pl], chain_us[fmt], w_us * busy });
+                // (runs of weight tiles only where they save rounds)
+                const uint32_t most = mmfw_run_ok(fmt, pl + 1, mt, L.groups, ks) ? static_cast<uint32_t>(std::min<uint64_t>(16, (items + static_cast<uint64_t>(cus) - 1) / static_cast<uint64_t>(cus))) : 1u;
+                for (uint32_t run = 1; run <= most; ++run) {
+                    const double us = std::ceil(static_cast<double>(m_tiles * ((tiles + run - 1) / run) * ks) / cus) * (run * tile + start) + meet;
+                    if (us < of[pl]) {
+                        of[pl] = us;
+                        of_mt[pl] = mt;
+                        of_run[pl] = run;
+                    }
                 }
             }
         }
         if (of[0] + of[1] < best) {
             best = of[0] + of[1];
             L.mt = of_mt[L.planes - 1];
+            L.run_tiles = of_run[L.planes - 1];
             L.ksplit = ks;
             L.bps = bps;
             L.run = run;
@@ -1311,7 +1327,9 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
         P.ksplit = L.ksplit;
         P.blocks_per_split = L.bps;
         P.run_mask = L.run ? L.run - 1u : ~0u;
-        P.items = P.m_tiles * P.n_tiles * L.ksplit;
+        P.run_tiles = std::min(mmfw_run_ok(fmt, hi_only ? 1 : 2, L.mt, L.groups, L.ksplit) ? std::max(1u, ctx->mmfw_run ? ctx->mmfw_run : L.run_tiles) : 1u, P.n_tiles);
+        P.n_runs = (P.n_tiles + P.run_tiles - 1u) / P.run_tiles;
+        P.items = P.m_tiles * P.n_runs * L.ksplit;
         P.band = std::min(L.band, P.m_tiles);
         P.elem = elem_y;
         float *part = reinterpret_cast<float *>(scratch + L.img_bytes + L.inv_bytes);
@@ -2143,6 +2161,7 @@ int gllmq_set_option(gllmq_ctx *ctx, const char *name, long value)
     else if (n == "mmfw_small_min_m") ctx->mmfw_small_min_m = std::max(1u, u);
     else if (n == "mmfw_mt") ctx->mmfw_mt = std::min(u, static_cast<uint32_t>(gq::MMFW_MAX_MT));
     else if (n == "mmfw_ksplit") ctx->mmfw_ksplit = u;
+    else if (n == "mmfw_run") ctx->mmfw_run = u;
     else if (n == "mmfr_min_rows") ctx->mmfr_min_rows = std::max(1u, u);
     else if (n == "chain") ctx->use_chain = value != 0;
     else if (n == "chain_dependent") ctx->chain_dependent = value != 0;
@@ -3193,9 +3212,11 @@ int run_moe_wide(gllmq_ctx *ctx, const Format &fg, const void *gate, size_t gate
             P.n_tiles += static_cast<uint32_t>((mats[i].n + gq::MMFW_TILE_ROWS - 1) / gq::MMFW_TILE_ROWS);
         }
         P.max_jobs = W.max_jobs;
+        P.run_tiles = 1;
+        P.n_runs = P.n_tiles;
         uint32_t lds = 0;
         for (uint32_t mt = 1; mt <= static_cast<uint32_t>(gq::MMFW_MAX_MT); ++mt) lds = std::max(lds, mmfw_lds_bytes(fmt, hi ? 1 : 2, mt));
-        return launch(ctx, ctx->moe_mmf[fmt][hi ? 1 : 0], (W.max_jobs + 7u) / 8u * 8u * P.n_tiles, gq::MMFW_WAVES * 64, lds, stream, &P,
+        return launch(ctx, ctx->moe_mmf[fmt][hi ? 1 : 0], (W.max_jobs + 7u) / 8u * 8u * P.n_runs, gq::MMFW_WAVES * 64, lds, stream, &P,
                       sizeof P, true);
     };
     {

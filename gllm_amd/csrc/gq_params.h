@@ -572,6 +572,12 @@ struct MmfwUnitShape {
     }
 };
 
+// A workgroup may take several weight tiles against its activation rows one after the other: the requests go on into the next
+// tile, so its first loads, the arguments and the way in are not waited for again.  Prompts of 16-bit elements: 2048 rows of 28672 x
+// 4096 Q4_K, seven rounds of workgroups 532 us, seven tiles a workgroup 502; of 6144 x 4096 141, 133 (three).  Two planes and
+// Q6_K lose 1 to 3 % to the registers it takes, for experts (tiles of unequal length) it came to nothing: 645, 642.
+constexpr bool mmfw_may_run(int fmt, int planes, int mt, bool grouped) { return fmt <= 1 && planes == 1 && mt >= 2 && !grouped; }
+
 template <int FMT, int PL, int MT> constexpr uint32_t mmfw_lds()
 {
     if constexpr (mmfw_units(FMT, PL, MT)) return MmfwUnitShape<FMT, PL, MT>::total > MmfwShape<FMT, PL, MT>::total ? MmfwUnitShape<FMT, PL, MT>::total : MmfwShape<FMT, PL, MT>::total;
@@ -596,7 +602,9 @@ struct MmfwParams {
     uint32_t m_tiles, n_tiles; // workgroup tiles of activation rows and of weight rows (all matrices)
     uint32_t ksplit, blocks_per_split;
     uint32_t run_mask;         // blocks whose sums are taken in one run, less one (a power of two less one; all ones: a slice's all)
-    uint32_t items;            // m_tiles * n_tiles * ksplit
+    uint32_t run_tiles;        // weight tiles that a workgroup multiplies one after the other (more than one: all of K, an even number of four or more blocks)
+    uint32_t n_runs;           // runs of them: ceil(n_tiles / run_tiles)
+    uint32_t items;            // m_tiles * n_runs * ksplit
     uint32_t band;             // activation tiles that neighbouring workgroups share a weight tile over
     uint32_t elem;             // element type of y
     // Grouped launch (experts): jobs[0 .. counters[2]) take the place of the activation tiles, row r of job J

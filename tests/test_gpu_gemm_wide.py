@@ -55,6 +55,30 @@ def test_weights_in_units(torch, oracle, dtype, tiles, blocks):
             check_close(got, want, f"dtype={dtype} m={m} n={n} k={k} bf16={bf16}")
 
 
+@pytest.mark.parametrize("dtype", [Q4_K, Q5_K])
+@pytest.mark.parametrize("tiles", [2, 3, 4])
+@pytest.mark.parametrize("run", [2, 3, 16])
+def test_runs_of_weight_tiles(torch, dtype, tiles, run):
+    """A workgroup takes several weight tiles one after the other, across matrices and up to a ragged last one: the bits of a
+    tile per workgroup, for the shortest rows that allow it and longer ones."""
+    from gllm_amd.backend import HipBackend
+    one, several = (HipBackend(0, options={"mmfw_mt": tiles, "mmfw_ksplit": 1, "mmfw_run": r}) for r in (1, run))
+    for m, k in ((65, 1024), (130, 1536 - 64), (200, 1280)):  # (the last: an odd number of blocks, no runs)
+        x = torch.from_numpy(random_activations(m, k, seed=k)).cuda().to(torch.bfloat16)
+        ws = [torch.from_numpy(random_weight(dtype, n, k, seed=n)).cuda() for n in (513, 256, 300)]
+        outs = []
+        for hip in (one, several):
+            print(f"runs dtype={dtype} tiles={tiles} run={run} m={m} k={k}", flush=True)
+            y = [torch.full((m, n), float("nan"), device="cuda", dtype=torch.bfloat16) for n in (513, 256, 300)]
+            hip.quantized_matmul_batch([(w, x, o, dtype, m, o.shape[1], k) for w, o in zip(ws, y)])
+            single = torch.full((m, 513), float("nan"), device="cuda", dtype=torch.bfloat16)
+            hip.quantized_matmul(ws[0], x, single, dtype, m, 513, k)
+            torch.cuda.synchronize()
+            outs.append(y + [single])
+        for a, b in zip(*outs):
+            assert torch.equal(a, b) and bool(torch.isfinite(a.float()).all())
+
+
 @pytest.mark.parametrize("tiles", [1, 2, 3])
 @pytest.mark.parametrize("tail", [1, 3, 4, 5, 7, 8])
 def test_q8_0_short_last_groups(torch, oracle, tiles, tail):
