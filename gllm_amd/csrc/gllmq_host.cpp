@@ -1183,21 +1183,25 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
     L.planes = hi_only ? 1u : 2u;
     L.n_tiles = static_cast<uint32_t>(tiles);
     const uint32_t row_tiles = static_cast<uint32_t>((m + 31) / 32);
-    // Activation tiles per workgroup and slices of K by a cost model (us): a block of K takes a
-    // workgroup its products (Q6_K, Q8_0: and their scales), the way of one wave's block through
-    // unpacking and LDS, which a tile or two do not cover, or the weights' way from memory, whichever
-    // is longest; a workgroup starts and ends in `start`; the slices of K meet through memory.  Slopes over
-    // K measured with one tile on 16 CUs: 1.5 (Q4_K), 2.7 (Q6_K), 2.4 (Q8_0) a block; two tiles,
-    // one plane and two: 1.8 and 2.4, 2.9 and 3.9, 3.4 and 4.2.
+    // Activation tiles per workgroup and slices of K by a cost model (us): a block of K takes a workgroup what the table says, or
+    // the weights' way from memory where that is longer; a workgroup starts and ends in `start`; the slices of K meet
+    // through memory.  The numbers are fitted to what they decide: 135 000 calls of 6852 shapes (9 to 2048 rows, 512 to 28672 x 1024
+    // to 14336, all formats, f32 and bf16; every number of tiles and up to 20 slices) were timed, half of the shapes
+    // searched for the numbers whose choices are shortest, the other half kept to check: choices 0.50 % longer than the best
+    // one in the mean, 1.43 % with block times measured one by one before (1.5 to 2.7 us for one tile).
     // Slices and runs decide the order of the sums, tiles do not; so a call of 16-bit elements has the slices of the f32 call
     // whose bits it has to give: those with which the two together are shortest.  (3000 plans of 9 to 2048 rows by the
     // model, against slices of their own: 0.5 % longer in the mean, one in a hundred by more than a tenth.)
     const double cus = ctx->num_cus;
-    const double w_us = find_format(dtype)->group_bytes * 256.0 * cus / 5.0e6; // 5 TB/s over all CUs
-    static const double chain_us[4] = { 1.5, 1.6, 2.7, 2.4 };
-    double tile_us[2];
-    for (uint32_t pl = 1; pl <= 2; ++pl) tile_us[pl - 1] = fmt >= 2 ? (fmt == 3 ? 1.2 : 1.45) + 0.45 * pl : 0.25 + 0.62 * pl;
-    const double start = 5.0, bar = mmfw_chain_bar(ctx, fmt, n, count, k);
+    const double w_us = find_format(dtype)->group_bytes * 256.0 * cus / 5.85e6; // 5.85 TB/s over all CUs
+    static const double block_us[4][2][gq::MMFW_MAX_MT] = { // [Q4_K, Q5_K, Q6_K, Q8_0][one plane, two][tiles - 1]
+        { { 1.65, 2.07, 2.88, 3.96 }, { 1.50, 2.98, 4.69, 5.95 } },
+        { { 1.76, 2.11, 2.95, 3.13 }, { 1.92, 2.98, 4.03, 5.36 } },
+        { { 2.70, 3.80, 5.41, 7.22 }, { 2.97, 4.70, 7.05, 9.40 } },
+        { { 3.45, 3.46, 4.16, 6.34 }, { 2.21, 5.04, 6.30, 7.98 } },
+    };
+    const double crowd_us = fmt == 0 ? 0.4 : 0.0; // more per block with every CU busy
+    const double start = 5.64, bar = mmfw_chain_bar(ctx, fmt, n, count, k);
     double best = 1e300;
     for (uint32_t ks = 1; ks <= std::min(L.groups, 32u); ++ks) {
         const uint32_t bps = (L.groups + ks - 1) / ks;
@@ -1205,7 +1209,7 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
         if (ctx->mmfw_ksplit && ks != std::min(ctx->mmfw_ksplit, L.groups)) continue;
         const size_t slices = ks > 1 ? static_cast<size_t>(ks) * n_sum * 4 : 0;
         if (slices * m > mmfw_most_slices(ctx, m) && !ctx->mmfw_ksplit) continue;
-        const double meet = ks > 1 ? 4.0 + 2.0 * ks * static_cast<double>(m) * static_cast<double>(n_sum) * 4.0 / 4.0e6 : 0.0;
+        const double meet = ks > 1 ? 0.64 + 2.2 * ks * static_cast<double>(m) * static_cast<double>(n_sum) / 1.0e6 : 0.0;
         const uint32_t run = mmfw_run(bps, ks, bar);
         double of[2] = { 1e300, 1e300 }; // one plane, two
         uint32_t of_mt[2] = { 0, 0 }, of_run[2] = { 1, 1 };
@@ -1220,7 +1224,7 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
                 continue;
             const double busy = std::min(1.0, static_cast<double>(items) / cus);
             for (int pl = 0; pl < 2; ++pl) {
-                const double tile = bps * std::max({ mt * tile_us[pl], chain_us[fmt], w_us * busy });
+                const double tile = bps * (std::max(block_us[fmt][pl][mt - 1], w_us * busy) + crowd_us * busy);
                 // (runs of weight tiles only where they save rounds)
                 const uint32_t most = mmfw_run_ok(fmt, pl + 1, mt, L.groups, ks) ? static_cast<uint32_t>(std::min<uint64_t>(16, (items + static_cast<uint64_t>(cus) - 1) / static_cast<uint64_t>(cus))) : 1u;
                 for (uint32_t run = 1; run <= most; ++run) {
