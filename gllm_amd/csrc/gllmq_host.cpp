@@ -118,6 +118,20 @@ uint32_t mmfw_lds_bytes(int fmt, int planes, uint32_t mt)
     return kTotal[fmt][planes - 1][mt - 1];
 }
 
+// ... where a workgroup makes its images itself: blocks of K that its slice may have, LDS
+uint32_t mmfw_own_blocks(int fmt, int planes)
+{
+    static const uint32_t kBlocks[4][2] = { { gq::mmfw_own_blocks<0, 1>(), gq::mmfw_own_blocks<0, 2>() }, { gq::mmfw_own_blocks<1, 1>(), gq::mmfw_own_blocks<1, 2>() },
+                                            { gq::mmfw_own_blocks<2, 1>(), gq::mmfw_own_blocks<2, 2>() }, { gq::mmfw_own_blocks<3, 1>(), gq::mmfw_own_blocks<3, 2>() } };
+    return kBlocks[fmt][planes - 1];
+}
+uint32_t mmfw_own_lds(int fmt, int planes)
+{
+    static const uint32_t kTotal[4][2] = { { gq::mmfw_own_lds<0, 1>(), gq::mmfw_own_lds<0, 2>() }, { gq::mmfw_own_lds<1, 1>(), gq::mmfw_own_lds<1, 2>() },
+                                           { gq::mmfw_own_lds<2, 1>(), gq::mmfw_own_lds<2, 2>() }, { gq::mmfw_own_lds<3, 1>(), gq::mmfw_own_lds<3, 2>() } };
+    return kTotal[fmt][planes - 1];
+}
+
 // Formats of the int8 matrix-core kernels, in the order of the kernel tables below.
 // (the grouped MoE kernels exist for the first MM8_MOE_KINDS of them)
 enum Mm8Kind { MM8_Q4K = 0, MM8_Q6K = 1, MM8_Q5K = 2, MM8_Q8_0 = 3, MM8_KINDS = 4, MM8_MOE_KINDS = 3 };
@@ -218,6 +232,8 @@ struct gllmq_ctx {
     hipFunction_t mmf_q4k[4][2][2] = {};        // f16 matrix-core GEMM [0 = Q4_K, 1 = Q5_K, 2 = Q6_K, 3 = Q8_0][32-row activation tiles - 1][bf16 mode]
     hipFunction_t mmfw[4][4][2] = {};           // the GEMM for more rows [format as above][32-row activation tiles - 1][0 = hi and lo plane, 1 = hi only]
     hipFunction_t moe_mmf[4][2] = {};           // the same over experts' rows [format][plane]
+    hipFunction_t mmfw_own[4][2] = {};          // ... of one tile, which prepares the activations itself [format][0 = hi and lo plane, 1 = hi only]
+    bool use_mmfw_own = true;                   // "mmfw_own" = 0: always a launch that prepares them
     hipFunction_t mmfw_prep[2] = {};            // its activation images [hi and lo plane, hi only]
     bool use_mmfw = true;                       // "mmfw" = 0: 64-row passes of the other forms
     uint32_t mmfw_min_m = 33;                   // "mmfw_min_m": fewest activation rows that take it
@@ -1254,6 +1270,14 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
     return L;
 }
 
+// Whether workgroups prepare their activations themselves (MmfwOwn): one row tile, slices short enough for the images to stay in
+// LDS, rows that sixteen-byte loads take piece by piece.  Where it can be done it is ahead, by 3 to 4 us of 13 to 25 (MmfwOwn).
+bool mmfw_takes_own(const gllmq_ctx *ctx, const MmfwPlan &L, int fmt, size_t m, size_t k, size_t ldx, size_t x_bytes)
+{
+    return ctx->use_mmfw_own && L.mt == 1 && L.bps <= mmfw_own_blocks(fmt, static_cast<int>(L.planes)) && k * x_bytes % 16 == 0 && ldx * x_bytes % 16 == 0 &&
+           m * ldx * x_bytes <= 0xFFFFFFFFull;
+}
+
 // The sums of K slices of a feed-forward block's gate and up rows, left in the scratch for the preparation of the down
 // projection, which adds them up while it applies the gate: a launch less, and the sums' way to memory and back.
 struct MmfwSlices {
@@ -1292,6 +1316,8 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
     uint8_t *scratch = static_cast<uint8_t *>(S.mmf) + (take ? take->used : 0);
     const int fmt = mmf_format(f.dtype);
     const uint32_t ldx = row_stride_x(ctx, k);
+    const size_t x_bytes = elem_x ? 2 : 4;
+    const bool own = mmfw_takes_own(ctx, L, fmt, m, k, ldx, x_bytes) && !take && !ctx->call_glu && !act_bf16;
     for (size_t m0 = 0; m0 < m; m0 += L.rows) {
         const uint32_t mm = static_cast<uint32_t>(std::min(L.rows, m - m0));
         gq::MmfwPrepParams Q{};
@@ -1314,11 +1340,16 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
             Q.slice_ld = static_cast<uint32_t>(m * k);
         }
         const uint32_t row_tiles = (mm + 31u) / 32u;
-        rc = launch2d(ctx, ctx->mmfw_prep[hi_only ? 1 : 0], L.groups, row_tiles, gq::MMFW_PREP_WAVES * 64, 0, stream, &Q, sizeof Q, true);
+        if (!own) rc = launch2d(ctx, ctx->mmfw_prep[hi_only ? 1 : 0], L.groups, row_tiles, gq::MMFW_PREP_WAVES * 64, 0, stream, &Q, sizeof Q, true);
         if (rc != GLLMQ_OK) return rc;
         gq::MmfwParams P{};
         P.ximg = scratch;
         P.inv = Q.inv;
+        if (own) {
+            P.x = reinterpret_cast<const uint8_t *>(Q.x);
+            P.x_row_bytes = static_cast<uint32_t>(ldx * x_bytes);
+            P.x_elem = Q.elem;
+        }
         P.segs = static_cast<uint32_t>(count);
         P.groups = L.groups;
         P.row_bytes = static_cast<uint32_t>(gllmq_row_bytes(f.dtype, k));
@@ -1348,8 +1379,8 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
             tile0 += (G.n + gq::MMFW_TILE_ROWS - 1u) / gq::MMFW_TILE_ROWS;
             part += static_cast<size_t>(L.ksplit) * mm * G.n;
         }
-        rc = launch(ctx, ctx->mmfw[fmt][L.mt - 1][hi_only ? 1 : 0], (P.items + 7u) / 8u * 8u, gq::MMFW_WAVES * 64, mmfw_lds_bytes(fmt, hi_only ? 1 : 2, L.mt),
-                    stream, &P, sizeof P, true);
+        rc = launch(ctx, own ? ctx->mmfw_own[fmt][hi_only ? 1 : 0] : ctx->mmfw[fmt][L.mt - 1][hi_only ? 1 : 0], (P.items + 7u) / 8u * 8u, gq::MMFW_WAVES * 64,
+                    own ? mmfw_own_lds(fmt, hi_only ? 1 : 2) : mmfw_lds_bytes(fmt, hi_only ? 1 : 2, L.mt), stream, &P, sizeof P, true);
         if (leaves) {
             leave->at = P.seg[0].partial;
             leave->slices = L.ksplit;
@@ -1962,6 +1993,11 @@ int gllmq_init(gllmq_ctx **out, int device)
             }
     for (int q = 0; q < 4 && rc == GLLMQ_OK; ++q)
         for (int b = 0; b < 2 && rc == GLLMQ_OK; ++b) {
+            snprintf(name, sizeof name, "gq_mmf_%s_w1_own%s", q == 3 ? "q8_0" : q == 2 ? "q6k" : q == 1 ? "q5k" : "q4k", b ? "_hi" : "");
+            rc = get_function(ctx, &ctx->mmfw_own[q][b], name);
+        }
+    for (int q = 0; q < 4 && rc == GLLMQ_OK; ++q)
+        for (int b = 0; b < 2 && rc == GLLMQ_OK; ++b) {
             snprintf(name, sizeof name, "gq_moe_mmf_%s%s", q == 3 ? "q8_0" : q == 2 ? "q6k" : q == 1 ? "q5k" : "q4k", b ? "_hi" : "");
             rc = get_function(ctx, &ctx->moe_mmf[q][b], name);
         }
@@ -2166,6 +2202,7 @@ int gllmq_set_option(gllmq_ctx *ctx, const char *name, long value)
     else if (n == "mmfw_mt") ctx->mmfw_mt = std::min(u, static_cast<uint32_t>(gq::MMFW_MAX_MT));
     else if (n == "mmfw_ksplit") ctx->mmfw_ksplit = u;
     else if (n == "mmfw_run") ctx->mmfw_run = u;
+    else if (n == "mmfw_own") ctx->use_mmfw_own = value != 0;
     else if (n == "mmfr_min_rows") ctx->mmfr_min_rows = std::max(1u, u);
     else if (n == "chain") ctx->use_chain = value != 0;
     else if (n == "chain_dependent") ctx->chain_dependent = value != 0;

@@ -435,16 +435,17 @@ template <> struct MmfwFormat<3> { // half groups: 136 bytes a row
     static constexpr bool SUMS = false;
 };
 
-template <int FMT, int PL, int MT, bool LO_FIRST = false>
+template <int FMT, int PL, int MT, bool LO_FIRST = false, bool OWN = false>
 struct MmfwShape {
     using F = MmfwFormat<FMT>;
     static_assert(!LO_FIRST || mmfw_lo_first(FMT, PL, MT), "");
+    static_assert(!OWN || MT == 1, "");
     // Activations move in chunks of UC units (32 elements of K) through a ring of R chunk slots in LDS.
     static constexpr int UC = MT == 4 ? (PL == 2 ? 1 : 2) : MT == 3 ? (PL == 2 ? 2 : 4) : MT == 2 ? (PL == 2 ? 2 : 4) : (PL == 2 ? 4 : 8);
     static constexpr int R = MT == 3 ? 3 : 4;
     static constexpr int C = 8 / UC;                   // chunks per block
     static constexpr int PIECES = MT * PL * 2 * UC;    // KiB per chunk
-    static constexpr int NA = PIECES / MMFW_WAVES;     // wave-loads per wave and chunk
+    static constexpr int NA = OWN ? 0 : PIECES / MMFW_WAVES; // wave-loads per wave and chunk
     static_assert(PIECES % MMFW_WAVES == 0, "every wave requests the same number of pieces");
     static constexpr uint32_t CHUNK = PIECES * 1024u;
     static constexpr uint32_t TILE_CHUNK = 2u * UC * PL * 1024u; // a row tile's share: contiguous in its image
@@ -452,7 +453,11 @@ struct MmfwShape {
     static constexpr uint32_t EXTRA = ((F::SUMS ? MT : 0) + 1) * 1024u;
     static constexpr uint32_t stage = 4u * EXTRA;
     static constexpr uint32_t ring = stage + MMFW_WAVES * F::STAGE;
-    static constexpr uint32_t total = ring + R * CHUNK;
+    // OWN: the images of a slice's blocks are made here, all of them ahead of the first product, and take the ring's place
+    // (four places of sums and scales: one more than blocks, read past the last)
+    static constexpr int OWN_FIT = (160u * 1024u - ring) / (C * CHUNK), OWN_BLOCKS = OWN_FIT < 3 ? OWN_FIT : 3;
+    static constexpr uint32_t RING = OWN ? OWN_BLOCKS * C * CHUNK : R * CHUNK;
+    static constexpr uint32_t total = ring + RING;
     static_assert(total <= 160u * 1024u, "LDS");
 
     // ---- A block is NS stages of SG operand slots (a K step of one plane) for all row tiles; Q6_K, Q8_0:
@@ -471,7 +476,7 @@ struct MmfwShape {
     // stage 0 the extra of the block after next, first); then, in the last stage of a chunk, the
     // next chunk is acquired: its arrival is waited for and NA pieces of the chunk R - 1 further on
     // are requested.
-    static constexpr int stage_loads(int s) { return (s == 0 ? 1 + F::HEAD : 0) + (part_of(s) >= 0 ? F::PART : 0); }
+    static constexpr int stage_loads(int s) { return (s == 0 ? (OWN ? 0 : 1) + F::HEAD : 0) + (part_of(s) >= 0 ? F::PART : 0); }
     static constexpr int after_weights(int s) // position behind stage s's weight requests
     {
         int p = 0;
@@ -578,6 +583,10 @@ struct MmfwUnitShape {
 // Q6_K lose 1 to 3 % to the registers it takes, for experts (tiles of unequal length) it came to nothing: 645, 642.
 constexpr bool mmfw_may_run(int fmt, int planes, int mt, bool grouped) { return fmt <= 1 && planes == 1 && mt >= 2 && !grouped; }
 
+// A workgroup of one row tile whose slice of K is this short makes its images itself.
+template <int FMT, int PL> constexpr uint32_t mmfw_own_blocks() { return MmfwShape<FMT, PL, 1, false, true>::OWN_BLOCKS; }
+template <int FMT, int PL> constexpr uint32_t mmfw_own_lds() { return MmfwShape<FMT, PL, 1, false, true>::total; }
+
 template <int FMT, int PL, int MT> constexpr uint32_t mmfw_lds()
 {
     if constexpr (mmfw_units(FMT, PL, MT)) return MmfwUnitShape<FMT, PL, MT>::total > MmfwShape<FMT, PL, MT>::total ? MmfwUnitShape<FMT, PL, MT>::total : MmfwShape<FMT, PL, MT>::total;
@@ -608,9 +617,16 @@ struct MmfwParams {
     uint32_t band;             // activation tiles that neighbouring workgroups share a weight tile over
     uint32_t elem;             // element type of y
     // Grouped launch (experts): jobs[0 .. counters[2]) take the place of the activation tiles, row r of job J
-    // is output row J.p0 + r.
-    const struct MoeWideJob *jobs;
-    const uint32_t *counters;
+    // is output row J.p0 + r.  Or, where a workgroup makes its images itself: the activations, bytes between their rows, their
+    // element type.
+    union {
+        const struct MoeWideJob *jobs;
+        const uint8_t *x;
+    };
+    union {
+        const uint32_t *counters;
+        struct { uint32_t x_row_bytes, x_elem; };
+    };
     uint32_t max_jobs;         // entries of `jobs` that exist at most
 };
 

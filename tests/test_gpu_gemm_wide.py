@@ -55,6 +55,38 @@ def test_weights_in_units(torch, oracle, dtype, tiles, blocks):
             check_close(got, want, f"dtype={dtype} m={m} n={n} k={k} bf16={bf16}")
 
 
+@pytest.mark.parametrize("dtype", ALL)
+@pytest.mark.parametrize("elem", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("slices, blocks", [(1, 1), (1, 2), (1, 3), (2, 2), (2, 3), (3, 3), (3, 4)])
+def test_images_made_by_the_workgroup(torch, dtype, elem, slices, blocks):
+    """Short slices of K, whose workgroups prepare their activations themselves: the bits of the launch that prepares them, with
+    blocks that K does not fill, a slice shorter than the rest, rows past the last, rows of zeros, tiny, huge and non-finite ones,
+    several matrices; blocks that do not fit take the launch."""
+    from gllm_amd.backend import HipBackend
+    t = getattr(torch, elem)
+    hips = [HipBackend(0, options={"mmfw_mt": 1, "mmfw_ksplit": slices, "mmfw_min_m": 9, "mmfw_own": v}) for v in (1, 0)]
+    k = 256 * slices * blocks - (256 if slices > 1 and blocks > 1 else 0)
+    for m, cut in ((33, 0), (9, 32 if dtype == Q8_0 and k > 256 else 0), (64, 224 if dtype == Q8_0 and k > 256 else 0)):
+        x = torch.from_numpy(random_activations(m, k - cut, seed=k + m)).cuda()
+        x[0] = 0.0
+        x[1] *= 1e-30
+        x[2] *= 2.0 ** 100
+        x[3, 5], x[m - 1, 0] = float("nan"), float("inf")
+        x = x.to(t)
+        sizes = (257, 64, 1)
+        ws = [torch.from_numpy(random_weight(dtype, n, k - cut, seed=n)).cuda() for n in sizes]
+        outs = []
+        for hip in hips:
+            print(f"own images dtype={dtype} {elem} slices={slices} blocks={blocks} m={m} k={k - cut}", flush=True)
+            ys = [torch.full((m, n), 7.0, device="cuda", dtype=t) for n in sizes]
+            hip.quantized_matmul(ws[0], x, ys[0], dtype, m, sizes[0], k - cut)
+            hip.quantized_matmul_batch([(w, x, y, dtype, m, y.shape[1], k - cut) for w, y in list(zip(ws, ys))[1:]])
+            torch.cuda.synchronize()
+            outs.append(ys)
+        for a, b in zip(*outs):
+            assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
 @pytest.mark.parametrize("dtype", [Q4_K, Q5_K])
 @pytest.mark.parametrize("tiles", [2, 3, 4])
 @pytest.mark.parametrize("run", [2, 3, 16])
