@@ -1217,6 +1217,11 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
         { { 3.45, 3.46, 4.16, 6.34 }, { 2.21, 5.04, 6.30, 7.98 } },
     };
     const double crowd_us = fmt == 0 ? 0.4 : 0.0; // more per block with every CU busy
+    // A launch that prepares the activations, where workgroups do not do it themselves.  It takes 3 to 4 us, but costs of that and more
+    // make slices too short where the numbers above are off: 300 shapes of 9 to 200 rows, against choices without it: 1.5 us 0.21 % shorter in
+    // the mean, the worst 1.8 % longer (65 x 8317 x 3840 Q6_K 39.8 us, 39.7, but 42.5 from 3 us on), the best 23 % shorter (37 x 7136 x 1056
+    // Q8_0 19.3, 15.1).
+    const double prepare_us = 1.5;
     const double start = 5.64, bar = mmfw_chain_bar(ctx, fmt, n, count, k);
     double best = 1e300;
     for (uint32_t ks = 1; ks <= std::min(L.groups, 32u); ++ks) {
@@ -1244,7 +1249,8 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
                 // (runs of weight tiles only where they save rounds)
                 const uint32_t most = mmfw_run_ok(fmt, pl + 1, mt, L.groups, ks) ? static_cast<uint32_t>(std::min<uint64_t>(16, (items + static_cast<uint64_t>(cus) - 1) / static_cast<uint64_t>(cus))) : 1u;
                 for (uint32_t run = 1; run <= most; ++run) {
-                    const double us = std::ceil(static_cast<double>(m_tiles * ((tiles + run - 1) / run) * ks) / cus) * (run * tile + start) + meet;
+                    const double prepare = mt == 1 && bps <= mmfw_own_blocks(fmt, pl + 1) ? 0.0 : prepare_us;
+                    const double us = std::ceil(static_cast<double>(m_tiles * ((tiles + run - 1) / run) * ks) / cus) * (run * tile + start) + meet + prepare;
                     if (us < of[pl]) {
                         of[pl] = us;
                         of_mt[pl] = mt;
