@@ -451,11 +451,12 @@ struct MmfwShape {
     static constexpr uint32_t TILE_CHUNK = 2u * UC * PL * 1024u; // a row tile's share: contiguous in its image
     static constexpr uint32_t extra = 0;               // [4][sums of MT tiles, inverse scales]
     static constexpr uint32_t EXTRA = ((F::SUMS ? MT : 0) + 1) * 1024u;
-    static constexpr uint32_t stage = 4u * EXTRA;
+    static constexpr uint32_t SLOTS = OWN ? 8u : 4u;
+    static constexpr uint32_t stage = SLOTS * EXTRA;
     static constexpr uint32_t ring = stage + MMFW_WAVES * F::STAGE;
     // OWN: the images of a slice's blocks are made here, all of them ahead of the first product, and take the ring's place
-    // (four places of sums and scales: one more than blocks, read past the last)
-    static constexpr int OWN_FIT = (160u * 1024u - ring) / (C * CHUNK), OWN_BLOCKS = OWN_FIT < 3 ? OWN_FIT : 3;
+    // (eight places of sums and scales: more than blocks, the next one is read past the last)
+    static constexpr int OWN_FIT = (160u * 1024u - ring) / (C * CHUNK), OWN_BLOCKS = OWN_FIT < 4 ? OWN_FIT : 4;
     static constexpr uint32_t RING = OWN ? OWN_BLOCKS * C * CHUNK : R * CHUNK;
     static constexpr uint32_t total = ring + RING;
     static_assert(total <= 160u * 1024u, "LDS");

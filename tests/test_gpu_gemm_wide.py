@@ -57,7 +57,7 @@ def test_weights_in_units(torch, oracle, dtype, tiles, blocks):
 
 @pytest.mark.parametrize("dtype", ALL)
 @pytest.mark.parametrize("elem", ["float32", "float16", "bfloat16"])
-@pytest.mark.parametrize("slices, blocks", [(1, 1), (1, 2), (1, 3), (2, 2), (2, 3), (3, 3), (3, 4)])
+@pytest.mark.parametrize("slices, blocks", [(1, 1), (1, 2), (1, 3), (1, 4), (1, 5), (2, 2), (2, 3), (3, 3), (3, 4)])
 def test_images_made_by_the_workgroup(torch, dtype, elem, slices, blocks):
     """Short slices of K, whose workgroups prepare their activations themselves: the bits of the launch that prepares them, with
     blocks that K does not fill, a slice shorter than the rest, rows past the last, rows of zeros, tiny, huge and non-finite ones,
