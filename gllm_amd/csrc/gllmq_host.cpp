@@ -1294,7 +1294,7 @@ struct MmfwSlices {
 };
 
 // The GEMM over `count` matrices of one format and K that share their activations: one launch that
-// prepares the activation images, one that multiplies, and one that adds the slices of K where
+// prepares the activation images (not where workgroups do: mmfw_takes_own), one that multiplies, and one that adds the slices of K where
 // there are any.  Returns -1 for what it does not take.
 // `elem_x`, `elem_y`: element types of the activations and of the outputs.
 // `leave`: the sums of slices may stay where they are (where both calls fit the scratch in one pass each); `take`: the
