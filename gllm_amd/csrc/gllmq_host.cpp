@@ -1220,7 +1220,7 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
     // A launch that prepares the activations, where workgroups do not do it themselves.  It takes 3 to 4 us, but costs of that and more
     // make slices too short where the numbers above are off: 300 shapes of 9 to 200 rows, against choices without it: 1.5 us 0.21 % shorter in
     // the mean, the worst 1.8 % longer (65 x 8317 x 3840 Q6_K 39.8 us, 39.7, but 42.5 from 3 us on), the best 23 % shorter (37 x 7136 x 1056
-    // Q8_0 19.3, 15.1).
+    // Q8_0 19.3, 15.1).  900 other shapes: no cost 0.17 % longer in the mean, the worst 29 %; 2.5 to 4.5 us level with 1.5.
     const double prepare_us = 1.5;
     const double start = 5.64, bar = mmfw_chain_bar(ctx, fmt, n, count, k);
     double best = 1e300;
