@@ -24,7 +24,8 @@
 #include <vector>
 
 // The code objects built from the kernels_*.hip translation units, placed in .rodata by the
-// assembler (GLLMQ_HSACO_DIR is the build directory).
+// assembler (GLLMQ_HSACO_DIR is the build directory).  A test of this file without a GPU has its own stand-ins.
+#ifndef GLLMQ_EMBED
 #define GLLMQ_EMBED(NAME)                                                              \
     __asm__(".section .rodata\n"                                                       \
             ".balign 4096\n"                                                           \
@@ -34,6 +35,7 @@
             ".byte 0\n"                                                                \
             ".previous\n");                                                            \
     extern "C" const unsigned char gllmq_co_##NAME[];
+#endif
 GLLMQ_EMBED(codec)
 GLLMQ_EMBED(mm8)
 GLLMQ_EMBED(mm8s)
@@ -1287,7 +1289,8 @@ bool mmfw_takes_own(const gllmq_ctx *ctx, const MmfwPlan &L, int fmt, size_t m, 
 // The sums of K slices of a feed-forward block's gate and up rows, left in the scratch for the preparation of the down
 // projection, which adds them up while it applies the gate: a launch less, and the sums' way to memory and back.
 struct MmfwSlices {
-    size_t next_need = 0;    // scratch that the down projection needs
+    size_t next_need = 0;    // scratch that the down projection needs,
+    size_t next_reserve = 0; // and that it grows the scratch to
     const float *at = nullptr;
     uint32_t slices = 0;     // 0: none were left
     size_t used = 0;         // bytes of the scratch in use
@@ -1297,7 +1300,8 @@ struct MmfwSlices {
 // prepares the activation images (not where workgroups do: mmfw_takes_own), one that multiplies, and one that adds the slices of K where
 // there are any.  Returns -1 for what it does not take.
 // `elem_x`, `elem_y`: element types of the activations and of the outputs.
-// `leave`: the sums of slices may stay where they are (where both calls fit the scratch in one pass each); `take`: the
+// `leave`: the sums of slices may stay where they are (where both calls fit the scratch in one pass each; it is not grown for that: what
+// it is grown to depends on rows and K alone, so that no call of as many or fewer rows frees what a graph holds); `take`: the
 // activations are such sums.
 int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats, int count, const float *x, uint32_t elem_x,
              uint32_t elem_y, size_t m, size_t k, bool act_bf16, void *stream, size_t min_m, MmfwSlices *leave = nullptr, const MmfwSlices *take = nullptr)
@@ -1315,7 +1319,7 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
     const bool may_leave = leave && L.ksplit > 1 && L.rows >= m;
     const size_t used = (L.need() + 255) & ~size_t(255);
     size_t reserve = std::max(L.need(), mmfw_reserve(ctx, m, k));
-    if (may_leave) reserve = std::max(reserve, used + leave->next_need);
+    if (may_leave) reserve = std::max(reserve, leave->next_reserve);
     if (!take && S.mmf_bytes < reserve && !S.fixed && !stream_is_capturing(stream)) rc = grow_scratch(ctx, S, &S.mmf, &S.mmf_bytes, reserve, stream, "quantized_matmul (GEMM)");
     if (rc != GLLMQ_OK) return rc;
     const bool leaves = may_leave && used + leave->next_need <= S.mmf_bytes;
@@ -2572,20 +2576,15 @@ int ffn_on_stream(gllmq_ctx *ctx, const void *gate_w, const void *up_w, size_t g
     // down 2 x 4096 x 14336, five bf16 rows 47.5, 61.1; eight 59.9, 61.7).
     const bool wide = m >= std::max(5u, std::min(ctx->mmfw_min_m, ctx->mmfw_small_min_m)) ||
                       (ctx->ffn_fused && 2 * ffn * hidden >= (64ull << 20) && mmfw_takes_few(ctx, dtype_gate_up, m)); // ("ffn_fused" off: up to 8 rows in separate steps)
-    auto down_fits = [&] {
-        MmfwPlan L = plan_mmfw(ctx, dtype_down, m, &hidden, 1, ffn, false);
-        return L.ok && mmfw_fit(ctx, S, L, stream);
-    };
-    auto gate_up_fits = [&] {
-        MmfwPlan L = plan_mmfw(ctx, dtype_gate_up, m, gate_up_n, 2, hidden, elem != 0);
-        return L.ok && mmfw_fit(ctx, S, L, stream);
-    };
-    if (wide && !ctx->mmfs_all && ffn % 4 == 0 && m * ffn <= 0xFFFFFFFFull && down_fits() && gate_up_fits()) {
+    auto fits = [&](MmfwPlan L) { return L.ok && mmfw_fit(ctx, S, L, stream); };
+    MmfwPlan down_plan;
+    if (wide && !ctx->mmfs_all && ffn % 4 == 0 && m * ffn <= 0xFFFFFFFFull) down_plan = plan_mmfw(ctx, dtype_down, m, &hidden, 1, ffn, false);
+    if (fits(down_plan) && fits(plan_mmfw(ctx, dtype_gate_up, m, gate_up_n, 2, hidden, elem != 0))) {
         const MmfwMatrix gate_up[2] = { { gw, gu, ffn }, { uw, gu + m * ffn, ffn } };
         MmfwSlices sums;
-        const MmfwPlan L = plan_mmfw(ctx, dtype_down, m, &hidden, 1, ffn, false);
-        sums.next_need = std::max(L.need(), mmfw_reserve(ctx, m, ffn)); // (what the down projection would grow the scratch to)
-        rc = run_mmfw(ctx, S, *fg, gate_up, 2, x, elem, 0, m, hidden, false, stream, 5, ctx->ffn_glu_load && L.rows >= m ? &sums : nullptr);
+        sums.next_need = down_plan.need();
+        sums.next_reserve = std::max(down_plan.need(), mmfw_reserve(ctx, m, ffn));
+        rc = run_mmfw(ctx, S, *fg, gate_up, 2, x, elem, 0, m, hidden, false, stream, 5, ctx->ffn_glu_load && down_plan.rows >= m ? &sums : nullptr);
         if (rc > 0) return rc;
         if (rc == GLLMQ_OK) {
             const MmfwMatrix down{ static_cast<const uint8_t *>(down_w), out, hidden };
@@ -3638,13 +3637,6 @@ int gllmq_reserve_ffn(gllmq_ctx *ctx, uint32_t dtype_gate_up, uint32_t dtype_dow
     Scratch *S = nullptr;
     rc = acquire_scratch(ctx, stream, &S);
     if (rc != GLLMQ_OK) return rc;
-    // (gate's and up's sums of slices beside what the down projection takes)
-    const size_t gate_up_n[2] = { ffn, ffn };
-    const MmfwPlan L = plan_mmfw(ctx, dtype_gate_up, m, gate_up_n, 2, hidden, false);
-    if (m >= 5 && L.ok && L.ksplit > 1) {
-        rc = grow_scratch(ctx, *S, &S->mmf, &S->mmf_bytes, ((L.need() + 255) & ~size_t(255)) + mmfw_reserve(ctx, m, ffn), stream, "reserve_ffn");
-        if (rc != GLLMQ_OK) return rc;
-    }
     return grow_scratch(ctx, *S, &S->ffn, &S->ffn_bytes, ffn_scratch_bytes(m, ffn), stream, "reserve_ffn");
 }
 

@@ -1,0 +1,221 @@
+// What the host code enqueues and allocates, on the CPU: the library's host source over stand-ins for the HIP runtime that record
+// launches (kernel, grid, arguments) and allocations.  Device pointers are numbers here; nothing follows them.
+//
+//   host_routes [check]     prints "ok" or what does not hold; exit status 0 or 1
+#define GLLMQ_EMBED(NAME) extern "C" const unsigned char gllmq_co_##NAME[1] = { 0 };
+#include "../../gllm_amd/csrc/gllmq_host.cpp"
+
+#include <functional>
+#include <map>
+#include <set>
+
+extern "C" int gq_noalloc_init(gllmq_ctx *, int) { return GLLMQ_OK; }
+
+namespace fake {
+
+struct Launch {
+    std::string kernel;
+    uint32_t grid;
+    std::vector<uint8_t> args;
+    gq::MmfwParams wide() const
+    {
+        gq::MmfwParams P;
+        if (args.size() != sizeof P) abort();
+        std::memcpy(static_cast<void *>(&P), args.data(), sizeof P);
+        return P;
+    }
+};
+
+std::set<std::string> names;
+std::vector<Launch> launches;
+std::map<void *, size_t> live; // device allocations
+size_t allocations = 0, frees = 0;
+uintptr_t next_address = uintptr_t(1) << 40;
+bool capturing = false;
+
+hipError_t record(hipFunction_t f, uint32_t grid, void **extra)
+{
+    size_t size = 0;
+    const uint8_t *args = nullptr;
+    for (int i = 0; extra[i] != HIP_LAUNCH_PARAM_END; i += 2) {
+        if (extra[i] == HIP_LAUNCH_PARAM_BUFFER_POINTER) args = static_cast<const uint8_t *>(extra[i + 1]);
+        if (extra[i] == HIP_LAUNCH_PARAM_BUFFER_SIZE) size = *static_cast<const size_t *>(extra[i + 1]);
+    }
+    launches.push_back({ *reinterpret_cast<const std::string *>(f), grid, std::vector<uint8_t>(args, args + size) });
+    return hipSuccess;
+}
+
+} // namespace fake
+
+extern "C" {
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
+hipError_t hipGetLastError(void) { return hipSuccess; }
+const char *hipGetErrorString(hipError_t) { return "error"; }
+hipError_t hipGetDeviceProperties(hipDeviceProp_t *p, int) // (the header's macro gives it its versioned name)
+{
+    std::memset(static_cast<void *>(p), 0, sizeof *p);
+    p->multiProcessorCount = 256;
+    std::strcpy(p->gcnArchName, "gfx950");
+    return hipSuccess;
+}
+hipError_t hipMalloc(void **p, size_t size)
+{
+    *p = reinterpret_cast<void *>(fake::next_address);
+    fake::next_address += (size + 4095) / 4096 * 4096;
+    fake::live[*p] = size;
+    ++fake::allocations;
+    return hipSuccess;
+}
+hipError_t hipFree(void *p)
+{
+    if (p && !fake::live.erase(p)) abort();
+    fake::frees += p != nullptr;
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void **p, size_t size, unsigned)
+{
+    *p = std::calloc(1, size);
+    return hipSuccess;
+}
+hipError_t hipHostFree(void *p)
+{
+    std::free(p);
+    return hipSuccess;
+}
+hipError_t hipMemset(void *, int, size_t) { return hipSuccess; }
+hipError_t hipMemcpy(void *, const void *, size_t, hipMemcpyKind) { return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *, unsigned) { return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *, unsigned) { return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *s)
+{
+    *s = fake::capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
+hipError_t hipModuleLoadData(hipModule_t *m, const void *)
+{
+    static int any;
+    *m = reinterpret_cast<hipModule_t>(&any);
+    return hipSuccess;
+}
+hipError_t hipModuleUnload(hipModule_t) { return hipSuccess; }
+hipError_t hipModuleGetFunction(hipFunction_t *f, hipModule_t, const char *name)
+{
+    *f = reinterpret_cast<hipFunction_t>(const_cast<std::string *>(&*fake::names.insert(name).first));
+    return hipSuccess;
+}
+hipError_t hipModuleLaunchKernel(hipFunction_t f, unsigned gx, unsigned, unsigned, unsigned, unsigned, unsigned, unsigned, hipStream_t, void **, void **extra)
+{
+    return fake::record(f, gx, extra);
+}
+hipError_t hipExtModuleLaunchKernel(hipFunction_t f, uint32_t gx, uint32_t, uint32_t, uint32_t bx, uint32_t, uint32_t, size_t, hipStream_t, void **, void **extra,
+                                    hipEvent_t, hipEvent_t, uint32_t)
+{
+    return fake::record(f, gx / bx, extra);
+}
+}
+
+namespace {
+
+int failures = 0;
+#define EXPECT(what, ...)                                   \
+    do {                                                    \
+        if (!(what) && ++failures <= 10) {                  \
+            std::printf("%s:%d: " #what ": ", __func__, __LINE__); \
+            std::printf(__VA_ARGS__);                       \
+            std::printf("\n");                              \
+        }                                                   \
+    } while (0)
+
+struct Context {
+    gllmq_ctx *ctx = nullptr;
+    Context() { gllmq_init(&ctx, 0); }
+    ~Context() { gllmq_destroy(ctx); }
+    operator gllmq_ctx *() const { return ctx; }
+};
+
+// addresses of a caller's own buffers, far from each other
+void *at(int i) { return reinterpret_cast<void *>((uintptr_t(1) << 44) + (uintptr_t(i) << 36)); }
+
+int ffn(gllmq_ctx *ctx, uint32_t gate_up, uint32_t down, size_t m, size_t hidden, size_t ffn, int elem = GLLMQ_ELEM_F32)
+{
+    fake::launches.clear();
+    return gllmq_ffn_swiglu_elem(ctx, at(1), at(2), ffn * gllmq_row_bytes(gate_up, hidden), gate_up, at(3), hidden * gllmq_row_bytes(down, ffn), down, at(4), at(5),
+                                 m, hidden, ffn, 0, elem, 0, nullptr);
+}
+
+size_t launched(const char *kernel)
+{
+    size_t n = 0;
+    for (const fake::Launch &l : fake::launches) n += l.kernel == kernel;
+    return n;
+}
+
+constexpr uint32_t kMixes[5][2] = { { T_Q4_K, T_Q6_K }, { T_Q5_K, T_Q6_K }, { T_Q6_K, T_Q6_K }, { T_Q8_0, T_Q8_0 }, { T_Q4_K, T_Q4_K } };
+constexpr size_t kLayers[5][2] = { { 4096, 14336 }, { 2048, 5632 }, { 1024, 2816 }, { 5120, 13824 }, { 2304, 6912 } };
+
+// The header's promise: what is reserved for, or grown by, one call serves every call of as many or fewer rows, so that a graph
+// captured behind it keeps the scratch it holds.
+void ffn_scratch_stays()
+{
+    for (const auto &mix : kMixes)
+        for (const auto &layer : kLayers)
+            for (size_t most : { 16u, 32u, 64u, 100u, 128u, 512u })
+                for (bool reserved : { false, true }) {
+                    Context ctx;
+                    if (reserved) EXPECT(gllmq_reserve_ffn(ctx, mix[0], mix[1], most, layer[0], layer[1], nullptr) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+                    else EXPECT(ffn(ctx, mix[0], mix[1], most, layer[0], layer[1]) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+                    const size_t before = fake::allocations, freed = fake::frees;
+                    for (size_t m = most; m >= 9; m = m > 40 ? m * 7 / 8 : m - 3) {
+                        for (int elem : { GLLMQ_ELEM_F32, GLLMQ_ELEM_BF16 }) {
+                            EXPECT(ffn(ctx, mix[0], mix[1], m, layer[0], layer[1], elem) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+                            EXPECT(fake::allocations == before && fake::frees == freed, "formats %u/%u, %zu x %zu: %zu rows grow the scratch of %zu", mix[0], mix[1],
+                                   layer[0], layer[1], m, most);
+                        }
+                        EXPECT(gllmq_reserve_ffn(ctx, mix[0], mix[1], m, layer[0], layer[1], nullptr) == GLLMQ_OK && fake::allocations == before,
+                               "formats %u/%u, %zu x %zu: reserving %zu rows grows the scratch of %zu", mix[0], mix[1], layer[0], layer[1], m, most);
+                        fake::capturing = true;
+                        EXPECT(ffn(ctx, mix[0], mix[1], m, layer[0], layer[1]) == GLLMQ_OK, "captured: %s", gllmq_last_error(ctx));
+                        fake::capturing = false;
+                    }
+                }
+}
+
+// Gate's and up's sums of K slices are left to the down projection's preparation where both fit the scratch as it is, and added up
+// by a launch of their own where they do not.
+void ffn_slices_are_left_where_there_is_room()
+{
+    Context ctx;
+    EXPECT(ffn(ctx, T_Q4_K, T_Q6_K, 32, 4096, 14336) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+    EXPECT(launched("gq_mmf_reduce") == 2, "%zu", launched("gq_mmf_reduce"));
+    EXPECT(ffn(ctx, T_Q4_K, T_Q6_K, 16, 4096, 14336) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+    EXPECT(launched("gq_mmf_reduce") == 1, "%zu", launched("gq_mmf_reduce"));
+    Context larger;
+    EXPECT(ffn(larger, T_Q4_K, T_Q6_K, 64, 4096, 14336) == GLLMQ_OK && ffn(larger, T_Q4_K, T_Q6_K, 32, 4096, 14336) == GLLMQ_OK, "%s", gllmq_last_error(larger));
+    EXPECT(launched("gq_mmf_reduce") == 1, "%zu", launched("gq_mmf_reduce"));
+}
+
+const std::map<std::string, std::function<void()>> kChecks = {
+    { "ffn_scratch_stays", ffn_scratch_stays },
+    { "ffn_slices_are_left_where_there_is_room", ffn_slices_are_left_where_there_is_room },
+};
+
+} // namespace
+
+int main(int argc, char **argv)
+{
+    if (argc > 1 && !kChecks.count(argv[1])) {
+        std::printf("no check %s\n", argv[1]);
+        return 1;
+    }
+    for (const auto &check : kChecks)
+        if (argc < 2 || check.first == argv[1]) check.second();
+    if (failures) std::printf("%d failures\n", failures);
+    else std::printf("ok\n");
+    return failures ? 1 : 0;
+}

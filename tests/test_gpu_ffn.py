@@ -233,3 +233,36 @@ def test_gate_and_up_left_as_sums_of_slices(torch, t_gu, t_dn, m, hidden, ffn, k
                 assert torch.equal(got, want), way
         torch.cuda.synchronize()
         assert torch.equal(got, want), way
+
+
+def test_smaller_calls_leave_a_graphs_scratch_alone(torch):
+    """What is reserved for one number of rows serves every smaller one, also where a smaller call has more slices of K: eager
+    calls of fewer rows take no device memory, and the graph captured behind the reservation goes on giving the eager bits."""
+    from gllm_amd.backend import HipBackend
+    hidden, ffn, most = 4096, 14336, 128
+    hip = HipBackend(0)
+    gate, up = dev_bytes(torch, random_weight(Q4_K, ffn, hidden, seed=1)), dev_bytes(torch, random_weight(Q4_K, ffn, hidden, seed=2))
+    down = dev_bytes(torch, random_weight(Q6_K, hidden, ffn, seed=3))
+    xs = {m: torch.from_numpy(random_activations(m, hidden, seed=m) * 1e-2).cuda() for m in (most, 33, 48, 64, 100)}
+    outs = {m: torch.zeros(m, hidden, device="cuda") for m in xs}
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        def call(m):
+            hip.ffn_swiglu(gate, up, Q4_K, down, Q6_K, xs[m], outs[m], m, hidden, ffn)
+        hip.reserve_ffn(Q4_K, Q6_K, most, hidden, ffn)
+        call(most)
+        torch.cuda.synchronize()
+        want = outs[most].clone()
+        with torch.cuda.graph(graph, stream=stream):
+            call(most)
+        free = torch.cuda.mem_get_info()[0]
+        for m in (33, 48, 64, 100):
+            print(f"ffn of {m} rows beside a graph of {most}", flush=True)
+            call(m)
+            torch.cuda.synchronize()
+            assert torch.cuda.mem_get_info()[0] == free, m
+            outs[most].fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(outs[most], want), m
