@@ -1078,6 +1078,13 @@ int run_mmf(gllmq_ctx *ctx, Scratch &S, const Format &f, const uint8_t *w, const
     return GLLMQ_OK;
 }
 
+// Whether [a, a + an) and [b, b + bn) share a byte.
+bool ranges_meet(const void *a, size_t an, const void *b, size_t bn)
+{
+    const uintptr_t a0 = reinterpret_cast<uintptr_t>(a), b0 = reinterpret_cast<uintptr_t>(b);
+    return a0 < b0 + bn && b0 < a0 + an;
+}
+
 // One weight matrix of a GEMM launch.
 struct MmfwMatrix {
     const uint8_t *w;
@@ -1327,7 +1334,9 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
     const int fmt = mmf_format(f.dtype);
     const uint32_t ldx = row_stride_x(ctx, k);
     const size_t x_bytes = elem_x ? 2 : 4;
-    const bool own = mmfw_takes_own(ctx, L, fmt, m, k, ldx, x_bytes) && !take && !ctx->call_glu && !act_bf16;
+    bool own = mmfw_takes_own(ctx, L, fmt, m, k, ldx, x_bytes) && !take && !ctx->call_glu && !act_bf16;
+    // outputs over the activations: what one workgroup stores another may still have to read
+    for (int i = 0; i < count && L.ksplit == 1; ++i) own = own && !ranges_meet(mats[i].y, m * mats[i].n * (elem_y ? 2 : 4), x, m * ldx * x_bytes);
     for (size_t m0 = 0; m0 < m; m0 += L.rows) {
         const uint32_t mm = static_cast<uint32_t>(std::min(L.rows, m - m0));
         gq::MmfwPrepParams Q{};
@@ -1606,13 +1615,6 @@ bool chain_entry_ok(const gllmq_ctx *ctx, const gllmq_matmul_desc &d, const gllm
     if (rb % f->w_align != 0 || d.w_bytes < d.n * rb) return false;
     const size_t cus = static_cast<size_t>(ctx->num_cus);
     return d.n > 0 && (d.n + cus - 1) / cus >= ctx->chain_min_rows; // rows of the largest share
-}
-
-// Whether [a, a + an) and [b, b + bn) share a byte.
-bool ranges_meet(const void *a, size_t an, const void *b, size_t bn)
-{
-    const uintptr_t a0 = reinterpret_cast<uintptr_t>(a), b0 = reinterpret_cast<uintptr_t>(b);
-    return a0 < b0 + bn && b0 < a0 + an;
 }
 
 constexpr size_t kChainBoxPairs = size_t(1) << 19; // 64-bit words of the mailbox (4 MiB per stream that runs such chains)

@@ -149,6 +149,23 @@ int ffn(gllmq_ctx *ctx, uint32_t gate_up, uint32_t down, size_t m, size_t hidden
                                  m, hidden, ffn, 0, elem, 0, nullptr);
 }
 
+int matmul(gllmq_ctx *ctx, uint32_t dtype, size_t m, size_t n, size_t k, int elem, void *x, void *y, int mode = GLLMQ_ACT_F32_SPLIT)
+{
+    fake::launches.clear();
+    const size_t bytes = n * gllmq_row_bytes(dtype, k);
+    if (elem != GLLMQ_ELEM_F32) return gllmq_quantized_matmul_elem(ctx, at(1), bytes, x, y, dtype, m, n, k, elem, nullptr);
+    return gllmq_quantized_matmul_ex(ctx, at(1), bytes, static_cast<const float *>(x), static_cast<float *>(y), dtype, m, n, k, mode, nullptr);
+}
+
+// the wide GEMM among the launches, if it is there
+const fake::Launch *wide_launch()
+{
+    for (const fake::Launch &l : fake::launches)
+        if (l.kernel.find("gq_mmf_") == 0 && l.kernel.find("_w") != std::string::npos) return &l;
+    return nullptr;
+}
+bool makes_own_images(const fake::Launch &l) { return l.kernel.find("_own") != std::string::npos; }
+
 size_t launched(const char *kernel)
 {
     size_t n = 0;
@@ -200,7 +217,33 @@ void ffn_slices_are_left_where_there_is_room()
     EXPECT(launched("gq_mmf_reduce") == 1, "%zu", launched("gq_mmf_reduce"));
 }
 
+// Outputs over the activations: workgroups that make their images themselves would read rows that others have stored over.  They
+// may only where the outputs are stored by the launch that adds up slices.
+void outputs_over_the_activations()
+{
+    Context ctx;
+    size_t apart = 0, in_place = 0;
+    for (const auto &f : kFormats)
+        for (size_t k : { 256u, 512u, 768u, 1024u, 2048u, 4096u })
+            for (size_t m : { 33u, 64u, 100u, 512u, 2048u })
+                for (int elem : { GLLMQ_ELEM_F32, GLLMQ_ELEM_BF16 })
+                    for (intptr_t shift : { intptr_t(-1), intptr_t(0), intptr_t(1) }) { // y from before x's end, x itself, x's last bytes
+                        const size_t e = elem == GLLMQ_ELEM_F32 ? 4 : 2, size = m * k * e;
+                        uint8_t *const x = static_cast<uint8_t *>(at(4)) + size;
+                        EXPECT(matmul(ctx, f.dtype, m, k, k, elem, x, x + size) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+                        const fake::Launch *l = wide_launch();
+                        EXPECT(l, "no wide launch");
+                        apart += l && makes_own_images(*l) && l->wide().ksplit == 1;
+                        EXPECT(matmul(ctx, f.dtype, m, k, k, elem, x, x + shift * static_cast<intptr_t>(size - 4)) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+                        l = wide_launch();
+                        EXPECT(l && (!makes_own_images(*l) || l->wide().ksplit > 1), "dtype %u, %zu rows of %zu in place: %s", f.dtype, m, k, l ? l->kernel.c_str() : "");
+                        in_place += l && makes_own_images(*l);
+                    }
+    EXPECT(apart > 20 && in_place > 20, "%zu and %zu calls make their images", apart, in_place);
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
+    { "outputs_over_the_activations", outputs_over_the_activations },
     { "ffn_scratch_stays", ffn_scratch_stays },
     { "ffn_slices_are_left_where_there_is_room", ffn_slices_are_left_where_there_is_room },
 };

@@ -87,6 +87,26 @@ def test_images_made_by_the_workgroup(torch, dtype, elem, slices, blocks):
             assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
 
 
+@pytest.mark.parametrize("dtype", ALL)
+@pytest.mark.parametrize("elem", ["float32", "bfloat16"])
+def test_outputs_over_the_activations(torch, dtype, elem):
+    """A square matmul in place, of a size whose workgroups make their images themselves where the outputs lie elsewhere: the same
+    bits."""
+    from gllm_amd.backend import HipBackend
+    t, hip = getattr(torch, elem), HipBackend(0, options={"mmfw_mt": 1, "mmfw_ksplit": 1})
+    for m, k in ((64, 512), (200, 512)):
+        print(f"in place dtype={dtype} {elem} m={m} k={k}", flush=True)
+        w = torch.from_numpy(random_weight(dtype, k, k, seed=k)).cuda()
+        x = torch.from_numpy(random_activations(m, k, seed=m)).cuda().to(t)
+        y = torch.zeros_like(x)
+        hip.quantized_matmul(w, x, y, dtype, m, k, k)
+        assert "_own" in hip.last_kernel_name(), hip.last_kernel_name()
+        hip.quantized_matmul(w, x, x, dtype, m, k, k)
+        assert "_own" not in hip.last_kernel_name(), hip.last_kernel_name()
+        torch.cuda.synchronize()
+        assert torch.equal(x, y)
+
+
 @pytest.mark.parametrize("dtype", [Q4_K, Q5_K])
 @pytest.mark.parametrize("tiles", [2, 3, 4])
 @pytest.mark.parametrize("run", [2, 3, 16])
