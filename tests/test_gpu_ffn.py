@@ -256,9 +256,9 @@ def test_smaller_calls_leave_a_graphs_scratch_alone(torch):
         want = outs[most].clone()
         with torch.cuda.graph(graph, stream=stream):
             call(most)
-        free = torch.cuda.mem_get_info()[0]
         for m in (33, 48, 64, 100):
             print(f"ffn of {m} rows beside a graph of {most}", flush=True)
+            free = torch.cuda.mem_get_info()[0]  # (each time: torch takes memory for the comparisons below)
             call(m)
             torch.cuda.synchronize()
             assert torch.cuda.mem_get_info()[0] == free, m
