@@ -1108,10 +1108,10 @@ struct MmfwPlan {
 int mmf_format(uint32_t dtype) { return dtype == T_Q8_0 ? 3 : dtype == T_Q6_K ? 2 : dtype == T_Q5_K ? 1 : 0; }
 
 // Whether a workgroup may take several weight tiles one after the other (mmfw_may_run): all of K, long enough for requests to reach
-// into the next tile only, and no unit of two blocks across its end.
+// into the next tile only.
 bool mmfw_run_ok(int fmt, int planes, uint32_t mt, uint32_t groups, uint32_t ksplit)
 {
-    return ksplit == 1 && groups >= 4 && groups % 2 == 0 && gq::mmfw_may_run(fmt, planes, static_cast<int>(mt), false);
+    return ksplit == 1 && groups >= 4 && gq::mmfw_may_run(fmt, planes, static_cast<int>(mt), false);
 }
 
 uint32_t mmfw_inv_ld(size_t rows) { return static_cast<uint32_t>((rows + 31) / 32 * 32); }

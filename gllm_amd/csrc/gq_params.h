@@ -614,7 +614,7 @@ struct MmfwParams {
     uint32_t m_tiles, n_tiles; // workgroup tiles of activation rows and of weight rows (all matrices)
     uint32_t ksplit, blocks_per_split;
     uint32_t run_mask;         // blocks whose sums are taken in one run, less one (a power of two less one; all ones: a slice's all)
-    uint32_t run_tiles;        // weight tiles that a workgroup multiplies one after the other (more than one: all of K, an even number of four or more blocks)
+    uint32_t run_tiles;        // weight tiles that a workgroup multiplies one after the other (more than one: all of K, four or more blocks)
     uint32_t n_runs;           // runs of them: ceil(n_tiles / run_tiles)
     uint32_t items;            // m_tiles * n_runs * ksplit
     uint32_t band;             // activation tiles that neighbouring workgroups share a weight tile over

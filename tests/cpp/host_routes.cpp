@@ -157,6 +157,16 @@ int matmul(gllmq_ctx *ctx, uint32_t dtype, size_t m, size_t n, size_t k, int ele
     return gllmq_quantized_matmul_ex(ctx, at(1), bytes, static_cast<const float *>(x), static_cast<float *>(y), dtype, m, n, k, mode, nullptr);
 }
 
+int batch(gllmq_ctx *ctx, uint32_t dtype, size_t m, const std::vector<size_t> &n, size_t k, int elem)
+{
+    fake::launches.clear();
+    const uint32_t flags = elem == GLLMQ_ELEM_F16 ? GLLMQ_DESC_ELEM_F16 : elem == GLLMQ_ELEM_BF16 ? GLLMQ_DESC_ELEM_BF16 : 0u;
+    std::vector<gllmq_matmul_desc> descs;
+    for (size_t i = 0; i < n.size(); ++i)
+        descs.push_back({ at(10 + static_cast<int>(i)), n[i] * gllmq_row_bytes(dtype, k), static_cast<const float *>(at(4)), static_cast<float *>(at(20 + static_cast<int>(i))), dtype, flags, m, n[i], k });
+    return gllmq_quantized_matmul_batch(ctx, descs.data(), descs.size(), nullptr);
+}
+
 // the wide GEMM among the launches, if it is there
 const fake::Launch *wide_launch()
 {
@@ -242,7 +252,40 @@ void outputs_over_the_activations()
     EXPECT(apart > 20 && in_place > 20, "%zu and %zu calls make their images", apart, in_place);
 }
 
+// Several weight tiles per workgroup: the calls of test_runs_of_weight_tiles (test_gpu_gemm_wide.py) take them, odd numbers of blocks among
+// them, and so do prompts by themselves; nothing that the kernel cannot do takes them.
+void runs_of_weight_tiles()
+{
+    for (uint32_t dtype : { T_Q4_K, T_Q5_K })
+        for (uint32_t tiles : { 2u, 3u, 4u })
+            for (uint32_t run : { 2u, 3u, 16u }) {
+                Context ctx;
+                gllmq_set_option(ctx, "mmfw_mt", tiles);
+                gllmq_set_option(ctx, "mmfw_ksplit", 1);
+                gllmq_set_option(ctx, "mmfw_run", run);
+                const size_t shapes[3][2] = { { 65, 1024 }, { 130, 1536 - 64 }, { 200, 1280 } };
+                for (const auto &s : shapes) {
+                    EXPECT(batch(ctx, dtype, s[0], { 513, 256, 300 }, s[1], GLLMQ_ELEM_BF16) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+                    const fake::Launch *l = wide_launch();
+                    EXPECT(l && l->wide().segs == 3 && l->wide().run_tiles == std::min(run, 6u), "K of %zu, three matrices", s[1]);
+                    EXPECT(matmul(ctx, dtype, s[0], 513, s[1], GLLMQ_ELEM_BF16, at(4), at(5)) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+                    l = wide_launch();
+                    EXPECT(l && l->wide().run_tiles == std::min(run, 3u) && l->wide().n_runs == (3 + run - 1) / run, "K of %zu", s[1]);
+                }
+            }
+    Context ctx;
+    for (const auto &f : kFormats)
+        for (size_t k : { 512u, 768u, 1024u, 1280u, 2304u, 4096u, 6912u, 8960u, 11008u })
+            for (int elem : { GLLMQ_ELEM_F32, GLLMQ_ELEM_BF16 }) {
+                EXPECT(matmul(ctx, f.dtype, 2048, 28672, k, elem, at(4), at(5)) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+                const fake::Launch *l = wide_launch();
+                const bool can = k >= 1024 && elem != GLLMQ_ELEM_F32 && (f.dtype == T_Q4_K || f.dtype == T_Q5_K);
+                EXPECT(l && (l->wide().run_tiles > 1) == can, "dtype %u, K of %zu, element type %d: %u tiles", f.dtype, k, elem, l ? l->wide().run_tiles : 0u);
+            }
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
+    { "runs_of_weight_tiles", runs_of_weight_tiles },
     { "outputs_over_the_activations", outputs_over_the_activations },
     { "ffn_scratch_stays", ffn_scratch_stays },
     { "ffn_slices_are_left_where_there_is_room", ffn_slices_are_left_where_there_is_room },

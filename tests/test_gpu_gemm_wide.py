@@ -115,7 +115,7 @@ def test_runs_of_weight_tiles(torch, dtype, tiles, run):
     tile per workgroup, for the shortest rows that allow it and longer ones."""
     from gllm_amd.backend import HipBackend
     one, several = (HipBackend(0, options={"mmfw_mt": tiles, "mmfw_ksplit": 1, "mmfw_run": r}) for r in (1, run))
-    for m, k in ((65, 1024), (130, 1536 - 64), (200, 1280)):  # (the last: an odd number of blocks, no runs)
+    for m, k in ((65, 1024), (130, 1536 - 64), (200, 1280)):  # (the last: an odd number of blocks)
         x = torch.from_numpy(random_activations(m, k, seed=k)).cuda().to(torch.bfloat16)
         ws = [torch.from_numpy(random_weight(dtype, n, k, seed=n)).cuda() for n in (513, 256, 300)]
         outs = []
