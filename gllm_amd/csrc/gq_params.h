@@ -534,13 +534,12 @@ struct MmfwUnitShape {
     static constexpr uint32_t STAGE = LW * 1024u;
     static constexpr int UC = W::UC, R = FMT == 1 && UB == 2 ? 3 : 4, C = W::C, NA = W::NA;      // the activations' ring, as above
     static constexpr uint32_t CHUNK = W::CHUNK, TILE_CHUNK = W::TILE_CHUNK, EXTRA = W::EXTRA, extra = 0;
-    static_assert(TILE_CHUNK % (NA * 1024u) == 0, "a wave's pieces of a chunk are neighbours");
+    static_assert(NA == 2 && TILE_CHUNK % (NA * 1024u) == 0, "a wave's pieces of a chunk are two neighbours");
     static constexpr uint32_t stage = 4u * EXTRA;
     static constexpr uint32_t ring = stage + MMFW_WAVES * STAGE;
     static constexpr uint32_t total = ring + R * CHUNK;
     static_assert(total <= 160u * 1024u, "LDS");
     static constexpr int SG = W::SG, NS = W::NS, SPC = W::SPC;
-    static constexpr int QL = NS / 4;              // K-quants: stages per quarter of a block
     static constexpr int T = UB * NS;              // stages of a unit
     static constexpr int REQUEST = 1;              // first stage that requests of the next unit; the last reads of this one are in stage 0
     static constexpr int SPREAD = T - 2 - REQUEST > LW ? LW : T - 2 - REQUEST; // stages that share the requests
