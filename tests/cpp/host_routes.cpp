@@ -284,9 +284,37 @@ void runs_of_weight_tiles()
             }
 }
 
+// The calls of test_images_made_by_the_workgroup (test_gpu_gemm_wide.py) make their images exactly where the blocks fit, single ones and
+// batches, and with the switch never.
+void own_images()
+{
+    const uint32_t most[4][2] = { { 4, 3 }, { 4, 3 }, { 4, 3 }, { 4, 2 } }; // blocks of a slice [format][one plane, two]
+    const uint32_t slices_blocks[9][2] = { { 1, 1 }, { 1, 2 }, { 1, 3 }, { 1, 4 }, { 1, 5 }, { 2, 2 }, { 2, 3 }, { 3, 3 }, { 3, 4 } };
+    for (const auto &f : kFormats)
+        for (int elem : { GLLMQ_ELEM_F32, GLLMQ_ELEM_F16, GLLMQ_ELEM_BF16 })
+            for (const auto &sb : slices_blocks)
+                for (bool on : { true, false }) {
+                    Context ctx;
+                    gllmq_set_option(ctx, "mmfw_mt", 1);
+                    gllmq_set_option(ctx, "mmfw_ksplit", sb[0]);
+                    gllmq_set_option(ctx, "mmfw_min_m", 9);
+                    gllmq_set_option(ctx, "mmfw_own", on);
+                    const size_t k = 256 * sb[0] * sb[1] - (sb[0] > 1 && sb[1] > 1 ? 256 : 0);
+                    const bool fits = sb[1] <= most[mmf_format(f.dtype)][elem == GLLMQ_ELEM_F32];
+                    for (size_t m : { 33u, 9u, 64u })
+                        for (bool group : { false, true }) {
+                            EXPECT((group ? batch(ctx, f.dtype, m, { 64, 1 }, k, elem) : matmul(ctx, f.dtype, m, 257, k, elem, at(4), at(5))) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+                            const fake::Launch *l = wide_launch();
+                            EXPECT(l && makes_own_images(*l) == (on && fits) && l->wide().ksplit == sb[0] && l->wide().blocks_per_split == sb[1],
+                                   "dtype %u, element type %d, %u slices of %u, %zu rows: %s", f.dtype, elem, sb[0], sb[1], m, l ? l->kernel.c_str() : "no wide launch");
+                        }
+                }
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
     { "runs_of_weight_tiles", runs_of_weight_tiles },
     { "outputs_over_the_activations", outputs_over_the_activations },
+    { "own_images", own_images },
     { "ffn_scratch_stays", ffn_scratch_stays },
     { "ffn_slices_are_left_where_there_is_room", ffn_slices_are_left_where_there_is_room },
 };

@@ -79,8 +79,11 @@ def test_images_made_by_the_workgroup(torch, dtype, elem, slices, blocks):
         for hip in hips:
             print(f"own images dtype={dtype} {elem} slices={slices} blocks={blocks} m={m} k={k - cut}", flush=True)
             ys = [torch.full((m, n), 7.0, device="cuda", dtype=t) for n in sizes]
+            own = hip is hips[0] and blocks <= (4 if elem != "float32" else 2 if dtype == Q8_0 else 3)  # (slices: test_host_routes.py)
             hip.quantized_matmul(ws[0], x, ys[0], dtype, m, sizes[0], k - cut)
+            assert slices > 1 or ("_w1_own" in hip.last_kernel_name()) == own, hip.last_kernel_name()
             hip.quantized_matmul_batch([(w, x, y, dtype, m, y.shape[1], k - cut) for w, y in list(zip(ws, ys))[1:]])
+            assert slices > 1 or ("_w1_own" in hip.last_kernel_name()) == own, hip.last_kernel_name()
             torch.cuda.synchronize()
             outs.append(ys)
         for a, b in zip(*outs):
