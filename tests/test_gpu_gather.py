@@ -105,6 +105,31 @@ def test_gather_16_bit_rows(hip, torch, oracle, dtype, hidden, count):
             assert torch.allclose(got[offset:offset + n].view(count, hidden).float(), want.to(elem).float(), rtol=0, atol=0, equal_nan=True)
 
 
+@pytest.mark.parametrize("elem", ["float16", "bfloat16"])
+def test_gather_rounds_16_bit_rows(hip, torch, elem):
+    """Rows times a scale round to the nearest 16-bit value, ties to even, as torch does: ties, the largest values, subnormal
+    ones, overflow, infinities and NaN, by the 127 quants times each."""
+    t, q = getattr(torch, elem), torch.arange(-128, 128, dtype=torch.int16).to(torch.int8)
+    blocks = torch.zeros(8, 34, dtype=torch.uint8)
+    blocks[:, :2] = torch.tensor([1.0]).half().view(torch.uint8)  # (the scale of each block of quants)
+    blocks[:, 2:] = q.view(torch.uint8).view(8, 32)
+    table, ids = blocks.view(-1).cuda(), torch.zeros(1, dtype=torch.int32, device="cuda")
+    bits = [0x3F808000, 0x3F818000, 0x3F808001, 0x3F807FFF, 0x3F801000, 0x3F803000, 0x7F7FFFFF, 0x7F7F8000, 0x7F7F7FFF, 0x477FEFFF, 0x477FF000,
+            0x00008000, 0x00018000, 0x00000001, 0x007FFFFF, 0x33000000, 0x33000001, 0x387FE000, 0x7F800000, 0x7FC00000, 0x7FA00001, 0x80000000]
+    bits += [int(b) for b in np.random.default_rng(1).integers(0, 2 ** 32, 100)]
+    for b in bits:
+        scale = float(np.array([b], np.uint32).view(np.float32)[0])
+        print(f"gather {elem} scale bits {b:08x}", flush=True)
+        wide, got = torch.empty(256, device="cuda"), torch.empty(256, dtype=t, device="cuda")
+        hip.quant_gather(table, Q8_0, 1, 256, ids, wide, scale=scale)
+        hip.quant_gather(table, Q8_0, 1, 256, ids, got, scale=scale)
+        torch.cuda.synchronize()
+        want = wide.cpu().to(t)
+        nan = torch.isnan(want)
+        assert torch.equal(torch.isnan(got.cpu()), nan)
+        assert torch.equal(got.cpu()[~nan].view(torch.int16), want[~nan].view(torch.int16)), f"{b:08x}"
+
+
 def test_gather_more_rows_than_one_grid_covers(hip, torch, oracle):
     # 70000 looked-up rows: the grid's second dimension ends at 65535 and walks the rest
     vocab, hidden, count = 500, 32, 70000
