@@ -1213,7 +1213,8 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
     // through memory.  The numbers are fitted to what they decide: 135 000 calls of 6852 shapes (9 to 2048 rows, 512 to 28672 x 1024
     // to 14336, all formats, f32 and bf16; every number of tiles and up to 20 slices) were timed, half of the shapes
     // searched for the numbers whose choices are shortest, the other half kept to check: choices 0.50 % longer than the best
-    // one in the mean, 1.43 % with block times measured one by one before (1.5 to 2.7 us for one tile).
+    // one in the mean, 1.43 % with block times measured one by one before (1.5 to 2.7 us for one tile).  So they are no times of a block: Q8_0
+    // in one tile has more for one plane than for two.  They were fitted ahead of workgroups that make their images (MmfwOwn); `prepare_us` is later.
     // Slices and runs decide the order of the sums, tiles do not; so a call of 16-bit elements has the slices of the f32 call
     // whose bits it has to give: those with which the two together are shortest.  (3000 plans of 9 to 2048 rows by the
     // model, against slices of their own: 0.5 % longer in the mean, one in a hundred by more than a tenth.)
@@ -1230,6 +1231,9 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
     // make slices too short where the numbers above are off: 300 shapes of 9 to 200 rows, against choices without it: 1.5 us 0.21 % shorter in
     // the mean, the worst 1.8 % longer (65 x 8317 x 3840 Q6_K 39.8 us, 39.7, but 42.5 from 3 us on), the best 23 % shorter (37 x 7136 x 1056
     // Q8_0 19.3, 15.1).  900 other shapes: no cost 0.17 % longer in the mean, the worst 29 %; 2.5 to 4.5 us level with 1.5.
+    // Calls that cannot do without the launch (gated activations, ones rounded to bf16) have the same plan: counted for those, it trades few
+    // slices of one row tile for about twice as many of two, one plan in eighty.  40 such shapes of 33 to 118 rows, whole feed-forward
+    // blocks 0.4 % shorter in the mean (2.8 shorter to 4.3 longer), rounded matmuls 2.4 % longer (3.2 shorter to 12.3 longer).
     const double prepare_us = 1.5;
     const double start = 5.64, bar = mmfw_chain_bar(ctx, fmt, n, count, k);
     double best = 1e300;
@@ -1257,13 +1261,13 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
                 const double tile = bps * (std::max(block_us[fmt][pl][mt - 1], w_us * busy) + crowd_us * busy);
                 // (runs of weight tiles only where they save rounds)
                 const uint32_t most = mmfw_run_ok(fmt, pl + 1, mt, L.groups, ks) ? static_cast<uint32_t>(std::min<uint64_t>(16, (items + static_cast<uint64_t>(cus) - 1) / static_cast<uint64_t>(cus))) : 1u;
-                for (uint32_t run = 1; run <= most; ++run) {
+                for (uint32_t in_row = 1; in_row <= most; ++in_row) {
                     const double prepare = mt == 1 && bps <= mmfw_own_blocks(fmt, pl + 1) ? 0.0 : prepare_us;
-                    const double us = std::ceil(static_cast<double>(m_tiles * ((tiles + run - 1) / run) * ks) / cus) * (run * tile + start) + meet + prepare;
+                    const double us = std::ceil(static_cast<double>(m_tiles * ((tiles + in_row - 1) / in_row) * ks) / cus) * (in_row * tile + start) + meet + prepare;
                     if (us < of[pl]) {
                         of[pl] = us;
                         of_mt[pl] = mt;
-                        of_run[pl] = run;
+                        of_run[pl] = in_row;
                     }
                 }
             }
@@ -1286,7 +1290,8 @@ MmfwPlan plan_mmfw(const gllmq_ctx *ctx, uint32_t dtype, size_t m, const size_t 
 }
 
 // Whether workgroups prepare their activations themselves (MmfwOwn): one row tile, slices short enough for the images to stay in
-// LDS, rows that sixteen-byte loads take piece by piece.  Where it can be done it is ahead, by 3 to 4 us of 13 to 25 (MmfwOwn).
+// LDS, rows that sixteen-byte loads take piece by piece.  Where it can be done it is ahead, by 0.8 to
+// 4.5 us of 13 to 30, by format and length of the slices (MmfwOwn).
 bool mmfw_takes_own(const gllmq_ctx *ctx, const MmfwPlan &L, int fmt, size_t m, size_t k, size_t ldx, size_t x_bytes)
 {
     return ctx->use_mmfw_own && L.mt == 1 && L.bps <= mmfw_own_blocks(fmt, static_cast<int>(L.planes)) && k * x_bytes % 16 == 0 && ldx * x_bytes % 16 == 0 &&
@@ -1787,17 +1792,17 @@ int dispatch_matmul(gllmq_ctx *ctx, Scratch &S, const Format &f, const uint8_t *
     rc = run_mmfs(ctx, S, f, w, x, y, m, n, k, bf16, stream);
     if (rc >= 0 || rc == kNeedPlainActivations) return rc;
     // 9 to 32 rows of what the streamed GEMMs leave: row tiles of the GEMM for more rows.  us per call with weights that are
-    // not in the caches, f32 and bf16, against run_mmf's in brackets.  32 rows: Q6_K 13824 x 5120 36.5, 34.6 (41.0, 40.8),
-    // 4096 x 4096 21.3, 20.7 (22.7, 22.6); Q8_0 14336 x 4096 31.7, 30.1 (36.5, 36.1); Q4_K 13824 x 5120 28.0, 26.0 (29.3,
-    // 28.6), 14336 x 4096 25.6, 23.7 (25.3, 24.3).  It is not ahead everywhere: of Q4_K and Q5_K with 17 to 32 rows f32 calls
-    // of k = 4096 are 1 to 8 % behind (28672 x 4096 34.3 (33.5), 39.8 (37.3)) where bf16 calls of Q4_K are up to 6 % ahead
-    // (31.2 (33.0)) and of Q5_K level (37.2 (37.1)); both take one kernel, so that they share their bits.
+    // not in the caches, f32 and bf16, against run_mmf's in brackets.  32 rows: Q6_K 13824 x 5120 35.0, 31.1 (41.3, 39.9),
+    // 4096 x 4096 18.4, 17.6 (23.6, 23.9); Q8_0 14336 x 4096 30.8, 25.4 (35.3, 35.5); Q4_K 13824 x 5120 28.4, 24.6 (28.9,
+    // 27.9), 14336 x 4096 26.1, 21.2 (24.0, 23.3).  It is not ahead everywhere: of Q4_K and Q5_K with 17 to 32 rows f32 calls
+    // of k = 4096 are 5 to 9 % behind (28672 x 4096 36.3 (34.7), 40.1 (38.3)) where bf16 calls are as much ahead (30.3 (33.5),
+    // 33.4 (36.9)); both take one kernel, so that they share their bits.
     // Five to eight rows beyond a pass of the int8 kernels: from 10240 elements a row and 40 M weights on.  f32, us per call, here and in
-    // brackets there (eight rows of Q5_K, seven of Q6_K and of Q8_0): 4096 x 10240 20.1 (21.4), 23.6 (24.2), 24.3 (24.9); 4096 x 11520 20.5 (24.6), 25.3
-    // (28.7), 25.2 (29.9); 14336 x 14336 54.7 (66.2), 71.6 (86.4), 69.6 (96.0); below, 2390 x 11520 23.4 (18.7), 26.9 (20.0), 26.4 (20.1); 4096 x 6144 17.6
-    // (16.6), 19.8 (17.7), 20.3 (18.3); 8192 x 8192 22.3 (23.3), 27.2 (27.6), 28.0 (29.5); 28672 x 8192 60.5 (57.5), 77.2 (79.1), 75.9 (89.9); 28672 x 4096
-    // 31.1 (30.3), 44.3 (40.5), 44.8 (47.0).  16-bit calls gain more (8192 x 8192 21.0 (27.4), 25.7 (31.5), 25.4 (33.3)), but share the f32 call's bits
-    // and so its kernel.  In a pass: Q8_0 six rows of 4096 x 14336 28.5 (24.0).
+    // brackets there (eight rows of Q5_K, seven of Q6_K and of Q8_0): 4096 x 10240 19.7 (21.9), 22.6 (24.9), 26.6 (26.1); 4096 x 11520 20.7 (26.1), 24.5
+    // (29.8), 27.8 (31.8); 14336 x 14336 56.8 (67.0), 66.3 (86.4), 68.2 (96.2); below, 2390 x 11520 17.1 (18.9), 22.8 (20.4), 21.5 (20.9); 4096 x 6144 15.2
+    // (16.1), 18.9 (18.6), 17.4 (18.9); 8192 x 8192 26.2 (24.6), 29.6 (29.1), 31.0 (31.4); 28672 x 8192 61.7 (58.8), 73.5 (79.0), 74.9 (90.2); 28672 x 4096
+    // 36.2 (32.4), 43.0 (41.7), 43.3 (46.8).  16-bit calls gain more (8192 x 8192 21.3 (28.8), 25.9 (33.0), 24.1 (35.3)), but share the f32 call's bits
+    // and so its kernel.  In a pass: Q8_0 six rows of 4096 x 14336 31.2 (26.4).
     if (!ctx->mmfs_all && (m >= ctx->mmfw_small_min_m || (!bf16 && k >= 10240 && n * k >= (40ull << 20) && mmfw_takes_few(ctx, f.dtype, m)))) {
         const MmfwMatrix one{ w, y, n };
         rc = run_mmfw(ctx, S, f, &one, 1, x, ctx->call_elem, ctx->call_elem, m, k, bf16, stream, 5);
@@ -2572,10 +2577,10 @@ int ffn_on_stream(gllmq_ctx *ctx, const void *gate_w, const void *up_w, size_t g
     // down projection's images are prepared from the two results.
     const size_t gate_up_n[2] = { ffn, ffn };
     // 5 to 8 rows, from 64 M gate and up weights on and whatever the element type (16-bit results are the f32 block's, rounded).
-    // us per call, int8 and GEMM, f32: Q5_K with Q6_K down eight rows 2 x 2048 x 5632 28.8, 35.1, 2 x 3072 x 8192 34.8, 40.3, 2 x 4096 x
-    // 8192 49.7, 43.6, 2 x 4096 x 14336 79, 67; Q6_K seven rows 44.1, 44.0 (3072 x 8192), 53.5, 51.3 (4096 x 8192), 88, 77 (4096 x 14336); Q8_0 45.7,
-    // 48.8, 54.3, 55.9, 95, 75.  16-bit blocks of fewer rows are ahead on the int8 kernels with conversions (Q4_K with Q6_K
-    // down 2 x 4096 x 14336, five bf16 rows 47.5, 61.1; eight 59.9, 61.7).
+    // us per call, int8 and GEMM, f32: Q5_K with Q6_K down eight rows 2 x 2048 x 5632 29.2, 32.5, 2 x 3072 x 8192 36.5, 42.5, 2 x 4096 x
+    // 8192 54.9, 47.8, 2 x 4096 x 14336 80, 65; Q6_K seven rows 49.1, 44.3 (3072 x 8192), 58.1, 51.0 (4096 x 8192), 89, 72 (4096 x 14336); Q8_0 50.5,
+    // 49.1, 60.0, 53.4, 96, 74.  16-bit blocks of fewer rows are ahead on the int8 kernels with conversions (Q4_K with Q6_K
+    // down 2 x 4096 x 14336, five bf16 rows 48.5, 56.2), of eight no more (60.4, 56.5).
     const bool wide = m >= std::max(5u, std::min(ctx->mmfw_min_m, ctx->mmfw_small_min_m)) ||
                       (ctx->ffn_fused && 2 * ffn * hidden >= (64ull << 20) && mmfw_takes_few(ctx, dtype_gate_up, m)); // ("ffn_fused" off: up to 8 rows in separate steps)
     auto fits = [&](MmfwPlan L) { return L.ok && mmfw_fit(ctx, S, L, stream); };
@@ -2871,11 +2876,11 @@ int run_group(gllmq_ctx *ctx, Scratch &S, const gllmq_matmul_desc *descs, size_t
     size_t n_sum = 0;
     for (size_t i = 0; i < len; ++i) n_sum += n[i];
     // The GEMM.  Up to eight rows it takes up to 72 and 48 weight tiles, beyond which its few slices of K leave the int8 kernels ahead: three f32
-    // rows Q4_K 3 x 6144 x 6144 33.1, 27.7, 3 x 8192 x 8192 39.8, 50.0, 2 x 14336 x 4352 26.0, 28.7; five rows 3 x 4096 x 4096 28.8, 20.2, 2 x 8192 x 4096 19.8,
-    // 21.9 (Q6_K 25.1, 27.2), 2 x 28672 x 4096 41.7, 50.0.
+    // rows Q4_K 3 x 6144 x 6144 35.1, 32.7, 3 x 8192 x 8192 42.6, 52.1, 2 x 14336 x 4352 27.7, 35.1; five rows 3 x 4096 x 4096 28.1, 21.8, 2 x 8192 x 4096 19.2,
+    // 23.7 (Q6_K 28.6, 29.0), 2 x 28672 x 4096 42.8, 51.2.
     if (first.m <= 8 && n_sum > (first.m <= 4 ? 72u : 48u) * gq::MMFW_TILE_ROWS) return -1;
-    // Nine to sixteen rows of Q4_K and Q5_K, which have a one-launch kernel alone: up to 128 M weights.  Nine f32 rows 2 x 14336 x 4096 31.3, 27.8 and 34.1, 33.9;
-    // 2 x 14336 x 8192 47.6, 53.0 and 53.7, 62.2; 2 x 28672 x 4096 48.9, 50.3 and 54.0, 57.6.
+    // Nine to sixteen rows of Q4_K and Q5_K, which have a one-launch kernel alone: up to 128 M weights.  Nine f32 rows 2 x 14336 x 4096 33.5, 33.3 and 35.8, 37.3
+    // (sixteen of Q4_K 37.6, 34.4); 2 x 14336 x 8192 47.2, 54.6 and 51.3, 62.1; 2 x 28672 x 4096 46.5, 52.0 and 50.7, 58.1.
     if (first.m >= 9 && first.m <= 16 && (first.ggml_dtype == T_Q4_K || first.ggml_dtype == T_Q5_K) && n_sum * first.k > (128ull << 20)) return -1;
     return run_mmfw(ctx, S, *f, mats, static_cast<int>(len), first.x_dev, elem, elem, first.m, first.k, false, stream, 2);
 }
@@ -3166,10 +3171,10 @@ MoeWidePlan plan_moe_wide(size_t pairs, size_t hidden, size_t ffn, size_t expert
     return W;
 }
 
-// From where the GEMM is ahead of jobs of eight tokens (us, whole call, jobs / GEMM): Q4_K with Q6_K down,
-// 128 experts of 4096 x 1536: 6 pairs per expert 472 / 590, 8: 617 / 602, 16: 884 / 616; 32 experts of
-// 2048 x 1024: 6: 96 / 90, 8: 124 / 96; 8 experts of 4096 x 2048: 8: 99 / 100, 12: 117 / 104.  Q8_0
-// experts, whose other form is the GEMV: 4: 1352 / 731, 129 / 94, 115 / 115.
+// From where the GEMM is ahead of jobs of eight tokens (us, without the router, jobs / GEMM): Q4_K with Q6_K down,
+// 128 experts of 4096 x 1536: 6 pairs per expert 469 / 552, 8: 602 / 556, 16: 881 / 580; 32 experts of
+// 2048 x 1024: 6: 82 / 61, 8: 97 / 63; 8 experts of 4096 x 2048: 8: 78 / 78, 12: 96 / 78.  Q8_0
+// experts, whose other form is the GEMV: 4: 1280 / 673, 112 / 71, 85 / 100.
 bool takes_moe_wide(const gllmq_ctx *ctx, uint32_t dtype_gu, uint32_t dtype_dn, const void *x, size_t hidden, size_t ffn, size_t experts,
                     size_t pairs)
 {
@@ -3181,8 +3186,8 @@ bool takes_moe_wide(const gllmq_ctx *ctx, uint32_t dtype_gu, uint32_t dtype_dn, 
         // int8 kernels do; those take time with every pair.  Estimates in us.  GEMM: a block of K 2.5 (Q6_K, Q8_0: 3.3), 0.6 more
         // with every CU busy, 5 for a workgroup's start and end, 20 for the launches beside the two.  int8: 25, the weights at 5
         // TB/s, the products at 100 TFLOP/s (Q5_K 60, Q8_0 26).  Measured / estimated, 8 experts of 3072 x 512, eight pairs each: Q4_K
-        // GEMM 60 / 67, int8 45 / 36; 8 of 4096 x 2048, sixteen: 104 / 104, 143 / 115; 32 of 2048 x 1024, eight: 78 / 70, 106 / 83; 128 of
-        // 4096 x 1536, eight: 570 / 575, 615 / 726, Q8_0 four: 685 / 651, 1272 / 1281; Q8_0 8 of 3072 x 512, four: 76 / 78, 47 / 45.
+        // GEMM 52 / 67, int8 37 / 36; 8 of 4096 x 2048, sixteen: 79 / 104, 99 / 115; 32 of 2048 x 1024, eight: 63 / 70, 97 / 83; 128 of
+        // 4096 x 1536, eight: 556 / 575, 602 / 726, Q8_0 four: 673 / 651, 1280 / 1281; Q8_0 8 of 3072 x 512, four: 67 / 78, 40 / 45.
         const double e = static_cast<double>(std::min(experts, pairs)), cus = ctx->num_cus;
         auto launch_us = [&](uint32_t dtype, size_t rows, size_t k) {
             const double wgs = std::ceil(rows / 256.0) * e, block = (dtype == T_Q6_K || dtype == T_Q8_0 ? 3.3 : 2.5) + 0.6 * std::min(1.0, wgs / cus);

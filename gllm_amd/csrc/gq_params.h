@@ -510,7 +510,7 @@ struct MmfwShape {
 
 // Few row tiles: a wave's weights come in units, whole rows of one block of K, or of two (Q4_K and Q5_K against one tile of one
 // plane), and a unit is read into registers before the next one is requested into the same place.  What that is for is the
-// CU's requests: 32 rows x 32 bytes a wave-load, as the parts have them, keep its address unit busy 79 % of a launch that streams
+// CU's requests, which take longer the more lines a wave-load touches, 32 rows x 32 bytes as the parts have them
 // (a stream of 28672 x 4096 Q4_K weights alone, eight waves a CU: 17.5 us so, whole rows 14.3, two blocks of a row 13.0).
 // us a launch, parts, units of one block, of two (bits are the same):
 //   Q4_K 16 rows 28672 x 4096, one plane        26.9, 27.1, 25.1     Q5_K 16 rows 13824 x 5120, one plane  21.5, 21.2, 19.8
@@ -520,8 +520,8 @@ struct MmfwShape {
 //   Q6_K 16 rows 4096 x 14336, two planes       26.2, 24.5           Q6_K 64 rows 14336 x 4096, one plane  31.4, 28.5
 //   Q6_K 2048 rows 4096 x 14336, two planes     610, 585             Q6_K 48 rows 14336 x 4096, two planes 35.3, 32.6
 //   Q8_0 64 rows 28672 x 4096, one plane        48.4, 50.6           (its rows' quants are off any alignment in LDS)
-// Q5_K against two planes keeps the parts: in calls one after the other with other work between, 48 rows of 13824 x 5120 33.1 us
-// in parts, 33.6 in units.
+// Q5_K against two planes keeps the parts: calls of 160 drawn shapes of 9 to 130 rows are level (in the mean up to 16 rows parts 0.5 %
+// shorter, above within 0.2 %; single ones 5 % either way).
 constexpr bool mmfw_units(int fmt, int planes, int mt) { return fmt == 2 ? mt <= 2 : fmt == 1 ? planes == 1 && mt == 1 : fmt == 0 && mt <= planes; }
 template <int FMT, int PL, int MT>
 struct MmfwUnitShape {

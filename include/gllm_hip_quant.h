@@ -104,7 +104,7 @@ const char *gllmq_version(void);
  * Development switches (UNSTABLE: they exist so that the test-suite and the measurements can reach
  * every kernel family through the public entry points; names and meaning may change with any
  * version, and a production caller should set none of them):
- *   kernel families on/off: "gemv_f32", "mm8", "mmf", "mm8s", "mm8s_q8_0", "mmfs", "mmfr", "mmfw",
+ *   kernel families on/off: "gemv_f32", "mm8", "mmf", "mm8s", "mm8s_q8_0", "mmfs", "mmfr", "mmfw", "mmfw_own",
  *     "moe_wide", "moe_mm8", "moe_mm8_q6k", "moe_mm8_rows", "moe_glu", "moe_streamed", "lm_head_fused",
  *     "elem_fused", "ffn_glu_load", "ffn_streamed", "mm8s_areg", "mm8s_fold", "mm8s_split",
  *     "mm8_small_to_gemv"
