@@ -174,6 +174,7 @@ struct Scratch {
     void *elem = nullptr;        // 16-bit activations and outputs as f32, for the kernels that do not convert themselves
     size_t elem_bytes = 0;
     void *box = nullptr;         // the chained launch's mailbox [kChainBoxPairs] of 64-bit words, zero when allocated
+    std::vector<void *> in_graph; // the allocations there were when a call that uses scratch was last captured: a graph may hold them
 };
 
 constexpr size_t kScratchArriveBytes = 4096; // MM8_SPLIT_MAX_LISTS words, padded; the chain kernel's counters behind them
@@ -302,6 +303,8 @@ struct gllmq_ctx {
     } overlap;
     std::recursive_mutex call_mutex;
     std::vector<Scratch> scratch;               // one set per stream the context has been used on
+    std::vector<void *> kept;                   // scratch that was given up while a graph may hold it
+    Scratch *call_scratch = nullptr;            // the set of the call being enqueued, until it has been looked at for a capture (call_mutex held)
     uint64_t use_counter = 0;
     std::vector<CachedWeights> weights;         // host-slice calls: uploaded weights by (pointer, length)
     size_t weights_cache_limit = size_t(64) << 30; // bytes kept before the least recently used goes
@@ -425,16 +428,29 @@ void carve_fixed(Scratch &S, void *base)
     S.mm8_part = reinterpret_cast<float *>(b + kScratchArriveBytes + kScratchKeysBytes);
 }
 
-void free_scratch(Scratch &S)
+// Gives an allocation of a scratch set back.  What a graph may hold stays until the context goes: graphs are replayed when their
+// owner likes, and the context does not learn of their end.  That is one set of allocations per capture at most.
+void drop_scratch(gllmq_ctx *ctx, const Scratch &S, void *p)
+{
+    if (!p) return;
+    if (std::find(S.in_graph.begin(), S.in_graph.end(), p) != S.in_graph.end()) ctx->kept.push_back(p);
+    else (void)hipFree(p);
+}
+
+void free_scratch(gllmq_ctx *ctx, Scratch &S)
 {
     if (S.fixed) return;
-    if (S.base) (void)hipFree(S.base);
-    if (S.mmf) (void)hipFree(S.mmf);
-    if (S.ffn) (void)hipFree(S.ffn);
-    if (S.moe) (void)hipFree(S.moe);
-    if (S.elem) (void)hipFree(S.elem);
-    if (S.box) (void)hipFree(S.box);
+    for (void *p : { S.base, S.mmf, S.ffn, S.moe, S.elem, S.box }) drop_scratch(ctx, S, p);
     S = Scratch{};
+}
+
+// A launch of the current call uses its scratch set: where the stream is being captured, a graph will hold it.  Once a call, and only
+// for calls that use scratch (the question takes 50 ns).
+void note_scratch_use(gllmq_ctx *ctx, void *stream)
+{
+    Scratch *S = ctx->call_scratch;
+    ctx->call_scratch = nullptr;
+    if (S && stream_is_capturing(stream)) S->in_graph = { S->base, S->mmf, S->ffn, S->moe, S->elem, S->box };
 }
 
 // The scratch set of `stream` on this context (call_mutex held).  A stream the context has not
@@ -446,7 +462,7 @@ int acquire_scratch(gllmq_ctx *ctx, void *stream, Scratch **out)
     for (Scratch &S : ctx->scratch)
         if (S.stream == static_cast<hipStream_t>(stream)) {
             S.last_use = ctx->use_counter;
-            *out = &S;
+            *out = ctx->call_scratch = &S;
             return GLLMQ_OK;
         }
     if (stream_is_capturing(stream))
@@ -459,7 +475,7 @@ int acquire_scratch(gllmq_ctx *ctx, void *stream, Scratch **out)
         for (size_t i = 1; i < ctx->scratch.size(); ++i)
             if (ctx->scratch[i].last_use < ctx->scratch[lru].last_use) lru = i;
         GLLMQ_HIP(ctx, hipDeviceSynchronize()); // its stream may be gone: wait for everything
-        free_scratch(ctx->scratch[lru]);
+        free_scratch(ctx, ctx->scratch[lru]);
         ctx->scratch.erase(ctx->scratch.begin() + static_cast<long>(lru));
     }
     Scratch S;
@@ -473,16 +489,20 @@ int acquire_scratch(gllmq_ctx *ctx, void *stream, Scratch **out)
     }
     carve_fixed(S, S.base);
     ctx->scratch.push_back(S);
-    *out = &ctx->scratch.back();
+    *out = ctx->call_scratch = &ctx->scratch.back();
     return GLLMQ_OK;
 }
 
-// Makes *buf hold at least `need` bytes.  Growing waits for the stream's earlier work (which may
+// Makes *buf, one of S's, hold at least `need` bytes for the call being enqueued.  Growing waits for the stream's earlier work (which may
 // still use the old buffer; other streams have their own scratch), so it cannot happen while the
 // stream is being captured, and never happens for a set of fixed size.
 int grow_scratch(gllmq_ctx *ctx, const Scratch &S, void **buf, size_t *have, size_t need, void *stream, const char *what)
 {
-    if (*have >= need || ctx->probe) return GLLMQ_OK; // (a dry run of the dispatch allocates nothing)
+    if (ctx->probe) return GLLMQ_OK; // (a dry run of the dispatch allocates nothing)
+    if (*have >= need) {
+        note_scratch_use(ctx, stream);
+        return GLLMQ_OK;
+    }
     if (S.fixed)
         return fail(ctx, GLLMQ_ERR_BAD_SHAPE, "%s needs %zu bytes of scratch, the fixed scratch of this entry point has %zu",
                     what, need, *have);
@@ -493,7 +513,7 @@ int grow_scratch(gllmq_ctx *ctx, const Scratch &S, void **buf, size_t *have, siz
     GLLMQ_HIP(ctx, hipSetDevice(ctx->device));
     if (*buf) {
         GLLMQ_HIP(ctx, hipStreamSynchronize(static_cast<hipStream_t>(stream)));
-        GLLMQ_HIP(ctx, hipFree(*buf));
+        drop_scratch(ctx, S, *buf);
         *buf = nullptr;
         *have = 0;
     }
@@ -517,6 +537,7 @@ int launch2d(gllmq_ctx *ctx, hipFunction_t f, uint32_t grid_x, uint32_t grid_y, 
         ctx->probe_fn = f;
         return GLLMQ_OK;
     }
+    if (uses_scratch) note_scratch_use(ctx, stream);
     void *config[] = { HIP_LAUNCH_PARAM_BUFFER_POINTER, params, HIP_LAUNCH_PARAM_BUFFER_SIZE,
                        &params_size, HIP_LAUNCH_PARAM_END };
     gllmq_ctx::Overlap &ov = ctx->overlap;
@@ -1144,7 +1165,8 @@ size_t mmfw_most_slices(const gllmq_ctx *ctx, size_t m) { return static_cast<siz
 
 // Scratch that any call of up to `m` rows of `k` elements fits, in one pass, and from 33 rows on any call of more rows in passes:
 // what is grown for one call or reserved serves every other one of as many rows, whatever its weight rows, matrices, slices
-// and element type.
+// and element type.  (The one-launch GEMM of 9 to 16 rows has sums of 64 bytes per weight row and 2048 of K: beyond 2^28 weights they
+// may be more than this.)
 size_t mmfw_reserve(const gllmq_ctx *ctx, size_t m, size_t k)
 {
     const size_t groups = (k + 255) / 256, tiles = m <= 32 ? 1 : std::max<size_t>((m + 31) / 32, gq::MMFW_MAX_MT);
@@ -2171,7 +2193,8 @@ int gllmq_init(gllmq_ctx **out, int device)
 void gllmq_destroy(gllmq_ctx *ctx)
 {
     if (!ctx) return;
-    for (Scratch &S : ctx->scratch) free_scratch(S);
+    for (Scratch &S : ctx->scratch) free_scratch(ctx, S);
+    for (void *p : ctx->kept) (void)hipFree(p);
     for (CachedWeights &W : ctx->weights)
         if (W.dev) (void)hipFree(W.dev);
     if (ctx->identity_rows) (void)hipFree(ctx->identity_rows);
@@ -2376,8 +2399,8 @@ int gllmq_argmax(gllmq_ctx *ctx, const float *logits, size_t rows, size_t n, siz
         P.logits = logits + r0 * ld;
         P.token = token + r0;
         P.value = value ? value + r0 : nullptr;
-        int rc = launch2d(ctx, ctx->argmax_part, P.parts, rr, 256, 0, stream, &P, sizeof P);
-        if (rc == GLLMQ_OK && P.parts > 1) rc = launch(ctx, ctx->argmax_final, rr, 256, 0, stream, &P, sizeof P);
+        int rc = launch2d(ctx, ctx->argmax_part, P.parts, rr, 256, 0, stream, &P, sizeof P, P.parts > 1);
+        if (rc == GLLMQ_OK && P.parts > 1) rc = launch(ctx, ctx->argmax_final, rr, 256, 0, stream, &P, sizeof P, true);
         if (rc != GLLMQ_OK) return rc;
     }
     return GLLMQ_OK;
@@ -3543,6 +3566,7 @@ int gq_quantized_matmul_on_block(gllmq_ctx *ctx, const void *w, size_t w_bytes, 
         return fail(ctx, GLLMQ_ERR_INVALID, "quantized_matmul: scratch block missing, misaligned or under %zu bytes", kScratchFixedBytes);
     static_assert(kScratchArriveBytes == GQ_BLOCK_ZEROED_BYTES, "the arrival counters are the zeroed head of the block");
     Scratch S;
+    ctx->call_scratch = nullptr; // (the block is the caller's)
     S.stream = static_cast<hipStream_t>(stream);
     S.fixed = true;
     carve_fixed(S, block);

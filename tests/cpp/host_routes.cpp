@@ -142,19 +142,19 @@ struct Context {
 // addresses of a caller's own buffers, far from each other
 void *at(int i) { return reinterpret_cast<void *>((uintptr_t(1) << 44) + (uintptr_t(i) << 36)); }
 
-int ffn(gllmq_ctx *ctx, uint32_t gate_up, uint32_t down, size_t m, size_t hidden, size_t ffn, int elem = GLLMQ_ELEM_F32)
+int ffn(gllmq_ctx *ctx, uint32_t gate_up, uint32_t down, size_t m, size_t hidden, size_t ffn, int elem = GLLMQ_ELEM_F32, void *stream = nullptr)
 {
     fake::launches.clear();
     return gllmq_ffn_swiglu_elem(ctx, at(1), at(2), ffn * gllmq_row_bytes(gate_up, hidden), gate_up, at(3), hidden * gllmq_row_bytes(down, ffn), down, at(4), at(5),
-                                 m, hidden, ffn, 0, elem, 0, nullptr);
+                                 m, hidden, ffn, 0, elem, 0, stream);
 }
 
-int matmul(gllmq_ctx *ctx, uint32_t dtype, size_t m, size_t n, size_t k, int elem, void *x, void *y, int mode = GLLMQ_ACT_F32_SPLIT)
+int matmul(gllmq_ctx *ctx, uint32_t dtype, size_t m, size_t n, size_t k, int elem, void *x, void *y, int mode = GLLMQ_ACT_F32_SPLIT, void *stream = nullptr)
 {
     fake::launches.clear();
     const size_t bytes = n * gllmq_row_bytes(dtype, k);
-    if (elem != GLLMQ_ELEM_F32) return gllmq_quantized_matmul_elem(ctx, at(1), bytes, x, y, dtype, m, n, k, elem, nullptr);
-    return gllmq_quantized_matmul_ex(ctx, at(1), bytes, static_cast<const float *>(x), static_cast<float *>(y), dtype, m, n, k, mode, nullptr);
+    if (elem != GLLMQ_ELEM_F32) return gllmq_quantized_matmul_elem(ctx, at(1), bytes, x, y, dtype, m, n, k, elem, stream);
+    return gllmq_quantized_matmul_ex(ctx, at(1), bytes, static_cast<const float *>(x), static_cast<float *>(y), dtype, m, n, k, mode, stream);
 }
 
 int batch(gllmq_ctx *ctx, uint32_t dtype, size_t m, const std::vector<size_t> &n, size_t k, int elem)
@@ -311,7 +311,47 @@ void own_images()
                 }
 }
 
+// Scratch that a captured call has used stays, whatever eager calls of more rows, and calls on many other streams, do afterwards;
+// what no graph can hold is given back as it is outgrown, and everything with the context.
+void scratch_of_graphs_stays()
+{
+    const auto elsewhere = [](int i) { return reinterpret_cast<void *>(uintptr_t(i + 1) << 8); };
+    for (int call = 0; call < 5; ++call)
+        for (bool captured : { true, false }) {
+            const size_t before = fake::live.size();
+            {
+                Context ctx;
+                const size_t n = call == 3 ? 1000 : 4096;
+                const auto run = [&](size_t m, void *stream) {
+                    int rc = 0;
+                    if (call == 0) rc = matmul(ctx, T_Q6_K, m, n, 4096, GLLMQ_ELEM_F32, at(4), at(5), GLLMQ_ACT_F32_SPLIT, stream); // GEMM
+                    else if (call == 1) rc = ffn(ctx, T_Q4_K, T_Q6_K, m, 1024, 2816, GLLMQ_ELEM_BF16, stream);
+                    else if (call == 2) rc = ffn(ctx, T_Q4_K, T_Q6_K, std::min<size_t>(m, 16) / 4, 1024, 2816, GLLMQ_ELEM_F32, stream); // (four rows at most)
+                    else if (call == 3) rc = matmul(ctx, T_Q8_0, m == 16 ? 4 : 8, m == 16 ? n : 4 * n, 1024, GLLMQ_ELEM_BF16, at(4), at(5), GLLMQ_ACT_F32_SPLIT, stream); // converted
+                    else rc = gllmq_argmax(ctx, static_cast<const float *>(at(4)), 1, 128256, 128256, static_cast<uint32_t *>(at(5)), nullptr, stream);
+                    EXPECT(rc == GLLMQ_OK, "call %d: %s", call, gllmq_last_error(ctx));
+                };
+                const std::map<void *, size_t> first = fake::live;
+                run(16, elsewhere(0));
+                std::map<void *, size_t> held = fake::live;
+                for (const auto &b : first) held.erase(b.first);
+                EXPECT(!held.empty(), "call %d", call);
+                fake::capturing = captured;
+                run(16, elsewhere(0));
+                fake::capturing = false;
+                for (size_t m : { 64u, 512u, 2048u }) run(m, elsewhere(0));
+                if (call != 2 && call != 4) EXPECT(fake::live.size() == first.size() + held.size() + captured + (call == 1 && captured), "call %d: %zu allocations", call, fake::live.size() - first.size());
+                for (int other = 1; other <= 40; ++other) run(16, elsewhere(other));
+                size_t there = 0;
+                for (const auto &b : held) there += fake::live.count(b.first);
+                EXPECT(captured ? there == held.size() : there == 0, "call %d%s: %zu of %zu buffers are there", call, captured ? ", captured" : "", there, held.size());
+            }
+            EXPECT(fake::live.size() == before, "call %d: %zu allocations left", call, fake::live.size() - before);
+        }
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
+    { "scratch_of_graphs_stays", scratch_of_graphs_stays },
     { "runs_of_weight_tiles", runs_of_weight_tiles },
     { "outputs_over_the_activations", outputs_over_the_activations },
     { "own_images", own_images },

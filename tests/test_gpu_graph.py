@@ -104,3 +104,43 @@ def test_graph_replays_match_eager(hip, torch):
         torch.cuda.synchronize()
         for got, exp in zip(outs, want):
             assert torch.equal(got, exp), f"replay {seed} differs from the eager run"
+
+
+@pytest.mark.parametrize("call", ["matmul", "matmul converted", "ffn", "ffn of few rows"])
+def test_graph_keeps_the_scratch_that_later_calls_outgrow(torch, call):
+    """A graph of a small call replays with the eager bits between eager calls of many rows on its stream, which need more scratch
+    than there was."""
+    from gllm_amd.backend import HipBackend
+    hip, n, k, f = HipBackend(0), 1000, 1024, 1536
+    dev = lambda a: torch.from_numpy(np.asarray(a).view(np.uint8).reshape(-1)).cuda()
+    elem = torch.bfloat16 if "converted" in call else torch.float32
+    small, large = {"matmul": (16, 700), "matmul converted": (4, 8), "ffn": (12, 700), "ffn of few rows": (1, 300)}[call]
+    w, up, down = dev(random_weight(Q6_K, 4 * n, k, seed=1)), dev(random_weight(Q6_K, f, k, seed=2)), dev(random_weight(Q6_K, k, f, seed=3))
+    gate = dev(random_weight(Q6_K, f, k, seed=4))
+
+    def run(x, out):
+        if call.startswith("matmul"):
+            hip.quantized_matmul(w, x, out, Q6_K, x.shape[0], out.shape[1], k)
+        else:
+            hip.ffn_swiglu(gate, up, Q6_K, down, Q6_K, x, out, x.shape[0], k, f)
+
+    width = n if call.startswith("matmul") else k
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        x = torch.from_numpy(random_activations(small, k, seed=5)).cuda().to(elem)
+        want, got = (torch.empty(small, width, device="cuda", dtype=elem) for _ in range(2))
+        many = torch.from_numpy(random_activations(large, k, seed=6)).cuda().to(elem)
+        wide = torch.empty(large, 4 * n if call.startswith("matmul") else k, device="cuda", dtype=elem)
+        run(x, want)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            run(x, got)
+        for i in range(4):
+            print(f"{call}, replay {i}", flush=True)
+            if i:
+                run(many, wide)
+            got.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(got, want)
+    del graph
