@@ -120,6 +120,14 @@ uint32_t mmfw_lds_bytes(int fmt, int planes, uint32_t mt)
     return kTotal[fmt][planes - 1][mt - 1];
 }
 
+// ... with decoded weights (Q6_K, from two tiles on)
+uint32_t mmfx_lds_bytes(int planes, uint32_t mt)
+{
+    static const uint32_t kTotal[2][3] = { { gq::MmfxShape<1, 2>::total, gq::MmfxShape<1, 3>::total, gq::MmfxShape<1, 4>::total },
+                                           { gq::MmfxShape<2, 2>::total, gq::MmfxShape<2, 3>::total, gq::MmfxShape<2, 4>::total } };
+    return kTotal[planes - 1][mt - 2];
+}
+
 // ... where a workgroup makes its images itself: blocks of K that its slice may have, LDS
 uint32_t mmfw_own_blocks(int fmt, int planes)
 {
@@ -236,6 +244,9 @@ struct gllmq_ctx {
     hipFunction_t mmfw[4][4][2] = {};           // the GEMM for more rows [format as above][32-row activation tiles - 1][0 = hi and lo plane, 1 = hi only]
     hipFunction_t moe_mmf[4][2] = {};           // the same over experts' rows [format][plane]
     hipFunction_t mmfw_own[4][2] = {};          // ... of one tile, which prepares the activations itself [format][0 = hi and lo plane, 1 = hi only]
+    hipFunction_t mmfx_decode = nullptr;        // Q6_K weights to matrix-core operands, for prompts
+    hipFunction_t mmfx[gq::MMFW_MAX_MT - 1][2] = {}; // ... and their GEMM [tiles - 2][0 = hi and lo plane, 1 = hi only]
+    uint32_t mmfx_min_m = 1024;                 // "mmfx_min_m": from how many activation rows on (0: never)
     bool use_mmfw_own = true;                   // "mmfw_own" = 0: always a launch that prepares them
     hipFunction_t mmfw_prep[2] = {};            // its activation images [hi and lo plane, hi only]
     bool use_mmfw = true;                       // "mmfw" = 0: 64-row passes of the other forms
@@ -1163,6 +1174,10 @@ bool mmfw_shrink(MmfwPlan &L, size_t limit)
 // rows 0.6 % in the mean by the cost model, 16 MiB 1.3 %, 64 MiB 0.5 %.
 size_t mmfw_most_slices(const gllmq_ctx *ctx, size_t m) { return static_cast<size_t>(ctx->num_cus) * 1024u * (m <= 32 ? 32u : 128u); }
 
+// Decoded weights (mmfx.hip.inc): bytes, and the most that a call has of them at a time; a matrix beyond that goes in slabs of its rows.
+constexpr size_t kMmfxMaxBytes = size_t(128) << 20;
+size_t mmfx_bytes(size_t n, uint32_t groups) { return (n + 31) / 32 * groups * gq::MmfxRecord::bytes; }
+
 // Scratch that any call of up to `m` rows of `k` elements fits, in one pass, and from 33 rows on any call of more rows in passes:
 // what is grown for one call or reserved serves every other one of as many rows, whatever its weight rows, matrices, slices
 // and element type.  (The one-launch GEMM of 9 to 16 rows has sums of 64 bytes per weight row and 2048 of K: beyond 2^28 weights they
@@ -1170,7 +1185,8 @@ size_t mmfw_most_slices(const gllmq_ctx *ctx, size_t m) { return static_cast<siz
 size_t mmfw_reserve(const gllmq_ctx *ctx, size_t m, size_t k)
 {
     const size_t groups = (k + 255) / 256, tiles = m <= 32 ? 1 : std::max<size_t>((m + 31) / 32, gq::MMFW_MAX_MT);
-    return std::min(tiles * groups * gq::MmfwImage<2>::bytes, kMmfwMaxImages) + ((groups * tiles * 128 + 1024 + 255) & ~size_t(255)) + mmfw_most_slices(ctx, m);
+    return std::min(tiles * groups * gq::MmfwImage<2>::bytes, kMmfwMaxImages) + ((groups * tiles * 128 + 1024 + 255) & ~size_t(255)) + mmfw_most_slices(ctx, m) +
+           (ctx->mmfx_min_m && m >= ctx->mmfx_min_m ? kMmfxMaxBytes : 0);
 }
 
 // Additions one after the other, in the mean over the blocks, when `blocks` of them are added up in runs of `run`
@@ -1320,6 +1336,45 @@ bool mmfw_takes_own(const gllmq_ctx *ctx, const MmfwPlan &L, int fmt, size_t m, 
            m * ldx * x_bytes <= 0xFFFFFFFFull;
 }
 
+// How a GEMM over many activation rows of Q6_K decodes its weights first.  mt = 0: it does not.
+struct MmfxPlan {
+    uint32_t mt = 0;
+    size_t slab_rows = 0; // weight rows decoded at a time (several matrices: all of them)
+    size_t bytes = 0;     // of a slab
+};
+
+// From 1024 rows on: decoding costs 0.5 us per million weights, the GEMM then takes a fifth less.  us, decoding and GEMM, and without (f32, 4096 x
+// 14336): 2048 rows 30 + 520, 625; 1024 rows 30 + 262, 313; 14336 x 4096: 1000 rows 30 + 275, 323, 512 rows 30 + 139, 164; one plane, 2048 rows of
+// 4096 x 4096 9 + 108, 142.
+// `room`: bytes of the scratch that are left.  Without room (a capture cannot have more) the weights are multiplied as they are, with the same bits.
+MmfxPlan plan_mmfx(const gllmq_ctx *ctx, const MmfwPlan &L, int fmt, const size_t *n, int count, size_t m, size_t room)
+{
+    MmfxPlan X;
+    if (fmt != 2 || L.ksplit != 1 || !ctx->mmfx_min_m || m < ctx->mmfx_min_m || ctx->mmfw_mt == 1) return X;
+    if (count == 1) {
+        X.slab_rows = std::min(n[0], kMmfxMaxBytes / mmfx_bytes(32, L.groups) * 32 / gq::MMFW_TILE_ROWS * gq::MMFW_TILE_ROWS);
+        X.bytes = mmfx_bytes(X.slab_rows, L.groups);
+    } else {
+        for (int i = 0; i < count; ++i) X.bytes += mmfx_bytes(n[i], L.groups);
+        X.slab_rows = X.bytes <= kMmfxMaxBytes ? L.n_sum : 0;
+    }
+    if (X.slab_rows == 0 || (X.bytes > room && !ctx->probe)) return X;
+    // Tiles by rounds of workgroups; us per block of K as timed (14336 x 4096, 4096 x 14336).  They do not touch the order of the sums.
+    static const double block_us[2][gq::MMFW_MAX_MT - 1] = { { 3.3, 4.4, 6.4 }, { 4.6, 6.3, 8.4 } }; // [one plane, two][tiles - 2]
+    const uint32_t row_tiles = static_cast<uint32_t>((std::min(L.rows, m) + 31) / 32);
+    double best = 1e300;
+    for (uint32_t mt = 2; mt <= static_cast<uint32_t>(gq::MMFW_MAX_MT); ++mt) {
+        if (ctx->mmfw_mt ? mt != ctx->mmfw_mt : (L.run && !gq::mmfw_runs(static_cast<int>(mt)))) continue;
+        const double rounds = std::ceil(static_cast<double>((row_tiles + mt - 1) / mt) * L.n_tiles / ctx->num_cus);
+        const double us = rounds * (L.groups * block_us[L.planes - 1][mt - 2] + 5.6);
+        if (us < best) {
+            best = us;
+            X.mt = mt;
+        }
+    }
+    return X;
+}
+
 // The sums of K slices of a feed-forward block's gate and up rows, left in the scratch for the preparation of the down
 // projection, which adds them up while it applies the gate: a launch less, and the sums' way to memory and back.
 struct MmfwSlices {
@@ -1364,6 +1419,26 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
     bool own = mmfw_takes_own(ctx, L, fmt, m, k, ldx, x_bytes) && !take && !ctx->call_glu && !act_bf16;
     // outputs over the activations: what one workgroup stores another may still have to read
     for (int i = 0; i < count && L.ksplit == 1; ++i) own = own && !ranges_meet(mats[i].y, m * mats[i].n * (elem_y ? 2 : 4), x, m * ldx * x_bytes);
+    const size_t decoded_at = (take ? take->used : 0) + used;
+    const MmfxPlan X = plan_mmfx(ctx, L, fmt, n, count, m, S.mmf_bytes - std::min(S.mmf_bytes, decoded_at));
+    if (X.mt) own = false;
+    uint8_t *decoded = static_cast<uint8_t *>(S.mmf) + decoded_at;
+    const bool slabs = X.mt && count == 1 && X.slab_rows < n[0];
+    const uint32_t mt = X.mt ? X.mt : L.mt;
+    auto decode = [&](int i, size_t row0, size_t rows, size_t at) -> int {
+        const uint32_t row_bytes = static_cast<uint32_t>(gllmq_row_bytes(f.dtype, k));
+        gq::MmfxDecodeParams D{ mats[i].w + row0 * row_bytes, decoded + at, static_cast<uint32_t>(rows), L.groups, row_bytes };
+        return launch2d(ctx, ctx->mmfx_decode, (L.groups + gq::MMFX_DECODE_WAVES - 1) / gq::MMFX_DECODE_WAVES, static_cast<uint32_t>((rows + 31) / 32),
+                        gq::MMFX_DECODE_WAVES * 64, 0, stream, &D, sizeof D, true);
+    };
+    if (X.mt && !slabs) {
+        size_t at = 0;
+        for (int i = 0; i < count && rc == GLLMQ_OK; ++i) {
+            rc = decode(i, 0, n[i], at);
+            at += mmfx_bytes(n[i], L.groups);
+        }
+        if (rc != GLLMQ_OK) return rc;
+    }
     for (size_t m0 = 0; m0 < m; m0 += L.rows) {
         const uint32_t mm = static_cast<uint32_t>(std::min(L.rows, m - m0));
         gq::MmfwPrepParams Q{};
@@ -1403,7 +1478,7 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
         P.k = Q.k;
         P.row_tiles = row_tiles;
         P.inv_ld = Q.inv_ld;
-        P.m_tiles = (row_tiles + L.mt - 1u) / L.mt;
+        P.m_tiles = (row_tiles + mt - 1u) / mt;
         P.n_tiles = L.n_tiles;
         P.ksplit = L.ksplit;
         P.blocks_per_split = L.bps;
@@ -1424,6 +1499,28 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
             G.tile0 = tile0;
             tile0 += (G.n + gq::MMFW_TILE_ROWS - 1u) / gq::MMFW_TILE_ROWS;
             part += static_cast<size_t>(L.ksplit) * mm * G.n;
+        }
+        if (X.mt) {
+            size_t at = 0;
+            for (int i = 0; i < count; ++i) {
+                P.seg[i].w = decoded + at;
+                at += mmfx_bytes(n[i], L.groups);
+            }
+            for (size_t row0 = 0; row0 < L.n_sum; row0 += X.slab_rows) {
+                if (slabs) { // weight tile 0 of the launch is tile row0 / 256 of the matrix
+                    const size_t rows = std::min(X.slab_rows, n[0] - row0);
+                    const uint32_t first = static_cast<uint32_t>(row0 / gq::MMFW_TILE_ROWS);
+                    rc = decode(0, row0, rows, 0);
+                    if (rc != GLLMQ_OK) return rc;
+                    P.seg[0].first_record_row = static_cast<uint32_t>(row0 / 32);
+                    P.seg[0].tile0 = 0u - first;
+                    P.n_tiles = P.n_runs = static_cast<uint32_t>((rows + gq::MMFW_TILE_ROWS - 1) / gq::MMFW_TILE_ROWS);
+                    P.items = P.m_tiles * P.n_runs;
+                }
+                rc = launch(ctx, ctx->mmfx[mt - 2][hi_only ? 1 : 0], (P.items + 7u) / 8u * 8u, gq::MMFW_WAVES * 64, mmfx_lds_bytes(hi_only ? 1 : 2, mt), stream, &P, sizeof P, true);
+                if (rc != GLLMQ_OK) return rc;
+            }
+            continue;
         }
         rc = launch(ctx, own ? ctx->mmfw_own[fmt][hi_only ? 1 : 0] : ctx->mmfw[fmt][L.mt - 1][hi_only ? 1 : 0], (P.items + 7u) / 8u * 8u, gq::MMFW_WAVES * 64,
                     own ? mmfw_own_lds(fmt, hi_only ? 1 : 2) : mmfw_lds_bytes(fmt, hi_only ? 1 : 2, L.mt), stream, &P, sizeof P, true);
@@ -2035,6 +2132,12 @@ int gllmq_init(gllmq_ctx **out, int device)
             snprintf(name, sizeof name, "gq_mmf_%s_w1_own%s", q == 3 ? "q8_0" : q == 2 ? "q6k" : q == 1 ? "q5k" : "q4k", b ? "_hi" : "");
             rc = get_function(ctx, &ctx->mmfw_own[q][b], name);
         }
+    if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfx_decode, "gq_mmfx_decode_q6k");
+    for (int t = 2; t <= gq::MMFW_MAX_MT && rc == GLLMQ_OK; ++t)
+        for (int b = 0; b < 2 && rc == GLLMQ_OK; ++b) {
+            snprintf(name, sizeof name, "gq_mmf_q6k_w%d%s_dec", t, b ? "_hi" : "");
+            rc = get_function(ctx, &ctx->mmfx[t - 2][b], name);
+        }
     for (int q = 0; q < 4 && rc == GLLMQ_OK; ++q)
         for (int b = 0; b < 2 && rc == GLLMQ_OK; ++b) {
             snprintf(name, sizeof name, "gq_moe_mmf_%s%s", q == 3 ? "q8_0" : q == 2 ? "q6k" : q == 1 ? "q5k" : "q4k", b ? "_hi" : "");
@@ -2243,6 +2346,7 @@ int gllmq_set_option(gllmq_ctx *ctx, const char *name, long value)
     else if (n == "mmfw_ksplit") ctx->mmfw_ksplit = u;
     else if (n == "mmfw_run") ctx->mmfw_run = u;
     else if (n == "mmfw_own") ctx->use_mmfw_own = value != 0;
+    else if (n == "mmfx_min_m") ctx->mmfx_min_m = static_cast<uint32_t>(std::max(0L, value));
     else if (n == "mmfr_min_rows") ctx->mmfr_min_rows = std::max(1u, u);
     else if (n == "chain") ctx->use_chain = value != 0;
     else if (n == "chain_dependent") ctx->chain_dependent = value != 0;

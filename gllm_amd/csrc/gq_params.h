@@ -579,6 +579,48 @@ struct MmfwUnitShape {
     }
 };
 
+// Q6_K weights decoded once per call (mmfx.hip.inc).  A record: 32 weight rows x one block of K, [K step 0..15][lane] 16 bytes of
+// f16 operands (q - 32; lane = row + 32 half, elements 16 step + 8 half .. + 7), the rows' sixteen scales each, their d as f32; records lie
+// [32 rows][block].
+struct MmfxRecord {
+    static constexpr uint32_t scales = 16u * 1024u, d = scales + 512u, bytes = d + 128u;
+};
+constexpr int MMFX_DECODE_WAVES = 4; // records of a workgroup that decodes
+struct MmfxDecodeParams {
+    const uint8_t *w; // first row of the slab
+    uint8_t *out;
+    uint32_t n, groups, row_bytes; // rows of the slab
+};
+template <int PL, int MT>
+struct MmfxShape {
+    using W = MmfwShape<2, PL, MT>; // the activations' ring is as it is there
+    static constexpr int UC = W::UC, R = W::R, C = W::C, NA = W::NA, SPC = W::SPC;
+    static constexpr uint32_t CHUNK = W::CHUNK, TILE_CHUNK = W::TILE_CHUNK, EXTRA = W::EXTRA, extra = 0, ring = 4u * EXTRA, total = ring + R * CHUNK;
+    static constexpr int AHEAD = 8;  // K steps that weights are requested ahead
+    static constexpr int SCALES = 4; // unit that requests the next block's scales
+    // ---- the wave's sequence of loads, a block being a period: unit u requests the extra of the block after next (u = 0), scales and d (u =
+    // SCALES) and, behind its first step, a step's weights; then, in the last unit of a chunk, the next chunk is acquired, and NA pieces of
+    // the one R - 1 further on are requested; then the second step's weights.
+    static constexpr int own(int u) { return (u == 0 ? 1 : 0) + (u == SCALES ? 2 : 0) + 1; }
+    static constexpr bool acquires(int u) { return (u + 1) % SPC == 0; }
+    static constexpr int all(int u) { return own(u) + (acquires(u) ? NA : 0) + 1; }
+    static constexpr int ahead_of(int u) // loads ahead of unit u
+    {
+        int blk = 0, n = 0, period = 0;
+        while (u < 0) { u += 8; --blk; }
+        for (int i = 0; i < u; ++i) n += all(i);
+        for (int i = 0; i < 8; ++i) period += all(i);
+        return n + blk * period;
+    }
+    // loads that may be outstanding at unit u's acquisition (a block's extra is older than any chunk that is waited for before it is read)
+    static_assert((R - 1) * SPC <= 15, "extra");
+    static constexpr int chunk_wait(int u)
+    {
+        const int from = u - (R - 1) * SPC, n = ahead_of(u) + own(u) - (ahead_of(from) + own((from % 8 + 8) % 8) + NA);
+        return n < 63 ? n : 63;
+    }
+};
+
 // A workgroup may take several weight tiles against its activation rows one after the other: the requests go on into the next
 // tile, so its first loads, the arguments and the way in are not waited for again.  Prompts of 16-bit elements: 2048 rows of 28672 x
 // 4096 Q4_K, seven rounds of workgroups 532 us, seven tiles a workgroup 502; of 6144 x 4096 141, 133 (three).  Two planes and
@@ -600,6 +642,7 @@ struct MmfwSeg {
     float *y;
     float *partial;    // [ksplit][m][n] when ksplit > 1
     uint32_t n, tile0; // weight rows; index of the matrix's first 256-row tile in the launch
+    uint32_t first_record_row; // decoded weights: rows of 32 ahead of the first that `w` holds
     uint64_t expert_stride; // grouped: bytes between the experts' matrices
 };
 

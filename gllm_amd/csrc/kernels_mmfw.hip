@@ -10,3 +10,4 @@
 #undef GQ_TEMPLATES_ONLY
 
 #include "mmfw.hip.inc"
+#include "mmfx.hip.inc"

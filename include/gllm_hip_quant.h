@@ -109,7 +109,7 @@ const char *gllmq_version(void);
  *     "elem_fused", "ffn_glu_load", "ffn_streamed", "mm8s_areg", "mm8s_fold", "mm8s_split",
  *     "mm8_small_to_gemv"
  *   shape thresholds: "mm8s_min_rows", "mmfs_min_rows", "mmfr_min_rows", "chain_min_rows",
- *     "mmfw_min_m", "mmfw_small_min_m", "moe_wide_min",
+ *     "mmfw_min_m", "mmfw_small_min_m", "mmfx_min_m", "moe_wide_min",
  *     "mm8_q5k_min_m", "mm8_q6k_min_m", "mm8_q8_0_min_m", "mmf_small_min_m", "mm8_ksplit",
  *     "mm8s_all", "mmfs_all" (1: that form wherever the shape fits it, also where another was timed faster)
  *   launch parameters: "mmfw_mt", "mmfw_ksplit", "mmfw_run", "mm8s_depth", "moe_depth", "moe_slices", "prefetch_wgs", "prefetch_threads",

@@ -564,3 +564,66 @@ def test_lines_of_the_launch_over_several_matrices(torch, dtype, m, k, sizes, on
             assert float((a - b).norm() / b.norm()) <= 4e-6 # (the int8 kernels' 1.2e-6, twice, over the GEMM's)
         else:
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("elem", ["float32", "bf16 mode", "float16", "bfloat16"])
+@pytest.mark.parametrize("tiles, runs", [(2, 0), (3, 0), (4, 0), (0, 0), (0, 1)])
+def test_weights_decoded_first(torch, elem, tiles, runs):
+    """Q6_K weights that are decoded ahead of the GEMM: the bits of the GEMM that unpacks them, with one block of K, blocks that K does
+    not fill, long rows added up in runs, weight rows that are no whole tiles or records, several matrices, one that goes in slabs,
+    rows of zeros and non-finite ones."""
+    from gllm_amd.backend import ACT_BF16, ACT_F32_SPLIT, HipBackend
+    mode = ACT_BF16 if elem == "bf16 mode" else ACT_F32_SPLIT
+    t = torch.float32 if elem == "bf16 mode" else getattr(torch, elem)
+    options = {"mmfw_ksplit": 1, "mmfw_mt": tiles, "mmfw_min_m": 9}
+    hips = [HipBackend(0, options={**options, "mmfx_min_m": v}) for v in (33, 0)]
+    shapes = [(129, 257, 14336)] if runs else [(33, 257, 256), (131, 1, 512), (97, 1000, 832), (300, 545, 2304)]
+    if tiles == 0 and not runs:
+        shapes.append((64, 80000, 1024))  # more than 128 MiB of decoded weights
+    for m, n, k in shapes:
+        x = torch.from_numpy(random_activations(m, k, seed=k + m)).cuda()
+        x[0] = 0.0
+        x[1] *= 1e-30
+        x[3, 5], x[m - 1, 0] = float("nan"), float("inf")
+        x = x.to(t)
+        sizes = (n, n // 3 + 1, 40)
+        ws = [torch.from_numpy(random_weight(Q6_K, s, k, seed=s)).cuda() for s in sizes]
+        outs = []
+        for hip in hips:
+            print(f"decoded weights {elem} tiles={tiles} m={m} n={n} k={k}", flush=True)
+            ys = [torch.full((m, s), 7.0, device="cuda", dtype=t) for s in (n,) + sizes]
+            hip.quantized_matmul(ws[0], x, ys[0], Q6_K, m, n, k, mode)
+            assert hip.last_kernel_name().endswith("_dec") == (hip is hips[0]), hip.last_kernel_name()
+            if mode == ACT_F32_SPLIT and n < 80000:
+                hip.quantized_matmul_batch([(w, x, y, Q6_K, m, y.shape[1], k) for w, y in zip(ws, ys[1:])])
+                assert hip.last_kernel_name().endswith("_dec") == (hip is hips[0]), hip.last_kernel_name()
+            torch.cuda.synchronize()
+            outs.append(ys)
+        for a, b in zip(*outs):
+            assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+def test_weights_decoded_first_in_a_graph(torch):
+    """A captured block decodes where the scratch has room for it, also behind calls that outgrow that scratch, and gives the eager
+    bits on every replay."""
+    from gllm_amd.backend import HipBackend
+    hip = HipBackend(0, options={"mmfx_min_m": 64})
+    m, hidden, ffn = 96, 512, 1024
+    weights = [torch.from_numpy(random_weight(Q6_K, n, k, seed=n + i)).cuda() for i, (n, k) in enumerate(((ffn, hidden), (ffn, hidden), (hidden, ffn)))]
+    x = torch.from_numpy(random_activations(m, hidden, seed=5)).cuda()
+    want, got = torch.zeros(m, hidden, device="cuda"), torch.zeros(m, hidden, device="cuda")
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        call = lambda y: hip.ffn_swiglu(weights[0], weights[1], Q6_K, weights[2], Q6_K, x, y, m, hidden, ffn)
+        call(want)
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            call(got)
+        more = torch.zeros(4 * m, hidden, device="cuda")
+        for i in range(4):
+            got.fill_(7.0)
+            graph.replay()
+            hip.ffn_swiglu(weights[0], weights[1], Q6_K, weights[2], Q6_K, more, torch.zeros_like(more), 4 * m, hidden, ffn)
+            stream.synchronize()
+            assert torch.equal(want, got), i
