@@ -367,3 +367,25 @@ def test_plan_of_few_pairs_is_the_plan_of_many(torch, options, dtype):
             assert float((outs[0] - outs[1][:tokens]).norm()) <= 4e-6 * float(outs[0].norm())
         else:
             assert torch.equal(outs[0], outs[1][:tokens])
+
+
+@pytest.mark.parametrize("counts", [(0, 1, 31, 32, 33, 64, 65, 96, 97, 128), (129, 0, 224, 225, 256, 3, 2, 1), (300, 1), (0, 0, 500)])
+def test_jobs_of_every_number_of_tiles(hip, torch, oracle, counts):
+    """Experts' jobs are dealt out by their number of tiles: every expert's tokens are multiplied, whatever the last job holds."""
+    from gllm_amd.backend import HipBackend
+    hip = HipBackend(0, options={"moe_wide_min": 1})  # (the GEMM, whatever it is estimated to take)
+    hidden, ffn, experts = 256, 256, len(counts)
+    gu, dn = expert_weights(Q4_K, Q6_K, experts, hidden, ffn, seed=41)
+    re = np.random.default_rng(5).permutation(np.repeat(np.arange(experts), counts)).astype(np.uint32)[:, None]
+    rw, rl = np.ones(re.shape, np.float32), np.ones(len(re), np.uint32)
+    x = random_activations(len(re), hidden, seed=43)
+    got = run_gpu(hip, torch, gu, Q4_K, dn, Q6_K, x, hidden, ffn, experts, re, rw, rl)
+    for e in range(experts):
+        rows = np.flatnonzero(re[:, 0] == e)
+        if len(rows) == 0:
+            continue
+        g, d = row_bytes(Q4_K, hidden), row_bytes(Q6_K, ffn)
+        both = oracle.quantized_matmul(gu[e * 2 * ffn * g:(e + 1) * 2 * ffn * g], x[rows], Q4_K, len(rows), 2 * ffn, hidden, acc=oracle.ACC_F64, threads=8).astype(np.float64)
+        mid = (both[:, :ffn] / (1 + np.exp(np.minimum(-both[:, :ffn], 700))) * both[:, ffn:]).astype(np.float32)
+        want = oracle.quantized_matmul(dn[e * hidden * d:(e + 1) * hidden * d], mid, Q6_K, len(rows), hidden, ffn, acc=oracle.ACC_F64, threads=8)
+        check_close(got[rows], want, f"expert {e} of {counts}")
