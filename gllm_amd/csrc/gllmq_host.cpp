@@ -249,6 +249,7 @@ struct gllmq_ctx {
     uint32_t mmfx_min_m = 1024;                 // "mmfx_min_m": from how many activation rows on (0: never)
     bool use_mmfw_own = true;                   // "mmfw_own" = 0: always a launch that prepares them
     hipFunction_t mmfw_prep[2] = {};            // its activation images [hi and lo plane, hi only]
+    hipFunction_t mmfw_prep_e16 = nullptr;      // ... from 16-bit elements
     bool use_mmfw = true;                       // "mmfw" = 0: 64-row passes of the other forms
     uint32_t mmfw_min_m = 33;                   // "mmfw_min_m": fewest activation rows that take it
     bool batch_group = true;                    // "batch_group": independent entries over the same rows as one GEMM
@@ -1385,6 +1386,14 @@ struct MmfwSlices {
     size_t used = 0;         // bytes of the scratch in use
 };
 
+// The images of activation rows (mmfw.hip.inc).  16-bit elements have one plane and a launch of their own.
+int launch_mmfw_prep(gllmq_ctx *ctx, gq::MmfwPrepParams &Q, bool hi_only, uint32_t row_tiles, void *stream)
+{
+    const bool e16 = Q.elem != 0 && !Q.glu;
+    return launch2d(ctx, e16 ? ctx->mmfw_prep_e16 : ctx->mmfw_prep[hi_only ? 1 : 0], Q.groups, row_tiles, (e16 ? gq::MMFW_PREP16_WAVES : gq::MMFW_PREP_WAVES) * 64, 0,
+                    stream, &Q, sizeof Q, true);
+}
+
 // The GEMM over `count` matrices of one format and K that share their activations: one launch that
 // prepares the activation images (not where workgroups do: mmfw_takes_own), one that multiplies, and one that adds the slices of K where
 // there are any.  Returns -1 for what it does not take.
@@ -1461,7 +1470,7 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
             Q.slice_ld = static_cast<uint32_t>(m * k);
         }
         const uint32_t row_tiles = (mm + 31u) / 32u;
-        if (!own) rc = launch2d(ctx, ctx->mmfw_prep[hi_only ? 1 : 0], L.groups, row_tiles, gq::MMFW_PREP_WAVES * 64, 0, stream, &Q, sizeof Q, true);
+        if (!own) rc = launch_mmfw_prep(ctx, Q, hi_only, row_tiles, stream);
         if (rc != GLLMQ_OK) return rc;
         gq::MmfwParams P{};
         P.ximg = scratch;
@@ -2121,6 +2130,7 @@ int gllmq_init(gllmq_ctx **out, int device)
         }
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfw_prep[0], "gq_mmfw_prep");
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfw_prep[1], "gq_mmfw_prep_hi");
+    if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfw_prep_e16, "gq_mmfw_prep_e16");
     for (int q = 0; q < 4 && rc == GLLMQ_OK; ++q)
         for (int t = 0; t < gq::MMFW_MAX_MT && rc == GLLMQ_OK; ++t)
             for (int b = 0; b < 2 && rc == GLLMQ_OK; ++b) {
@@ -3368,7 +3378,7 @@ int run_moe_wide(gllmq_ctx *ctx, const Format &fg, const void *gate, size_t gate
         Q.tiles = plan.tiles;
         Q.counters = counters;
         Q.natural = fmt == 2 ? 1u : 0u;
-        int r = launch2d(ctx, ctx->mmfw_prep[hi ? 1 : 0], Q.groups, W.max_tiles, gq::MMFW_PREP_WAVES * 64, 0, stream, &Q, sizeof Q, true);
+        int r = launch_mmfw_prep(ctx, Q, hi, W.max_tiles, stream);
         if (r != GLLMQ_OK) return r;
         gq::MmfwParams P{};
         P.ximg = Q.ximg;

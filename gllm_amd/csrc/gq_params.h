@@ -390,6 +390,7 @@ constexpr int MMFW_MAX_SEGS = 3;                // weight matrices of one launch
 constexpr int MMFW_MAX_MT = 4;
 constexpr bool mmfw_runs(int mt) { return mt <= 3; } // Q6_K, Q8_0: registers for sums of runs (MmfwParams::run_mask)
 constexpr uint32_t MMFW_PREP_WAVES = 16;        // of a workgroup that prepares an image
+constexpr uint32_t MMFW_PREP16_WAVES = 8;       // ... from 16-bit elements, four rows a wave
 
 // Four tiles of Q4_K and Q5_K: no registers for sums of the lo plane's products, which therefore come ahead of the hi
 // plane's (a block's weights are unpacked twice).  In turn with them, where each costs the sum a rounding at its full size,
