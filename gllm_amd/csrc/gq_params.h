@@ -221,6 +221,7 @@ GQ_HD inline uint32_t mm8s_fold_first(uint32_t pair) { return 16u * (pair >> 3) 
 
 // `glu`: the gated kernels keep the sums of a gate tile (pairs x 64 floats) behind the partial sums
 // until the up tile of the same rows is summed.
+constexpr uint32_t MM8S_Q6K_ZEROS = 256u; // Q6_K: zeros ahead of the ring, a block of an operand's unused elements
 GQ_HD inline Mm8sLds mm8s_lds_layout(uint32_t groups, uint32_t m, uint32_t pairs, uint32_t item_bytes, uint32_t slots,
                                      uint32_t subs = 8u, bool glu = false)
 {
@@ -228,7 +229,7 @@ GQ_HD inline Mm8sLds mm8s_lds_layout(uint32_t groups, uint32_t m, uint32_t pairs
     L.prep = mm8_lds_layout(groups, m, pairs, subs, 0u);
     L.ctrl = (L.prep.red + 15u) & ~15u; // the area of mm8.hip.inc's partial sums and stages is not used here
     L.red = L.ctrl + static_cast<uint32_t>(sizeof(Mm8sCtrl));
-    L.ring = (L.red + MM8S_RED_BUFS * MM8S_CWAVES * pairs * 64u * 4u + (glu ? pairs * 64u * 4u : 0u) + 1023u) & ~1023u;
+    L.ring = (L.red + MM8S_RED_BUFS * MM8S_CWAVES * pairs * 64u * 4u + (glu ? pairs * 64u * 4u : 0u) + (subs == 16u ? MM8S_Q6K_ZEROS : 0u) + 1023u) & ~1023u;
     L.total = L.ring + slots * item_bytes;
     return L;
 }
