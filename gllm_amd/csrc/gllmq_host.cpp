@@ -150,13 +150,13 @@ int mm8_kind(uint32_t dtype)
     return dtype == T_Q4_K ? MM8_Q4K : dtype == T_Q6_K ? MM8_Q6K : dtype == T_Q5_K ? MM8_Q5K : dtype == T_Q8_0 ? MM8_Q8_0 : -1;
 }
 
-// Bytes of LDS the int8 matrix-core kernels need: Q6_K keeps 16 sub-block sums per block
-// instead of 8, Q8_0 none, and the weight stage of a wave differs by format.
+// Bytes of LDS the int8 matrix-core kernels need: Q4_K and Q5_K keep 8 sub-block sums per
+// block, Q6_K and Q8_0 none, and the weight stage of a wave differs by format.
 uint32_t mm8_lds_bytes(uint32_t groups, uint32_t m, uint32_t pairs, int kind = MM8_Q4K)
 {
     const uint32_t stage = kind == MM8_Q6K ? gq::MM8Q6_STAGE_BYTES : kind == MM8_Q8_0 ? gq::MM8Q8_STAGE_BYTES
                          : kind == MM8_Q5K ? gq::Mm8Format<1>::STAGE : gq::Mm8Format<0>::STAGE;
-    return gq::mm8_lds_layout(groups, m, pairs, kind == MM8_Q6K ? 16u : kind == MM8_Q8_0 ? 0u : 8u, stage).total;
+    return gq::mm8_lds_layout(groups, m, pairs, kind == MM8_Q6K || kind == MM8_Q8_0 ? 0u : 8u, stage).total;
 }
 
 } // namespace
@@ -716,7 +716,7 @@ int run_mm8s(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
     if (kind == MM8_Q8_0 && (ctx->mm8_q8_0_min_m == 0 || !ctx->mm8s_q8_0 || k % 256 != 0)) return -1;
     const int sfmt = kind == MM8_Q8_0 ? 3 : kind == MM8_Q6K ? 2 : kind == MM8_Q5K ? 1 : 0;
     const uint32_t pieces = sfmt == 3 ? gq::Mm8sFormat<3>::PIECES : sfmt == 2 ? gq::Mm8sFormat<2>::PIECES : sfmt == 1 ? gq::Mm8sFormat<1>::PIECES : gq::Mm8sFormat<0>::PIECES;
-    const uint32_t subs = sfmt == 3 ? 0u : sfmt == 2 ? 16u : 8u;
+    const uint32_t subs = sfmt >= 2 ? 0u : 8u, zeros = sfmt == 2 ? gq::Mm8sFormat<2>::ZEROS : 0u;
     if (!aligned(x, 16) || k % 8 != 0) return -1;
     const uint32_t cus = static_cast<uint32_t>(ctx->num_cus);
     const uint32_t groups = static_cast<uint32_t>((k + 255) / 256), tiles = static_cast<uint32_t>((n + 31) / 32);
@@ -768,7 +768,7 @@ int run_mm8s(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
     if (may_fold && !fold && n < static_cast<size_t>(ctx->mm8s_min_rows) * cus) return -1;
     const uint32_t ipt = fold ? gq::mm8s_fold_pairs(groups) : lds_groups; // items per tile
     const uint32_t item_bytes = (fold ? 2u : 1u) * tile_rows * pieces * 16u; // a row of an item in LDS: its 16-byte pieces side by side
-    const uint32_t fixed = gq::mm8s_lds_layout(lds_groups, mm, pairs, item_bytes, 0, subs, glu).total;
+    const uint32_t fixed = gq::mm8s_lds_layout(lds_groups, mm, pairs, item_bytes, 0, subs, glu, zeros).total;
     const uint32_t items = (glu ? 2u : 1u) * wg_tiles * ipt; // (gated: a gate tile and an up tile per tile of rows)
     uint32_t slots = std::min(items, (160u * 1024u - std::min(fixed, 160u * 1024u)) / item_bytes);
     if (slots < items) slots -= slots % gq::MM8S_LOADERS; // a reused ring is a whole number of rounds of the loaders
@@ -880,7 +880,7 @@ int run_mm8s(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
     P.wg_tiles = wg_tiles;
     P.last_wg_rows = P.n - (grid - 1u) * rows_per_wg;
     P.last_wg_tiles = (P.last_wg_rows + tile_rows - 1u) / tile_rows;
-    const gq::Mm8sLds L = gq::mm8s_lds_layout(lds_groups, mm, pairs, item_bytes, slots, subs, glu);
+    const gq::Mm8sLds L = gq::mm8s_lds_layout(lds_groups, mm, pairs, item_bytes, slots, subs, glu, zeros);
     P.lds_ctrl = L.ctrl;
     P.lds_ring = L.ring;
     P.depth = depth;
@@ -3596,12 +3596,12 @@ int moe_on_stream(gllmq_ctx *ctx, const void *gate, size_t gate_bytes, size_t ga
         if (streamed_jobs && ctx->moe_mm8s_fn[kind][glu ? 1 : 0] && aligned(xin, 16) && max_jobs * Q.g.tiles < 0x7FFFFFFFull) {
             const uint32_t sfmt = kind == MM8_Q6K ? 2u : kind == MM8_Q5K ? 1u : 0u;
             const uint32_t pieces = sfmt == 2 ? gq::Mm8sFormat<2>::PIECES : sfmt == 1 ? gq::Mm8sFormat<1>::PIECES : gq::Mm8sFormat<0>::PIECES;
-            const uint32_t subs = sfmt == 2 ? 16u : 8u, item_bytes = 32u * pieces * 16u, lds_bytes = 160u * 1024u;
+            const uint32_t subs = sfmt == 2 ? 0u : 8u, zeros = sfmt == 2 ? gq::Mm8sFormat<2>::ZEROS : 0u, item_bytes = 32u * pieces * 16u, lds_bytes = 160u * 1024u;
             const uint32_t items = (glu ? 2u : 1u) * Q.g.tiles * groups; // the longest piece: all tiles of a job
             gq::Mm8sLds L2, L4;
             uint32_t slots, depth;
-            if (gq::mm8s_ring(groups, 2, item_bytes, items, subs, glu, lds_bytes, ctx->moe_depth, L2, slots, depth) &&
-                gq::mm8s_ring(groups, 4, item_bytes, items, subs, glu, lds_bytes, ctx->moe_depth, L4, slots, depth)) {
+            if (gq::mm8s_ring(groups, 2, item_bytes, items, subs, glu, zeros, lds_bytes, ctx->moe_depth, L2, slots, depth) &&
+                gq::mm8s_ring(groups, 4, item_bytes, items, subs, glu, zeros, lds_bytes, ctx->moe_depth, L4, slots, depth)) {
                 Q.slices = 1;
                 Q.g.tile_rows = 32;
                 Q.g.lds_ring = lds_bytes; // the kernel carves it up per job

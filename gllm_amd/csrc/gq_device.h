@@ -109,7 +109,7 @@ __device__ __forceinline__ float argmax_key_value(uint64_t key)
 }
 
 // Block fixed point: the powers of two that turn a group of activations whose largest magnitude
-// has the biased exponent `e_raw` (0 .. 254) into integers below 2^BITS and back.
+// has the biased exponent `e_raw` (0 .. 254, with 23 bits also 255) into integers below 2^BITS and back.
 //   |x| < 2^(e-126)   ->   |x * pre * up| < 2^BITS,   down = 1 / (pre * up) = 2^(e - 126 - BITS)
 // With e >= BITS one multiplier does (pre = 1).  Smaller groups (down to subnormal ones, e = 1
 // covers them) need more than 2^127: pre lifts the values first, exactly, and `down` is then a
@@ -121,7 +121,7 @@ struct BlockScale {
 template <int BITS>
 __device__ __forceinline__ BlockScale block_scale(uint32_t e_raw)
 {
-    const uint32_t e = min(max(e_raw, 1u), 254u);
+    const uint32_t e = min(max(e_raw, 1u), BITS == 23 ? 255u : 254u);
     const bool tiny = e < static_cast<uint32_t>(BITS);
     BlockScale s;
     s.pre = tiny ? __builtin_bit_cast(float, (static_cast<uint32_t>(BITS) + 126u - e) << 23) : 1.0f;

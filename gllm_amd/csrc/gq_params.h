@@ -142,10 +142,10 @@ template <> struct Mm8Format<1> { // Q5_K
 // 32-row item, sub-block sums the preparation keeps per block.  In LDS a row of an item is its
 // pieces side by side, PIECES * 16 bytes.
 template <int FMT> struct Mm8sFormat;
-template <> struct Mm8sFormat<0> { static constexpr uint32_t BLOCK = 144, PIECES = 9, SUBS = 8; };   // Q4_K
-template <> struct Mm8sFormat<1> { static constexpr uint32_t BLOCK = 176, PIECES = 11, SUBS = 8; };  // Q5_K
-template <> struct Mm8sFormat<2> { static constexpr uint32_t BLOCK = 210, PIECES = 14, SUBS = 16; }; // Q6_K
-template <> struct Mm8sFormat<3> { static constexpr uint32_t BLOCK = 272, PIECES = 17, SUBS = 0; };   // Q8_0: a group of 8 blocks of 34 bytes (K a multiple of 256)
+template <> struct Mm8sFormat<0> { static constexpr uint32_t BLOCK = 144, PIECES = 9, SUBS = 8, ZEROS = 0; };   // Q4_K
+template <> struct Mm8sFormat<1> { static constexpr uint32_t BLOCK = 176, PIECES = 11, SUBS = 8, ZEROS = 0; };  // Q5_K
+template <> struct Mm8sFormat<2> { static constexpr uint32_t BLOCK = 210, PIECES = 14, SUBS = 0, ZEROS = 256; }; // Q6_K (ZEROS: bytes of zeros ahead of the ring, a block of an operand's unused elements)
+template <> struct Mm8sFormat<3> { static constexpr uint32_t BLOCK = 272, PIECES = 17, SUBS = 0, ZEROS = 0; };   // Q8_0: a group of 8 blocks of 34 bytes (K a multiple of 256)
 GQ_HD constexpr uint32_t mm8s_piece_offset(int fmt, uint32_t piece) { return (fmt == 2 && piece == 13u) ? 194u : 16u * piece; }
 
 // LDS carve-up (bytes) of the int8 matrix-core kernels.
@@ -159,8 +159,8 @@ struct Mm8Lds {
     uint32_t total;
 };
 
-// `subs`: sub-block sums kept per 256-element block (8 of 32 elements for Q4_K, 16 of 16 for
-// Q6_K, none for Q8_0); `stage_bytes`: one wave's weight stage.
+// `subs`: sub-block sums kept per 256-element block (8 of 32 elements for Q4_K and Q5_K, none for
+// Q6_K and Q8_0); `stage_bytes`: one wave's weight stage.
 GQ_HD inline Mm8Lds mm8_lds_layout(uint32_t groups, uint32_t m, uint32_t pairs, uint32_t subs = 8u,
                                    uint32_t stage_bytes = MM8_STAGE_BYTES)
 {
@@ -221,15 +221,14 @@ GQ_HD inline uint32_t mm8s_fold_first(uint32_t pair) { return 16u * (pair >> 3) 
 
 // `glu`: the gated kernels keep the sums of a gate tile (pairs x 64 floats) behind the partial sums
 // until the up tile of the same rows is summed.
-constexpr uint32_t MM8S_Q6K_ZEROS = 256u; // Q6_K: zeros ahead of the ring, a block of an operand's unused elements
 GQ_HD inline Mm8sLds mm8s_lds_layout(uint32_t groups, uint32_t m, uint32_t pairs, uint32_t item_bytes, uint32_t slots,
-                                     uint32_t subs = 8u, bool glu = false)
+                                     uint32_t subs, bool glu, uint32_t zeros)
 {
     Mm8sLds L;
     L.prep = mm8_lds_layout(groups, m, pairs, subs, 0u);
     L.ctrl = (L.prep.red + 15u) & ~15u; // the area of mm8.hip.inc's partial sums and stages is not used here
     L.red = L.ctrl + static_cast<uint32_t>(sizeof(Mm8sCtrl));
-    L.ring = (L.red + MM8S_RED_BUFS * MM8S_CWAVES * pairs * 64u * 4u + (glu ? pairs * 64u * 4u : 0u) + (subs == 16u ? MM8S_Q6K_ZEROS : 0u) + 1023u) & ~1023u;
+    L.ring = (L.red + MM8S_RED_BUFS * MM8S_CWAVES * pairs * 64u * 4u + (glu ? pairs * 64u * 4u : 0u) + zeros + 1023u) & ~1023u;
     L.total = L.ring + slots * item_bytes;
     return L;
 }
@@ -239,11 +238,11 @@ GQ_HD inline Mm8sLds mm8s_lds_layout(uint32_t groups, uint32_t m, uint32_t pairs
 // blocks: one or two rows keep one item per loader unconfirmed, three and four about
 // MM8S_DEPTH_BYTES.  False when the ring would be too short for the loaders to run ahead.
 // `want_depth` != 0: that many items per loader instead (a long stream gains from more of them).
-GQ_HD inline bool mm8s_ring(uint32_t groups, uint32_t m, uint32_t item_bytes, uint32_t items, uint32_t subs, bool glu,
+GQ_HD inline bool mm8s_ring(uint32_t groups, uint32_t m, uint32_t item_bytes, uint32_t items, uint32_t subs, bool glu, uint32_t zeros,
                             uint32_t lds_bytes, uint32_t want_depth, Mm8sLds &L, uint32_t &slots, uint32_t &depth)
 {
     const uint32_t pairs = m <= 2u ? 1u : 2u;
-    L = mm8s_lds_layout(groups, m, pairs, item_bytes, 0u, subs, glu);
+    L = mm8s_lds_layout(groups, m, pairs, item_bytes, 0u, subs, glu, zeros);
     if (L.total + item_bytes > lds_bytes) return false;
     slots = (lds_bytes - L.total) / item_bytes;
     if (slots >= items) slots = items;
