@@ -737,15 +737,26 @@ int run_mm8s(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
     // workgroup cost rows x K of preparation in each (and four rows of 14336 do not fit the LDS);
     // `ksplit` workgroups share a tile and take a slice of at least 16 blocks each.
     uint32_t ksplit = 1;
-    // (Q6_K: two rows; with three and four the fetch-and-compute form stays ahead, 14336 -> 4096 at
-    // three rows 19.8 against 22.5 us)
-    if (S && ctx->mm8s_split_on && !glu && !ctx->call_elem && mm >= 2 && mm <= (kind == MM8_Q6K && !ctx->mm8s_all ? 2u : 4u) &&
+    // (three and four rows of Q6_K: over fewer rows than that, 14336 -> 2048 14.9-15.3 against 17.0-18.5 us for the fetch-and-compute form,
+    // 8192 -> 1024 10.3 against 12.1; 14336 -> 4096 18.9-19.3 against 19.9-20.4)
+    if (S && ctx->mm8s_split_on && !glu && (!ctx->call_elem || kind == MM8_Q6K) && mm >= 2 && mm <= 4 &&
+        (kind != MM8_Q6K || mm == 2 || (tiles * 2u < cus && groups < 64) || ctx->mm8s_all) &&
         groups >= 32 && tiles * 2u <= cus && tiles <= gq::MM8_SPLIT_MAX_LISTS)
         ksplit = std::min(cus / tiles, groups / 16u);
+    // Slices of at least 8 blocks where those of 16 are for fewer than three quarters of the CUs (us, here and in brackets in the fetch-and-compute
+    // form; three rows 9216 -> 2048 Q4_K 10.5 (13.2), Q5_K 10.9 (13.9), Q6_K 11.2 (15.3), Q8_0 11.8 (17.4), 14336 -> 1024 11.6 (13.5), 12.0 (14.1),
+    // 12.3 (15.5), 12.7 (17.2)), below 64 blocks (16384 -> 1024 Q4_K 12.3 (10.7), Q8_0 13.4 (13.1)).  Q4_K and Q5_K: where the other form's slices are
+    // of three passes of 8 blocks and not of two, whose operands it keeps in registers (11008 -> 1280 10.7 (10.3)).  Two rows: from where the
+    // GEMV is not the other form, so that a call of 16-bit elements is of the f32 call's bits.
+    if (ksplit > 1 && groups < 64 && ksplit * tiles * 4u < cus * 3u && (mm > 2 || groups > 38) &&
+        (kind == MM8_Q6K || kind == MM8_Q8_0 || (groups + 7u) / 8u % 2u == 1u))
+        ksplit = std::min(cus / tiles, groups / 8u);
     while (ksplit > 1 && static_cast<size_t>(ksplit) * mm * n > gq::MM8_SPLIT_PART_FLOATS) --ksplit;
     // (slices for fewer than three quarters of the CUs leave too many of them idle: Q8_0 8192 -> 1024
-    // at two rows 10.9 against 9.6 us for the GEMV)
-    if (ksplit > 1 && !ctx->mm8s_all && ksplit * tiles * 4u < cus * 3u) ksplit = 1;
+    // at two rows 10.9 against 9.6 us for the GEMV; Q6_K at three rows 10.3 against 12.1)
+    if (ksplit > 1 && !ctx->mm8s_all && (kind != MM8_Q6K || (mm == 2 && groups <= 38)) && ksplit * tiles * 4u < cus * 3u) ksplit = 1;
+    // slices are of f32 activations: 16-bit ones are widened first (two rows as the kernels below have it)
+    if (ksplit > 1 && ctx->call_elem) return mm == 2 ? -1 : kNeedPlainActivations;
     const bool split = ksplit > 1;
     const uint32_t kslice = (groups + ksplit - 1u) / ksplit, lds_groups = split ? kslice : groups; // blocks a workgroup prepares
     uint32_t rows_per_wg = split ? 32u : static_cast<uint32_t>((n + cus - 1) / cus);
@@ -791,11 +802,7 @@ int run_mm8s(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
     const bool areg = ipt <= 16 && pi <= 1 && ctx->mm8s_areg && !(fold && ctx->call_glu) && !split;
     // Where the other kernels were timed faster (rows of 14336 and of 4096 elements over 4096 to
     // 128256 weight rows): several activation rows of long weight rows, whose preparation every
-    // workgroup repeats in full (Q4_K 2 x 14336 -> 4096: 13.0 against 12.2 us); Q6_K other than
-    // one long row (14336 -> 4096: 14.6 against 16.3 us, 11008 -> 4096: 11.7 against 14.4) or two
-    // short ones (4096 -> 14336: 12.9 against 16.0), the integer-dot GEMV being ahead for one short
-    // row (4096 -> 14336: 11.5 against 12.8 us) and the arithmetic of a Q6_K item costing the same
-    // for a low tile as for a full one.
+    // workgroup repeats in full (Q4_K 2 x 14336 -> 4096: 13.0 against 12.2 us).
     // Five to eight activation rows lead over at most 32 weight rows per CU or rows of at most 8
     // blocks (Q4_K 6 x 4096 -> 6144: 9.9 against 10.2 us, 8 x 2048 -> 14336: 10.6 against 12.0; 6 x
     // 4096 -> 14336: 15.0 against 14.3, 6 x 4096 -> 28672: 24.7 against 21.6), Q6_K over at most 32
@@ -803,7 +810,7 @@ int run_mm8s(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
     const bool few_rows = n <= static_cast<size_t>(32) * cus;
     if (!ctx->mm8s_all) {
         if (pi == 2 && !(few_rows || (groups <= 8 && kind != MM8_Q6K))) return -1;
-        if (mm >= 2 && groups > 16 && !split) return -1;
+        if (mm >= 2 && groups > 16 && !split && !(kind == MM8_Q6K && pi < 2)) return -1;
         // Tiles of fewer than 16 weight rows block by block, the matrix cores mostly idle, lose to
         // the K split of the other form for long rows (Q4_K 8192 -> 2048: 7.6 against 8.6 us) and
         // to the integer-dot GEMV for one row of Q5_K (4096 -> 2048: 4.8-5.2 against 5.6).  In
@@ -811,18 +818,22 @@ int run_mm8s(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
         // 14336 -> 2048 Q4_K 7.1 against 9.9; Q5_K 4096 -> 2048 4.5 against 4.7).
         if (!fold && kind != MM8_Q6K && groups > 16 && rows_per_wg < 16) return -1;
         if (!fold && kind == MM8_Q5K && mm == 1 && n < static_cast<size_t>(12) * cus) return -1;
-        // Q6_K: one row of 40 blocks and more, in pairs of blocks from 20 (5120 -> 4096: 6.4 against 8.1 us, 6144 -> 4096: 7.3 against
-        // 8.7 us for the GEMV, 8192 -> 4096: 9.1 against 10.2; 4096 -> 4096: 6.3 against 6.0), or two short rows
-        // three rows of K <= 4096 (4096 -> 14336: 14.7 against 16.6 us), four over at most 32 weight rows per
-        // CU or rows of at most 8 blocks (4096 -> 6144: 8.7 against 10.4; 4096 -> 14336: 17.4 against 16.7)
-        if (kind == MM8_Q6K && !((mm == 1 && (groups >= 40 || (fold && groups >= 20))) || ((mm == 2 || mm == 3) && areg) ||
-                                 (mm == 4 && areg && (few_rows || groups <= 8)) || pi == 2 || split))
-            return -1;
+        // Q6_K: two to four rows everywhere (us, here and in brackets in the other forms: two rows 5120 -> 4096 7.5 (11.7), -> 28672 25 (38), 14336 ->
+        // 6144 20 (26); three 5120 -> 6144 10.7 (13.5), four 4096 -> 14336 14.0 (17.0)).  One row: in pairs of blocks from 20 blocks on; from 40 on at
+        // all heights; of 17 to 39 blocks over more than 24 weight rows per CU (5120 -> 8192 9.3 (12.2), 4864 -> 32000 25 (35)), rows of 8192, where the
+        // GEMV's waves have all lanes at work, to 56 (14336 20.3 (21.8), 128256 153 (145)); up to 15 blocks (3072 -> 1024 5.0 (5.4-6.2), -> 8192 6.4
+        // (7.6), 2048 -> 14336 7.7 (8.4)), the shortest to 16 weight rows per CU and block (2048 -> 32000 12.2 (13.0), 128256 42 (40); 1024 -> 14336
+        // 5.9 (6.5), 28672 8.9 (8.7)).
+        if (kind == MM8_Q6K && mm == 1 && groups < 40 && !(fold && groups >= 20)) {
+            const size_t rows = (n + cus - 1) / cus;
+            if (groups >= 16 ? (groups == 16 || rows <= 24 || (groups == 32 && rows > 56)) : (groups <= 8 && rows > 16u * groups)) return -1;
+        }
         // Q8_0, two rows over at most 8 weight rows per CU: its GEMV stays ahead (4096 -> 1024: 5.9 against 7.1 us)
         if (kind == MM8_Q8_0 && mm == 2 && n <= static_cast<size_t>(8) * cus) return -1;
         // one short row over at most 4 weight rows per CU: the integer-dot GEMV stays ahead
         // (4096 -> 1024: Q4_K 4.6 against 5.0 us, Q5_K 4.9 against 5.0; 8192 -> 1024 Q4_K: 6.3 against 5.9 here)
-        if (mm == 1 && rows_per_wg <= 4 && groups <= 16) return -1;
+        // (Q6_K leads here, 3072 -> 1024: 4.9-5.1 against 5.4-6.2)
+        if (mm == 1 && rows_per_wg <= 4 && groups <= 16 && kind != MM8_Q6K) return -1;
     }
     const uint32_t steps = (((groups + 7u) / 8u + 1u) / 2u) * mm; // preparation steps per wave
     int variant;

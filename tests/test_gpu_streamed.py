@@ -222,3 +222,27 @@ def test_more_open_requests_per_loader_change_no_bit(hip, torch, dtype):
             got = gpu_matmul(deep, torch, w, x, dtype, m, n, k)
             assert deep.last_kernel_name() == name
             assert np.array_equal(got.view(np.uint32), base.view(np.uint32)), (dtype, m, n, k, depth)
+
+
+@pytest.mark.parametrize("dtype,m,rows,k,form", [
+    (Q6_K, 1, 5, 3072, "_f"), (Q6_K, 1, 16, 1024, "_a"), (Q6_K, 1, 65, 1024, "gemv"), (Q6_K, 1, 25, 4864 + 8, "_e2"), (Q6_K, 1, 24, 4864, "gemv"),
+    (Q6_K, 1, 57, 8192, "gemv"), (Q6_K, 2, 5, 5120 - 8, "_e4"), (Q6_K, 3, 25, 5120, "_e4"), (Q6_K, 4, 57, 4096, "_a"), (Q6_K, 2, 5, 8192, "_e4"),
+    (Q6_K, 3, 15, 14336, "_s"), (Q6_K, 4, 4, 9216 + 136, "_s"), (Q6_K, 2, 4, 14336, "_s"), (Q6_K, 3, 4, 16384, "mm8_"),
+    (Q4_K, 3, 8, 9216, "_s"), (Q4_K, 2, 5, 14336 - 8, "_s"), (Q5_K, 4, 4, 14336, "_s"), (8, 3, 8, 9216, "_s"), (8, 4, 8, 11008, "_s")])
+def test_default_choice_at_its_lines(torch, dtype, m, rows, k, form):
+    """Q6_K at one to four rows and the finer slices of K: the default choice just inside and outside its lines, a ragged last workgroup, against
+    the kernels that ran there before (which the other tests hold to the oracle), and a call of 16-bit elements as the rounded f32 result."""
+    from gllm_amd.backend import HipBackend
+    n = rows * cus(torch) - (3 if m != 1 and rows > 4 else 0)
+    default, plain = HipBackend(0), HipBackend(0, options={"mm8s": 0})
+    w, x = random_weight(dtype, n, k, seed=n + m), random_activations(m, k, seed=k)
+    xb = torch.from_numpy(x).to(torch.bfloat16)
+    x = xb.float().numpy()
+    y = gpu_matmul(default, torch, w, x, dtype, m, n, k)
+    name = default.last_kernel_name()
+    print(f"line dtype={dtype} m={m} n={n} k={k}: {name}", flush=True)
+    assert form in name and name.startswith("gq_mm8s_") == (form[0] == "_"), name
+    check_close(y, gpu_matmul(plain, torch, w, x, dtype, m, n, k), name)
+    out = torch.zeros(m, n, device="cuda", dtype=torch.bfloat16)
+    default.quantized_matmul(torch.from_numpy(w).cuda(), xb.cuda(), out, dtype, m, n, k)
+    assert torch.equal(out.cpu().view(torch.int16), torch.from_numpy(y).to(torch.bfloat16).view(torch.int16))
