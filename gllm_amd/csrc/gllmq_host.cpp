@@ -273,7 +273,7 @@ struct gllmq_ctx {
     hipFunction_t mmf_prep_lanes = nullptr;     // the images of the streamed form
     hipFunction_t mmf_prep[2] = {};             // its activation preparation [32-row activation tiles - 1]
     hipFunction_t mmf_reduce = nullptr;         // and the in-order sum of its K-split partial results
-    hipFunction_t moe_plan = nullptr, moe_plan_few = nullptr, moe_act = nullptr, moe_combine = nullptr, moe_route = nullptr;
+    hipFunction_t moe_plan = nullptr, moe_plan_wide = nullptr, moe_plan_few = nullptr, moe_act = nullptr, moe_combine = nullptr, moe_combine_v4 = nullptr, moe_route = nullptr;
     hipFunction_t moe_gemv[kNumFormats] = {};
     hipFunction_t moe_mm8_fn[MM8_KINDS][2] = {}; // grouped int8 matrix-core kernels [Mm8Kind][passes per tile - 1]
     hipFunction_t moe_mm8_q6k_rows = nullptr;   // Q6_K rows of at most 8 blocks: a wave per 32-row tile
@@ -2169,9 +2169,11 @@ int gllmq_init(gllmq_ctx **out, int device)
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfr[1][0], "gq_mmfr_q5k");
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfr[1][1], "gq_mmfr_q5k_e16");
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->moe_plan, "gq_moe_plan");
+    if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->moe_plan_wide, "gq_moe_plan_wide");
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->moe_plan_few, "gq_moe_plan_few");
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->moe_act, "gq_moe_act");
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->moe_combine, "gq_moe_combine");
+    if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->moe_combine_v4, "gq_moe_combine_v4");
     for (int i = 0; i < kNumFormats && rc == GLLMQ_OK; ++i) {
         snprintf(name, sizeof name, "gq_moe_gemv_%s", kFormats[i].tag);
         rc = get_function(ctx, &ctx->moe_gemv[i], name);
@@ -3266,6 +3268,15 @@ MoeWorkspace moe_workspace(size_t pairs, size_t hidden, size_t ffn)
     return W;
 }
 
+// The weighted sum of each token's routes.
+int launch_moe_combine(gllmq_ctx *ctx, MoeCombineParams C, void *stream)
+{
+    // Four columns a thread from 128 tokens on (512 tokens 15.0 us, 13.0; with 64 there are too few threads for it, 4.2, 4.3).  o is on a
+    // boundary of 256 bytes and hidden a multiple of 4 (moe_matvec refuses others), so o's rows are on one of 16.
+    const uint32_t per = C.tokens >= 128u ? 4u : 1u;
+    return launch2d(ctx, per == 4u ? ctx->moe_combine_v4 : ctx->moe_combine, (C.hidden + 256u * per - 1u) / (256u * per), C.tokens, 256, 0, stream, &C, sizeof C);
+}
+
 // Sorts the routed pairs by expert and writes the job tables that `P` points to.
 int launch_moe_plan(gllmq_ctx *ctx, MoePlanParams &P, const uint32_t *route_expert, const uint32_t *route_len, size_t tokens,
                     size_t top_k, size_t experts, void *stream)
@@ -3274,20 +3285,23 @@ int launch_moe_plan(gllmq_ctx *ctx, MoePlanParams &P, const uint32_t *route_expe
     P.route_len = route_len;
     P.tokens = static_cast<uint32_t>(tokens);
     P.top_k = static_cast<uint32_t>(top_k);
+    P.top_k_inverse = 0xFFFFFFFFu / P.top_k;
     P.experts = static_cast<uint32_t>(experts);
     P.pairs = static_cast<uint32_t>(tokens * top_k);
     if (P.pairs <= gq::MOE_PLAN_FEW) { // (from 256 pairs on the two take the same time)
         const uint32_t padded = (P.pairs + 63u) & ~63u;
         const uint32_t threads = std::max(padded, std::min(gq::MOE_PLAN_FEW_THREADS, (P.experts + 63u) & ~63u));
+        P.experts_per_thread = (P.experts + threads - 1u) / threads;
         return launch(ctx, ctx->moe_plan_few, 1, threads, (2u * P.experts + 2u * padded + 16u) * 4u, stream, &P, sizeof P);
     }
     // a wave per 64 pairs up to 16, as far as their counts (a word per expert each) fit the LDS; no
     // fewer than four, which share the rest of the work
     uint32_t waves = std::min<uint32_t>(gq::MOE_PLAN_THREADS / 64, std::max(4u, (P.pairs + 63u) / 64u));
     while (waves > 4u && (waves + 4u) * P.experts * 4u > 128u * 1024u) waves /= 2u;
-    const uint64_t words = static_cast<uint64_t>(waves + 4u) * P.experts + 16u, with_pairs = words + 2ull * P.pairs;
+    const uint64_t words = static_cast<uint64_t>(waves + 4u) * P.experts + 64u, with_pairs = words + 2ull * P.pairs;
     P.in_lds = with_pairs * 4u <= 128u * 1024u ? 1u : 0u;
-    return launch(ctx, ctx->moe_plan, 1, waves * 64u, static_cast<uint32_t>(P.in_lds ? with_pairs : words) * 4u, stream, &P, sizeof P);
+    P.experts_per_thread = (P.experts + waves * 64u - 1u) / (waves * 64u);
+    return launch(ctx, P.tiles ? ctx->moe_plan_wide : ctx->moe_plan, 1, waves * 64u, static_cast<uint32_t>(P.in_lds ? with_pairs : words) * 4u, stream, &P, sizeof P);
 }
 
 // ---- Many tokens per expert (prompts): the GEMM of mmfw.hip.inc over the experts' own rows
@@ -3373,7 +3387,8 @@ int run_moe_wide(gllmq_ctx *ctx, const Format &fg, const void *gate, size_t gate
     plan.wide = reinterpret_cast<gq::MoeWideJob *>(ws + W.jobs);
     plan.token = token;
     plan.counters = counters;
-    plan.job_rows = 32u * gq::MMFW_MAX_MT;
+    static_assert(32u * gq::MMFW_MAX_MT == 1u << 7, "rows of a job");
+    plan.job_shift = 7u;
     rc = launch_moe_plan(ctx, plan, route_expert, route_len, tokens, top_k, experts, stream);
     if (rc != GLLMQ_OK) return rc;
 
@@ -3444,7 +3459,7 @@ int run_moe_wide(gllmq_ctx *ctx, const Format &fg, const void *gate, size_t gate
     }
     MoeCombineParams C{ o, route_weight, route_len, plan.pair_pos, out, static_cast<uint32_t>(tokens), static_cast<uint32_t>(top_k),
                         static_cast<uint32_t>(hidden), elem };
-    return launch2d(ctx, ctx->moe_combine, static_cast<uint32_t>((hidden + 255) / 256), static_cast<uint32_t>(tokens), 256, 0, stream, &C, sizeof C);
+    return launch_moe_combine(ctx, C, stream);
 }
 
 // The expert matvec (call_mutex held).  x and out are of type `elem`; where the kernels of the shape take
@@ -3529,7 +3544,7 @@ int moe_on_stream(gllmq_ctx *ctx, const void *gate, size_t gate_bytes, size_t ga
         P.jobs = jobs;
         P.jobs8 = jobs8;
         P.counters = counters;
-        P.job_rows = 1u << job_shift;
+        P.job_shift = job_shift;
         rc = launch_moe_plan(ctx, P, route_expert, route_len, tokens, top_k, experts, stream);
         if (rc != GLLMQ_OK) return rc;
     }
@@ -3664,7 +3679,7 @@ int moe_on_stream(gllmq_ctx *ctx, const void *gate, size_t gate_bytes, size_t ga
     if (rc != GLLMQ_OK) return rc;
     MoeCombineParams C{ o, route_weight, route_len, pair_pos, out, static_cast<uint32_t>(tokens),
                         static_cast<uint32_t>(top_k), H, 0 };
-    return launch2d(ctx, ctx->moe_combine, (H + 255u) / 256u, static_cast<uint32_t>(tokens), 256, 0, stream, &C, sizeof C);
+    return launch_moe_combine(ctx, C, stream);
 }
 
 } // namespace

@@ -796,7 +796,9 @@ struct MoePlanParams {
     uint32_t *token;    // [pairs] token of each sorted position
     uint32_t *counters; // [0] jobs, [1] routed pairs, [2] matrix-core (or GEMM) jobs, [3] tiles of 32
     uint32_t tokens, top_k, experts, pairs;
-    uint32_t job_rows;  // a matrix-core job takes up to that many tokens of an expert
+    uint32_t top_k_inverse; // 2^32 / top_k, rounded down
+    uint32_t experts_per_thread; // rounded up
+    uint32_t job_shift; // a matrix-core job takes up to 1 << job_shift tokens of an expert
     uint32_t in_lds;    // the pairs' experts and the sorted order fit the LDS
 };
 

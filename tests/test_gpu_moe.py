@@ -389,3 +389,32 @@ def test_jobs_of_every_number_of_tiles(hip, torch, oracle, counts):
         mid = (both[:, :ffn] / (1 + np.exp(np.minimum(-both[:, :ffn], 700))) * both[:, ffn:]).astype(np.float32)
         want = oracle.quantized_matmul(dn[e * hidden * d:(e + 1) * hidden * d], mid, Q6_K, len(rows), hidden, ffn, acc=oracle.ACC_F64, threads=8)
         check_close(got[rows], want, f"expert {e} of {counts}")
+
+
+@pytest.mark.parametrize("hidden, top_k", [(256, 3), (260, 9), (1028, 8), (512, 2)])
+def test_combine_of_many_tokens_is_the_combine_of_few(torch, hidden, top_k):
+    """From 128 tokens on a thread adds up four columns.  The same tokens with others behind them that are
+    routed nowhere: the same bits, wherever the output lies; zeros for tokens without a route."""
+    from gllm_amd.backend import HipBackend
+    hip, ffn, experts, few, many = HipBackend(0, options={"moe_streamed": 0, "moe_wide": 0}), 256, 12, 100, 131
+    rng = np.random.default_rng(9)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    gate_up = dev(random_weight(Q4_K, experts * 2 * ffn, hidden, seed=1).view(np.uint8).reshape(-1))
+    down = dev(random_weight(Q4_K, experts * hidden, ffn, seed=2).view(np.uint8).reshape(-1))
+    x = dev(random_activations(many, hidden, seed=3) * 1e-3)
+    expert = np.stack([rng.permutation(experts)[:top_k] for _ in range(many)]).astype(np.int32)
+    expert[rng.random(expert.shape) < 0.1] = experts + 5  # (routes nowhere)
+    length = rng.integers(0, top_k + 1, many).astype(np.int32)
+    length[few:] = 0
+    weight = rng.uniform(0.1, 1.0, (many, top_k)).astype(np.float32)
+    for dtype, shifts in ((torch.float32, (0, 1, 2)), (torch.bfloat16, (0, 1, 2, 4))):
+        outs = []
+        for count, shift in [(few, 0)] + [(many, s) for s in shifts]:
+            flat = torch.full((count * hidden + 8,), float("nan"), device="cuda", dtype=dtype)
+            out = flat[shift:shift + count * hidden].view(count, hidden)
+            hip.moe_matvec(gate_up, Q4_K, down, Q4_K, x[:count].to(dtype), out, hidden, ffn, experts, dev(expert[:count]), dev(weight[:count]), dev(length[:count]))
+            assert bool(flat[:shift].isnan().all()) and bool(flat[shift + count * hidden:].isnan().all())
+            outs.append(out)
+        assert bool(outs[0].any())
+        for got in outs[1:]:
+            assert torch.equal(got[:few], outs[0]) and not bool(got[few:].any())
