@@ -15,6 +15,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+from types import SimpleNamespace
 
 import numpy as np
 
@@ -147,6 +148,23 @@ def load_library() -> C.CDLL:
     return L
 
 
+_step_calls = None
+
+
+def step_calls() -> dict:
+    """The entry points of a model's step as functions of plain numbers (``csrc/py_calls.cpp``): a call of a few microseconds
+    is bound by its way to the library, of which ctypes takes 0.9."""
+    global _step_calls
+    if _step_calls is None:
+        lib = load_library()
+        try:
+            from . import _calls
+        except ImportError as e:
+            raise HipError(f"gllm_amd/_calls.so cannot be loaded ({e}): build it with `python -m gllm_amd.build`") from e
+        _step_calls = {name: _calls.bind(name, C.cast(getattr(lib, name), C.c_void_p).value) for name in _calls.names}
+    return _step_calls
+
+
 EXPORTED_SYMBOLS = [
     "gllmq_init", "gllmq_destroy", "gllmq_last_error", "gllmq_status_string", "gllmq_version",
     "gllmq_block_size", "gllmq_block_bytes", "gllmq_row_bytes", "gllmq_dequantize",
@@ -192,6 +210,7 @@ class HipBackend:
         """``options``: kernel-family choices by name (``gllmq_set_option``), used by the tests to
         reach the kernels the default dispatch does not pick."""
         self._lib = load_library()
+        self._calls = SimpleNamespace(**{name.removeprefix("gllmq_"): fn for name, fn in step_calls().items()})
         import torch
         if not torch.cuda.is_available():
             raise HipError("no HIP device is visible; this backend has no CPU path")
@@ -210,6 +229,7 @@ class HipBackend:
         if rc != OK:
             raise HipError(f"gllmq_init(device={device}): {self._lib.gllmq_status_string(rc).decode()}")
         self._ctx = ctx
+        self._address = ctx.value
         for name, value in (options or {}).items():
             self.set_option(name, value)
 
@@ -249,7 +269,7 @@ class HipBackend:
     def close(self) -> None:
         if getattr(self, "_ctx", None):
             self._lib.gllmq_destroy(self._ctx)
-            self._ctx = None
+            self._ctx = self._address = None
 
     def __del__(self):
         try:
@@ -294,11 +314,11 @@ class HipBackend:
             if elem != ELEM_F32:
                 if act_mode != ACT_F32_SPLIT:
                     raise Unimplemented("quantized_matmul: the bf16 activation mode is for f32 tensors")
-                rc = self._lib.gllmq_quantized_matmul_elem(self._ctx, w.data_ptr(), w.nbytes, x.data_ptr(), y.data_ptr(), dt, m, n, k,
-                                                           elem, self._raw_stream(self.device))
+                rc = self._calls.quantized_matmul_elem(self._address, w.data_ptr(), w.nbytes, x.data_ptr(), y.data_ptr(), dt, m, n, k,
+                                                       elem, self._raw_stream(self.device))
             else:
-                rc = self._lib.gllmq_quantized_matmul_ex(self._ctx, w.data_ptr(), w.nbytes, x.data_ptr(), y.data_ptr(), dt, m, n, k,
-                                                         act_mode, self._raw_stream(self.device))
+                rc = self._calls.quantized_matmul_ex(self._address, w.data_ptr(), w.nbytes, x.data_ptr(), y.data_ptr(), dt, m, n, k,
+                                                     act_mode, self._raw_stream(self.device))
         else:
             w = _host_bytes(weight_blocks)
             x = np.ascontiguousarray(input, np.float32).reshape(-1)
@@ -337,8 +357,8 @@ class HipBackend:
             b, o = block_data, output
             if not (b.is_cuda and o.is_cuda and o.dtype == self._torch.float32):
                 raise OtherError("dequantize: tensors must live on the GPU, output f32")
-            rc = self._lib.gllmq_dequantize(self._ctx, b.data_ptr(), b.nbytes,
-                                            o.data_ptr(), o.numel(), dt, self._stream())
+            rc = self._calls.dequantize(self._address, b.data_ptr(), b.nbytes,
+                                        o.data_ptr(), o.numel(), dt, self._stream())
         else:
             b = _host_bytes(block_data)
             if not (isinstance(output, np.ndarray) and output.dtype == np.float32 and output.flags.c_contiguous):
@@ -371,8 +391,7 @@ class HipBackend:
         count = len(arr) - start if count is None else count
         if start < 0 or count < 0 or start + count > len(arr):
             raise OtherError("run_batch: range outside the descriptor array")
-        first = C.cast(C.byref(arr, start * C.sizeof(MatmulDesc)), C.POINTER(MatmulDesc))
-        rc = self._lib.gllmq_quantized_matmul_batch(self._ctx, first, count, self._stream())
+        rc = self._calls.quantized_matmul_batch(self._address, C.addressof(arr) + start * C.sizeof(MatmulDesc), count, self._stream())
         if rc != OK:
             self._raise(rc, "quantized_matmul_batch")
 
@@ -402,13 +421,13 @@ class HipBackend:
         if output.numel() < count * hidden_dim:
             raise OtherError("quant_gather: output shorter than len(ids) * hidden_dim")
         if elem == ELEM_F32:
-            rc = self._lib.gllmq_quant_gather(self._ctx, table.data_ptr(), table.nbytes, dt,
-                                              vocab_size, hidden_dim, token_ids.data_ptr(), count,
-                                              1.0 if scale is None else float(scale), output.data_ptr(), self._stream())
+            rc = self._calls.quant_gather(self._address, table.data_ptr(), table.nbytes, dt,
+                                          vocab_size, hidden_dim, token_ids.data_ptr(), count,
+                                          1.0 if scale is None else float(scale), output.data_ptr(), self._stream())
         else:
-            rc = self._lib.gllmq_quant_gather_elem(self._ctx, table.data_ptr(), table.nbytes, dt,
-                                                   vocab_size, hidden_dim, token_ids.data_ptr(), count,
-                                                   1.0 if scale is None else float(scale), output.data_ptr(), elem, self._stream())
+            rc = self._calls.quant_gather_elem(self._address, table.data_ptr(), table.nbytes, dt,
+                                               vocab_size, hidden_dim, token_ids.data_ptr(), count,
+                                               1.0 if scale is None else float(scale), output.data_ptr(), elem, self._stream())
         if rc != OK:
             self._raise(rc, "quant_gather")
 
@@ -429,15 +448,15 @@ class HipBackend:
             raise OtherError("ffn_swiglu: x/out shorter than m * hidden")
         gb, ub = gate.nbytes, up.nbytes
         if elem == ELEM_F32 and not accumulate:
-            rc = self._lib.gllmq_ffn_swiglu(self._ctx, gate.data_ptr(), up.data_ptr(), min(gb, ub), _dtype_id(dtype_gate_up),
-                                            down.data_ptr(), down.nbytes, _dtype_id(dtype_down),
-                                            x.data_ptr(), out.data_ptr(), m, hidden, ffn, 1 if relu_gate else 0,
-                                            self._stream())
+            rc = self._calls.ffn_swiglu(self._address, gate.data_ptr(), up.data_ptr(), min(gb, ub), _dtype_id(dtype_gate_up),
+                                        down.data_ptr(), down.nbytes, _dtype_id(dtype_down),
+                                        x.data_ptr(), out.data_ptr(), m, hidden, ffn, 1 if relu_gate else 0,
+                                        self._stream())
         else:
-            rc = self._lib.gllmq_ffn_swiglu_elem(self._ctx, gate.data_ptr(), up.data_ptr(), min(gb, ub), _dtype_id(dtype_gate_up),
-                                                 down.data_ptr(), down.nbytes, _dtype_id(dtype_down),
-                                                 x.data_ptr(), out.data_ptr(), m, hidden, ffn, 1 if relu_gate else 0,
-                                                 elem, OUT_ACCUMULATE if accumulate else 0, self._stream())
+            rc = self._calls.ffn_swiglu_elem(self._address, gate.data_ptr(), up.data_ptr(), min(gb, ub), _dtype_id(dtype_gate_up),
+                                             down.data_ptr(), down.nbytes, _dtype_id(dtype_down),
+                                             x.data_ptr(), out.data_ptr(), m, hidden, ffn, 1 if relu_gate else 0,
+                                             elem, OUT_ACCUMULATE if accumulate else 0, self._stream())
         if rc != OK:
             self._raise(rc, "ffn_swiglu")
 
@@ -454,8 +473,8 @@ class HipBackend:
         ld = lg.stride(0) if rows > 1 else max(n, 1)
         if token.numel() < rows or (value is not None and value.numel() < rows):
             raise OtherError("argmax: token/value shorter than the number of rows")
-        rc = self._lib.gllmq_argmax(self._ctx, lg.data_ptr(), rows, n, ld, token.data_ptr(),
-                                    value.data_ptr() if value is not None else None, self._stream())
+        rc = self._calls.argmax(self._address, lg.data_ptr(), rows, n, ld, token.data_ptr(),
+                                value.data_ptr() if value is not None else None, self._stream())
         if rc != OK:
             self._raise(rc, "argmax")
 
@@ -474,10 +493,10 @@ class HipBackend:
             raise OtherError("lm_head_argmax: logits must be a contiguous device f32 tensor of n entries")
         if value is not None and not (value.is_cuda and value.dtype == self._torch.float32 and value.numel() >= 1):
             raise OtherError("lm_head_argmax: value must be a device f32 tensor")
-        rc = self._lib.gllmq_lm_head_argmax(self._ctx, w.data_ptr(), w.nbytes, x.data_ptr(),
-                                            _dtype_id(quant_type), n, k, logits.data_ptr() if logits is not None else None,
-                                            token.data_ptr(), value.data_ptr() if value is not None else None,
-                                            self._stream())
+        rc = self._calls.lm_head_argmax(self._address, w.data_ptr(), w.nbytes, x.data_ptr(),
+                                        _dtype_id(quant_type), n, k, logits.data_ptr() if logits is not None else None,
+                                        token.data_ptr(), value.data_ptr() if value is not None else None,
+                                        self._stream())
         if rc != OK:
             self._raise(rc, "lm_head_argmax")
 
@@ -493,9 +512,9 @@ class HipBackend:
         if route_expert.numel() < tokens * top_k or route_weight.numel() < tokens * top_k or route_len.numel() < tokens:
             raise OtherError("moe_route: outputs shorter than tokens * top_k / tokens")
         opt = [t.data_ptr() if t is not None else None for t in (route_pos, expert_counts, overflow)]
-        rc = self._lib.gllmq_moe_route(self._ctx, logits.data_ptr(), tokens, experts, top_k, float(capacity_factor),
-                                       route_expert.data_ptr(), route_weight.data_ptr(), route_len.data_ptr(),
-                                       opt[0], opt[1], opt[2], self._stream())
+        rc = self._calls.moe_route(self._address, logits.data_ptr(), tokens, experts, top_k, float(capacity_factor),
+                                   route_expert.data_ptr(), route_weight.data_ptr(), route_len.data_ptr(),
+                                   opt[0], opt[1], opt[2], self._stream())
         if rc != OK:
             self._raise(rc, "moe_route")
 
@@ -520,14 +539,14 @@ class HipBackend:
         else:
             gate_ptr, gate_b, gate_st = gate_up.data_ptr(), gbytes, each
             up_ptr, up_b, up_st = up.data_ptr(), up.nbytes, each
-        args = (self._ctx, gate_ptr, gate_b, gate_st, up_ptr, up_b, up_st, dgu,
+        args = (self._address, gate_ptr, gate_b, gate_st, up_ptr, up_b, up_st, dgu,
                 down.data_ptr(), down.nbytes, hidden * row_bytes(ddn, ffn) if supported(ddn) else 0, ddn,
                 x.data_ptr(), out.data_ptr(), tokens, hidden, ffn, experts, top_k, route_expert.data_ptr(),
                 route_weight.data_ptr(), route_len.data_ptr(), int(relu_gate))
         if elem == ELEM_F32 and not accumulate:
-            rc = self._lib.gllmq_moe_matvec(*args, self._stream())
+            rc = self._calls.moe_matvec(*args, self._stream())
         else:
-            rc = self._lib.gllmq_moe_matvec_elem(*args, elem, OUT_ACCUMULATE if accumulate else 0, self._stream())
+            rc = self._calls.moe_matvec_elem(*args, elem, OUT_ACCUMULATE if accumulate else 0, self._stream())
         if rc != OK:
             self._raise(rc, "moe_matvec")
 

@@ -2,18 +2,20 @@
 
     python -m gllm_amd.build
 
-Three steps, all plain compiler invocations (no cmake, no JIT cache):
+Three steps and one beside them, all plain compiler invocations (no cmake, no JIT cache):
   1. hipcc --genco --offload-arch=gfx950   csrc/kernels_*.hip -> csrc/build/kernels_*.hsaco, side by side
   2. hipcc -c --offload-arch=gfx950        csrc/gllmq_noalloc.hip -> csrc/build/gllmq_noalloc.o (host code plus the
                                            device array behind the entry point that allocates nothing)
   3. hipcc (host only)                     csrc/gllmq_host.cpp, csrc/gguf_reader.cpp + the object of step 2 + the code
                                            objects of step 1 embedded with .incbin -> gllm_amd/libgllm_hip_quant.so
+and g++ for csrc/py_calls.cpp, the way from Python to the library's entry points -> gllm_amd/_calls.so
 """
 from __future__ import annotations
 
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -22,6 +24,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(CSRC, "build")
 KERNEL_UNITS = ["codec", "mm8", "mm8s", "mm8s_q8_0", "mm8c", "mm8_q6k_q8_0", "mmf", "mmfs", "mmfw", "moe"]  # csrc/kernels_<unit>.hip, one code object each
 LIB = os.path.join(HERE, "libgllm_hip_quant.so")
+CALLS = os.path.join(HERE, "_calls.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 
@@ -71,9 +74,17 @@ def build_host() -> str:
     return LIB
 
 
+def build_calls() -> str:
+    """The Python functions of a step's entry points (they are bound to the loaded library's addresses: nothing is linked)."""
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wextra", "-I", sysconfig.get_paths()["include"],
+          "-I", os.path.join(ROOT, "include"), os.path.join(CSRC, "py_calls.cpp"), "-o", CALLS])
+    return CALLS
+
+
 def build() -> str:
     build_kernels()
     build_noalloc()
+    build_calls()
     return build_host()
 
 
@@ -107,6 +118,7 @@ if __name__ == "__main__":
         build_kernels(sorted(set(sys.argv[1:]) | set(stale_units())))
         if not os.path.exists(NOALLOC_OBJ):
             build_noalloc()
+        build_calls()
         build_host()
     else:
         build()
