@@ -168,3 +168,17 @@ def test_route_without_drops_and_without_places(hip, torch, oracle):
         assert np.array_equal(rw.cpu().numpy().view(np.uint32), np.ascontiguousarray(full["weight"]).view(np.uint32))
         assert (rl.cpu().numpy() == min(top_k, experts)).all()
         check_against_oracle(oracle, full, logits, top_k, float(experts), f"{tokens} {experts} {top_k}")
+
+
+@pytest.mark.parametrize("experts", [1, 2, 63, 64, 65, 127, 128, 129, 511, 512, 513])
+def test_edges_of_the_registers_with_ties(hip, torch, oracle, experts):
+    """Choices from two, eight or no registers a lane: equal logits within a lane, in two lanes, in all of them."""
+    rng = np.random.default_rng(experts)
+    logits = rng.standard_normal((7, experts)).astype(np.float32)
+    logits[1] = 0.5
+    logits[2] = np.round(logits[2])
+    logits[3, ::64] = 9.0
+    logits[4, -3:] = 9.0
+    logits[5] = np.where(rng.random(experts) < 0.7, -np.inf, logits[5])
+    for top_k in sorted({1, min(8, experts), min(64, experts)}):
+        check_against_oracle(oracle, route(hip, torch, logits, top_k, capacity_factor=float(experts)), logits, top_k, float(experts), f"{experts} experts, top {top_k}")
