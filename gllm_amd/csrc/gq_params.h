@@ -598,6 +598,7 @@ struct MmfxShape {
     static constexpr int UC = W::UC, R = W::R, C = W::C, NA = W::NA, SPC = W::SPC;
     static constexpr uint32_t CHUNK = W::CHUNK, TILE_CHUNK = W::TILE_CHUNK, EXTRA = W::EXTRA, extra = 0, ring = 4u * EXTRA, total = ring + R * CHUNK;
     static constexpr int AHEAD = 8;  // K steps that weights are requested ahead
+    static constexpr int BEHIND = 1; // of those ahead of the loop, steps requested behind the last chunk, as a unit has it
     static constexpr int SCALES = 4; // unit that requests the next block's scales
     // ---- the wave's sequence of loads, a block being a period: unit u requests the extra of the block after next (u = 0), scales and d (u =
     // SCALES) and, behind its first step, a step's weights; then, in the last unit of a chunk, the next chunk is acquired, and NA pieces of
@@ -620,7 +621,31 @@ struct MmfxShape {
         const int from = u - (R - 1) * SPC, n = ahead_of(u) + own(u) - (ahead_of(from) + own((from % 8 + 8) % 8) + NA);
         return n < 63 ? n : 63;
     }
+    // Every load of a wave in its order, the ones ahead of the loop and three blocks': is there any acquisition whose chunk could still be
+    // on its way by its wait alone?  (The compiler's waits for weights, which it puts ahead of a step's products, are tighter today; nothing
+    // promises that.)
+    static constexpr bool waits_cover()
+    {
+        int issued = 0, behind[3 * 8 / SPC + R] = {}; // behind[q]: loads up to the last piece of chunk q
+        issued += 2 + 2 + AHEAD - BEHIND; // scales and d, extras, weights
+        for (int q = 0; q < R - 1; ++q) behind[q] = issued += NA;
+        const int landed = issued;
+        behind[R - 1] = issued += NA;
+        issued += BEHIND;
+        for (int u = 0; u < 3 * 8; ++u) {
+            issued += own(u % 8);
+            if (acquires(u % 8)) {
+                const int q = (u + 1) / SPC;
+                if (behind[q] > landed && issued - behind[q] < chunk_wait(u % 8)) return false;
+                behind[q + R - 1] = issued += NA;
+            }
+            ++issued;
+        }
+        return true;
+    }
 };
+static_assert(MmfxShape<1, 2>::waits_cover() && MmfxShape<1, 3>::waits_cover() && MmfxShape<1, 4>::waits_cover() && MmfxShape<2, 2>::waits_cover() &&
+              MmfxShape<2, 3>::waits_cover() && MmfxShape<2, 4>::waits_cover(), "a chunk is read before it is sure to have arrived");
 
 // A workgroup may take several weight tiles against its activation rows one after the other: the requests go on into the next
 // tile, so its first loads, the arguments and the way in are not waited for again.  Prompts of 16-bit elements: 2048 rows of 28672 x
