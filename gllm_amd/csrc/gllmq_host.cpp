@@ -739,7 +739,7 @@ int run_mm8s(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
     uint32_t ksplit = 1;
     // (three and four rows of Q6_K: over fewer rows than that, 14336 -> 2048 14.9-15.3 against 17.0-18.5 us for the fetch-and-compute form,
     // 8192 -> 1024 10.3 against 12.1; 14336 -> 4096 18.9-19.3 against 19.9-20.4)
-    if (S && ctx->mm8s_split_on && !glu && (!ctx->call_elem || kind == MM8_Q6K) && mm >= 2 && mm <= 4 &&
+    if (S && ctx->mm8s_split_on && !glu && mm >= 2 && mm <= 4 &&
         (kind != MM8_Q6K || mm == 2 || (tiles * 2u < cus && groups < 64) || ctx->mm8s_all) &&
         groups >= 32 && tiles * 2u <= cus && tiles <= gq::MM8_SPLIT_MAX_LISTS)
         ksplit = std::min(cus / tiles, groups / 16u);
@@ -747,7 +747,7 @@ int run_mm8s(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
     // form; three rows 9216 -> 2048 Q4_K 10.5 (13.2), Q5_K 10.9 (13.9), Q6_K 11.2 (15.3), Q8_0 11.8 (17.4), 14336 -> 1024 11.6 (13.5), 12.0 (14.1),
     // 12.3 (15.5), 12.7 (17.2)), below 64 blocks (16384 -> 1024 Q4_K 12.3 (10.7), Q8_0 13.4 (13.1)).  Q4_K and Q5_K: where the other form's slices are
     // of three passes of 8 blocks and not of two, whose operands it keeps in registers (11008 -> 1280 10.7 (10.3)).  Two rows: from where the
-    // GEMV is not the other form, so that a call of 16-bit elements is of the f32 call's bits.
+    // GEMV, which reads 16-bit elements itself, is not the other form.
     if (ksplit > 1 && groups < 64 && ksplit * tiles * 4u < cus * 3u && (mm > 2 || groups > 38) &&
         (kind == MM8_Q6K || kind == MM8_Q8_0 || (groups + 7u) / 8u % 2u == 1u))
         ksplit = std::min(cus / tiles, groups / 8u);
@@ -755,8 +755,8 @@ int run_mm8s(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
     // (slices for fewer than three quarters of the CUs leave too many of them idle: Q8_0 8192 -> 1024
     // at two rows 10.9 against 9.6 us for the GEMV; Q6_K at three rows 10.3 against 12.1)
     if (ksplit > 1 && !ctx->mm8s_all && (kind != MM8_Q6K || (mm == 2 && groups <= 38)) && ksplit * tiles * 4u < cus * 3u) ksplit = 1;
-    // slices are of f32 activations: 16-bit ones are widened first (two rows as the kernels below have it)
-    if (ksplit > 1 && ctx->call_elem) return mm == 2 ? -1 : kNeedPlainActivations;
+    // slices are of f32 activations: 16-bit ones are widened first, so that their call is of the f32 call's bits
+    if (ksplit > 1 && ctx->call_elem) return kNeedPlainActivations;
     const bool split = ksplit > 1;
     const uint32_t kslice = (groups + ksplit - 1u) / ksplit, lds_groups = split ? kslice : groups; // blocks a workgroup prepares
     uint32_t rows_per_wg = split ? 32u : static_cast<uint32_t>((n + cus - 1) / cus);

@@ -311,6 +311,32 @@ void own_images()
                 }
 }
 
+// A call of 16-bit elements is the f32 call on the widened activations, rounded, bit for bit: up to eight rows it multiplies with the f32 call's
+// kernel over as many workgroups, in the form that reads such elements or between launches that convert.
+void elements_take_the_f32_kernels()
+{
+    Context ctx;
+    const auto multiplies = [&](uint32_t dtype, size_t m, size_t n, size_t k, int elem) {
+        EXPECT(matmul(ctx, dtype, m, n, k, elem, at(4), at(5)) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+        std::string all;
+        for (const fake::Launch &l : fake::launches) {
+            std::string name = l.kernel;
+            if (name.find("prep") != std::string::npos || name == "gq_convert_elem") continue; // (images are of the same bits wherever they are made)
+            for (const char *form : { "_e16", "_hi", "_own" })
+                if (const size_t p = name.find(form); p != std::string::npos) name.erase(p, std::strlen(form));
+            all += name + " " + std::to_string(l.grid) + " ";
+        }
+        return all;
+    };
+    for (const auto &f : kFormats)
+        for (size_t m = 1; m <= 8; ++m)
+            for (size_t n : { 1u, 777u, 1024u, 1280u, 2048u, 3073u, 3500u, 4096u, 5120u, 8192u, 14336u, 128256u })
+                for (size_t k : { 256u, 1024u, 2880u, 4096u, 4864u, 5120u, 7936u, 8192u, 9216u, 9728u, 9984u, 11008u, 14336u, 16384u }) {
+                    const std::string f32 = multiplies(f.dtype, m, n, k, GLLMQ_ELEM_F32), bf16 = multiplies(f.dtype, m, n, k, GLLMQ_ELEM_BF16);
+                    EXPECT(f32 == bf16, "dtype %u, %zu rows, %zu x %zu: %s, not %s", f.dtype, m, n, k, bf16.c_str(), f32.c_str());
+                }
+}
+
 // Scratch that a captured call has used stays, whatever eager calls of more rows, and calls on many other streams, do afterwards;
 // what no graph can hold is given back as it is outgrown, and everything with the context.
 void scratch_of_graphs_stays()
@@ -352,6 +378,7 @@ void scratch_of_graphs_stays()
 
 const std::map<std::string, std::function<void()>> kChecks = {
     { "scratch_of_graphs_stays", scratch_of_graphs_stays },
+    { "elements_take_the_f32_kernels", elements_take_the_f32_kernels },
     { "runs_of_weight_tiles", runs_of_weight_tiles },
     { "outputs_over_the_activations", outputs_over_the_activations },
     { "own_images", own_images },
