@@ -2,8 +2,11 @@
 refuse what it refuses."""
 import ctypes as C
 import random
+import warnings
 
+import numpy as np
 import pytest
+import torch
 
 from gllm_amd import _calls
 from gllm_amd.backend import load_library, step_calls
@@ -60,3 +63,48 @@ def test_bound_to_the_loaded_library():
         lib.gllmq_quantized_matmul_ex(None, None, 0, None, None, 12, 1, 1, 256, 0, None) != 0
     with pytest.raises(KeyError):
         _calls.bind("gllmq_nothing", 1)
+
+
+class Index:
+    def __index__(self):
+        return 2 ** 33 + 6
+
+
+class Parameter:
+    _as_parameter_ = 9
+
+
+def through(fn, args, seen):
+    """What arrives, or that it is refused."""
+    seen.clear()
+    try:
+        with warnings.catch_warnings():
+            warnings.simplefilter("ignore")
+            rc = fn(*args)
+    except Exception as e:
+        assert not seen
+        return type(e)
+    return rc, seen[0]
+
+
+@pytest.mark.parametrize("name", _calls.names)
+def test_whatever_ctypes_takes_or_refuses(name):
+    """Integers of numpy's, torch scalars, ctypes objects, anything that says what it is as an index or a parameter, and what is none of
+    those: accepted with the same value as through ctypes, or refused with the same exception."""
+    argtypes = [C.c_void_p if isinstance(t, type) and issubclass(t, C._Pointer) else t for t in getattr(load_library(), name).argtypes]
+    fn, address, seen = receiver(argtypes, 3)
+    call, plain = _calls.bind(name, address), C.CFUNCTYPE(C.c_int, *argtypes)(address)
+    good = [1.0 if t is C.c_float else 1 for t in argtypes]
+    values = [np.int64(5), np.uint32(7), np.int8(-1), np.bool_(True), np.float32(2.5), np.array(3), np.zeros(2, np.int64), torch.tensor(3), torch.tensor(3.5),
+              torch.tensor([1, 2]), C.c_size_t(2 ** 40), C.c_uint32(4), C.c_int(-4), C.c_float(4.5), C.c_void_p(2 ** 40), C.c_void_p(None), Index(), Parameter(),
+              2 ** 70, -1, None, True, 1.5, 3, "a", [], object()]
+    accepted = 0
+    for i, t in enumerate(argtypes):
+        for v in values:
+            if isinstance(v, str) and t is C.c_void_p:
+                continue  # (a pointer to a copy of the text, which differs from call to call)
+            args = good[:i] + [v] + good[i + 1:]
+            got, want = through(call, args, seen), through(plain, args, seen)
+            assert got == want, (i, t, v)
+            accepted += isinstance(got, tuple)
+    assert accepted > 6 * len(argtypes)
