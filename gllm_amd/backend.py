@@ -151,17 +151,24 @@ def load_library() -> C.CDLL:
 _step_calls = None
 
 
+_STEP_CALLS = ["gllmq_quantized_matmul_ex", "gllmq_quantized_matmul_elem", "gllmq_quantized_matmul_batch", "gllmq_dequantize", "gllmq_quant_gather",
+               "gllmq_quant_gather_elem", "gllmq_ffn_swiglu", "gllmq_ffn_swiglu_elem", "gllmq_argmax", "gllmq_lm_head_argmax", "gllmq_moe_route",
+               "gllmq_moe_matvec", "gllmq_moe_matvec_elem"]
+
+
 def step_calls() -> dict:
     """The entry points of a model's step as functions of plain numbers (``csrc/py_calls.cpp``): a call of a few microseconds
-    is bound by its way to the library, of which ctypes takes 0.9."""
+    is bound by its way to the library, of which ctypes takes 0.9.  The same functions through ctypes where that module was not built."""
     global _step_calls
     if _step_calls is None:
         lib = load_library()
+        address = {name: C.cast(getattr(lib, name), C.c_void_p).value for name in _STEP_CALLS}
         try:
             from . import _calls
-        except ImportError as e:
-            raise HipError(f"gllm_amd/_calls.so cannot be loaded ({e}): build it with `python -m gllm_amd.build`") from e
-        _step_calls = {name: _calls.bind(name, C.cast(getattr(lib, name), C.c_void_p).value) for name in _calls.names}
+            _step_calls = {name: _calls.bind(name, at) for name, at in address.items()}
+        except ImportError:
+            plain = lambda t: C.c_void_p if issubclass(t, C._Pointer) else t
+            _step_calls = {name: C.CFUNCTYPE(C.c_int, *map(plain, getattr(lib, name).argtypes))(at) for name, at in address.items()}
     return _step_calls
 
 

@@ -8,7 +8,8 @@ Three steps and one beside them, all plain compiler invocations (no cmake, no JI
                                            device array behind the entry point that allocates nothing)
   3. hipcc (host only)                     csrc/gllmq_host.cpp, csrc/gguf_reader.cpp + the object of step 2 + the code
                                            objects of step 1 embedded with .incbin -> gllm_amd/libgllm_hip_quant.so
-and g++ for csrc/py_calls.cpp, the way from Python to the library's entry points -> gllm_amd/_calls.so
+and behind them csrc/py_calls.cpp, a shorter way from Python to the library's entry points -> gllm_amd/_calls.abi3.so (where there is no
+Python.h it is left out: the library does not need it, and the Python package then goes through ctypes).
 """
 from __future__ import annotations
 
@@ -24,7 +25,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(CSRC, "build")
 KERNEL_UNITS = ["codec", "mm8", "mm8s", "mm8s_q8_0", "mm8c", "mm8_q6k_q8_0", "mmf", "mmfs", "mmfw", "moe"]  # csrc/kernels_<unit>.hip, one code object each
 LIB = os.path.join(HERE, "libgllm_hip_quant.so")
-CALLS = os.path.join(HERE, "_calls.so")
+CALLS = os.path.join(HERE, "_calls.abi3.so")  # Python's limited interface: not one interpreter version's
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 
@@ -74,18 +75,23 @@ def build_host() -> str:
     return LIB
 
 
-def build_calls() -> str:
+def build_calls() -> str | None:
     """The Python functions of a step's entry points (they are bound to the loaded library's addresses: nothing is linked)."""
-    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wextra", "-I", sysconfig.get_paths()["include"],
-          "-I", os.path.join(ROOT, "include"), os.path.join(CSRC, "py_calls.cpp"), "-o", CALLS])
+    include = sysconfig.get_paths()["include"]
+    if not os.path.exists(os.path.join(include, "Python.h")):
+        print(f"no {include}/Python.h: {os.path.basename(CALLS)} is not built, Python calls go through ctypes", flush=True)
+        return None
+    _run([HIPCC, "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wextra", "-I", include, "-I", os.path.join(ROOT, "include"),
+          os.path.join(CSRC, "py_calls.cpp"), "-o", CALLS])
     return CALLS
 
 
 def build() -> str:
     build_kernels()
     build_noalloc()
+    lib = build_host()
     build_calls()
-    return build_host()
+    return lib
 
 
 def stale_units() -> list[str]:
@@ -118,8 +124,8 @@ if __name__ == "__main__":
         build_kernels(sorted(set(sys.argv[1:]) | set(stale_units())))
         if not os.path.exists(NOALLOC_OBJ):
             build_noalloc()
-        build_calls()
         build_host()
+        build_calls()
     else:
         build()
     print(LIB)

@@ -6,7 +6,9 @@
 // prototypes.  The interpreter's lock is released around the call.
 //
 // The functions are bound to addresses in the library that is already loaded (bind(name, address)); this module links nothing of it.
+// It keeps to Python's limited interface, so that interpreters from 3.10 on load one build of it.
 #define PY_SSIZE_T_CLEAN
+#define Py_LIMITED_API 0x030A0000
 #include <Python.h>
 
 #include <cstdint>

@@ -108,3 +108,18 @@ def test_whatever_ctypes_takes_or_refuses(name):
             assert got == want, (i, t, v)
             accepted += isinstance(got, tuple)
     assert accepted > 6 * len(argtypes)
+
+
+def test_without_the_module(monkeypatch):
+    """The backend's calls are there, with the same results, where the module was not built."""
+    import sys
+    from gllm_amd import backend
+    want = backend.step_calls()["gllmq_moe_route"](None, None, 1, 1, 1, 1.0, None, None, None, None, None, None, None)
+    monkeypatch.setattr(backend, "_step_calls", None)
+    monkeypatch.setitem(sys.modules, "gllm_amd._calls", None)
+    monkeypatch.delattr("gllm_amd._calls")
+    calls = backend.step_calls()
+    assert set(calls) == set(_calls.names) and not any(type(fn) is type(_calls.bind) for fn in calls.values())
+    assert calls["gllmq_moe_route"](None, None, 1, 1, 1, 1.0, None, None, None, None, None, None, None) == want != 0
+    arr = (backend.MatmulDesc * 1)()
+    assert calls["gllmq_quantized_matmul_batch"](None, C.addressof(arr), 1, None) != 0
