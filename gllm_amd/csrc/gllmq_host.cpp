@@ -173,7 +173,7 @@ struct Scratch {
     uint32_t *mm8_arrive = nullptr; // [MM8_SPLIT_MAX_LISTS]
     uint64_t *argmax_keys = nullptr; // [ARGMAX_MAX_ROWS][ARGMAX_MAX_PARTS]
     void *base = nullptr;        // the allocation that holds the three above
-    void *mmf = nullptr;         // GEMM: activation images, then partial sums of K-split workgroups
+    void *mmf = nullptr;         // GEMM: activation images, then partial sums of K-split workgroups or decoded weights
     size_t mmf_bytes = 0;
     void *ffn = nullptr;         // gllmq_ffn_swiglu: gated activations, then gate/up results
     size_t ffn_bytes = 0;
@@ -1197,8 +1197,7 @@ size_t mmfx_bytes(size_t n, uint32_t groups) { return (n + 31) / 32 * groups * g
 size_t mmfw_reserve(const gllmq_ctx *ctx, size_t m, size_t k)
 {
     const size_t groups = (k + 255) / 256, tiles = m <= 32 ? 1 : std::max<size_t>((m + 31) / 32, gq::MMFW_MAX_MT);
-    return std::min(tiles * groups * gq::MmfwImage<2>::bytes, kMmfwMaxImages) + ((groups * tiles * 128 + 1024 + 255) & ~size_t(255)) + mmfw_most_slices(ctx, m) +
-           (ctx->mmfx_min_m && m >= ctx->mmfx_min_m ? kMmfxMaxBytes : 0);
+    return std::min(tiles * groups * gq::MmfwImage<2>::bytes, kMmfwMaxImages) + ((groups * tiles * 128 + 1024 + 255) & ~size_t(255)) + mmfw_most_slices(ctx, m);
 }
 
 // Additions one after the other, in the mean over the blocks, when `blocks` of them are added up in runs of `run`
@@ -1348,6 +1347,33 @@ bool mmfw_takes_own(const gllmq_ctx *ctx, const MmfwPlan &L, int fmt, size_t m, 
            m * ldx * x_bytes <= 0xFFFFFFFFull;
 }
 
+// Makes the GEMM's scratch hold `need` bytes where decoded weights are to go, the call's own matrices' (`need` depends on them), if they can be had: not
+// under capture, and where the allocation is refused the scratch stays what it is.  The call then goes without, with the same bits.
+void grow_for_decoded(gllmq_ctx *ctx, Scratch &S, size_t need, void *stream)
+{
+    if (S.mmf_bytes >= need || S.fixed || ctx->probe || stream_is_capturing(stream)) return;
+    void *buf = nullptr;
+    if (hipSetDevice(ctx->device) != hipSuccess || hipMalloc(&buf, need) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+    }
+    if (S.mmf && hipStreamSynchronize(static_cast<hipStream_t>(stream)) != hipSuccess) { // (earlier work's error, which the next launch reports)
+        (void)hipFree(buf);
+        return;
+    }
+    drop_scratch(ctx, S, S.mmf);
+    S.mmf = buf;
+    S.mmf_bytes = need;
+}
+
+// ... enough for any call of up to `m` rows and `n` weight rows in up to MMFW_MAX_SEGS matrices
+size_t mmfx_reserve(const gllmq_ctx *ctx, uint32_t dtype, size_t m, size_t n, size_t k)
+{
+    if (mmf_format(dtype) != 2 || !ctx->use_mmf || !ctx->use_mmfw || !ctx->mmfx_min_m || m < ctx->mmfx_min_m) return 0;
+    return mmfw_reserve(ctx, m, k) - mmfw_most_slices(ctx, m) + 256 +
+           std::min(mmfx_bytes(n + 32u * (gq::MMFW_MAX_SEGS - 1), static_cast<uint32_t>((k + 255) / 256)), kMmfxMaxBytes);
+}
+
 // How a GEMM over many activation rows of Q6_K decodes its weights first.  mt = 0: it does not.
 struct MmfxPlan {
     uint32_t mt = 0;
@@ -1358,8 +1384,7 @@ struct MmfxPlan {
 // From 1024 rows on: decoding costs 0.5 us per million weights, the GEMM then takes a fifth less.  us, decoding and GEMM, and without (f32, 4096 x
 // 14336): 2048 rows 30 + 520, 625; 1024 rows 30 + 262, 313; 14336 x 4096: 1000 rows 30 + 275, 323, 512 rows 30 + 139, 164; one plane, 2048 rows of
 // 4096 x 4096 9 + 108, 142.
-// `room`: bytes of the scratch that are left.  Without room (a capture cannot have more) the weights are multiplied as they are, with the same bits.
-MmfxPlan plan_mmfx(const gllmq_ctx *ctx, const MmfwPlan &L, int fmt, const size_t *n, int count, size_t m, size_t room)
+MmfxPlan plan_mmfx(const gllmq_ctx *ctx, const MmfwPlan &L, int fmt, const size_t *n, int count, size_t m)
 {
     MmfxPlan X;
     if (fmt != 2 || L.ksplit != 1 || !ctx->mmfx_min_m || m < ctx->mmfx_min_m || ctx->mmfw_mt == 1) return X;
@@ -1370,7 +1395,7 @@ MmfxPlan plan_mmfx(const gllmq_ctx *ctx, const MmfwPlan &L, int fmt, const size_
         for (int i = 0; i < count; ++i) X.bytes += mmfx_bytes(n[i], L.groups);
         X.slab_rows = X.bytes <= kMmfxMaxBytes ? L.n_sum : 0;
     }
-    if (X.slab_rows == 0 || (X.bytes > room && !ctx->probe)) return X;
+    if (X.slab_rows == 0) return X;
     // Tiles by rounds of workgroups; us per block of K as timed (14336 x 4096, 4096 x 14336).  They do not touch the order of the sums.
     static const double block_us[2][gq::MMFW_MAX_MT - 1] = { { 3.3, 4.4, 6.4 }, { 4.6, 6.3, 8.4 } }; // [one plane, two][tiles - 2]
     const uint32_t row_tiles = static_cast<uint32_t>((std::min(L.rows, m) + 31) / 32);
@@ -1429,18 +1454,20 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
     const size_t used = (L.need() + 255) & ~size_t(255);
     size_t reserve = std::max(L.need(), mmfw_reserve(ctx, m, k));
     if (may_leave) reserve = std::max(reserve, leave->next_reserve);
+    const int fmt = mmf_format(f.dtype);
+    MmfxPlan X = plan_mmfx(ctx, L, fmt, n, count, m);
+    const size_t decoded_at = (take ? take->used : 0) + used;
+    if (X.mt && !take) grow_for_decoded(ctx, S, std::max(reserve, decoded_at + X.bytes), stream);
     if (!take && S.mmf_bytes < reserve && !S.fixed && !stream_is_capturing(stream)) rc = grow_scratch(ctx, S, &S.mmf, &S.mmf_bytes, reserve, stream, "quantized_matmul (GEMM)");
     if (rc != GLLMQ_OK) return rc;
+    if (decoded_at + X.bytes > S.mmf_bytes && !ctx->probe) X.mt = 0;
     const bool leaves = may_leave && used + leave->next_need <= S.mmf_bytes;
     uint8_t *scratch = static_cast<uint8_t *>(S.mmf) + (take ? take->used : 0);
-    const int fmt = mmf_format(f.dtype);
     const uint32_t ldx = row_stride_x(ctx, k);
     const size_t x_bytes = elem_x ? 2 : 4;
     bool own = mmfw_takes_own(ctx, L, fmt, m, k, ldx, x_bytes) && !take && !ctx->call_glu && !act_bf16;
     // outputs over the activations: what one workgroup stores another may still have to read
     for (int i = 0; i < count && L.ksplit == 1; ++i) own = own && !ranges_meet(mats[i].y, m * mats[i].n * (elem_y ? 2 : 4), x, m * ldx * x_bytes);
-    const size_t decoded_at = (take ? take->used : 0) + used;
-    const MmfxPlan X = plan_mmfx(ctx, L, fmt, n, count, m, S.mmf_bytes - std::min(S.mmf_bytes, decoded_at));
     if (X.mt) own = false;
     uint8_t *decoded = static_cast<uint8_t *>(S.mmf) + decoded_at;
     const bool slabs = X.mt && count == 1 && X.slab_rows < n[0];
@@ -3794,6 +3821,7 @@ int gllmq_reserve_matmul(gllmq_ctx *ctx, uint32_t dtype, size_t m, size_t n, siz
     if (ctx->use_mmf && ctx->use_mmfw) need = std::max(need, mmfw_reserve(ctx, m, k));
     const MmfsPlan Ls = plan_mmfs(ctx, *find_format(dtype), m, n, k);
     if (Ls.ok) need = std::max(need, Ls.need);
+    if (const size_t decoded = mmfx_reserve(ctx, dtype, m, n, k)) grow_for_decoded(ctx, *S, std::max(need, decoded), stream); // (refused: calls go without)
     return grow_scratch(ctx, *S, &S->mmf, &S->mmf_bytes, need, stream, "reserve_matmul");
 }
 

@@ -123,7 +123,10 @@ const char *gllmq_last_kernel_name(const gllmq_ctx *ctx);
  * nothing (needed before a stream capture).  What the GEMM needs depends on m and k alone, and 33 rows
  * serve any number (a captured call of more goes in passes, with the same bits), so one reserved or
  * eager call per k covers other matrices, element types and batches over the same rows too (but 9 to 16 rows of
- * Q4_K and Q5_K against matrices of more than 2^28 weights: reserve those by their own shape).  No
+ * Q4_K and Q5_K against matrices of more than 2^28 weights: reserve those by their own shape).  From 1024
+ * rows of Q6_K on the weights are decoded first where there is scratch for that, 17 KiB per 32 x 256 of them and
+ * at most 128 MiB: what is reserved, or grown by an eager call, is for as large matrices (a batch's together).
+ * Without it (captured, or an allocation that is refused) they are multiplied as they are: the same bits, later.  No
  * counterpart in the reference, whose scratch is
  * sized when the graph is compiled (src/compat/gpu_backend_macro.rs:82-87). */
 int gllmq_reserve_matmul(gllmq_ctx *ctx, uint32_t ggml_dtype, size_t m, size_t n, size_t k, void *stream);

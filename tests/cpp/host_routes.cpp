@@ -32,6 +32,7 @@ std::map<void *, size_t> live; // device allocations
 size_t allocations = 0, frees = 0;
 uintptr_t next_address = uintptr_t(1) << 40;
 bool capturing = false;
+size_t refuse_from = SIZE_MAX; // allocations of as many bytes are refused
 
 hipError_t record(hipFunction_t f, uint32_t grid, void **extra)
 {
@@ -61,6 +62,7 @@ hipError_t hipGetDeviceProperties(hipDeviceProp_t *p, int) // (the header's macr
 }
 hipError_t hipMalloc(void **p, size_t size)
 {
+    if (size >= fake::refuse_from) return hipErrorOutOfMemory;
     *p = reinterpret_cast<void *>(fake::next_address);
     fake::next_address += (size + 4095) / 4096 * 4096;
     fake::live[*p] = size;
@@ -376,7 +378,63 @@ void scratch_of_graphs_stays()
         }
 }
 
+// A prompt's decoded weights take as much scratch as the call's matrices need: other formats allocate nothing for them, a call that cannot
+// have it goes without, and a reservation is enough for a captured call to have it.
+void decoded_weights_scratch()
+{
+    const auto held = [] {
+        size_t bytes = 0;
+        for (const auto &b : fake::live) bytes += b.second;
+        return bytes;
+    };
+    const auto decodes = [] { return launched("gq_mmfx_decode_q6k"); };
+    for (const auto &f : kFormats)
+        for (size_t m : { 1023u, 1024u, 2048u })
+            for (const auto &s : std::vector<std::vector<size_t>>{ { 100, 1024 }, { 4096, 4096 }, { 4096, 14336 }, { 14336, 4096 }, { 28672, 4096 }, { 128256, 2048 } }) {
+                size_t total[2], need = std::min<size_t>((s[0] + 31) / 32 * (s[1] / 256) * gq::MmfxRecord::bytes, size_t(128) << 20);
+                for (int decoded = 0; decoded < 2; ++decoded) {
+                    Context ctx;
+                    if (!decoded) gllmq_set_option(ctx, "mmfx_min_m", 0);
+                    for (int elem : { GLLMQ_ELEM_F32, GLLMQ_ELEM_BF16 }) {
+                        EXPECT(matmul(ctx, f.dtype, m, s[0], s[1], elem, at(4), at(5)) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+                        EXPECT((decodes() > 0) == (decoded && f.dtype == T_Q6_K && m >= 1024 && s[0] > 100), "dtype %u, %zu rows, %zu x %zu: %zu", f.dtype, m, s[0], s[1], decodes());
+                    }
+                    total[decoded] = held();
+                }
+                EXPECT(total[1] >= total[0] && total[1] - total[0] <= (f.dtype == T_Q6_K && m >= 1024 ? need : 0), "dtype %u, %zu rows, %zu x %zu: %zu bytes more, the weights need %zu",
+                       f.dtype, m, s[0], s[1], total[1] - total[0], need);
+            }
+    for (bool reserved : { false, true }) {
+        Context ctx;
+        // no room: the weights as they are, in the scratch that there was
+        EXPECT(matmul(ctx, T_Q6_K, 1024, 4096, 4096, GLLMQ_ELEM_F32, at(4), at(5)) == GLLMQ_OK && decodes() == 1, "%s", gllmq_last_error(ctx));
+        fake::refuse_from = size_t(100) << 20;
+        const size_t before = held(), frees = fake::frees;
+        EXPECT(matmul(ctx, T_Q6_K, 1024, 14336, 4096, GLLMQ_ELEM_F32, at(4), at(5)) == GLLMQ_OK && decodes() == 0 && wide_launch(), "%s", gllmq_last_error(ctx));
+        EXPECT(gllmq_reserve_matmul(ctx, T_Q6_K, 1024, 14336, 4096, nullptr) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+        EXPECT(matmul(ctx, T_Q6_K, 1024, 4096, 4096, GLLMQ_ELEM_F32, at(4), at(5)) == GLLMQ_OK && decodes() == 1 && held() == before && fake::frees == frees, "%zu bytes", held());
+        fake::refuse_from = SIZE_MAX;
+        // captured: with what there is
+        fake::capturing = true;
+        EXPECT(matmul(ctx, T_Q6_K, 1024, 14336, 4096, GLLMQ_ELEM_F32, at(4), at(5)) == GLLMQ_OK && decodes() == 0, "%s", gllmq_last_error(ctx));
+        EXPECT(matmul(ctx, T_Q6_K, 1024, 4096, 4096, GLLMQ_ELEM_F32, at(4), at(5)) == GLLMQ_OK && decodes() == 1, "%s", gllmq_last_error(ctx));
+        fake::capturing = false;
+        const std::map<void *, size_t> captured = fake::live;
+        for (size_t m : { 1024u, 1500u, 2048u })
+            for (int elem : { GLLMQ_ELEM_F32, GLLMQ_ELEM_BF16 }) {
+                if (reserved) EXPECT(gllmq_reserve_ffn(ctx, T_Q6_K, T_Q6_K, m, 4096, 7000 / 256 * 256, nullptr) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+                else EXPECT(ffn(ctx, T_Q6_K, T_Q6_K, m, 4096, 7000 / 256 * 256, elem) == GLLMQ_OK && decodes() == 3, "%zu: %s", decodes(), gllmq_last_error(ctx));
+                for (const auto &b : captured) EXPECT(fake::live.count(b.first), "%zu bytes that a graph holds are gone", b.second);
+                const size_t allocations = fake::allocations;
+                fake::capturing = true;
+                EXPECT(ffn(ctx, T_Q6_K, T_Q6_K, m, 4096, 7000 / 256 * 256, GLLMQ_ELEM_BF16) == GLLMQ_OK && decodes() == 3 && fake::allocations == allocations, "%zu: %s", decodes(), gllmq_last_error(ctx));
+                fake::capturing = false;
+            }
+    }
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
+    { "decoded_weights_scratch", decoded_weights_scratch },
     { "scratch_of_graphs_stays", scratch_of_graphs_stays },
     { "elements_take_the_f32_kernels", elements_take_the_f32_kernels },
     { "runs_of_weight_tiles", runs_of_weight_tiles },
