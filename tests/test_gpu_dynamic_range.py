@@ -214,3 +214,40 @@ def test_moe_over_the_dynamic_range(torch, oracle):
         got = run_gpu(hip, torch, gu, Q4_K, dn, Q6_K, x, hidden, ffn, experts, r["expert"], r["weight"], r["len"])
         assert np.isfinite(got).all()
         check_moe(got, want, f"moe {kind}")
+
+
+@pytest.mark.parametrize("m, k, options, form", [
+    (1, 3072, {}, "gq_mm8s_q6k_p1_e1_a_f"), (1, 14336, {}, "gq_mm8s_q6k_p1_e4_f"), (1, 512, {}, "gq_mm8s_q6k_p1_e1_a"), (2, 1024, {}, "gq_mm8s_q6k_p1_e2_a"),
+    (4, 1024, {}, "gq_mm8s_q6k_p2_e4_a"), (6, 1024, {}, "gq_mm8s_q6k_p4"), (3, 14336, {}, "gq_mm8s_q6k_p2_e4_s"), (3, 1024, {"mm8s": 0}, "gq_mm8_q6k_p2"), (6, 1024, {"mm8s": 0}, "gq_mm8_q6k_p4"), (6, 4096, {"mm8s": 0}, "gq_mm8_q6k_p4")])
+def test_q6k_activations_have_23_bits(torch, m, k, options, form):
+    """Weight rows of one 1 and zeros give back activations as the int8 kernels of Q6_K hold them: a block's values rounded to whole
+    numbers of 2^(e - 149), e its largest value's exponent, or one more from the mantissa 0x7EFE00 on, where the whole number would not fit
+    three signed digits.  Largest values on both sides of that line, up to the exponent above the last one; nothing but that rounding."""
+    from gllm_amd.backend import HipBackend
+    from tests.packing import pack_q6_k
+    hip, n = HipBackend(0, options=options), max(1024, 2048 * 512 // k)
+    rng = np.random.default_rng(m + k)
+    tops = [(e, f) for e in (24, 60, 127, 253, 254) for f in (0x000000, 0x000001, 0x7EFDFE, 0x7EFDFF, 0x7EFE00, 0x7EFE01, 0x7FFFF0)]
+    x, grid = np.zeros((m, k), np.float32), np.zeros((m, k))
+    for r in range(m):
+        for b in range(k // 256):
+            e, f = tops[int(rng.integers(len(tops)))]
+            top = float(np.array([e << 23 | f], np.uint32).view(np.float32)[0])
+            step = 2.0 ** (e + (f >= 0x7EFE00) - 149)
+            v = rng.uniform(-1, 1, 256) * top * rng.choice([1.0, 1e-3], 256)
+            v[:64] = (np.floor(v[:64] / step) + 0.5) * step  # halves of a step, which go up
+            v = np.clip(v, -top, top).astype(np.float32)
+            v[rng.integers(64, 256)] = top * rng.choice([-1.0, 1.0])
+            x[r, 256 * b:256 * b + 256], grid[r, 256 * b:256 * b + 256] = v, step
+    zero = pack_q6_k(1.0, np.ones(16), np.zeros(256))
+    w, per = np.tile(zero, (n, k // 256, 1)), max(1, k // n)
+    at = (np.arange(n) * per + np.arange(n) % per) % k
+    for row, element in enumerate(at):
+        one = np.zeros(256)
+        one[element % 256] = 1
+        w[row, element // 256] = pack_q6_k(1.0, np.ones(16), one)
+    print(f"23 bits m={m} k={k} {options}", flush=True)
+    y = gpu_matmul(hip, torch, w.reshape(-1), x, Q6_K, m, n, k)
+    assert form in hip.last_kernel_name(), hip.last_kernel_name()
+    want = np.floor(x.astype(np.float64) / grid + 0.5) * grid
+    assert np.array_equal(y.astype(np.float64), want[:, at])
