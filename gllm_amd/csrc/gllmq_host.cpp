@@ -820,13 +820,16 @@ int run_mm8s(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
         if (!fold && kind == MM8_Q5K && mm == 1 && n < static_cast<size_t>(12) * cus) return -1;
         // Q6_K: two to four rows everywhere (us, here and in brackets in the other forms: two rows 5120 -> 4096 7.5 (11.7), -> 28672 25 (38), 14336 ->
         // 6144 20 (26); three 5120 -> 6144 10.7 (13.5), four 4096 -> 14336 14.0 (17.0)).  One row: in pairs of blocks from 20 blocks on; from 40 on at
-        // all heights; of 17 to 39 blocks over more than 24 weight rows per CU (5120 -> 8192 9.3 (12.2), 4864 -> 32000 25 (35)), rows of 8192, where the
-        // GEMV's waves have all lanes at work, to 56 (14336 20.3 (21.8), 128256 153 (145)); up to 15 blocks (3072 -> 1024 5.0 (5.4-6.2), -> 8192 6.4
-        // (7.6), 2048 -> 14336 7.7 (8.4)), the shortest to 16 weight rows per CU and block (2048 -> 32000 12.2 (13.0), 128256 42 (40); 1024 -> 14336
-        // 5.9 (6.5), 28672 8.9 (8.7)).
+        // all heights; of 17 to 39 blocks over more than 24 weight rows per CU (5120 -> 8192 9.3 (12.2), 4864 -> 32000 25 (35)); up to 16 blocks
+        // (3072 -> 1024 5.0 (5.4-6.2), -> 8192 6.4 (7.6), 2048 -> 14336 7.7 (8.4)), the shortest to 16 weight rows per CU and block (2048 -> 32000
+        // 12.2 (13.0), 128256 42 (40); 1024 -> 14336 5.9 (6.5), 28672 8.9 (8.7)).  A wave of the GEMV takes 4096 elements of K, and where all its lanes
+        // are at work it is ahead: rows of 4096, rows of 8192 over more than 56 weight rows per CU (14336 20.3 (21.8), 128256 153 (145)), and over more
+        // than 64 also rows that fill all but a part of a block of it (3968 -> 8192 7.0 (7.6), 32000 22.7 (22.3), 64000 44.6 (40.8); 8064 -> 16384
+        // 22.3 (23.9), 64000 82 (78)).
         if (kind == MM8_Q6K && mm == 1 && groups < 40 && !(fold && groups >= 20)) {
             const size_t rows = (n + cus - 1) / cus;
-            if (groups >= 16 ? (groups == 16 || rows <= 24 || (groups == 32 && rows > 56)) : (groups <= 8 && rows > 16u * groups)) return -1;
+            const size_t most = k % 4096 == 0 ? (groups == 16 ? 0u : 56u) : groups % 16 == 0 ? 64u : groups <= 8 ? 16u * groups : SIZE_MAX;
+            if (rows > most || (groups > 16 && rows <= 24)) return -1;
         }
         // Q8_0, two rows over at most 8 weight rows per CU: its GEMV stays ahead (4096 -> 1024: 5.9 against 7.1 us)
         if (kind == MM8_Q8_0 && mm == 2 && n <= static_cast<size_t>(8) * cus) return -1;

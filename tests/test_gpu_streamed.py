@@ -229,6 +229,7 @@ def test_more_open_requests_per_loader_change_no_bit(hip, torch, dtype):
     (Q6_K, 1, 57, 8192, "gemv"), (Q6_K, 2, 5, 5120 - 8, "_e4"), (Q6_K, 3, 25, 5120, "_e4"), (Q6_K, 4, 57, 4096, "_a"), (Q6_K, 2, 5, 8192, "_e4"),
     (Q6_K, 3, 15, 14336, "_s"), (Q6_K, 4, 4, 9216 + 136, "_s"), (Q6_K, 2, 4, 14336, "_s"), (Q6_K, 3, 4, 16384, "mm8_"),
     (Q4_K, 3, 8, 9216, "_s"), (Q4_K, 2, 5, 14336 - 8, "_s"), (Q5_K, 4, 4, 14336, "_s"), (8, 3, 8, 9216, "_s"), (8, 4, 8, 11008, "_s"),
+    (Q6_K, 1, 64, 3968, "_a"), (Q6_K, 1, 65, 4096 - 8, "gemv"), (Q6_K, 1, 16, 4096, "gemv"), (Q6_K, 1, 57, 7944, "_e2"),
     (Q6_K, 2, 16, 8192, "_s"), (Q6_K, 2, 12, 9728, "_s"), (8, 2, 16, 8192, "_s"), (8, 2, 13, 9728, "_s")])
 def test_default_choice_at_its_lines(torch, dtype, m, rows, k, form):
     """Q6_K at one to four rows and the finer slices of K: the default choice just inside and outside its lines, a ragged last workgroup, against
