@@ -1420,6 +1420,7 @@ MmfxPlan plan_mmfx(const gllmq_ctx *ctx, const MmfwPlan &L, int fmt, const size_
 struct MmfwSlices {
     size_t next_need = 0;    // scratch that the down projection needs,
     size_t next_reserve = 0; // and that it grows the scratch to
+    size_t next_decoded = 0; // bytes of its decoded weights, which it cannot grow the scratch for with the sums there
     const float *at = nullptr;
     uint32_t slices = 0;     // 0: none were left
     size_t used = 0;         // bytes of the scratch in use
@@ -1461,6 +1462,7 @@ int run_mmfw(gllmq_ctx *ctx, Scratch &S, const Format &f, const MmfwMatrix *mats
     MmfxPlan X = plan_mmfx(ctx, L, fmt, n, count, m);
     const size_t decoded_at = (take ? take->used : 0) + used;
     if (X.mt && !take) grow_for_decoded(ctx, S, std::max(reserve, decoded_at + X.bytes), stream);
+    if (may_leave && leave->next_decoded) grow_for_decoded(ctx, S, std::max(reserve, used + ((leave->next_need + 255) & ~size_t(255)) + leave->next_decoded), stream);
     if (!take && S.mmf_bytes < reserve && !S.fixed && !stream_is_capturing(stream)) rc = grow_scratch(ctx, S, &S.mmf, &S.mmf_bytes, reserve, stream, "quantized_matmul (GEMM)");
     if (rc != GLLMQ_OK) return rc;
     if (decoded_at + X.bytes > S.mmf_bytes && !ctx->probe) X.mt = 0;
@@ -2771,6 +2773,7 @@ int ffn_on_stream(gllmq_ctx *ctx, const void *gate_w, const void *up_w, size_t g
         MmfwSlices sums;
         sums.next_need = down_plan.need();
         sums.next_reserve = std::max(down_plan.need(), mmfw_reserve(ctx, m, ffn));
+        sums.next_decoded = plan_mmfx(ctx, down_plan, mmf_format(dtype_down), &hidden, 1, m).bytes;
         rc = run_mmfw(ctx, S, *fg, gate_up, 2, x, elem, 0, m, hidden, false, stream, 5, ctx->ffn_glu_load && down_plan.rows >= m ? &sums : nullptr);
         if (rc > 0) return rc;
         if (rc == GLLMQ_OK) {

@@ -404,6 +404,14 @@ void decoded_weights_scratch()
                 EXPECT(total[1] >= total[0] && total[1] - total[0] <= (f.dtype == T_Q6_K && m >= 1024 ? need : 0), "dtype %u, %zu rows, %zu x %zu: %zu bytes more, the weights need %zu",
                        f.dtype, m, s[0], s[1], total[1] - total[0], need);
             }
+    // a down projection behind sums that gate and up leave, which the scratch cannot grow around: room for it is made ahead of them
+    for (const auto &s : std::vector<std::vector<size_t>>{ { 1024, 8192, 1024 }, { 1536, 4096, 1024 }, { 3000, 5120, 512 } }) {
+        Context ctx;
+        EXPECT(ffn(ctx, T_Q4_K, T_Q6_K, s[0], s[1], s[2]) == GLLMQ_OK && launched("gq_mmf_reduce") == 0 && decodes() == 1, "%zu rows, %zu x %zu: %zu", s[0], s[1], s[2], decodes());
+        fake::refuse_from = 1;
+        EXPECT(ffn(ctx, T_Q4_K, T_Q6_K, s[0], s[1], s[2]) == GLLMQ_OK && decodes() == 1, "%s", gllmq_last_error(ctx));
+        fake::refuse_from = SIZE_MAX;
+    }
     for (bool reserved : { false, true }) {
         Context ctx;
         // no room: the weights as they are, in the scratch that there was
