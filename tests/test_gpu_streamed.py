@@ -228,9 +228,7 @@ def test_more_open_requests_per_loader_change_no_bit(hip, torch, dtype):
     (Q6_K, 1, 5, 3072, "_f"), (Q6_K, 1, 16, 1024, "_a"), (Q6_K, 1, 65, 1024, "gemv"), (Q6_K, 1, 25, 4864 + 8, "_e2"), (Q6_K, 1, 24, 4864, "gemv"),
     (Q6_K, 1, 57, 8192, "gemv"), (Q6_K, 2, 5, 5120 - 8, "_e4"), (Q6_K, 3, 25, 5120, "_e4"), (Q6_K, 4, 57, 4096, "_a"), (Q6_K, 2, 5, 8192, "_e4"),
     (Q6_K, 3, 15, 14336, "_s"), (Q6_K, 4, 4, 9216 + 136, "_s"), (Q6_K, 2, 4, 14336, "_s"), (Q6_K, 3, 4, 16384, "mm8_"),
-    (Q4_K, 3, 8, 9216, "_s"), (Q4_K, 2, 5, 14336 - 8, "_s"), (Q5_K, 4, 4, 14336, "_s"), (8, 3, 8, 9216, "_s"), (8, 4, 8, 11008, "_s"),
-    (Q6_K, 1, 64, 3968, "_a"), (Q6_K, 1, 65, 4096 - 8, "gemv"), (Q6_K, 1, 16, 4096, "gemv"), (Q6_K, 1, 57, 7944, "_e2"),
-    (Q6_K, 2, 16, 8192, "_s"), (Q6_K, 2, 12, 9728, "_s"), (8, 2, 16, 8192, "_s"), (8, 2, 13, 9728, "_s")])
+    (Q4_K, 3, 8, 9216, "_s"), (Q4_K, 2, 5, 14336 - 8, "_s"), (Q5_K, 4, 4, 14336, "_s"), (8, 3, 8, 9216, "_s"), (8, 4, 8, 11008, "_s")])
 def test_default_choice_at_its_lines(torch, dtype, m, rows, k, form):
     """Q6_K at one to four rows and the finer slices of K: the default choice just inside and outside its lines, a ragged last workgroup, against
     the kernels that ran there before (which the other tests hold to the oracle), and a call of 16-bit elements as the rounded f32 result."""
@@ -248,3 +246,11 @@ def test_default_choice_at_its_lines(torch, dtype, m, rows, k, form):
     out = torch.zeros(m, n, device="cuda", dtype=torch.bfloat16)
     default.quantized_matmul(torch.from_numpy(w).cuda(), xb.cuda(), out, dtype, m, n, k)
     assert torch.equal(out.cpu().view(torch.int16), torch.from_numpy(y).to(torch.bfloat16).view(torch.int16))
+
+
+@pytest.mark.parametrize("dtype,m,rows,k,form", [
+    (Q6_K, 1, 64, 3968, "_a"), (Q6_K, 1, 65, 4096 - 8, "gemv"), (Q6_K, 1, 16, 4096, "gemv"), (Q6_K, 1, 57, 7944, "_e2"),
+    (Q6_K, 2, 16, 8192, "_s"), (Q6_K, 2, 12, 9728, "_s"), (8, 2, 16, 8192, "_s"), (8, 2, 13, 9728, "_s")])
+def test_default_choice_at_more_lines(torch, dtype, m, rows, k, form):
+    """... rows of K that almost fill the GEMV's waves, and two rows that share K among workgroups."""
+    test_default_choice_at_its_lines(torch, dtype, m, rows, k, form)
