@@ -192,6 +192,16 @@ constexpr size_t kScratchPartBytes = sizeof(float) * gq::MM8_SPLIT_PART_FLOATS;
 constexpr size_t kScratchFixedBytes = kScratchArriveBytes + kScratchKeysBytes + kScratchPartBytes;
 constexpr size_t kMaxScratchSlots = 16;
 
+// The greedy token behind a one-row matmul's outputs `y` (gllmq_lm_head_argmax).
+struct TokenChoice {
+    const float *y;
+    size_t n;
+    uint64_t *keys;
+    uint32_t *ticket, *token;
+    float *value;
+    bool made; // the launch makes it
+};
+
 // Weights that a host-slice call uploaded, kept for the next call with the same slice
 // (the reference keeps its uploaded weight blob the same way, src/compat/hip_backend.rs:141-156).
 struct CachedWeights {
@@ -232,6 +242,7 @@ struct gllmq_ctx {
     // streamed form (loader waves + arithmetic waves) [0 = Q4_K, 1 = Q5_K, 2 = Q6_K, 3 = Q8_0][variant]: register
     // operands p1_e1, p1_e2, p2_e4, then LDS operands p1_e2, p2_e4, p4_e4
     hipFunction_t mm8s[4][7] = {};
+    hipFunction_t mm8s_token[4][4] = {};        // one row, ending in the greedy token choice [format as above][p1_e1_a, p1_e2_a, p1_e2, p1_e4]
     bool use_mm8s = true;                       // "mm8s" = 0: the fetch-and-compute kernels throughout
     bool batch_overlap = true;                  // "batch_overlap" = 0: the kernels of a batch run strictly one after the other
     bool mm8s_all = false;                      // "mm8s_all" = 1: the streamed form wherever it fits, also where another was timed faster
@@ -330,6 +341,7 @@ struct gllmq_ctx {
     // activations of the matmul being enqueued that are a gated product: x[r][i] = act(x[r][i]) * x[r][i + call_glu_off],
     // rows call_ldx elements apart (the input of a feed-forward block's down projection); 0 = plain
     uint32_t call_glu = 0, call_glu_off = 0, call_ldx = 0;
+    TokenChoice *call_token = nullptr; // the one-row matmul being enqueued ends in the greedy token where its kernel can
     bool ffn_glu_load = true;   // "ffn_glu_load" = 0: the gate activation always runs as a kernel of its own
     hipFunction_t mm8s_gated[2][6] = {};        // streamed gate/up kernels with act(g) * u at the end of a tile pair [Q4_K, Q5_K][p1_e1_a, p1_e2_a, p2_e4_a, p1_e2, p2_e4, p1_e4]
     bool ffn_streamed = true;                   // "ffn_streamed" = 0: gllmq_ffn_swiglu never uses them
@@ -911,6 +923,12 @@ int run_mm8s(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
         P.kslice_groups = kslice;
         P.part = S->mm8_part;
         P.arrive = S->mm8_arrive;
+    }
+    if (TokenChoice *c = ctx->call_token; c && c->y == y && c->n == n && mm == 1 && !split && !fold && !glu && !ctx->call_glu && !ctx->call_elem &&
+                                          grid <= gq::ARGMAX_MAX_PARTS * gq::ARGMAX_MAX_ROWS) {
+        gq::Mm8sTokenParams T{ P, c->keys, c->ticket, c->token, c->value };
+        c->made = true;
+        return launch(ctx, ctx->mm8s_token[sfmt][variant <= 1 ? variant : variant == 3 ? 2 : 3], grid, (gq::MM8S_CWAVES + gq::MM8S_LOADERS) * 64, lds, stream, &T, sizeof T, true);
     }
     return launch(ctx, fn, grid * ksplit, (gq::MM8S_CWAVES + gq::MM8S_LOADERS) * 64, lds, stream, &P, sizeof P, split);
 }
@@ -2284,6 +2302,12 @@ int gllmq_init(gllmq_ctx **out, int device)
                 snprintf(name, sizeof name, "gq_mm8s_%s_%s", kMm8sFormat[q], kMm8s[v]);
                 rc = get_function(ctx, &ctx->mm8s[q][v], name);
             }
+        static const char *const kMm8sToken[4] = { "p1_e1_a", "p1_e2_a", "p1_e2", "p1_e4" };
+        for (int q = 0; q < 4; ++q)
+            for (int v = 0; v < 4 && rc == GLLMQ_OK; ++v) {
+                snprintf(name, sizeof name, "gq_mm8s_%s_%s_token", kMm8sFormat[q], kMm8sToken[v]);
+                rc = get_function(ctx, &ctx->mm8s_token[q][v], name);
+            }
         static const char *const kMm8sGated[6] = { "p1_e1_a", "p1_e2_a", "p2_e4_a", "p1_e2", "p2_e4", "p1_e4" };
         for (int q = 0; q < 2; ++q)
             for (int v = 0; v < 6 && rc == GLLMQ_OK; ++v) {
@@ -2581,11 +2605,12 @@ int gllmq_lm_head_argmax(gllmq_ctx *ctx, const void *w, size_t w_bytes, const fl
     Scratch *S = nullptr;
     rc = acquire_scratch(ctx, stream, &S);
     if (rc != GLLMQ_OK) return rc;
-    // The matvec whose workgroups leave their best candidate behind: the one-row GEMV of Q6_K and
-    // Q8_0 (the types of GGUF output matrices) where one launch covers K; the workgroup that
-    // finishes last picks among the candidates.  With a logits buffer it runs where the GEMV is
+    // The matvec whose workgroups leave their best candidate behind; the workgroup that
+    // finishes last picks among the candidates.  The one-row GEMV of Q6_K and
+    // Q8_0 (the types of GGUF output matrices) where one launch covers K: with a logits buffer where the GEMV is
     // the kernel gllmq_quantized_matmul gives the shape anyway (dispatch_choice() asks the dispatch
-    // itself), so that the logits are that call's bit for bit; without one, always.
+    // itself), so that the logits are that call's bit for bit; without one, always.  With a logits buffer, of any
+    // format, the streamed kernel where that is the one the shape gets (run_mm8s sees the choice that is wanted).
     const size_t rb = gllmq_row_bytes(dtype, k);
     const bool gemv_type = dtype == 14u || dtype == 8u;
     bool gemv_anyway = true;
@@ -2616,8 +2641,11 @@ int gllmq_lm_head_argmax(gllmq_ctx *ctx, const void *w, size_t w_bytes, const fl
         return fail(ctx, GLLMQ_ERR_UNIMPLEMENTED,
                     "lm_head_argmax: this matrix (ggml dtype %u, k = %zu) goes through the matmul and the token choice one "
                     "after the other, which needs a logits buffer of n floats", dtype, k);
+    TokenChoice choice{ logits, n, S->argmax_keys, S->mm8_arrive + kLmHeadTicketAt, token, value, false };
+    if (ctx->lm_head_fused) ctx->call_token = &choice;
     rc = dispatch_matmul(ctx, *S, *f, static_cast<const uint8_t *>(w), x, logits, 1, n, k, false, stream);
-    if (rc != GLLMQ_OK) return rc;
+    ctx->call_token = nullptr;
+    if (rc != GLLMQ_OK || choice.made) return rc;
     return gllmq_argmax(ctx, logits, 1, n, n, token, value, stream);
 }
 

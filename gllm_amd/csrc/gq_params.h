@@ -83,6 +83,16 @@ struct Mm8Params {
     unsigned long long progress_seq;
 };
 
+// The launch that ends in the greedy token (gq_mm8s_*_token): the workgroups' candidates (argmax_key), how many workgroups have left
+// theirs (zero between launches), the token, and (or null) its value.
+struct Mm8sTokenParams {
+    Mm8Params p;
+    uint64_t *keys;
+    uint32_t *ticket;
+    uint32_t *token;
+    float *value;
+};
+
 // Several weight matrices over the same activations in one streamed launch: the row ranges of a matrix are
 // those of workgroups first_wg .. up to the next matrix's; p.w, p.y, p.n and p.ldy are each workgroup's own.
 constexpr int MM8S_MAX_SEGS = 3;
@@ -199,8 +209,11 @@ struct Mm8sCtrl {                    // counters in LDS, all start at zero
     uint32_t done[MM8S_CWAVES];      // per arithmetic wave: items consumed
     uint32_t arrived[MM8S_RED_BUFS]; // per partial-sum buffer: waves that left their sums
     uint32_t reduced;                // tiles summed and stored
-    uint32_t finished;               // K split: arithmetic waves whose slice sums have reached coherent memory
-    uint32_t pad[2];
+    uint32_t finished;               // K split: arithmetic waves whose slice sums have reached coherent memory; token choice: that are through
+    union {
+        uint32_t pad[2];
+        uint64_t best;               // token choice: the workgroup's largest candidate
+    };
 };
 
 // LDS carve-up of the streamed kernels: the preparation's planes, sums and scales as in

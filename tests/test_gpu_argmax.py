@@ -150,6 +150,41 @@ def test_lm_head_and_token_in_one_call(hip, torch, oracle, dt, n, k):
     assert want[int(tok[0])] >= want.max() - 2e-3 * np.abs(want).max()
 
 
+@pytest.mark.parametrize("dt", [8, 12, 13, 14])
+@pytest.mark.parametrize("n, k", [(6145, 2048), (8192 + 31, 4096), (9001, 4608), (12000, 8192), (5000, 1280), (70000, 256)])
+def test_token_from_the_streamed_kernel(hip, torch, oracle, dt, n, k):
+    """The output matrix as one launch that ends in the token (gq_mm8s_*_token), planes in registers and in LDS, ragged last workgroups: logits and
+    token of the two calls bit for bit, twice in a row (the count of workgroups is back at zero); equal rows in several workgroups give the last
+    one; a NaN activation leaves no candidate."""
+    from gllm_amd.synth import random_activations, random_weight
+    w = np.asarray(random_weight(dt, n, k, seed=n)).view(np.uint8).reshape(n, -1).copy()
+    x = random_activations(1, k, seed=k)
+    xd = torch.from_numpy(x).cuda()
+    xn = xd.clone()
+    xn[0, k // 2] = NAN
+    y, y2 = torch.empty(1, n, device="cuda"), torch.empty(n, device="cuda")
+    tok, val = torch.zeros(2, dtype=torch.int32, device="cuda"), torch.zeros(2, device="cuda")
+    for tied in (False, True):
+        if tied:
+            top = int(tok[0])
+            w[[0, n // 2, n - 2]] = w[top]
+        wd = torch.from_numpy(w.reshape(-1)).cuda()
+        for acts in (xd, xd, xn):
+            print(f"token dtype={dt} n={n} k={k} tied={tied}", flush=True)
+            hip.quantized_matmul(wd, acts, y, dt, 1, n, k)
+            streamed = "mm8s" in hip.last_kernel_name() and "_f" not in hip.last_kernel_name()
+            hip.argmax(y, tok[:1], val[:1])
+            hip.lm_head_argmax(wd, acts, dt, n, k, tok[1:], logits=y2, value=val[1:])
+            assert hip.last_kernel_name().endswith(("_token",) if streamed else ("_argmax", "gq_argmax_final", "gq_argmax_part")), hip.last_kernel_name()
+            torch.cuda.synchronize()
+            assert torch.equal(y2.view(torch.int32), y[0].view(torch.int32))
+            assert int(tok[0]) == int(tok[1]) and torch.equal(val[:1].view(torch.int32), val[1:].view(torch.int32))
+            if tied and acts is xd:
+                assert int(tok[1]) == max(top, n - 2)
+        hip.argmax(y.new_zeros(1, 1).copy_(y2[:1].view(1, 1)), tok[:1])  # (another use of the scratch keys in between)
+        hip.lm_head_argmax(wd, xd, dt, n, k, tok[:1], logits=y2, value=val[:1])
+
+
 def test_lm_head_token_with_ties_and_nan(hip, torch, oracle):
     """Rows of equal weights give equal logits (the LAST of them is the token), and a NaN activation
     leaves no candidate at all."""
