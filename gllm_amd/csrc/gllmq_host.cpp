@@ -120,6 +120,16 @@ uint32_t mmfw_lds_bytes(int fmt, int planes, uint32_t mt)
     return kTotal[fmt][planes - 1][mt - 1];
 }
 
+// ... over experts' jobs (`few`: in workgroups of four waves)
+uint32_t mmfw_grouped_lds(int fmt, int planes, bool few)
+{
+#define GQ_ROW(F, PL) { gq::mmfw_grouped_lds<F, PL, gq::MMFW_EXPERTS>(), gq::mmfw_grouped_lds<F, PL, gq::MMFW_EXPERTS_FEW>() }
+    static const uint32_t kTotal[4][2][2] = { { GQ_ROW(0, 1), GQ_ROW(0, 2) }, { GQ_ROW(1, 1), GQ_ROW(1, 2) },
+                                              { GQ_ROW(2, 1), GQ_ROW(2, 2) }, { GQ_ROW(3, 1), GQ_ROW(3, 2) } };
+#undef GQ_ROW
+    return kTotal[fmt][planes - 1][few ? 1 : 0];
+}
+
 // ... with decoded weights (Q6_K, from two tiles on)
 uint32_t mmfx_lds_bytes(int planes, uint32_t mt)
 {
@@ -254,6 +264,7 @@ struct gllmq_ctx {
     hipFunction_t mmf_q4k[4][2][2] = {};        // f16 matrix-core GEMM [0 = Q4_K, 1 = Q5_K, 2 = Q6_K, 3 = Q8_0][32-row activation tiles - 1][bf16 mode]
     hipFunction_t mmfw[4][4][2] = {};           // the GEMM for more rows [format as above][32-row activation tiles - 1][0 = hi and lo plane, 1 = hi only]
     hipFunction_t moe_mmf[4][2] = {};           // the same over experts' rows [format][plane]
+    hipFunction_t moe_mmf_few[4][2] = {};       // ... in workgroups of four waves
     hipFunction_t mmfw_own[4][2] = {};          // ... of one tile, which prepares the activations itself [format][0 = hi and lo plane, 1 = hi only]
     hipFunction_t mmfx_decode = nullptr;        // Q6_K weights to matrix-core operands, for prompts
     hipFunction_t mmfx[gq::MMFW_MAX_MT - 1][2] = {}; // ... and their GEMM [tiles - 2][0 = hi and lo plane, 1 = hi only]
@@ -312,6 +323,7 @@ struct gllmq_ctx {
     uint32_t moe_streamed = 1;                  // "moe_streamed": the grouped kernels in the streamed form: 0 never, 1 while experts see few tokens each, 2 always
     bool moe_wide = true;                       // "moe_wide" = 0: experts with many tokens stay on the eight-token jobs
     bool moe_wide_cost = true;                  // ... and only where it is estimated to be ahead (off once "moe_wide_min" is set)
+    uint32_t moe_wide_few = 1;                  // "moe_wide_few" = 0 / 2: its workgroups of four waves never / always
     uint32_t moe_wide_min = 8;                  // "moe_wide_min": fewest pairs per expert (on average) that take the GEMM
     uint32_t moe_depth = 0;                     // "moe_depth": items a loader of the streamed grouped kernels keeps unconfirmed (0 = as the dense launches)
 
@@ -2214,6 +2226,9 @@ int gllmq_init(gllmq_ctx **out, int device)
         for (int b = 0; b < 2 && rc == GLLMQ_OK; ++b) {
             snprintf(name, sizeof name, "gq_moe_mmf_%s%s", q == 3 ? "q8_0" : q == 2 ? "q6k" : q == 1 ? "q5k" : "q4k", b ? "_hi" : "");
             rc = get_function(ctx, &ctx->moe_mmf[q][b], name);
+            if (rc != GLLMQ_OK) break;
+            strncat(name, "_few", sizeof name - strlen(name) - 1);
+            rc = get_function(ctx, &ctx->moe_mmf_few[q][b], name);
         }
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfr[0][0], "gq_mmfr_q4k");
     if (rc == GLLMQ_OK) rc = get_function(ctx, &ctx->mmfr[0][1], "gq_mmfr_q4k_e16");
@@ -2459,6 +2474,7 @@ int gllmq_set_option(gllmq_ctx *ctx, const char *name, long value)
     else if (n == "moe_glu") ctx->moe_glu = value != 0;
     else if (n == "moe_streamed") ctx->moe_streamed = u;
     else if (n == "moe_wide") ctx->moe_wide = value != 0;
+    else if (n == "moe_wide_few") ctx->moe_wide_few = u;
     else if (n == "moe_wide_min") {
         ctx->moe_wide_min = std::max(1u, u);
         ctx->moe_wide_cost = false;
@@ -3426,6 +3442,20 @@ bool takes_moe_wide(const gllmq_ctx *ctx, uint32_t dtype_gu, uint32_t dtype_dn, 
     return aligned(x, 16) && pairs * ffn <= 0xFFFFFFFFull && tiles * groups * gq::MmfwImage<2>::bytes <= 0xFFFFFFFFull;
 }
 
+// Whether a launch over experts takes the workgroups of four waves (MMFW_EXPERTS_FEW); wgs: workgroups of eight waves it would have
+// at one job an expert.  170 drawn layers (8 to 128 experts of 1024 to 4096 x 512 to 2048, 6 to 512 pairs an expert), change of the call by one
+// launch's form: more than one workgroup a CU, up to 40 pairs an expert -2.1 % in the mean (128 experts of 4096 x 1536, top 8 of 256 tokens 496 us,
+// 473; Q5_K of two planes -0.2 %, single ones +6; above 40 pairs, jobs of three tiles and more, -0.6 and +7).  At most half a workgroup a CU, where
+// it fills the device: -2.9 % up to 40 pairs, with two planes -5.4 % up to 100 (8 experts of 4096 x 2048, 100 pairs each 160, 135), with one +1.9.
+// Between them the eight waves have a CU to themselves either way: +0.3 %.  By this rule 115 of the 170 calls change, 4 % shorter in the mean.
+bool moe_wide_few(const gllmq_ctx *ctx, int fmt, int planes, size_t wgs, size_t pairs, size_t experts)
+{
+    if (ctx->moe_wide_few != 1) return ctx->moe_wide_few == 2;
+    const size_t cus = ctx->num_cus;
+    if (2 * wgs <= cus) return pairs <= (planes == 2 ? 100u : 40u) * experts;
+    return wgs > cus && pairs <= 40 * experts && !(fmt == 1 && planes == 2);
+}
+
 int run_moe_wide(gllmq_ctx *ctx, const Format &fg, const void *gate, size_t gate_stride, const void *up, size_t up_stride, const Format &fd,
                  const void *down, size_t down_stride, const float *x, float *out, uint32_t elem, size_t tokens, size_t hidden, size_t ffn,
                  size_t experts, size_t top_k, const uint32_t *route_expert, const float *route_weight, const uint32_t *route_len,
@@ -3481,21 +3511,23 @@ int run_moe_wide(gllmq_ctx *ctx, const Format &fg, const void *gate, size_t gate
         P.blocks_per_split = Q.groups;
         P.jobs = plan.wide;
         P.counters = counters;
+        size_t wgs = 0;
+        for (int i = 0; i < count; ++i) wgs += (mats[i].n + gq::MMFW_TILE_ROWS - 1) / gq::MMFW_TILE_ROWS;
+        const bool few = moe_wide_few(ctx, fmt, hi ? 1 : 2, wgs * std::min(experts, pairs), pairs, experts);
+        const uint32_t waves = gq::mmfw_waves(few ? gq::MMFW_EXPERTS_FEW : gq::MMFW_EXPERTS), tile_rows = 32 * waves;
         for (int i = 0; i < count; ++i) {
             P.seg[i].w = mats[i].w;
             P.seg[i].y = mats[i].y;
             P.seg[i].n = static_cast<uint32_t>(mats[i].n);
             P.seg[i].tile0 = P.n_tiles;
             P.seg[i].expert_stride = strides[i];
-            P.n_tiles += static_cast<uint32_t>((mats[i].n + gq::MMFW_TILE_ROWS - 1) / gq::MMFW_TILE_ROWS);
+            P.n_tiles += static_cast<uint32_t>((mats[i].n + tile_rows - 1) / tile_rows);
         }
         P.max_jobs = W.max_jobs;
         P.run_tiles = 1;
         P.n_runs = P.n_tiles;
-        uint32_t lds = 0;
-        for (uint32_t mt = 1; mt <= static_cast<uint32_t>(gq::MMFW_MAX_MT); ++mt) lds = std::max(lds, mmfw_lds_bytes(fmt, hi ? 1 : 2, mt));
-        return launch(ctx, ctx->moe_mmf[fmt][hi ? 1 : 0], (W.max_jobs + 7u) / 8u * 8u * P.n_runs, gq::MMFW_WAVES * 64, lds, stream, &P,
-                      sizeof P, true);
+        return launch(ctx, (few ? ctx->moe_mmf_few : ctx->moe_mmf)[fmt][hi ? 1 : 0], (W.max_jobs + 7u) / 8u * 8u * P.n_runs, waves * 64,
+                      mmfw_grouped_lds(fmt, hi ? 1 : 2, few), stream, &P, sizeof P, true);
     };
     {
         gq::MmfwPrepParams Q{};

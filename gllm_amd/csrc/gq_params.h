@@ -399,6 +399,10 @@ constexpr uint32_t MMFR_RED_WAVE = 2u * 64u * 16u; // bytes of a tile's sums in 
 // lanes hold them (MmfwImage), the weight matrices of one launch share the activations.
 constexpr int MMFW_WAVES = 8;
 constexpr int MMFW_TILE_ROWS = 32 * MMFW_WAVES; // weight rows per workgroup
+// What a launch multiplies: activation tiles, experts' jobs, or experts' jobs of one and two tiles in workgroups of four waves, two a CU
+// (moe_wide_few).
+constexpr int MMFW_DENSE = 0, MMFW_EXPERTS = 1, MMFW_EXPERTS_FEW = 2;
+constexpr int mmfw_waves(int grouped) { return grouped == MMFW_EXPERTS_FEW ? MMFW_WAVES / 2 : MMFW_WAVES; }
 constexpr int MMFW_MAX_SEGS = 3;                // weight matrices of one launch
 constexpr int MMFW_MAX_MT = 4;
 constexpr bool mmfw_runs(int mt) { return mt <= 3; } // Q6_K, Q8_0: registers for sums of runs (MmfwParams::run_mask)
@@ -449,25 +453,27 @@ template <> struct MmfwFormat<3> { // half groups: 136 bytes a row
     static constexpr bool SUMS = false;
 };
 
-template <int FMT, int PL, int MT, bool LO_FIRST = false, bool OWN = false>
+template <int FMT, int PL, int MT, bool LO_FIRST = false, bool OWN = false, int NWAVES = MMFW_WAVES>
 struct MmfwShape {
     using F = MmfwFormat<FMT>;
+    static constexpr int WAVES = NWAVES;
+    static_assert(WAVES == MMFW_WAVES || MT <= 2, "workgroups of four waves: one and two tiles");
     static_assert(!LO_FIRST || mmfw_lo_first(FMT, PL, MT), "");
     static_assert(!OWN || MT == 1, "");
     // Activations move in chunks of UC units (32 elements of K) through a ring of R chunk slots in LDS.
-    static constexpr int UC = MT == 4 ? (PL == 2 ? 1 : 2) : MT == 3 ? (PL == 2 ? 2 : 4) : MT == 2 ? (PL == 2 ? 2 : 4) : (PL == 2 ? 4 : 8);
+    static constexpr int UC = (MT == 4 ? (PL == 2 ? 1 : 2) : MT == 3 ? (PL == 2 ? 2 : 4) : MT == 2 ? (PL == 2 ? 2 : 4) : (PL == 2 ? 4 : 8)) * WAVES / MMFW_WAVES;
     static constexpr int R = MT == 3 ? 3 : 4;
     static constexpr int C = 8 / UC;                   // chunks per block
     static constexpr int PIECES = MT * PL * 2 * UC;    // KiB per chunk
-    static constexpr int NA = OWN ? 0 : PIECES / MMFW_WAVES; // wave-loads per wave and chunk
-    static_assert(PIECES % MMFW_WAVES == 0, "every wave requests the same number of pieces");
+    static constexpr int NA = OWN ? 0 : PIECES / WAVES; // wave-loads per wave and chunk
+    static_assert(PIECES % WAVES == 0, "every wave requests the same number of pieces");
     static constexpr uint32_t CHUNK = PIECES * 1024u;
     static constexpr uint32_t TILE_CHUNK = 2u * UC * PL * 1024u; // a row tile's share: contiguous in its image
     static constexpr uint32_t extra = 0;               // [4][sums of MT tiles, inverse scales]
     static constexpr uint32_t EXTRA = ((F::SUMS ? MT : 0) + 1) * 1024u;
     static constexpr uint32_t SLOTS = OWN ? 8u : 4u;
     static constexpr uint32_t stage = SLOTS * EXTRA;
-    static constexpr uint32_t ring = stage + MMFW_WAVES * F::STAGE;
+    static constexpr uint32_t ring = stage + WAVES * F::STAGE;
     // OWN: the images of a slice's blocks are made here, all of them ahead of the first product, and take the ring's place
     // (eight places of sums and scales: more than blocks, the next one is read past the last)
     static constexpr int OWN_FIT = (160u * 1024u - ring) / (C * CHUNK), OWN_BLOCKS = OWN_FIT < 4 ? OWN_FIT : 4;
@@ -536,11 +542,18 @@ struct MmfwShape {
 //   Q8_0 64 rows 28672 x 4096, one plane        48.4, 50.6           (its rows' quants are off any alignment in LDS)
 // Q5_K against two planes keeps the parts: calls of 160 drawn shapes of 9 to 130 rows are level (in the mean up to 16 rows parts 0.5 %
 // shorter, above within 0.2 %; single ones 5 % either way).
-constexpr bool mmfw_units(int fmt, int planes, int mt) { return fmt == 2 ? mt <= 2 : fmt == 1 ? planes == 1 && mt == 1 : fmt == 0 && mt <= planes; }
-template <int FMT, int PL, int MT>
+// Experts, all of whose CUs stream weights at once, take units against two tiles of one plane as well (512 tokens, top 8 of 128 experts of
+// 4096 x 1536, the call: Q4_K 589 us, so 585, Q5_K 628, 619; with workgroups of four waves 581, 572 and 622, 605).
+constexpr bool mmfw_units(int fmt, int planes, int mt, int grouped)
+{
+    if (grouped && fmt <= 1 && planes == 1 && mt == 2) return true;
+    return fmt == 2 ? mt <= 2 : fmt == 1 ? planes == 1 && mt == 1 : fmt == 0 && mt <= planes;
+}
+template <int FMT, int PL, int MT, int NWAVES = MMFW_WAVES>
 struct MmfwUnitShape {
     using F = MmfwFormat<FMT>;
-    using W = MmfwShape<FMT, PL, MT>;
+    using W = MmfwShape<FMT, PL, MT, false, false, NWAVES>;
+    static constexpr int WAVES = NWAVES;
     static constexpr int UB = FMT <= 1 && PL == 1 ? 2 : 1;                            // blocks of K in a unit
     static constexpr uint32_t ROW = FMT == 2 ? 224u : UB * F::BLOCK;                  // bytes of a row in LDS (Q6_K: 208 and a window of 16 that ends with the block)
     static constexpr int ROW_PIECES = ROW / 16u;
@@ -550,7 +563,7 @@ struct MmfwUnitShape {
     static constexpr uint32_t CHUNK = W::CHUNK, TILE_CHUNK = W::TILE_CHUNK, EXTRA = W::EXTRA, extra = 0;
     static_assert(NA == 2 && TILE_CHUNK % (NA * 1024u) == 0, "a wave's pieces of a chunk are two neighbours");
     static constexpr uint32_t stage = 4u * EXTRA;
-    static constexpr uint32_t ring = stage + MMFW_WAVES * STAGE;
+    static constexpr uint32_t ring = stage + WAVES * STAGE;
     static constexpr uint32_t total = ring + R * CHUNK;
     static_assert(total <= 160u * 1024u, "LDS");
     static constexpr int SG = W::SG, NS = W::NS, SPC = W::SPC;
@@ -670,10 +683,24 @@ constexpr bool mmfw_may_run(int fmt, int planes, int mt, bool grouped) { return 
 template <int FMT, int PL> constexpr uint32_t mmfw_own_blocks() { return MmfwShape<FMT, PL, 1, false, true>::OWN_BLOCKS; }
 template <int FMT, int PL> constexpr uint32_t mmfw_own_lds() { return MmfwShape<FMT, PL, 1, false, true>::total; }
 
-template <int FMT, int PL, int MT> constexpr uint32_t mmfw_lds()
+template <int FMT, int PL, int MT, int GROUPED = MMFW_DENSE> constexpr uint32_t mmfw_lds()
 {
-    if constexpr (mmfw_units(FMT, PL, MT)) return MmfwUnitShape<FMT, PL, MT>::total > MmfwShape<FMT, PL, MT>::total ? MmfwUnitShape<FMT, PL, MT>::total : MmfwShape<FMT, PL, MT>::total;
-    else return MmfwShape<FMT, PL, MT>::total;
+    using W = MmfwShape<FMT, PL, MT, false, false, mmfw_waves(GROUPED)>;
+    using U = MmfwUnitShape<FMT, PL, MT, mmfw_waves(GROUPED)>;
+    if constexpr (mmfw_units(FMT, PL, MT, GROUPED)) return U::total > W::total ? U::total : W::total;
+    else return W::total;
+}
+// ... of a grouped launch, whose jobs have any number of tiles
+template <int FMT, int PL, int GROUPED> constexpr uint32_t mmfw_grouped_lds()
+{
+    constexpr uint32_t one = mmfw_lds<FMT, PL, 1, GROUPED>(), two = mmfw_lds<FMT, PL, 2, GROUPED>(), few = one > two ? one : two;
+    if constexpr (GROUPED == MMFW_EXPERTS_FEW) {
+        static_assert(few <= 80u * 1024u, "two workgroups a CU");
+        return few;
+    } else {
+        constexpr uint32_t three = mmfw_lds<FMT, PL, 3, GROUPED>(), four = mmfw_lds<FMT, PL, 4, GROUPED>(), many = three > four ? three : four;
+        return few > many ? few : many;
+    }
 }
 
 struct MmfwSeg {

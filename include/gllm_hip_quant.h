@@ -112,7 +112,7 @@ const char *gllmq_version(void);
  *     "mmfw_min_m", "mmfw_small_min_m", "mmfx_min_m", "moe_wide_min",
  *     "mm8_q5k_min_m", "mm8_q6k_min_m", "mm8_q8_0_min_m", "mmf_small_min_m", "mm8_ksplit",
  *     "mm8s_all", "mmfs_all" (1: that form wherever the shape fits it, also where another was timed faster)
- *   launch parameters: "mmfw_mt", "mmfw_ksplit", "mmfw_run", "mm8s_depth", "moe_depth", "moe_slices", "prefetch_wgs", "prefetch_threads",
+ *   launch parameters: "mmfw_mt", "mmfw_ksplit", "mmfw_run", "mm8s_depth", "moe_depth", "moe_slices", "moe_wide_few", "prefetch_wgs", "prefetch_threads",
  *     "prefetch_timeout_us", "prefetch_flags", "prefetch_announce", "prefetch_min_kib" */
 int gllmq_set_option(gllmq_ctx *ctx, const char *name, long value);
 /* Name of the kernel the context launched last ("" before the first launch): lets a profile be

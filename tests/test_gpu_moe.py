@@ -391,6 +391,34 @@ def test_jobs_of_every_number_of_tiles(hip, torch, oracle, counts):
         check_close(got[rows], want, f"expert {e} of {counts}")
 
 
+@pytest.mark.parametrize("t_gu, t_dn, hidden, ffn", [(Q4_K, Q6_K, 512, 384), (Q5_K, Q4_K, 768, 520), (Q6_K, Q5_K, 256, 2048), (8, 8, 288, 352)])
+@pytest.mark.parametrize("elem", ["float32", "bfloat16"])
+def test_workgroups_of_four_waves_give_the_bits_of_eight(torch, t_gu, t_dn, hidden, ffn, elem):
+    """Jobs of every number of tiles, matrices of whole and broken tiles of 128 rows, rows of one to nine blocks.  Four tiles of Q4_K and Q5_K in f32
+    add the products of the lo plane in another order there: both orders are within 2.5e-7 of the sum, and a down projection behind one another such."""
+    from gllm_amd.backend import HipBackend
+    counts = (0, 1, 31, 32, 33, 64, 65, 96, 97, 128, 129, 200)
+    experts, t = len(counts), getattr(torch, elem)
+    gu, dn = expert_weights(t_gu, t_dn, experts, hidden, ffn, seed=71)
+    re = np.random.default_rng(6).permutation(np.repeat(np.arange(experts), counts)).astype(np.int32)[:, None]
+    x = (torch.from_numpy(random_activations(len(re), hidden, seed=73)) * 1e-2).to(t).cuda()
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    args = dev(gu), dev(dn), dev(re), torch.ones(re.shape, device="cuda"), torch.ones(len(re), dtype=torch.int32, device="cuda")
+    outs = []
+    for form in (0, 2):
+        print(f"four waves {t_gu}/{t_dn} {hidden} x {ffn} {elem} form={form}", flush=True)
+        hip = HipBackend(0, options={"moe_wide_min": 1, "moe_wide_few": form})
+        out = torch.full((len(re), hidden), float("nan"), dtype=t, device="cuda")
+        hip.moe_matvec(args[0], t_gu, args[1], t_dn, x, out, hidden, ffn, experts, args[2], args[3], args[4])
+        torch.cuda.synchronize()
+        outs.append(out.float().cpu())
+    assert bool(torch.isfinite(outs[0]).all())
+    large = torch.from_numpy(np.isin(re[:, 0], [e for e, c in enumerate(counts) if c > 96]))
+    assert torch.equal(outs[0][~large], outs[1][~large])
+    bar = 1e-6 if elem == "float32" else 2.0 ** -8  # (bf16: a sum between two values may round either way)
+    assert float((outs[0] - outs[1])[large].norm()) <= bar * float(outs[0][large].norm())
+
+
 @pytest.mark.parametrize("hidden, top_k", [(256, 3), (260, 9), (1028, 8), (512, 2)])
 def test_combine_of_many_tokens_is_the_combine_of_few(torch, hidden, top_k):
     """From 128 tokens on a thread adds up four columns.  The same tokens with others behind them that are
