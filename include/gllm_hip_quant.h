@@ -244,10 +244,10 @@ int gllmq_reserve_matmul_elem(gllmq_ctx *ctx, uint32_t ggml_dtype, size_t m, siz
  * value_dev as in gllmq_argmax (one row).  logits_dev (n f32) receives the logits; it may be
  * NULL when only the token is wanted and the matrix is Q6_K or Q8_0 with k <= 16384: there
  * every workgroup of the matvec leaves its best candidate behind and the one that finishes last
- * picks among them (one launch), so the logits are neither written nor read again.  Other matrices run
- * gllmq_quantized_matmul and gllmq_argmax one after the other and need logits_dev, and so do
- * shapes with a logits buffer for which gllmq_quantized_matmul has a faster kernel than that
- * matvec (Q8_0 rows of whole 256-element groups, a few long Q6_K rows).  With logits_dev the
+ * picks among them (one launch), so the logits are neither written nor read again.  Other matrices need
+ * logits_dev.  With it, where gllmq_quantized_matmul takes the streamed kernel (Q4_K, Q5_K, Q8_0 rows of whole
+ * 256-element groups, short Q6_K rows) that kernel ends in the token, one launch too; what remains runs
+ * gllmq_quantized_matmul and gllmq_argmax one after the other.  With logits_dev the
  * logits and the token are those of the two calls made separately, bit for bit; without it the
  * token is the choice among that matvec's own logits, which agree with the other kernels' to the
  * matmul's tolerance. */
