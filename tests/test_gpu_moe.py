@@ -446,3 +446,49 @@ def test_combine_of_many_tokens_is_the_combine_of_few(torch, hidden, top_k):
         assert bool(outs[0].any())
         for got in outs[1:]:
             assert torch.equal(got[:few], outs[0]) and not bool(got[few:].any())
+
+
+@pytest.mark.parametrize("elem", ["float32", "float16"])
+@pytest.mark.parametrize("t_gu, t_dn, hidden, ffn, experts, top_k, tokens", [
+    (Q4_K, Q6_K, 1024, 512, 16, 4, 8),     # two pairs an expert
+    (Q4_K, Q4_K, 1280, 1024, 16, 2, 40),   # five
+    (Q5_K, Q6_K, 512, 512, 128, 8, 111),   # just under seven, as many experts as the measured line has
+    (Q5_K, Q6_K, 512, 512, 129, 8, 111),   # one more: the jobs' side below eight
+    (8, 8, 1024, 512, 64, 2, 33),          # Q8_0 from one pair on
+    (8, 8, 1024, 512, 160, 2, 320),        # Q8_0, more experts: at four
+])
+def test_layers_about_the_line_fit_what_is_reserved(torch, t_gu, t_dn, hidden, ffn, experts, top_k, tokens, elem):
+    """Few pairs an expert, on both sides of the line between the GEMM and the jobs: captured behind the reservation alone, replayed between
+    eager work, the bits of the eager call; GEMM and jobs are each within 1e-5 of the sums, and in f16 a rounding of 2^-11 apart from them besides."""
+    from gllm_amd.backend import HipBackend
+    t = getattr(torch, elem)
+    gu, dn = expert_weights(t_gu, t_dn, experts, hidden, ffn, seed=experts)
+    rng = np.random.default_rng(tokens)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    re = dev(np.stack([rng.permutation(experts)[:top_k] for _ in range(tokens)]).astype(np.int32))
+    args = (dev(gu), t_gu, dev(dn), t_dn, (torch.from_numpy(random_activations(tokens, hidden, seed=5)) * 1e-3).to(t).cuda())
+    route = (hidden, ffn, experts, re, torch.full(re.shape, 0.5, device="cuda"), torch.full((tokens,), top_k, dtype=torch.int32, device="cuda"))
+    outs = []
+    for options in ({}, {"moe_wide": 0}):
+        print(f"line {t_gu}/{t_dn} {experts} x {hidden} x {ffn} top {top_k} of {tokens} {elem} {options}", flush=True)
+        hip = HipBackend(0, options=options)
+        out = torch.full((tokens, hidden), float("nan"), dtype=t, device="cuda")
+        hip.moe_matvec(*args, out, *route)
+        torch.cuda.synchronize()
+        outs.append(out.float())
+    assert float((outs[0] - outs[1]).norm()) <= (2e-5 if elem == "float32" else 2.0 ** -10) * float(outs[1].norm())
+    if elem != "float32":
+        return
+    hip, out = HipBackend(0), torch.empty(tokens, hidden, device="cuda")
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        hip.reserve_moe(tokens, top_k, hidden, ffn)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        hip.moe_matvec(*args, out, *route)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, outs[0])
