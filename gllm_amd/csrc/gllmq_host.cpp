@@ -3415,8 +3415,8 @@ MoeWidePlan plan_moe_wide(size_t pairs, size_t hidden, size_t ffn, size_t expert
 constexpr size_t kMoeLineExperts = 128, kMoeLineHidden = 4096, kMoeLineFfn = 2048;
 
 // Whether the GEMM is ahead of jobs of eight tokens (of Q8_0, whose other form is the GEMV, of those).
-bool takes_moe_wide(const gllmq_ctx *ctx, uint32_t dtype_gu, uint32_t dtype_dn, const void *x, uint32_t elem, size_t hidden, size_t ffn, size_t experts,
-                    size_t pairs)
+// Without the element type: the two forms round differently, and a call of 16-bit elements gives the bits of the f32 call.
+bool takes_moe_wide(const gllmq_ctx *ctx, uint32_t dtype_gu, uint32_t dtype_dn, const void *x, size_t hidden, size_t ffn, size_t experts, size_t pairs)
 {
     const bool q8 = dtype_gu == T_Q8_0 || dtype_dn == T_Q8_0;
     if (!ctx->moe_wide || !ctx->use_mmf || !ctx->use_mmfw || ctx->moe_streamed == 2 || pairs < (q8 ? (ctx->moe_wide_min + 1) / 2 : ctx->moe_wide_min) * experts)
@@ -3424,17 +3424,17 @@ bool takes_moe_wide(const gllmq_ctx *ctx, uint32_t dtype_gu, uint32_t dtype_dn, 
     if ((dtype_gu == T_Q8_0 && hidden < 256) || (dtype_dn == T_Q8_0 && ffn < 256)) return false; // the Q8_0 window is a whole group
     if (ctx->moe_wide_cost) {
         // Few experts, or small ones, do not fill the device with one workgroup per 256 weight rows and all of K, which the
-        // int8 kernels do; those take time with every pair.  Estimates in us, fitted to 410 drawn layers in both forms (8 to 128 experts of 1024 to 4096 x
-        // 512 to 2048, 1.2 to 14 pairs an expert; within 8 and 14 %).  GEMM: a block of K 0.3 (Q5_K 0.6, Q6_K 1.1, Q8_0 1.6), 2 more with every
-        // CU busy and 0.6 for the second plane of gate and up, 4 for a workgroup's start and end, 22 for the launches beside the two.  The others: 31, 5.5 for 16-bit
-        // elements, the weights at 12 TB/s (whose pairs' time holds the rest of theirs), the products at 59 TFLOP/s (Q5_K 54, Q8_0 18).  A tenth in favour of
-        // the other form.  Below 8 pairs (4) calls of fewer than 32 pairs stay there (8 experts of 1024 x 512, 18 pairs: GEMM 31, jobs 27), and f32 rows
-        // of a device twice full (128 experts of 3584 x 512 Q5_K, 6 pairs an expert 223, 196; of 4096 x 1792 Q4_K, 4 pairs 604, 486).  Of 443 such layers, 200 of them not
-        // fitted to, 99 go to the GEMM, 22 % shorter in the mean and none slower by more than 1 %: 16 experts of 1792 x 1792, 6 pairs, Q4_K f16 78,
-        // so 55; 60 of 2048 x 768 Q5_K bf16, 7 pairs 118, 93.
+        // int8 kernels do; those take time with every pair.  Estimates in us of an f32 call, fitted to 410 drawn layers in both forms (8 to 128 experts of 1024
+        // to 4096 x 512 to 2048, 1.2 to 14 pairs an expert; within 8 and 14 %).  GEMM: a block of K 0.3 (Q5_K 0.6, Q6_K 1.1, Q8_0 1.6), 2 more with every
+        // CU busy and 0.6 for the second plane of gate and up, 4 for a workgroup's start and end, 22 for the launches beside the two.  The others: 31,
+        // the weights at 12 TB/s (whose pairs' time holds the rest of theirs), the products at 59 TFLOP/s (Q5_K 54, Q8_0 18).  A tenth in favour of
+        // the other form.  Below 8 pairs (4) calls of fewer than 32 pairs stay there (8 experts of 1024 x 512, 18 pairs: GEMM 31, jobs 27), and those
+        // of a device twice full (128 experts of 3584 x 512 Q5_K, 6 pairs an expert 223, 196; of 4096 x 1792 Q4_K, 4 pairs 604, 486).  A call of 16-bit elements
+        // has more of the GEMM (one plane of gate and up; the jobs' rows are converted) and follows the f32 call: by an estimate of its own the bf16 calls of
+        // 7385 layers of that range were 4.6 % shorter in the mean, and not the f32 call's results rounded.
         const size_t cus_whole = static_cast<size_t>(ctx->num_cus), gu_wgs = (2 * ffn + 255) / 256 * std::min(experts, pairs);
         if (pairs < (q8 ? 4u : 8u) * experts &&
-            (pairs < 32 || experts > kMoeLineExperts || hidden > kMoeLineHidden || ffn > kMoeLineFfn || (!elem && !q8 && gu_wgs >= 2 * cus_whole)))
+            (pairs < 32 || experts > kMoeLineExperts || hidden > kMoeLineHidden || ffn > kMoeLineFfn || (!q8 && gu_wgs >= 2 * cus_whole)))
             return false;
         const double e = static_cast<double>(std::min(experts, pairs)), cus = ctx->num_cus;
         auto launch_us = [&](uint32_t dtype, size_t rows, size_t k, double planes) {
@@ -3442,10 +3442,10 @@ bool takes_moe_wide(const gllmq_ctx *ctx, uint32_t dtype_gu, uint32_t dtype_dn, 
             const double block = (dtype == T_Q8_0 ? 1.6 : dtype == T_Q6_K ? 1.1 : dtype == T_Q5_K ? 0.6 : 0.3) + 2.0 * std::min(1.0, wgs / cus) + planes;
             return std::ceil(wgs / cus) * (static_cast<double>((k + 255) / 256) * block + 4.0);
         };
-        const double wide = 22.0 + launch_us(dtype_gu, 2 * ffn, hidden, elem ? 0.0 : 0.6) + launch_us(dtype_dn, hidden, ffn, 0.0);
+        const double wide = 22.0 + launch_us(dtype_gu, 2 * ffn, hidden, 0.6) + launch_us(dtype_dn, hidden, ffn, 0.0);
         const double bytes = e * (2.0 * ffn * gllmq_row_bytes(dtype_gu, hidden) + static_cast<double>(hidden) * gllmq_row_bytes(dtype_dn, ffn));
         const double rate = q8 ? 18e6 : dtype_gu == T_Q5_K || dtype_dn == T_Q5_K ? 54e6 : 59e6;
-        if (1.1 * wide > (elem ? 36.5 : 31.0) + bytes / 12e6 + 6.0 * pairs * static_cast<double>(hidden) * ffn / rate) return false;
+        if (1.1 * wide > 31.0 + bytes / 12e6 + 6.0 * pairs * static_cast<double>(hidden) * ffn / rate) return false;
     }
     const size_t tiles = pairs / 32 + std::min(experts, pairs), groups = std::max((hidden + 255) / 256, (ffn + 255) / 256);
     return aligned(x, 16) && pairs * ffn <= 0xFFFFFFFFull && tiles * groups * gq::MmfwImage<2>::bytes <= 0xFFFFFFFFull;
@@ -3614,7 +3614,7 @@ int moe_on_stream(gllmq_ctx *ctx, const void *gate, size_t gate_bytes, size_t ga
     if (!aligned(x, 16) || !aligned(out, 4))
         return fail(ctx, GLLMQ_ERR_BAD_ALIGNMENT, "moe_matvec: x must be 16-byte and out 4-byte aligned");
 
-    if (takes_moe_wide(ctx, dtype_gu, dtype_dn, x, elem, hidden, ffn, experts, pairs))
+    if (takes_moe_wide(ctx, dtype_gu, dtype_dn, x, hidden, ffn, experts, pairs))
         return run_moe_wide(ctx, *fg, gate, gate_expert_stride, up, up_expert_stride, *fd, down, down_expert_stride, x, out, elem, tokens,
                             hidden, ffn, experts, top_k, route_expert, route_weight, route_len, relu_gate, stream);
     if (elem) return kNeedPlainActivations;

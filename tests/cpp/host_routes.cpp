@@ -169,6 +169,23 @@ int batch(gllmq_ctx *ctx, uint32_t dtype, size_t m, const std::vector<size_t> &n
     return gllmq_quantized_matmul_batch(ctx, descs.data(), descs.size(), nullptr);
 }
 
+// experts' matrices in one stack a role
+int moe(gllmq_ctx *ctx, uint32_t gate_up, uint32_t down, size_t tokens, size_t top_k, size_t hidden, size_t ffn, size_t experts, int elem = GLLMQ_ELEM_F32, int flags = 0)
+{
+    fake::launches.clear();
+    const size_t one = ffn * gllmq_row_bytes(gate_up, hidden), dn = hidden * gllmq_row_bytes(down, ffn);
+    uint8_t *const w = static_cast<uint8_t *>(at(1));
+    return gllmq_moe_matvec_elem(ctx, w, (2 * experts - 1) * one, 2 * one, w + one, (2 * experts - 1) * one, 2 * one, gate_up, at(3), experts * dn, dn, down, at(4), at(5), tokens, hidden,
+                                 ffn, experts, top_k, static_cast<const uint32_t *>(at(6)), static_cast<const float *>(at(7)), static_cast<const uint32_t *>(at(8)), 0, elem, flags, nullptr);
+}
+// ... its products were the GEMM's
+bool moe_gemm()
+{
+    for (const fake::Launch &l : fake::launches)
+        if (l.kernel.find("gq_moe_mmf_") == 0) return true;
+    return false;
+}
+
 // the wide GEMM among the launches, if it is there
 const fake::Launch *wide_launch()
 {
@@ -339,6 +356,32 @@ void elements_take_the_f32_kernels()
                 }
 }
 
+// Experts' calls of 16-bit elements, with and without accumulation, take the f32 call's form, and so its bits, on both sides of every line
+// between the GEMM and the jobs.
+void elements_take_the_f32_experts()
+{
+    Context ctx;
+    size_t gemms = 0, jobs = 0;
+    for (const auto &mix : kMixes)
+        for (size_t experts : { 8u, 16u, 60u, 128u, 160u })
+            for (size_t top_k : { 2u, 8u })
+                for (const auto &layer : std::vector<std::vector<size_t>>{ { 1024, 512 }, { 1280, 768 }, { 2048, 1024 }, { 4096, 1536 }, { 4096, 2048 }, { 5120, 1536 }, { 4096, 14336 } })
+                    for (size_t pairs = experts; pairs <= 16 * experts && pairs <= 4096; pairs += std::max(experts, top_k)) {
+                        const size_t tokens = pairs / top_k;
+                        if (tokens == 0) continue;
+                        EXPECT(moe(ctx, mix[0], mix[1], tokens, top_k, layer[0], layer[1], experts) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+                        const bool f32 = moe_gemm();
+                        (f32 ? gemms : jobs)++;
+                        for (int elem : { GLLMQ_ELEM_F32, GLLMQ_ELEM_F16, GLLMQ_ELEM_BF16 })
+                            for (int flags : { 0, int(GLLMQ_OUT_ACCUMULATE) }) {
+                                EXPECT(moe(ctx, mix[0], mix[1], tokens, top_k, layer[0], layer[1], experts, elem, flags) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+                                EXPECT(moe_gemm() == f32, "formats %u/%u, %zu tokens, top %zu of %zu experts of %zu x %zu, element type %d, flags %d: GEMM %d, f32 %d", mix[0], mix[1], tokens,
+                                       top_k, experts, layer[0], layer[1], elem, flags, !f32, f32);
+                            }
+                    }
+    EXPECT(gemms > 200 && jobs > 200, "%zu calls on the GEMM, %zu on the jobs", gemms, jobs);
+}
+
 // Scratch that a captured call has used stays, whatever eager calls of more rows, and calls on many other streams, do afterwards;
 // what no graph can hold is given back as it is outgrown, and everything with the context.
 void scratch_of_graphs_stays()
@@ -445,6 +488,7 @@ const std::map<std::string, std::function<void()>> kChecks = {
     { "decoded_weights_scratch", decoded_weights_scratch },
     { "scratch_of_graphs_stays", scratch_of_graphs_stays },
     { "elements_take_the_f32_kernels", elements_take_the_f32_kernels },
+    { "elements_take_the_f32_experts", elements_take_the_f32_experts },
     { "runs_of_weight_tiles", runs_of_weight_tiles },
     { "outputs_over_the_activations", outputs_over_the_activations },
     { "own_images", own_images },

@@ -120,6 +120,44 @@ def test_expert_matvec(hip, torch, oracle, elem, accumulate):
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("elem", [F16, BF16])
+@pytest.mark.parametrize("t_gu, t_dn, hidden, ffn, experts, top_k, tokens", [
+    (Q4_K, Q6_K, 1024, 512, 8, 2, 16),    # jobs of eight tokens, where a 16-bit call by itself would be ahead on the GEMM
+    (Q5_K, Q6_K, 1280, 768, 16, 4, 24),   # ... six pairs an expert
+    (Q4_K, Q4_K, 1792, 1024, 16, 4, 28),  # seven
+    (Q8_0, Q8_0, 1024, 512, 16, 2, 33),   # Q8_0: four
+    (Q4_K, Q4_K, 512, 384, 8, 2, 400),    # the GEMM: two planes in workgroups of four waves, one plane in those of eight, jobs of four tiles
+    (Q5_K, Q5_K, 512, 384, 8, 2, 400),
+    (Q6_K, Q6_K, 512, 384, 8, 2, 130),
+])
+def test_expert_calls_about_the_lines(hip, torch, oracle, t_gu, t_dn, hidden, ffn, experts, top_k, tokens, elem):
+    """Whichever form the layer takes, 16-bit elements give the f32 call's results, rounded; added to an output too."""
+    print(f"moe line elem={elem} {t_gu}/{t_dn} {experts} x {hidden} x {ffn} top {top_k} of {tokens}", flush=True)
+    gu = np.concatenate([np.asarray(random_weight(t_gu, 2 * ffn, hidden, seed=140 + e)).view(np.uint8).reshape(-1) for e in range(experts)])
+    dn = np.concatenate([np.asarray(random_weight(t_dn, hidden, ffn, seed=160 + e)).view(np.uint8).reshape(-1) for e in range(experts)])
+    gud, dnd = dev_bytes(torch, gu), dev_bytes(torch, dn)
+    x32 = representable(random_activations(tokens, hidden, seed=141) * 2.0 ** -7, elem)
+    old32 = representable(random_activations(tokens, hidden, seed=143), elem)
+    logits = torch.from_numpy(random_gate_logits(tokens, experts, seed=142)).cuda()
+    re_ = torch.empty(tokens, top_k, dtype=torch.int32, device="cuda")
+    rw = torch.empty(tokens, top_k, device="cuda")
+    rl = torch.empty(tokens, dtype=torch.int32, device="cuda")
+    hip.moe_route(logits, top_k, re_, rw, rl, capacity_factor=float(experts))
+    xf, rf = to_dev(torch, x32, None), torch.full((tokens, hidden), float("nan"), device="cuda")
+    hip.moe_matvec(gud, t_gu, dnd, t_dn, xf, rf, hidden, ffn, experts, re_, rw, rl)
+    torch.cuda.synchronize()
+    result32 = rf.cpu().numpy()
+    few = min(tokens, 40)
+    check_close(result32[:few], oracle.moe_ffn(gu, t_gu, dn, t_dn, x32[:few], hidden, ffn, experts, re_[:few].cpu().numpy().astype(np.uint32), rw[:few].cpu().numpy(),
+                                               rl[:few].cpu().numpy().astype(np.uint32)), "the f32 expert matvec")
+    for accumulate in (False, True):
+        xe, oe = to_dev(torch, x32, elem), to_dev(torch, old32, elem)
+        hip.moe_matvec(gud, t_gu, dnd, t_dn, xe, oe, hidden, ffn, experts, re_, rw, rl, accumulate=accumulate)
+        torch.cuda.synchronize()
+        got, want = as_f32(torch, oe), expected(result32, old32, elem, accumulate)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), f"accumulate={accumulate}"
+
+
 def test_shared_expert_on_top_of_routed_experts_and_residual(hip, torch, oracle):
     """The layer's sequence (build_graph.inc.rs:2076-2170): routed experts into the accumulator, the
     shared expert's block added to it, the sum added to the residual stream; against numpy adds of
