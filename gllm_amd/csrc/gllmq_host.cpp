@@ -849,11 +849,11 @@ int run_mm8s(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
         // 12.2 (13.0), 128256 42 (40); 1024 -> 14336 5.9 (6.5), 28672 8.9 (8.7)).  A wave of the GEMV takes 4096 elements of K, and where all its lanes
         // are at work it is ahead: rows of 4096, rows of 8192 over more than 56 weight rows per CU (14336 20.3 (21.8), 128256 153 (145)), and over more
         // than 64 also rows that fill all but a part of a block of it (3968 -> 8192 7.0 (7.6), 32000 22.7 (22.3), 64000 44.6 (40.8); 8064 -> 16384
-        // 22.3 (23.9), 64000 82 (78)).  Rows of 14 and 15 blocks leave few of its lanes idle: ahead over more than 100 weight rows per CU (3584 -> 16384
-        // 11.4 (11.7), 32000 21.2 (20.4), 64000 40.7 (36.3), 128256 74.1 (69.2); 3840 -> 32000 22.5 (21.2), 128256 78.3 (74.1); 3328 68.3 (68.7)).
+        // 22.3 (23.9), 64000 82 (78)).  Rows of 14 and 15 blocks stay here, also where it is ahead (3584 -> 128256 74.1 (69.2)): its activations have a
+        // bit less and its offset comes off in f32, for nearly twice the error (3584 normal activations 1.6e-7, 2.9e-7).
         if (kind == MM8_Q6K && mm == 1 && groups < 40 && !(fold && groups >= 20)) {
             const size_t rows = (n + cus - 1) / cus;
-            const size_t most = k % 4096 == 0 ? (groups == 16 ? 0u : 56u) : groups % 16 == 0 ? 64u : groups <= 8 ? 16u * groups : groups == 14 || groups == 15 ? 100u : SIZE_MAX;
+            const size_t most = k % 4096 == 0 ? (groups == 16 ? 0u : 56u) : groups % 16 == 0 ? 64u : groups <= 8 ? 16u * groups : SIZE_MAX;
             if (rows > most || (groups > 16 && rows <= 24)) return -1;
         }
         // Q8_0, two rows over at most 8 weight rows per CU: its GEMV stays ahead (4096 -> 1024: 5.9 against 7.1 us)

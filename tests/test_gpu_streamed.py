@@ -254,3 +254,25 @@ def test_default_choice_at_its_lines(torch, dtype, m, rows, k, form):
 def test_default_choice_at_more_lines(torch, dtype, m, rows, k, form):
     """... rows of K that almost fill the GEMV's waves, and two rows that share K among workgroups."""
     test_default_choice_at_its_lines(torch, dtype, m, rows, k, form)
+
+
+@pytest.mark.parametrize("n, k", [(32000, 3584), (25601, 3840), (33000, 3584 - 8), (128256, 3840)])
+def test_long_columns_of_q6_k_keep_the_streamed_kernels_bits(torch, n, k):
+    """One row of 14 and 15 blocks over more than 100 weight rows per CU: the error against 64 bits is no larger than in the streamed kernel (both are
+    root mean squares over n outputs of one activation row, which differ by less than 3 % between draws), and so with the greedy token behind it."""
+    from gllm_amd.backend import HipBackend
+    w = torch.from_numpy(random_weight(Q6_K, n, k, seed=n).view(np.uint8).reshape(-1)).cuda()
+    x = torch.from_numpy(random_activations(1, k, seed=k)).cuda()
+    deq = torch.zeros(n, -(-k // 256) * 256, device="cuda")
+    HipBackend(0).dequantize(w, deq, Q6_K)
+    want = deq[:, :k].double() @ x.double()[0]
+    found = []
+    for options in ({"mm8s_all": 1}, {}):
+        for token in (False, True):
+            print(f"long columns {n} x {k} {options} token={token}", flush=True)
+            hip, y, tok = HipBackend(0, options=options), torch.full((1, n), float("nan"), device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+            if token: hip.lm_head_argmax(w, x, Q6_K, n, k, tok, logits=y[0])
+            else: hip.quantized_matmul(w, x, y, Q6_K, 1, n, k)
+            found.append(float((y[0].double() - want).norm() / want.norm()))
+    print(f"errors {[f'{e:.2e}' for e in found]}", flush=True)
+    assert max(found) <= 1.03 * found[0]
