@@ -3411,16 +3411,18 @@ MoeWidePlan plan_moe_wide(size_t pairs, size_t hidden, size_t ffn, size_t expert
     return W;
 }
 
+constexpr size_t kMoeMaxExperts = 4096; // of a call
+
 // Layers whose line between the two forms was measured below 8 pairs an expert (Q8_0: 4); others have it there.
 constexpr size_t kMoeLineExperts = 128, kMoeLineHidden = 4096, kMoeLineFfn = 2048;
 
 // Whether the GEMM is ahead of jobs of eight tokens (of Q8_0, whose other form is the GEMV, of those).
-// Without the element type: the two forms round differently, and a call of 16-bit elements gives the bits of the f32 call.
-bool takes_moe_wide(const gllmq_ctx *ctx, uint32_t dtype_gu, uint32_t dtype_dn, const void *x, size_t hidden, size_t ffn, size_t experts, size_t pairs)
+// Without the element type: the two forms round differently, and a call of 16-bit elements gives the bits of the f32 call.  A call that has it
+// ahead has it so with more pairs too (moe_wide_reserve).
+bool moe_wide_ahead(const gllmq_ctx *ctx, uint32_t dtype_gu, uint32_t dtype_dn, size_t hidden, size_t ffn, size_t experts, size_t pairs)
 {
     const bool q8 = dtype_gu == T_Q8_0 || dtype_dn == T_Q8_0;
-    if (!ctx->moe_wide || !ctx->use_mmf || !ctx->use_mmfw || ctx->moe_streamed == 2 || pairs < (q8 ? (ctx->moe_wide_min + 1) / 2 : ctx->moe_wide_min) * experts)
-        return false;
+    if (pairs < (q8 ? (ctx->moe_wide_min + 1) / 2 : ctx->moe_wide_min) * experts) return false;
     if ((dtype_gu == T_Q8_0 && hidden < 256) || (dtype_dn == T_Q8_0 && ffn < 256)) return false; // the Q8_0 window is a whole group
     if (ctx->moe_wide_cost) {
         // Few experts, or small ones, do not fill the device with one workgroup per 256 weight rows and all of K, which the
@@ -3447,8 +3449,24 @@ bool takes_moe_wide(const gllmq_ctx *ctx, uint32_t dtype_gu, uint32_t dtype_dn, 
         const double rate = q8 ? 18e6 : dtype_gu == T_Q5_K || dtype_dn == T_Q5_K ? 54e6 : 59e6;
         if (1.1 * wide > 31.0 + bytes / 12e6 + 6.0 * pairs * static_cast<double>(hidden) * ffn / rate) return false;
     }
+    return true;
+}
+
+bool takes_moe_wide(const gllmq_ctx *ctx, uint32_t dtype_gu, uint32_t dtype_dn, const void *x, size_t hidden, size_t ffn, size_t experts, size_t pairs)
+{
+    if (!ctx->moe_wide || !ctx->use_mmf || !ctx->use_mmfw || ctx->moe_streamed == 2 || !moe_wide_ahead(ctx, dtype_gu, dtype_dn, hidden, ffn, experts, pairs)) return false;
     const size_t tiles = pairs / 32 + std::min(experts, pairs), groups = std::max((hidden + 255) / 256, (ffn + 255) / 256);
     return aligned(x, 16) && pairs * ffn <= 0xFFFFFFFFull && tiles * groups * gq::MmfwImage<2>::bytes <= 0xFFFFFFFFull;
+}
+
+// Scratch for any call of that many pairs or fewer: the GEMM takes the more the more experts, so that of the most, in any formats, which take it.
+size_t moe_wide_reserve(const gllmq_ctx *ctx, size_t pairs, size_t hidden, size_t ffn)
+{
+    for (size_t experts = std::min<size_t>(kMoeMaxExperts, pairs / ((ctx->moe_wide_min + 1) / 2)); experts > 0; --experts)
+        for (const Format &gu : kFormats)
+            for (const Format &dn : kFormats)
+                if (moe_wide_ahead(ctx, gu.dtype, dn.dtype, hidden, ffn, experts, pairs)) return plan_moe_wide(pairs, hidden, ffn, experts, false).total;
+    return 0;
 }
 
 // Whether a launch over experts takes the workgroups of four waves (MMFW_EXPERTS_FEW); wgs: workgroups of eight waves it would have
@@ -3586,7 +3604,7 @@ int moe_on_stream(gllmq_ctx *ctx, const void *gate, size_t gate_bytes, size_t ga
     const size_t pairs = tokens * top_k;
     // The plan kernel keeps the pair list and three words per expert in LDS, and a launch
     // covers at most 16384 elements of K.
-    if (pairs > 16384 || experts > 4096)
+    if (pairs > 16384 || experts > kMoeMaxExperts)
         return fail(ctx, GLLMQ_ERR_UNIMPLEMENTED,
                     "moe_matvec: tokens*top_k = %zu (max 16384) or experts = %zu (max 4096) is beyond this build", pairs,
                     experts);
@@ -3922,11 +3940,7 @@ int gllmq_reserve_moe(gllmq_ctx *ctx, size_t tokens, size_t top_k, size_t hidden
     Scratch *S = nullptr;
     int rc = acquire_scratch(ctx, stream, &S);
     if (rc != GLLMQ_OK || tokens == 0 || top_k == 0) return rc;
-    // (the GEMM form is for calls with at least moe_wide_min pairs per expert, half as many of Q8_0, and takes the more the more experts;
-    // takes_moe_wide has more experts than kMoeLineExperts go there from 8 and 4)
-    const size_t pairs = tokens * top_k, any = 2 * pairs / ctx->moe_wide_min;
-    const size_t most_experts = std::max<size_t>(1, ctx->moe_wide_cost ? std::max(std::min(any, kMoeLineExperts), pairs / 4) : any);
-    const size_t need = std::max(moe_workspace(pairs, hidden, ffn).total, plan_moe_wide(pairs, hidden, ffn, most_experts, false).total);
+    const size_t pairs = tokens * top_k, need = std::max(moe_workspace(pairs, hidden, ffn).total, moe_wide_reserve(ctx, pairs, hidden, ffn));
     return grow_scratch(ctx, *S, &S->moe, &S->moe_bytes, need, stream, "reserve_moe");
 }
 

@@ -5,6 +5,7 @@
 #define GLLMQ_EMBED(NAME) extern "C" const unsigned char gllmq_co_##NAME[1] = { 0 };
 #include "../../gllm_amd/csrc/gllmq_host.cpp"
 
+#include <array>
 #include <functional>
 #include <map>
 #include <set>
@@ -382,6 +383,43 @@ void elements_take_the_f32_experts()
     EXPECT(gemms > 200 && jobs > 200, "%zu calls on the GEMM, %zu on the jobs", gemms, jobs);
 }
 
+// What is reserved for experts is what the calls of so many pairs need, in any formats and over any number of experts, and no more; a
+// captured call of as many or fewer pairs finds it.
+void experts_scratch_is_reserved()
+{
+    const auto held = [](const gllmq_ctx *) {
+        size_t bytes = 0;
+        for (const auto &b : fake::live) bytes += b.second;
+        return bytes;
+    };
+    std::vector<std::array<uint32_t, 2>> mixes;
+    for (const auto &gu : kFormats)
+        for (const auto &dn : kFormats) mixes.push_back({ gu.dtype, dn.dtype });
+    for (const auto &layer : std::vector<std::vector<size_t>>{ { 1024, 512 }, { 2048, 1024 }, { 4096, 1536 }, { 4096, 14336 }, { 5120, 13824 }, { 7168, 2048 } })
+        for (const auto &call : std::vector<std::vector<size_t>>{ { 1, 8 }, { 16, 2 }, { 16, 8 }, { 64, 2 }, { 128, 4 }, { 100, 6 } }) {
+            const size_t tokens = call[0], top_k = call[1], pairs = tokens * top_k;
+            Context used, reserved;
+            const size_t nothing = held(used);
+            std::vector<size_t> counts;
+            for (size_t e = 1; e <= pairs; e += 1 + e / 24) counts.push_back(e);
+            for (size_t e = 8; e <= pairs; e += 8) counts.push_back(e);
+            counts.push_back(pairs);
+            for (size_t experts : counts)
+                for (const auto &mix : mixes) EXPECT(moe(used, mix[0], mix[1], tokens, top_k, layer[0], layer[1], experts) == GLLMQ_OK, "%s", gllmq_last_error(used));
+            const size_t needed = held(used) - nothing;
+            EXPECT(gllmq_reserve_moe(reserved, tokens, top_k, layer[0], layer[1], nullptr) == GLLMQ_OK, "%s", gllmq_last_error(reserved));
+            const size_t taken = held(reserved) - nothing - needed;
+            // (a count of experts between the tried ones may take it: 4 % more at most)
+            EXPECT(taken >= needed && taken <= needed + needed / 25, "%zu tokens, top %zu, %zu x %zu: %zu bytes, calls need %zu", tokens, top_k, layer[0], layer[1], taken, needed);
+            fake::capturing = true;
+            for (size_t t = tokens; t > 0; t = t * 3 / 4)
+                for (size_t experts : counts)
+                    for (const auto &mix : mixes)
+                        EXPECT(moe(reserved, mix[0], mix[1], t, top_k, layer[0], layer[1], experts) == GLLMQ_OK, "%zu tokens behind %zu: %s", t, tokens, gllmq_last_error(reserved));
+            fake::capturing = false;
+        }
+}
+
 // Scratch that a captured call has used stays, whatever eager calls of more rows, and calls on many other streams, do afterwards;
 // what no graph can hold is given back as it is outgrown, and everything with the context.
 void scratch_of_graphs_stays()
@@ -489,6 +527,7 @@ const std::map<std::string, std::function<void()>> kChecks = {
     { "scratch_of_graphs_stays", scratch_of_graphs_stays },
     { "elements_take_the_f32_kernels", elements_take_the_f32_kernels },
     { "elements_take_the_f32_experts", elements_take_the_f32_experts },
+    { "experts_scratch_is_reserved", experts_scratch_is_reserved },
     { "runs_of_weight_tiles", runs_of_weight_tiles },
     { "outputs_over_the_activations", outputs_over_the_activations },
     { "own_images", own_images },
