@@ -383,6 +383,39 @@ void elements_take_the_f32_experts()
     EXPECT(gemms > 200 && jobs > 200, "%zu calls on the GEMM, %zu on the jobs", gemms, jobs);
 }
 
+// A layer that is an eighth larger, in any direction, has its line between the jobs and the GEMM where the layer itself has it, to a pair an
+// expert (where the GEMM's workgroups go round the device as often, by which its time is estimated).
+void experts_line_has_no_edges()
+{
+    Context ctx;
+    const auto line = [&](const uint32_t *mix, size_t hidden, size_t ffn, size_t experts) {
+        size_t per = 1;
+        for (; per < 16; ++per) {
+            EXPECT(moe(ctx, mix[0], mix[1], per * experts / 2, 2, hidden, ffn, experts) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+            if (moe_gemm()) break;
+        }
+        return per;
+    };
+    const auto rounds = [](size_t rows, size_t experts) { return ((rows + 255) / 256 * experts + 255) / 256; };
+    const auto full = [](size_t ffn, size_t experts) { return (2 * ffn + 255) / 256 * experts >= 512; };
+    size_t compared = 0, below = 0;
+    for (const auto &mix : kMixes)
+        for (size_t hidden : { 1024u, 2048u, 2560u, 4096u, 5120u, 7168u })
+            for (size_t ffn : { 512u, 1024u, 1792u, 2048u, 4096u, 8192u })
+                for (size_t experts : { 8u, 16u, 32u, 64u, 128u, 256u })
+                    for (int way = 0; way < 3; ++way) {
+                        const size_t h = hidden + (way == 0 ? hidden / 8 : 0), f = ffn + (way == 1 ? ffn / 8 : 0), e = experts + (way == 2 ? experts / 8 : 0);
+                        if (rounds(2 * ffn, experts) != rounds(2 * f, e) || rounds(hidden, experts) != rounds(h, e) || full(ffn, experts) != full(f, e)) continue;
+                        const size_t at = line(mix, hidden, ffn, experts), larger = line(mix, h, f, e);
+                        if (std::min(at, larger) > 8) continue; // (few small experts: a pair is little of the jobs' time)
+                        EXPECT(at <= larger + 1 && larger <= at + 1, "formats %u/%u: %zu experts of %zu x %zu from %zu pairs on, %zu of %zu x %zu from %zu", mix[0], mix[1], experts, hidden, ffn,
+                               at, e, h, f, larger);
+                        ++compared;
+                        below += at < 8;
+                    }
+    EXPECT(compared > 200 && below > 100, "%zu layers, %zu below eight pairs", compared, below);
+}
+
 // What is reserved for experts is what the calls of so many pairs need, in any formats and over any number of experts, and no more; a
 // captured call of as many or fewer pairs finds it.
 void experts_scratch_is_reserved()
@@ -527,6 +560,7 @@ const std::map<std::string, std::function<void()>> kChecks = {
     { "scratch_of_graphs_stays", scratch_of_graphs_stays },
     { "elements_take_the_f32_kernels", elements_take_the_f32_kernels },
     { "elements_take_the_f32_experts", elements_take_the_f32_experts },
+    { "experts_line_has_no_edges", experts_line_has_no_edges },
     { "experts_scratch_is_reserved", experts_scratch_is_reserved },
     { "runs_of_weight_tiles", runs_of_weight_tiles },
     { "outputs_over_the_activations", outputs_over_the_activations },
