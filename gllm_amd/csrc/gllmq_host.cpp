@@ -3427,17 +3427,16 @@ bool moe_wide_ahead(const gllmq_ctx *ctx, uint32_t dtype_gu, uint32_t dtype_dn, 
         // to 4096 x 512 to 2048, 1.2 to 14 pairs an expert; within 8 and 14 %).  GEMM: a block of K 0.3 (Q5_K 0.6, Q6_K 1.1, Q8_0 1.6), 2 more with every
         // CU busy and 0.6 for the second plane of gate and up, 4 for a workgroup's start and end, 22 for the launches beside the two.  The others: 31,
         // the weights at 12 TB/s (whose pairs' time holds the rest of theirs), the products at 59 TFLOP/s (Q5_K 54, Q8_0 18).  A tenth in favour of
-        // the other form.  Below 8 pairs (4) calls of fewer than 32 pairs stay there (8 experts of 1024 x 512, 18 pairs: GEMM 31, jobs 27), and those
-        // of a device twice full (128 experts of 3584 x 512 Q5_K, 6 pairs an expert 223, 196; of 4096 x 1792 Q4_K, 4 pairs 604, 486).  A call of 16-bit elements
-        // has more of the GEMM (one plane of gate and up; the jobs' rows are converted) and follows the f32 call: by an estimate of its own the bf16 calls of
-        // 7385 layers of that range were 4.6 % shorter in the mean, and not the f32 call's results rounded.
-        // Layers of other sizes (1882 drawn ones: 8 to 384 experts of 1024 to 8192 x 512 to 14336, 1.2 to 32 pairs) have the same line: with eight pairs (four)
-        // 74 of 865 go to the GEMM that the estimate before left to the jobs, f32 50 % shorter in the mean, none slower by more than 2 %; below 53 of
-        // 1017, 37 % shorter, one slower by 4 %.
+        // the other form.  Below 8 pairs an expert (Q8_0: 4) calls of fewer than 32 pairs stay there (8 experts of 1024 x 512, 18 pairs: GEMM 31, jobs 27),
+        // and K-quants whose gate and up fill the device twice (128 experts of 3584 x 512 Q5_K, 6 pairs an expert 223, 196; of 4096 x 1792 Q4_K, 4 pairs 604, 486);
+        // from two thirds of the CUs on 15 % in favour of the other form (16 experts of 3840 x 2048 Q4_K, 72 pairs, GEMM 104.5, jobs 91.4).
+        // By this 400 of 2303 other layers of that range with eight pairs (four) and more go to the GEMM that the estimate before left to the other form, f32
+        // 30 % shorter in the mean, and 411 of 5082 with fewer, 24 %, seven of them slower by 2 to 6 %; of larger layers (to 384 experts,
+        // 8192 and 14336) 74 of 865, 50 %, and 48 of 1017, 37 %, one slower by 1 %.  A call of 16-bit elements has more of the GEMM (one plane of gate and up; the jobs'
+        // rows are converted) and follows the f32 call: by an estimate of its own bf16 calls were 4.6 % shorter in the mean, and not the f32 call's results rounded.
         const size_t cus_whole = static_cast<size_t>(ctx->num_cus), gu_wgs = (2 * ffn + 255) / 256 * std::min(experts, pairs);
-        if (pairs < (q8 ? 4u : 8u) * experts &&
-            (pairs < 32 || (!q8 && gu_wgs >= 2 * cus_whole)))
-            return false;
+        const bool few = pairs < (q8 ? 4u : 8u) * experts;
+        if (few && (pairs < 32 || (!q8 && gu_wgs >= 2 * cus_whole))) return false;
         const double e = static_cast<double>(std::min(experts, pairs)), cus = ctx->num_cus;
         auto launch_us = [&](uint32_t dtype, size_t rows, size_t k, double planes) {
             const double wgs = std::ceil(rows / 256.0) * e;
@@ -3447,7 +3446,7 @@ bool moe_wide_ahead(const gllmq_ctx *ctx, uint32_t dtype_gu, uint32_t dtype_dn, 
         const double wide = 22.0 + launch_us(dtype_gu, 2 * ffn, hidden, 0.6) + launch_us(dtype_dn, hidden, ffn, 0.0);
         const double bytes = e * (2.0 * ffn * gllmq_row_bytes(dtype_gu, hidden) + static_cast<double>(hidden) * gllmq_row_bytes(dtype_dn, ffn));
         const double rate = q8 ? 18e6 : dtype_gu == T_Q5_K || dtype_dn == T_Q5_K ? 54e6 : 59e6;
-        if (1.1 * wide > 31.0 + bytes / 12e6 + 6.0 * pairs * static_cast<double>(hidden) * ffn / rate) return false;
+        if ((few && !q8 && 3 * gu_wgs >= 2 * cus_whole ? 1.15 : 1.1) * wide > 31.0 + bytes / 12e6 + 6.0 * pairs * static_cast<double>(hidden) * ffn / rate) return false;
     }
     return true;
 }

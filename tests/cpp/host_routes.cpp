@@ -416,6 +416,21 @@ void experts_line_has_no_edges()
     EXPECT(compared > 200 && below > 100, "%zu layers, %zu below eight pairs", compared, below);
 }
 
+// f32 layers of few pairs an expert as they were timed in both forms: the GEMM is not taken where it is slower by 8 % and more.
+void experts_take_the_faster_form()
+{
+    struct Timed { uint32_t gate_up, down; size_t tokens, top_k, hidden, ffn, experts; double jobs, gemm; };
+    const Timed layers[] = {
+        { T_Q4_K, T_Q6_K, 36, 2, 3840, 2048, 16, 91.4, 104.5 }, { T_Q4_K, T_Q6_K, 210, 2, 3840, 768, 64, 154.1, 171.5 }, { T_Q5_K, T_Q6_K, 40, 2, 3072, 1792, 16, 86.3, 94.8 },
+        { T_Q4_K, T_Q6_K, 42, 2, 3072, 1536, 16, 76.7, 83.9 },  { T_Q5_K, T_Q6_K, 114, 2, 2560, 1536, 32, 130.4, 141.3 },
+    };
+    Context ctx;
+    for (const Timed &l : layers) {
+        EXPECT(moe(ctx, l.gate_up, l.down, l.tokens, l.top_k, l.hidden, l.ffn, l.experts) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+        EXPECT(!moe_gemm(), "formats %u/%u, %zu experts of %zu x %zu, %zu tokens: GEMM %.1f us, jobs %.1f", l.gate_up, l.down, l.experts, l.hidden, l.ffn, l.tokens, l.gemm, l.jobs);
+    }
+}
+
 // What is reserved for experts is what the calls of so many pairs need, in any formats and over any number of experts, and no more; a
 // captured call of as many or fewer pairs finds it.
 void experts_scratch_is_reserved()
@@ -561,6 +576,7 @@ const std::map<std::string, std::function<void()>> kChecks = {
     { "elements_take_the_f32_kernels", elements_take_the_f32_kernels },
     { "elements_take_the_f32_experts", elements_take_the_f32_experts },
     { "experts_line_has_no_edges", experts_line_has_no_edges },
+    { "experts_take_the_faster_form", experts_take_the_faster_form },
     { "experts_scratch_is_reserved", experts_scratch_is_reserved },
     { "runs_of_weight_tiles", runs_of_weight_tiles },
     { "outputs_over_the_activations", outputs_over_the_activations },
