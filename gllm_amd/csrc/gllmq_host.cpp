@@ -1381,24 +1381,26 @@ bool mmfw_takes_own(const gllmq_ctx *ctx, const MmfwPlan &L, int fmt, size_t m, 
            m * ldx * x_bytes <= 0xFFFFFFFFull;
 }
 
-// Makes the GEMM's scratch hold `need` bytes where decoded weights are to go, the call's own matrices' (`need` depends on them), if they can be had: not
-// under capture, and where the allocation is refused the scratch stays what it is.  The call then goes without, with the same bits.
-void grow_for_decoded(gllmq_ctx *ctx, Scratch &S, size_t need, void *stream)
+// Makes one of the stream's buffers hold `need` bytes if they can be had: not under capture, and where the allocation is refused it stays what it is.
+void grow_if_possible(gllmq_ctx *ctx, const Scratch &S, void **have, size_t *have_bytes, size_t need, void *stream)
 {
-    if (S.mmf_bytes >= need || S.fixed || ctx->probe || stream_is_capturing(stream)) return;
+    if (*have_bytes >= need || S.fixed || ctx->probe || stream_is_capturing(stream)) return;
     void *buf = nullptr;
     if (hipSetDevice(ctx->device) != hipSuccess || hipMalloc(&buf, need) != hipSuccess) {
         (void)hipGetLastError();
         return;
     }
-    if (S.mmf && hipStreamSynchronize(static_cast<hipStream_t>(stream)) != hipSuccess) { // (earlier work's error, which the next launch reports)
+    if (*have && hipStreamSynchronize(static_cast<hipStream_t>(stream)) != hipSuccess) { // (earlier work's error, which the next launch reports)
         (void)hipFree(buf);
         return;
     }
-    drop_scratch(ctx, S, S.mmf);
-    S.mmf = buf;
-    S.mmf_bytes = need;
+    drop_scratch(ctx, S, *have);
+    *have = buf;
+    *have_bytes = need;
 }
+
+// ... the GEMM's, where decoded weights are to go, the call's own matrices' (`need` depends on them).  Without, the call has the same bits.
+void grow_for_decoded(gllmq_ctx *ctx, Scratch &S, size_t need, void *stream) { grow_if_possible(ctx, S, &S.mmf, &S.mmf_bytes, need, stream); }
 
 // ... enough for any call of up to `m` rows and `n` weight rows in up to MMFW_MAX_SEGS matrices
 size_t mmfx_reserve(const gllmq_ctx *ctx, uint32_t dtype, size_t m, size_t n, size_t k)
@@ -3413,6 +3415,9 @@ MoeWidePlan plan_moe_wide(size_t pairs, size_t hidden, size_t ffn, size_t expert
 
 constexpr size_t kMoeMaxExperts = 4096; // of a call
 
+// Few pairs an expert: the GEMM takes the call only where there is scratch for it (run_moe_wide).
+bool moe_few_pairs(uint32_t dtype_gu, uint32_t dtype_dn, size_t experts, size_t pairs) { return pairs < (dtype_gu == T_Q8_0 || dtype_dn == T_Q8_0 ? 4u : 8u) * experts; }
+
 // Whether the GEMM is ahead of jobs of eight tokens (of Q8_0, whose other form is the GEMV, of those).
 // Without the element type: the two forms round differently, and a call of 16-bit elements gives the bits of the f32 call.  A call that has it
 // ahead has it so with more pairs too (moe_wide_reserve).
@@ -3435,7 +3440,7 @@ bool moe_wide_ahead(const gllmq_ctx *ctx, uint32_t dtype_gu, uint32_t dtype_dn, 
         // 8192 and 14336) 74 of 865, 50 %, and 48 of 1017, 37 %, one slower by 1 %.  A call of 16-bit elements has more of the GEMM (one plane of gate and up; the jobs'
         // rows are converted) and follows the f32 call: by an estimate of its own bf16 calls were 4.6 % shorter in the mean, and not the f32 call's results rounded.
         const size_t cus_whole = static_cast<size_t>(ctx->num_cus), gu_wgs = (2 * ffn + 255) / 256 * std::min(experts, pairs);
-        const bool few = pairs < (q8 ? 4u : 8u) * experts;
+        const bool few = moe_few_pairs(dtype_gu, dtype_dn, experts, pairs);
         if (few && (pairs < 32 || (!q8 && gu_wgs >= 2 * cus_whole))) return false;
         const double e = static_cast<double>(std::min(experts, pairs)), cus = ctx->num_cus;
         auto launch_us = [&](uint32_t dtype, size_t rows, size_t k, double planes) {
@@ -3458,13 +3463,14 @@ bool takes_moe_wide(const gllmq_ctx *ctx, uint32_t dtype_gu, uint32_t dtype_dn, 
     return aligned(x, 16) && pairs * ffn <= 0xFFFFFFFFull && tiles * groups * gq::MmfwImage<2>::bytes <= 0xFFFFFFFFull;
 }
 
-// Scratch for any call of that many pairs or fewer: the GEMM takes the more the more experts, so that of the most, in any formats, which take it.
-size_t moe_wide_reserve(const gllmq_ctx *ctx, size_t pairs, size_t hidden, size_t ffn)
+// Scratch for any call of that many pairs or fewer: the GEMM takes the more the more experts, so that of the most, in any formats, which take it
+// (`few`: with few pairs too).
+size_t moe_wide_reserve(const gllmq_ctx *ctx, size_t pairs, size_t hidden, size_t ffn, bool few)
 {
     for (size_t experts = std::min<size_t>(kMoeMaxExperts, pairs / ((ctx->moe_wide_min + 1) / 2)); experts > 0; --experts)
         for (const Format &gu : kFormats)
             for (const Format &dn : kFormats)
-                if (moe_wide_ahead(ctx, gu.dtype, dn.dtype, hidden, ffn, experts, pairs)) return plan_moe_wide(pairs, hidden, ffn, experts, false).total;
+                if (moe_wide_ahead(ctx, gu.dtype, dn.dtype, hidden, ffn, experts, pairs) && (few || !moe_few_pairs(gu.dtype, dn.dtype, experts, pairs))) return plan_moe_wide(pairs, hidden, ffn, experts, false).total;
     return 0;
 }
 
@@ -3482,6 +3488,9 @@ bool moe_wide_few(const gllmq_ctx *ctx, int fmt, int planes, size_t wgs, size_t 
     return wgs > cus && pairs <= 40 * experts && !(fmt == 1 && planes == 2);
 }
 
+// With few pairs an expert, of which the jobs take less scratch: kNoRoomForGemm, nothing enqueued, where that cannot be had (captured behind a
+// smaller reservation, or refused).
+constexpr int kNoRoomForGemm = -3;
 int run_moe_wide(gllmq_ctx *ctx, const Format &fg, const void *gate, size_t gate_stride, const void *up, size_t up_stride, const Format &fd,
                  const void *down, size_t down_stride, const float *x, float *out, uint32_t elem, size_t tokens, size_t hidden, size_t ffn,
                  size_t experts, size_t top_k, const uint32_t *route_expert, const float *route_weight, const uint32_t *route_len,
@@ -3493,6 +3502,11 @@ int run_moe_wide(gllmq_ctx *ctx, const Format &fg, const void *gate, size_t gate
     Scratch *Sp = nullptr;
     int rc = acquire_scratch(ctx, stream, &Sp);
     if (rc != GLLMQ_OK) return rc;
+    if (moe_few_pairs(fg.dtype, fd.dtype, experts, pairs)) {
+        const size_t f32_total = plan_moe_wide(pairs, hidden, ffn, experts, false).total; // (a 16-bit call in the f32 call's form)
+        grow_if_possible(ctx, *Sp, &Sp->moe, &Sp->moe_bytes, f32_total, stream);
+        if (Sp->moe_bytes < f32_total) return kNoRoomForGemm;
+    }
     rc = grow_scratch(ctx, *Sp, &Sp->moe, &Sp->moe_bytes, W.total, stream, "moe_matvec");
     if (rc != GLLMQ_OK) return rc;
     uint8_t *ws = static_cast<uint8_t *>(Sp->moe);
@@ -3631,13 +3645,15 @@ int moe_on_stream(gllmq_ctx *ctx, const void *gate, size_t gate_bytes, size_t ga
     if (!aligned(x, 16) || !aligned(out, 4))
         return fail(ctx, GLLMQ_ERR_BAD_ALIGNMENT, "moe_matvec: x must be 16-byte and out 4-byte aligned");
 
+    int rc = kNoRoomForGemm;
     if (takes_moe_wide(ctx, dtype_gu, dtype_dn, x, hidden, ffn, experts, pairs))
-        return run_moe_wide(ctx, *fg, gate, gate_expert_stride, up, up_expert_stride, *fd, down, down_expert_stride, x, out, elem, tokens,
-                            hidden, ffn, experts, top_k, route_expert, route_weight, route_len, relu_gate, stream);
+        rc = run_moe_wide(ctx, *fg, gate, gate_expert_stride, up, up_expert_stride, *fd, down, down_expert_stride, x, out, elem, tokens,
+                          hidden, ffn, experts, top_k, route_expert, route_weight, route_len, relu_gate, stream);
+    if (rc != kNoRoomForGemm) return rc;
     if (elem) return kNeedPlainActivations;
     const MoeWorkspace W = moe_workspace(pairs, hidden, ffn);
     Scratch *Sp = nullptr;
-    int rc = acquire_scratch(ctx, stream, &Sp);
+    rc = acquire_scratch(ctx, stream, &Sp);
     if (rc != GLLMQ_OK) return rc;
     rc = grow_scratch(ctx, *Sp, &Sp->moe, &Sp->moe_bytes, W.total, stream, "moe_matvec");
     if (rc != GLLMQ_OK) return rc;
@@ -3939,7 +3955,9 @@ int gllmq_reserve_moe(gllmq_ctx *ctx, size_t tokens, size_t top_k, size_t hidden
     Scratch *S = nullptr;
     int rc = acquire_scratch(ctx, stream, &S);
     if (rc != GLLMQ_OK || tokens == 0 || top_k == 0) return rc;
-    const size_t pairs = tokens * top_k, need = std::max(moe_workspace(pairs, hidden, ffn).total, moe_wide_reserve(ctx, pairs, hidden, ffn));
+    const size_t pairs = tokens * top_k;
+    grow_if_possible(ctx, *S, &S->moe, &S->moe_bytes, moe_wide_reserve(ctx, pairs, hidden, ffn, true), stream); // (refused: those calls go without)
+    const size_t need = std::max(moe_workspace(pairs, hidden, ffn).total, moe_wide_reserve(ctx, pairs, hidden, ffn, false));
     return grow_scratch(ctx, *S, &S->moe, &S->moe_bytes, need, stream, "reserve_moe");
 }
 

@@ -126,7 +126,8 @@ const char *gllmq_last_kernel_name(const gllmq_ctx *ctx);
  * Q4_K and Q5_K against matrices of more than 2^28 weights: reserve those by their own shape).  From 1024
  * rows of Q6_K on the weights are decoded first where there is scratch for that, 17 KiB per 32 x 256 of them and
  * at most 128 MiB: what is reserved, or grown by an eager call, is for as large matrices (a batch's together).
- * Without it (captured, or an allocation that is refused) they are multiplied as they are: the same bits, later.  No
+ * Without it (captured, or an allocation that is refused) they are multiplied as they are: the same bits, later.  Experts' calls
+ * of fewer than eight pairs an expert (Q8_0: four) that would take the GEMM run their other form without the scratch for it.  No
  * counterpart in the reference, whose scratch is
  * sized when the graph is compiled (src/compat/gpu_backend_macro.rs:82-87). */
 int gllmq_reserve_matmul(gllmq_ctx *ctx, uint32_t ggml_dtype, size_t m, size_t n, size_t k, void *stream);
@@ -376,7 +377,7 @@ int gllmq_moe_route(gllmq_ctx *ctx, const float *logits_dev, size_t tokens, size
  * Q6_K rows of at most 4096 elements run on the int8 matrix cores, all tokens of an expert
  * (eight per pass) against one read of its weights, Q4_K / Q5_K gate and up with the activation
  * in the same launch; other shapes run the integer-dot GEMV, two tokens per pass.  A prompt's many
- * tokens per expert (about eight and more, four of Q8_0, where the experts are large or many enough)
+ * tokens per expert (from two, of Q8_0 one, to about eight on, by an estimate of both forms)
  * run the f16 matrix-core GEMM of gllmq_quantized_matmul over each expert's rows.
  * Expert e's gate rows ([ffn x hidden] blocks of dtype_gate_up) start at gate_dev +
  * e * gate_expert_stride, its up rows at up_dev + e * up_expert_stride, its down rows

@@ -468,6 +468,49 @@ void experts_scratch_is_reserved()
         }
 }
 
+// Few pairs an expert, whose jobs need less scratch than the GEMM: where that is not to be had the call goes on the jobs, of any element type, and
+// what is reserved is what there is room for.  With eight pairs (Q8_0: four) the GEMM or an error, as the reservation is for.
+void experts_without_room_take_the_jobs()
+{
+    struct Layer { uint32_t gate_up, down; size_t few, many, top_k, hidden, ffn, experts; };
+    for (const Layer &l : { Layer{ T_Q4_K, T_Q4_K, 27, 200, 2, 4096, 2048, 8 }, Layer{ T_Q8_0, T_Q8_0, 24, 200, 2, 4096, 2048, 16 }, Layer{ T_Q5_K, T_Q6_K, 56, 200, 2, 2560, 1024, 16 } })
+        for (int elem : { GLLMQ_ELEM_F32, GLLMQ_ELEM_BF16 }) {
+            Context ctx;
+            EXPECT(moe(ctx, l.gate_up, l.down, l.few, l.top_k, l.hidden, l.ffn, l.experts, elem) == GLLMQ_OK && moe_gemm(), "%u: %s", l.gate_up, gllmq_last_error(ctx));
+            size_t gemm = 0;
+            for (const auto &b : fake::live) gemm = std::max(gemm, b.second); // (the largest: of the call)
+            EXPECT(moe(ctx, l.gate_up, l.down, l.few, l.top_k, l.hidden, l.ffn, l.experts) == GLLMQ_OK && moe_gemm(), "%s", gllmq_last_error(ctx));
+            for (const auto &b : fake::live) EXPECT(b.second <= gemm, "the f32 call grows what element type %d took", elem);
+            Context small;
+            gllmq_set_option(small, "moe_wide", 0);
+            EXPECT(moe(small, l.gate_up, l.down, l.few, l.top_k, l.hidden, l.ffn, l.experts, elem) == GLLMQ_OK && !moe_gemm(), "%s", gllmq_last_error(small));
+            gllmq_set_option(small, "moe_wide", 1);
+            const std::map<void *, size_t> before = fake::live;
+            fake::capturing = true;
+            EXPECT(moe(small, l.gate_up, l.down, l.few, l.top_k, l.hidden, l.ffn, l.experts, elem) == GLLMQ_OK && !moe_gemm(), "captured: %s", gllmq_last_error(small));
+            fake::capturing = false;
+            EXPECT(fake::live == before, "captured: allocations");
+            fake::refuse_from = gemm;
+            Context refused;
+            EXPECT(moe(refused, l.gate_up, l.down, l.few, l.top_k, l.hidden, l.ffn, l.experts, elem) == GLLMQ_OK && !moe_gemm(), "refused: %s", gllmq_last_error(refused));
+            EXPECT(moe(refused, l.gate_up, l.down, l.many, l.top_k, l.hidden, l.ffn, l.experts, elem) != GLLMQ_OK, "%u: many pairs", l.gate_up);
+            fake::refuse_from = SIZE_MAX;
+            Context all, less;
+            size_t most = 0, held = 0;
+            const std::map<void *, size_t> there = fake::live;
+            EXPECT(gllmq_reserve_moe(all, l.few, l.top_k, l.hidden, l.ffn, nullptr) == GLLMQ_OK, "%s", gllmq_last_error(all));
+            for (const auto &b : fake::live)
+                if (!there.count(b.first)) most = std::max(most, b.second);
+            fake::refuse_from = most;
+            const std::map<void *, size_t> then = fake::live;
+            EXPECT(gllmq_reserve_moe(less, l.few, l.top_k, l.hidden, l.ffn, nullptr) == GLLMQ_OK, "refused: %s", gllmq_last_error(less));
+            fake::refuse_from = SIZE_MAX;
+            for (const auto &b : fake::live)
+                if (!then.count(b.first)) held = std::max(held, b.second);
+            EXPECT(held > 0 && held < most, "%zu of %zu bytes", held, most);
+        }
+}
+
 // Scratch that a captured call has used stays, whatever eager calls of more rows, and calls on many other streams, do afterwards;
 // what no graph can hold is given back as it is outgrown, and everything with the context.
 void scratch_of_graphs_stays()
@@ -578,6 +621,7 @@ const std::map<std::string, std::function<void()>> kChecks = {
     { "experts_line_has_no_edges", experts_line_has_no_edges },
     { "experts_take_the_faster_form", experts_take_the_faster_form },
     { "experts_scratch_is_reserved", experts_scratch_is_reserved },
+    { "experts_without_room_take_the_jobs", experts_without_room_take_the_jobs },
     { "runs_of_weight_tiles", runs_of_weight_tiles },
     { "outputs_over_the_activations", outputs_over_the_activations },
     { "own_images", own_images },
