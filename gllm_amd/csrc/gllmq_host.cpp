@@ -252,7 +252,7 @@ struct gllmq_ctx {
     // streamed form (loader waves + arithmetic waves) [0 = Q4_K, 1 = Q5_K, 2 = Q6_K, 3 = Q8_0][variant]: register
     // operands p1_e1, p1_e2, p2_e4, then LDS operands p1_e2, p2_e4, p4_e4
     hipFunction_t mm8s[4][7] = {};
-    hipFunction_t mm8s_token[4][4] = {};        // one row, ending in the greedy token choice [format as above][p1_e1_a, p1_e2_a, p1_e2, p1_e4]
+    hipFunction_t mm8s_token[4][3] = {};        // one row, ending in the greedy token choice [format as above][p1_e1_a, p1_e2, p1_e4]
     bool use_mm8s = true;                       // "mm8s" = 0: the fetch-and-compute kernels throughout
     bool batch_overlap = true;                  // "batch_overlap" = 0: the kernels of a batch run strictly one after the other
     bool mm8s_all = false;                      // "mm8s_all" = 1: the streamed form wherever it fits, also where another was timed faster
@@ -938,10 +938,11 @@ int run_mm8s(gllmq_ctx *ctx, const Format &f, const uint8_t *w, const float *x, 
         P.arrive = S->mm8_arrive;
     }
     if (TokenChoice *c = ctx->call_token; c && c->y == y && c->n == n && mm == 1 && !split && !fold && !glu && !ctx->call_glu && !ctx->call_elem &&
-                                          grid <= gq::ARGMAX_MAX_PARTS * gq::ARGMAX_MAX_ROWS) {
+                                          grid <= gq::ARGMAX_MAX_PARTS * gq::ARGMAX_MAX_ROWS && (variant == 0 || variant == 3 || variant == 6)) {
+        // (register operands are of at most 16 blocks, which one row prepares in one step: never p1_e2_a)
         gq::Mm8sTokenParams T{ P, c->keys, c->ticket, c->token, c->value };
         c->made = true;
-        return launch(ctx, ctx->mm8s_token[sfmt][variant <= 1 ? variant : variant == 3 ? 2 : 3], grid, (gq::MM8S_CWAVES + gq::MM8S_LOADERS) * 64, lds, stream, &T, sizeof T, true);
+        return launch(ctx, ctx->mm8s_token[sfmt][variant / 3], grid, (gq::MM8S_CWAVES + gq::MM8S_LOADERS) * 64, lds, stream, &T, sizeof T, true);
     }
     return launch(ctx, fn, grid * ksplit, (gq::MM8S_CWAVES + gq::MM8S_LOADERS) * 64, lds, stream, &P, sizeof P, split);
 }
@@ -2320,9 +2321,9 @@ int gllmq_init(gllmq_ctx **out, int device)
                 snprintf(name, sizeof name, "gq_mm8s_%s_%s", kMm8sFormat[q], kMm8s[v]);
                 rc = get_function(ctx, &ctx->mm8s[q][v], name);
             }
-        static const char *const kMm8sToken[4] = { "p1_e1_a", "p1_e2_a", "p1_e2", "p1_e4" };
+        static const char *const kMm8sToken[3] = { "p1_e1_a", "p1_e2", "p1_e4" };
         for (int q = 0; q < 4; ++q)
-            for (int v = 0; v < 4 && rc == GLLMQ_OK; ++v) {
+            for (int v = 0; v < 3 && rc == GLLMQ_OK; ++v) {
                 snprintf(name, sizeof name, "gq_mm8s_%s_%s_token", kMm8sFormat[q], kMm8sToken[v]);
                 rc = get_function(ctx, &ctx->mm8s_token[q][v], name);
             }

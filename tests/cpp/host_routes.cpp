@@ -431,6 +431,25 @@ void experts_take_the_faster_form()
     }
 }
 
+// Every kernel that ends in the greedy token is some output matrix's.
+void token_kernels_are_reached()
+{
+    Context ctx;
+    std::set<std::string> reached, unreached;
+    for (const auto &f : kFormats)
+        for (size_t n : { 6145u, 12000u, 32000u, 128256u })
+            for (size_t k = 256; k <= 16384; k += 256) {
+                fake::launches.clear();
+                EXPECT(gllmq_lm_head_argmax(ctx, at(1), n * gllmq_row_bytes(f.dtype, k), static_cast<const float *>(at(4)), f.dtype, n, k, static_cast<float *>(at(5)),
+                                            static_cast<uint32_t *>(at(6)), static_cast<float *>(at(7)), nullptr) == GLLMQ_OK, "%s", gllmq_last_error(ctx));
+                for (const fake::Launch &l : fake::launches) reached.insert(l.kernel);
+            }
+    for (const std::string &name : fake::names)
+        if (name.find("_token") != std::string::npos && !reached.count(name)) unreached.insert(name);
+    for (const std::string &name : unreached) EXPECT(false, "%s", name.c_str());
+    EXPECT(reached.count("gq_mm8s_q8_0_p1_e4_token"), "no streamed token");
+}
+
 // What is reserved for experts is what the calls of so many pairs need, in any formats and over any number of experts, and no more; a
 // captured call of as many or fewer pairs finds it.
 void experts_scratch_is_reserved()
@@ -618,6 +637,7 @@ const std::map<std::string, std::function<void()>> kChecks = {
     { "scratch_of_graphs_stays", scratch_of_graphs_stays },
     { "elements_take_the_f32_kernels", elements_take_the_f32_kernels },
     { "elements_take_the_f32_experts", elements_take_the_f32_experts },
+    { "token_kernels_are_reached", token_kernels_are_reached },
     { "experts_line_has_no_edges", experts_line_has_no_edges },
     { "experts_take_the_faster_form", experts_take_the_faster_form },
     { "experts_scratch_is_reserved", experts_scratch_is_reserved },

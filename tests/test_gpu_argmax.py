@@ -185,6 +185,64 @@ def test_token_from_the_streamed_kernel(hip, torch, oracle, dt, n, k):
         hip.lm_head_argmax(wd, xd, dt, n, k, tok[:1], logits=y2, value=val[:1])
 
 
+@pytest.mark.parametrize("dt, name", [(8, "q8_0"), (12, "q4k"), (13, "q5k"), (14, "q6k")])
+@pytest.mark.parametrize("n, k, form", [(6145, 2048, "p1_e1_a"), (12000, 4608, "p1_e2"), (9001, 8448, "p1_e4"), (12000, 10240, "p1_e4"), (10003, 10240 - 32, "p1_e4"), (6200, 16384, "p1_e4")])
+def test_every_token_kernel(hip, torch, dt, name, n, k, form):
+    """Each kernel that ends in the greedy token by its name: logits and token of the two calls bit for bit, in an eager call, in a graph replayed
+    between eager calls of other activations, and on two streams at once (the count of workgroups is each stream's own, back at zero after a launch)."""
+    from gllm_amd.synth import random_activations, random_weight
+    if dt == 8: k = k // 256 * 256  # (other rows of Q8_0 are the GEMV's)
+    w = torch.from_numpy(np.asarray(random_weight(dt, n, k, seed=n)).view(np.uint8).reshape(-1)).cuda()
+    x = [torch.from_numpy(random_activations(1, k, seed=s)).cuda() for s in (1, 2, 3)]
+    want = []
+    for xs in x:
+        y, tok = torch.empty(1, n, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+        hip.quantized_matmul(w, xs, y, dt, 1, n, k)
+        hip.argmax(y, tok)
+        want.append((y[0], tok))
+    print(f"token kernel {dt} {n} x {k}", flush=True)
+
+    def buffers():
+        return torch.full((n,), NAN, device="cuda"), torch.full((1,), -1, dtype=torch.int32, device="cuda")
+
+    def check(got, i):
+        assert torch.equal(got[0].view(torch.int32), want[i][0].view(torch.int32)) and torch.equal(got[1], want[i][1])
+
+    got = buffers()
+    hip.lm_head_argmax(w, x[0], dt, n, k, got[1], logits=got[0])
+    assert hip.last_kernel_name() == f"gq_mm8s_{name}_{form}_token"
+    torch.cuda.synchronize()
+    check(got, 0)
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    held, held_x = buffers(), x[0].clone()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        hip.lm_head_argmax(w, held_x, dt, n, k, held[1], logits=held[0])
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=side):
+        hip.lm_head_argmax(w, held_x, dt, n, k, held[1], logits=held[0])
+    for i in (1, 2, 0):
+        held_x.copy_(x[i])
+        held[0].fill_(NAN)
+        graph.replay()
+        torch.cuda.synchronize()
+        check(held, i)
+        got = buffers()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            hip.lm_head_argmax(w, x[(i + 1) % 3], dt, n, k, got[1], logits=got[0])
+        torch.cuda.synchronize()
+        check(got, (i + 1) % 3)
+    streams, outs = (side, torch.cuda.Stream()), [buffers() for _ in range(8)]
+    torch.cuda.synchronize()
+    for i, o in enumerate(outs):
+        with torch.cuda.stream(streams[i % 2]):
+            hip.lm_head_argmax(w, x[i % 3], dt, n, k, o[1], logits=o[0])
+    torch.cuda.synchronize()
+    for i, o in enumerate(outs):
+        check(o, i % 3)
+
+
 def test_lm_head_token_with_ties_and_nan(hip, torch, oracle):
     """Rows of equal weights give equal logits (the LAST of them is the token), and a NaN activation
     leaves no candidate at all."""
