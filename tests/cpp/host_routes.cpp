@@ -450,6 +450,37 @@ void token_kernels_are_reached()
     EXPECT(reached.count("gq_mm8s_q8_0_p1_e4_token"), "no streamed token");
 }
 
+// The workgroups of four waves are the option's, and by themselves some calls' and not others'; workgroups cover all weight rows in either form.
+void experts_workgroups_by_option()
+{
+    size_t with[3] = {}, without[3] = {};
+    for (int option = 0; option < 3; ++option) {
+        Context ctx;
+        gllmq_set_option(ctx, "moe_wide_min", 1);
+        gllmq_set_option(ctx, "moe_wide_few", option);
+        for (const auto &mix : kMixes)
+            for (const auto &layer : std::vector<std::vector<size_t>>{ { 512, 384 }, { 768, 520 }, { 288, 352 }, { 4096, 1536 }, { 4096, 2048 } })
+                for (size_t experts : { 8u, 12u, 64u, 128u })
+                    for (size_t per : { 8u, 32u, 64u, 110u })
+                        for (int elem : { GLLMQ_ELEM_F32, GLLMQ_ELEM_BF16 }) {
+                            EXPECT(moe(ctx, mix[0], mix[1], per * experts / 2, 2, layer[0], layer[1], experts, elem) == GLLMQ_OK && moe_gemm(), "%s", gllmq_last_error(ctx));
+                            for (const fake::Launch &l : fake::launches) {
+                                if (l.kernel.find("gq_moe_mmf_") != 0) continue;
+                                const bool few = l.kernel.find("_few") != std::string::npos;
+                                (few ? with : without)[option]++;
+                                uint32_t tiles = 0;
+                                for (uint32_t i = 0; i < l.wide().segs; ++i) {
+                                    EXPECT(l.wide().seg[i].tile0 == tiles, "%s", l.kernel.c_str());
+                                    tiles += (l.wide().seg[i].n + (few ? 127 : 255)) / (few ? 128 : 256);
+                                }
+                                EXPECT(l.wide().n_tiles == tiles && l.grid == (l.wide().max_jobs + 7) / 8 * 8 * tiles, "%s: %u workgroups, %u tiles", l.kernel.c_str(), l.grid, l.wide().n_tiles);
+                            }
+                        }
+    }
+    EXPECT(with[0] == 0 && without[2] == 0 && with[1] > 100 && without[1] > 100, "%zu, %zu and %zu of four waves, %zu, %zu and %zu of eight", with[0], with[1], with[2], without[0],
+           without[1], without[2]);
+}
+
 // What is reserved for experts is what the calls of so many pairs need, in any formats and over any number of experts, and no more; a
 // captured call of as many or fewer pairs finds it.
 void experts_scratch_is_reserved()
@@ -637,6 +668,7 @@ const std::map<std::string, std::function<void()>> kChecks = {
     { "scratch_of_graphs_stays", scratch_of_graphs_stays },
     { "elements_take_the_f32_kernels", elements_take_the_f32_kernels },
     { "elements_take_the_f32_experts", elements_take_the_f32_experts },
+    { "experts_workgroups_by_option", experts_workgroups_by_option },
     { "token_kernels_are_reached", token_kernels_are_reached },
     { "experts_line_has_no_edges", experts_line_has_no_edges },
     { "experts_take_the_faster_form", experts_take_the_faster_form },

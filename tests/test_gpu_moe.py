@@ -419,6 +419,30 @@ def test_workgroups_of_four_waves_give_the_bits_of_eight(torch, t_gu, t_dn, hidd
     assert float((outs[0] - outs[1])[large].norm()) <= bar * float(outs[0][large].norm())
 
 
+@pytest.mark.parametrize("t_gu, t_dn, hidden, ffn", [(Q4_K, Q6_K, 1280, 520), (Q5_K, Q4_K, 512, 1152), (Q6_K, Q5_K, 768, 384), (8, 8, 1312, 352)])
+def test_workgroups_of_four_waves_against_the_oracle(torch, oracle, t_gu, t_dn, hidden, ffn):
+    """Jobs of one to four tiles, passes of two and one of them, rows of more than three blocks (units) and fewer (parts).  Which form the option gives is
+    checked on the CPU (tests/cpp/host_routes.cpp, experts_workgroups_by_option)."""
+    from gllm_amd.backend import HipBackend
+    hip = HipBackend(0, options={"moe_wide_min": 1, "moe_wide_few": 2})
+    counts = (0, 1, 33, 64, 65, 97, 128, 130)
+    experts = len(counts)
+    gu, dn = expert_weights(t_gu, t_dn, experts, hidden, ffn, seed=81)
+    re = np.random.default_rng(8).permutation(np.repeat(np.arange(experts), counts)).astype(np.uint32)[:, None]
+    x = random_activations(len(re), hidden, seed=83) * 1e-2
+    print(f"four waves {t_gu}/{t_dn} {hidden} x {ffn}", flush=True)
+    got = run_gpu(hip, torch, gu, t_gu, dn, t_dn, x, hidden, ffn, experts, re, np.ones(re.shape, np.float32), np.ones(len(re), np.uint32))
+    for e in range(experts):
+        rows = np.flatnonzero(re[:, 0] == e)
+        if len(rows) == 0:
+            continue
+        g, d = row_bytes(t_gu, hidden), row_bytes(t_dn, ffn)
+        both = oracle.quantized_matmul(gu[e * 2 * ffn * g:(e + 1) * 2 * ffn * g], x[rows], t_gu, len(rows), 2 * ffn, hidden, acc=oracle.ACC_F64, threads=8).astype(np.float64)
+        mid = (both[:, :ffn] / (1 + np.exp(np.minimum(-both[:, :ffn], 700))) * both[:, ffn:]).astype(np.float32)
+        want = oracle.quantized_matmul(dn[e * hidden * d:(e + 1) * hidden * d], mid, t_dn, len(rows), hidden, ffn, acc=oracle.ACC_F64, threads=8)
+        check_close(got[rows], want, f"expert {e} of {counts}")
+
+
 @pytest.mark.parametrize("hidden, top_k", [(256, 3), (260, 9), (1028, 8), (512, 2)])
 def test_combine_of_many_tokens_is_the_combine_of_few(torch, hidden, top_k):
     """From 128 tokens on a thread adds up four columns.  The same tokens with others behind them that are
@@ -492,3 +516,54 @@ def test_layers_about_the_line_fit_what_is_reserved(torch, t_gu, t_dn, hidden, f
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, outs[0])
+
+
+@pytest.mark.parametrize("elem", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("t_gu, t_dn, hidden, ffn, experts, top_k, tokens, gemm", [
+    (Q4_K, Q4_K, 1280, 768, 32, 4, 56, True),     # seven pairs an expert
+    (Q4_K, Q4_K, 2560, 1024, 16, 2, 56, True),
+    (Q5_K, Q6_K, 2560, 1024, 16, 4, 28, True),
+    (8, 8, 2048, 1024, 64, 4, 48, True),          # Q8_0: three
+    (Q4_K, Q6_K, 1024, 512, 16, 2, 24, False),    # three: jobs of eight tokens
+    (Q5_K, Q6_K, 1536, 512, 128, 8, 111, False),  # seven, a device four times full
+])
+def test_few_pairs_are_captured_in_the_form_that_they_take(torch, t_gu, t_dn, hidden, ffn, experts, top_k, tokens, gemm, elem):
+    """Below eight pairs an expert (Q8_0: four), behind the reservation alone (the jobs of 16-bit elements: an eager call, for what they are converted
+    in): every replay gives the eager call's bits, which are those of the form that the layer takes and not the other's."""
+    from gllm_amd.backend import HipBackend
+    t = getattr(torch, elem)
+    gu, dn = expert_weights(t_gu, t_dn, experts, hidden, ffn, seed=experts)
+    rng = np.random.default_rng(tokens)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    re = dev(np.stack([rng.permutation(experts)[:top_k] for _ in range(tokens)]).astype(np.int32))
+    x = (torch.from_numpy(random_activations(tokens, hidden, seed=5)) * 2.0 ** -9).to(t).cuda()
+    args = (dev(gu), t_gu, dev(dn), t_dn, x)
+    route = (hidden, ffn, experts, re, torch.full(re.shape, 0.5, device="cuda"), torch.full((tokens,), top_k, dtype=torch.int32, device="cuda"))
+    outs = []
+    for options in ({}, {"moe_wide_min": 1}, {"moe_wide": 0}):
+        print(f"few pairs {t_gu}/{t_dn} {experts} x {hidden} x {ffn} top {top_k} of {tokens} {elem} {options}", flush=True)
+        out = torch.full((tokens, hidden), float("nan"), dtype=t, device="cuda")
+        hip = HipBackend(0, options=options)
+        hip.moe_matvec(*args, out, *route)
+        torch.cuda.synchronize()
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1 if gemm else 2])
+    if elem == "float32":  # (rounded to 16 bits the two forms may be the same)
+        assert not torch.equal(outs[0], outs[2 if gemm else 1])
+    hip, out, stream, graph = HipBackend(0), torch.empty(tokens, hidden, dtype=t, device="cuda"), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        hip.reserve_moe(tokens, top_k, hidden, ffn)
+        if not gemm and elem != "float32":
+            hip.moe_matvec(*args, out, *route)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        hip.moe_matvec(*args, out, *route)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, outs[0])
+        with torch.cuda.stream(stream):  # (eager work on the graph's scratch in between)
+            hip.moe_matvec(*args, torch.empty_like(out), *route)
+        torch.cuda.synchronize()

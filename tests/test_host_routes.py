@@ -9,7 +9,7 @@ CPP = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
 CHECKS = ["ffn_scratch_stays", "ffn_slices_are_left_where_there_is_room", "outputs_over_the_activations",
           "runs_of_weight_tiles", "own_images", "scratch_of_graphs_stays"]
 CHECKS += ["elements_take_the_f32_kernels", "decoded_weights_scratch"]
-CHECKS += ["elements_take_the_f32_experts", "experts_scratch_is_reserved", "experts_line_has_no_edges", "experts_take_the_faster_form", "experts_without_room_take_the_jobs", "token_kernels_are_reached"]
+CHECKS += ["elements_take_the_f32_experts", "experts_scratch_is_reserved", "experts_line_has_no_edges", "experts_take_the_faster_form", "experts_without_room_take_the_jobs", "token_kernels_are_reached", "experts_workgroups_by_option"]
 
 
 @pytest.fixture(scope="module")
