@@ -3439,7 +3439,7 @@ bool moe_wide_ahead(const gllmq_ctx *ctx, uint32_t dtype_gu, uint32_t dtype_dn, 
         // By this 400 of 2303 other layers of that range with eight pairs (four) and more go to the GEMM that the estimate before left to the other form, f32
         // 30 % shorter in the mean, and 411 of 5082 with fewer, 24 %, seven of them slower by 2 to 6 %; of larger layers (to 384 experts,
         // 8192 and 14336) 74 of 865, 50 %, and 48 of 1017, 37 %, one slower by 1 %.  A call of 16-bit elements has more of the GEMM (one plane of gate and up; the jobs'
-        // rows are converted) and follows the f32 call: by an estimate of its own bf16 calls were 4.6 % shorter in the mean, and not the f32 call's results rounded.
+        // rows are converted) and follows the f32 call: by an estimate of its own bf16 calls were 5 % shorter in the mean, and not the f32 call's results rounded.
         const size_t cus_whole = static_cast<size_t>(ctx->num_cus), gu_wgs = (2 * ffn + 255) / 256 * std::min(experts, pairs);
         const bool few = moe_few_pairs(dtype_gu, dtype_dn, experts, pairs);
         if (few && (pairs < 32 || (!q8 && gu_wgs >= 2 * cus_whole))) return false;
@@ -3481,6 +3481,8 @@ size_t moe_wide_reserve(const gllmq_ctx *ctx, size_t pairs, size_t hidden, size_
 // 473; Q5_K of two planes -0.2 %, single ones +6; above 40 pairs, jobs of three tiles and more, -0.6 and +7).  At most half a workgroup a CU, where
 // it fills the device: -2.9 % up to 40 pairs, with two planes -5.4 % up to 100 (8 experts of 4096 x 2048, 100 pairs each 160, 135), with one +1.9.
 // Between them the eight waves have a CU to themselves either way: +0.3 %.  By this rule 115 of the 170 calls change, 4 % shorter in the mean.
+// Uneven routing, by which single experts have jobs of four tiles in two passes: 3995 calls whose experts' logits are spread by 0.7 and 1.4, 2.7 to 5.4 % shorter in
+// the mean by format, 13 longer by 5 to 7 %, nine of them Q8_0.
 bool moe_wide_few(const gllmq_ctx *ctx, int fmt, int planes, size_t wgs, size_t pairs, size_t experts)
 {
     if (ctx->moe_wide_few != 1) return ctx->moe_wide_few == 2;

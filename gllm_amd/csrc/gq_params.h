@@ -539,7 +539,7 @@ struct MmfwShape {
 //   Q4_K 64 rows 28672 x 4096, two planes       43.2, 40.8, 44.1     Q4_K 64 rows, one plane               32.8, 33.2, 33.4
 //   Q6_K 16 rows 4096 x 14336, two planes       26.2, 24.5           Q6_K 64 rows 14336 x 4096, one plane  31.4, 28.5
 //   Q6_K 2048 rows 4096 x 14336, two planes     610, 585             Q6_K 48 rows 14336 x 4096, two planes 35.3, 32.6
-//   Q8_0 64 rows 28672 x 4096, one plane        48.4, 50.6           (its rows' quants are off any alignment in LDS)
+//   Q8_0 64 rows 28672 x 4096, one plane        48.4, 50.6           (both while its quants were read off any alignment; not timed since)
 // Q5_K against two planes keeps the parts: calls of 160 drawn shapes of 9 to 130 rows are level (in the mean up to 16 rows parts 0.5 %
 // shorter, above within 0.2 %; single ones 5 % either way).
 // Experts, all of whose CUs stream weights at once, take units against two tiles of one plane as well (512 tokens, top 8 of 128 experts of
